@@ -171,7 +171,7 @@ def served_burst(ctx, q, db, eval_, batch, nslots=2, bursts=4, wait_us=0):
     """All of q's queries submitted at once to a serving loop over the resident
     database (budget for the whole database per request, so that a tick can
     batch them), `bursts` times on one server (its slots keep their buffers,
-    tuned grid sizes and graphs, as a long-running server's do); the last
+    and graphs, as a long-running server's do); the last
     burst is measured: GCUPS over first submit -> last done, latency
     percentiles, the largest tick."""
     import cother_amd
@@ -210,7 +210,7 @@ def batch_phase(args, threads, tdist):
     ctx.upload_db(db)
     cells = float(q.lens().sum()) * db.npos
     ctx.search(0, 2, eval=args.eval)                    # warmup
-    ctx.search(eval=args.eval, batch=True)              # autotune + graph capture
+    ctx.search(eval=args.eval, batch=True)              # graph capture
     reps = 3
     t0 = time.perf_counter()
     for _ in range(reps):

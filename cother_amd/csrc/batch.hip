@@ -27,11 +27,6 @@
 // lists' order varies, the hit order is restored by the (log E-value,
 // profile) sort.
 //
-// The persistent grids' sizes (wavefronts per compute unit of the phase-1
-// DP and of the later stages) are chosen by a small autotuner: the first
-// batch of a shape runs once per candidate with events around it, and the
-// fastest candidate is kept for that shape (database size and pair count).
-//
 // Covered: the FP32 contraction and databases whose profiles fit the LDS
 // boundary rows (CTH_DP_LDS_ROW_MAX positions); other searches, and queries
 // whose buffers alone exceed the budget, run through cth_search.
@@ -57,7 +52,8 @@ extern "C" int cth_score_rows_per_tile(int ddms);
 extern "C" int cth_launch_dp_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq,
                                    const cth_bpair* pairs, const int* list, const int* count, int n, int* next,
                                    int ltmax, int64_t ldsc, const float* scores, uint8_t* btck, cth_dpres* res,
-                                   int grid, hipStream_t st);
+                                   float* grow, int grid, int W, hipStream_t st);
+extern "C" size_t cth_dp_batch_row_bytes(int grid, int ltmax);
 extern "C" int cth_launch_stats_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq,
                                       const cth_bpair* pairs, const int* list, const int* count, int64_t ldsc,
                                       const float* scores, const cth_dpres* dpres, int ssemodel, double* out,
@@ -180,7 +176,7 @@ struct batch_layout {
   float* scores; float* mods; float* post; uint8_t* btck;
   // small
   cth_bquery* bq; cth_bytile* ytab; cth_bpair* pairs; cth_dpres* res; double* stats; cth_mapres* mres;
-  int* cand; int* passed; int* hitl; int* ctr; double* zrow; cth_hit* hits; char* alnout;
+  int* cand; int* passed; int* hitl; int* ctr; double* zrow; cth_hit* hits; char* alnout; float* grow;
 };
 
 // One batch's description on the host.
@@ -194,9 +190,28 @@ struct batch_plan {
   int ddms = 1;                     // 0: no cell of the batch has a DDMS term
 };
 
+// Grids of the persistent launches (workgroups) and wavefronts per pair of
+// the two DP passes.
 struct launch_shape {
-  int dp_grid, small_grid;
+  int dp_grid, dp_waves, small_grid, trace_waves;
 };
+
+// One wavefront per pair where the pairs fill the chip (128,000 pairs of 99 x
+// 231 positions: 6.8 ms, against 7.4 and 9.6 ms with two and three, whose
+// wavefronts past a pair's last stripe wait), else one per stripe.  16
+// workgroups per compute unit, more than are resident: those that start late
+// take the pairs that are left (8 per unit: 7.2 ms, 10: 6.9, 12: 6.9, 16:
+// 6.8).  Boundary rows in global memory are reserved per workgroup, so half
+// as many then.  The traceback pass has few pairs: one wavefront per stripe.
+launch_shape choose_shape(int ncu, int npairs, int lqmax, int ltmax) {
+  launch_shape S;
+  const int stripes = std::min(8, std::max(1, (lqmax + 63) / 64));
+  S.dp_waves = npairs >= ncu * 8 ? 1 : stripes;
+  S.trace_waves = stripes;
+  S.dp_grid = ncu * (ltmax > CTH_DP_GLOBAL_FROM ? 8 : 16);
+  S.small_grid = ncu * 4;
+  return S;
+}
 
 int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, const cth_search_opts* opt,
                       int64_t ldsc, int ltmax, int rowcap, const launch_shape& S, bool capture, bool timing) {
@@ -215,14 +230,16 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
       return -1;
     if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[1], st));
     if (cth_launch_dp_batch(&c->q.d, &db.d, L.bq, L.pairs, nullptr, nullptr, npairs, L.ctr + kCtrNext1, ltmax, ldsc,
-                            L.scores, nullptr, L.res, std::min(S.dp_grid, npairs), st))
+                            L.scores, nullptr, L.res, L.grow, std::min(S.dp_grid, npairs),
+                            S.dp_waves, st))
       return -1;
     const int sel_grid = std::max(1, std::min(1024, (npairs + 255) / 256));
     hipLaunchKernelGGL(k_select_cand, dim3(sel_grid), dim3(256), 0, st, L.bq, L.pairs, npairs, L.res, L.cand,
                        L.ctr + kCtrCand);
     CTH_HIP_CHECK(hipGetLastError());
     if (cth_launch_dp_batch(&c->q.d, &db.d, L.bq, L.pairs, L.cand, L.ctr + kCtrCand, 0, L.ctr + kCtrNext2, ltmax,
-                            ldsc, L.scores, L.btck, L.res, std::min(S.small_grid, npairs), st))
+                            ldsc, L.scores, L.btck, L.res, L.grow, std::min(S.small_grid, npairs),
+                            S.trace_waves, st))
       return -1;
     hipLaunchKernelGGL(k_select_passed, dim3(sel_grid), dim3(256), 0, st, L.res, L.cand, L.ctr + kCtrCand, L.passed,
                        L.ctr + kCtrPassed);
@@ -423,22 +440,25 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
     const size_t cells = (size_t)P.cells;
     const size_t cbytes = up256(4 * cells) * (opt->do_map ? 3 : 2) + up256(cells);
     const int small_max = std::max(1, std::min(npairs, ncu * 32));
+    const launch_shape S = choose_shape(ncu, npairs, P.lqmax, ltmax);
+    const size_t growbytes = cth_dp_batch_row_bytes(std::min(npairs, std::max(S.dp_grid, S.small_grid)), ltmax);
     const size_t sbytes = up256(sizeof(cth_bquery) * P.bq.size()) + up256(sizeof(cth_bytile) * P.ytab.size()) +
                           up256(sizeof(cth_bpair) * npairs) + up256(sizeof(cth_dpres) * npairs) +
                           up256(sizeof(double) * CTH_STATS_NOUT * npairs) + up256(sizeof(cth_mapres) * npairs) +
                           3 * up256(sizeof(int) * npairs) + up256(sizeof(int) * kNCtr) +
                           up256(sizeof(double) * (size_t)small_max * P.lqmax) + up256(sizeof(cth_hit) * npairs) +
-                          up256(alnbytes);
+                          up256(alnbytes) + up256(growbytes);
     if (cth_ctx_reserve(c, &c->bcells, &c->cap_bcells, cbytes)) return -1;
     if (cth_ctx_reserve(c, &c->bsmall, &c->cap_bsmall, sbytes)) return -1;
     batch_layout L{};
     {
       uint8_t* o = (uint8_t*)c->bcells;
       auto take = [&](size_t n) { uint8_t* p = o; o += up256(n); return p; };
+      // (traceback bytes first: the DP sweeps read up to 8 floats to either side of the scores)
+      L.btck = take(cells);
       L.scores = (float*)take(4 * cells);
       L.mods = (float*)take(4 * cells);
       L.post = opt->do_map ? (float*)take(4 * cells) : nullptr;
-      L.btck = take(cells);
       uint8_t* s = (uint8_t*)c->bsmall;
       auto takes = [&](size_t n) { uint8_t* p = s; s += up256(n); return p; };
       L.bq = (cth_bquery*)takes(sizeof(cth_bquery) * P.bq.size());
@@ -454,6 +474,7 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
       L.zrow = (double*)takes(sizeof(double) * (size_t)small_max * P.lqmax);
       L.hits = (cth_hit*)takes(sizeof(cth_hit) * npairs);
       L.alnout = alnbytes ? (char*)takes(alnbytes) : nullptr;
+      L.grow = growbytes ? (float*)takes(growbytes) : nullptr;
     }
     // the batch's tables (outside the graph: a replayed graph reads the current ones)
     CTH_HIP_CHECK(hipMemcpyAsync(L.bq, P.bq.data(), sizeof(cth_bquery) * P.bq.size(), hipMemcpyHostToDevice, c->st));
@@ -461,67 +482,6 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
                                  c->st));
     CTH_HIP_CHECK(hipMemcpyAsync(L.pairs, P.pairs.data(), sizeof(cth_bpair) * npairs, hipMemcpyHostToDevice, c->st));
     const double t0 = now_ms();
-    // persistent grid sizes: tuned once per class of shapes (database size
-    // and pair count rounded up to a power of two), so that batches of
-    // similar size (a serving loop's ticks) share the tuning instead of each
-    // paying for its candidates; shared contexts use their parent's table
-    uint64_t pbucket = 1;
-    while (pbucket < (uint64_t)npairs) pbucket <<= 1;
-    const uint64_t tkey = ((uint64_t)npos << 24) ^ pbucket;
-    cth_ctx* tc = c->borrowed ? c->parent : c;
-    launch_shape S{ncu * 20, ncu * 8};
-    bool tuned = false;
-    {
-      std::lock_guard<std::mutex> g(tc->tune_mu);
-      for (int k = 0; k < tc->nbtune && k < 32; k++)
-        if (tc->btune[k].key == tkey) {
-          S = launch_shape{tc->btune[k].dp_grid, tc->btune[k].small_grid};
-          tuned = true;
-        }
-    }
-    if (!tuned) {
-      // wavefronts per compute unit for the phase-1 DP: measured on 128,000
-      // pairs of <= 150 x <= 400 positions (LDS for 14 per unit), 4: 47.5 ms,
-      // 6: 32.5, 8: 25.9, 10: 23.8, 12: 28.2, 14: 29.4.  The batch runs once
-      // with the first candidate (its results stand); then the DP's first
-      // pass alone runs again per candidate on the scores in place (it
-      // rewrites the same maxima), so that tuning a class costs one batch and
-      // a few DP passes, not a batch per candidate (with distance lists the
-      // score stage is most of a batch)
-      const int dp_cand[] = {ncu * 8, ncu * 10, ncu * 20};
-      hipEvent_t e0, e1;
-      CTH_HIP_CHECK(hipEventCreate(&e0));
-      CTH_HIP_CHECK(hipEventCreate(&e1));
-      S = launch_shape{dp_cand[0], ncu * 4};
-      if (capture_or_launch(c, P, L, opt, ldsc, ltmax, rowcap, S, false, false)) return -1;
-      // (each candidate twice, the faster run counting: single runs of
-      // candidates a few percent apart are not told apart reliably)
-      float best = 1e30f;
-      for (int rep = 0; rep < 2; rep++)
-        for (const int g : dp_cand) {
-          CTH_HIP_CHECK(hipMemsetAsync(L.ctr + kCtrNext1, 0, sizeof(int), c->st));
-          CTH_HIP_CHECK(hipEventRecord(e0, c->st));
-          if (cth_launch_dp_batch(&c->q.d, &db.d, L.bq, L.pairs, nullptr, nullptr, npairs, L.ctr + kCtrNext1,
-                                  ltmax, ldsc, L.scores, nullptr, L.res, std::min(g, npairs), c->st))
-            return -1;
-          CTH_HIP_CHECK(hipEventRecord(e1, c->st));
-          CTH_HIP_CHECK(hipEventSynchronize(e1));
-          float ms = 0.0f;
-          CTH_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-          if (ms < best) { best = ms; S.dp_grid = g; }
-        }
-      (void)hipEventDestroy(e0);
-      (void)hipEventDestroy(e1);
-      // the table keeps the last 32 classes (another slot may have added
-      // this one meanwhile: then its entry stays)
-      std::lock_guard<std::mutex> g(tc->tune_mu);
-      bool have = false;
-      for (int k = 0; k < tc->nbtune && k < 32; k++) have |= tc->btune[k].key == tkey;
-      if (!have) {
-        tc->btune[tc->nbtune % 32] = cth_btune{tkey, S.dp_grid, S.small_grid, best};
-        tc->nbtune++;
-      }
-    }
     // the graph: replayed when everything its launches captured is the same
     // (buffers and their layout, sizes, options, the uploaded sets)
     uint32_t mp;
@@ -531,7 +491,8 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
                         (uint64_t)P.cells, (uint64_t)P.lqmax | ((uint64_t)rowcap << 32),
                         (uint64_t)S.dp_grid | ((uint64_t)S.small_grid << 32),
                         (uint64_t)opt->do_map | ((uint64_t)opt->ssemodel << 8) | ((uint64_t)(alnbytes != 0) << 17) |
-                            ((uint64_t)P.ddms << 18) | ((uint64_t)mp << 32),
+                            ((uint64_t)P.ddms << 18) | ((uint64_t)S.dp_waves << 20) |
+                            ((uint64_t)S.trace_waves << 24) | ((uint64_t)mp << 32),
                         fnv(&db.d, sizeof db.d), fnv(&c->q.d, sizeof c->q.d),
                         (uint64_t)(uintptr_t)c->q.ddoff, (uint64_t)(uintptr_t)c->dtab};
     if (timing) {

@@ -59,7 +59,6 @@ extern "C" int cth_ctx_create(int device, const char* envdir, cth_ctx** out) {
   cth_ctx* c = (cth_ctx*)calloc(1, sizeof(cth_ctx));
   if (!c) { cth_set_error("out of host memory"); return -1; }
   new (&c->nshared) std::atomic<int>(0);
-  new (&c->tune_mu) std::mutex();
   c->device = device;
   int rc = cth_tables_load(envdir, &c->htab);
   if (rc) { cth_set_error("cannot load score tables from %s (code %d)", envdir, rc); free(c); return -1; }
@@ -88,7 +87,6 @@ extern "C" int cth_ctx_create_shared(cth_ctx* parent, cth_ctx** out) {
   cth_ctx* c = (cth_ctx*)calloc(1, sizeof(cth_ctx));
   if (!c) { cth_set_error("out of host memory"); return -1; }
   new (&c->nshared) std::atomic<int>(0);
-  new (&c->tune_mu) std::mutex();
   c->device = parent->device;
   c->borrowed = 1;
   c->parent = parent;
@@ -139,7 +137,6 @@ extern "C" void cth_ctx_destroy(cth_ctx* c) {
   if (c->bcells) (void)hipFree(c->bcells);
   if (c->bsmall) (void)hipFree(c->bsmall);
   if (c->st) (void)hipStreamDestroy(c->st);
-  c->tune_mu.~mutex();
   free(c);
 }
 
@@ -247,7 +244,7 @@ extern "C" int cth_score_block(cth_ctx* c, int qidx, int p0, int p1, float* h_sc
   return cth_score_block_ex(c, qidx, p0, p1, 0, h_scores, h_mods);
 }
 
-extern "C" int cth_launch_dp(const cth_dpset* q, int qp, const cth_dpset* db, int p0, int np, int ltmax,
+extern "C" int cth_launch_dp(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int np, int ltmax,
                              int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck, float scorethld,
                              cth_dpres* res, float* grow, hipStream_t st);
 extern "C" size_t cth_dp_row_bytes(int np, int ltmax);
@@ -270,17 +267,17 @@ extern "C" int cth_phase1_block(cth_ctx* c, int qidx, int p0, int p1, float scor
   const size_t need = sizeof(float) * (size_t)lq * ldsc;
   int ltmax = 0;
   for (int p = p0; p < p1; p++) ltmax = c->db.h_len[p] > ltmax ? c->db.h_len[p] : ltmax;
-  if (cth_ctx_reserve(c, (void**)&c->scores, &c->cap_scores, need)) return -1;
+  if (cth_ctx_reserve(c, (void**)&c->scores, &c->cap_scores, need + 2 * CTH_SCORE_PAD * sizeof(float))) return -1;
   if (cth_ctx_reserve(c, (void**)&c->mods, &c->cap_mods, need)) return -1;
   if (cth_ctx_reserve(c, (void**)&c->btck, &c->cap_btck, (size_t)lq * ldsc)) return -1;
   if (cth_ctx_reserve(c, (void**)&c->dpout, &c->cap_dpout, sizeof(cth_dpres) * (size_t)(p1 - p0))) return -1;
-  if (cth_launch_score(&c->q.d, c->q.ddoff, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores, c->mods, 0,
+  if (cth_launch_score(&c->q.d, c->q.ddoff, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores + CTH_SCORE_PAD, c->mods, 0,
                        ddms_of(c, qidx, p0, p1), c->st))
     return -1;
   // boundary rows in global memory for profiles over the LDS row limit
   const size_t rows = cth_dp_row_bytes(p1 - p0, ltmax);
   if (rows && cth_ctx_reserve(c, (void**)&c->grow, &c->cap_grow, rows)) return -1;
-  if (cth_launch_dp(&c->q.d, qidx, &c->db.d, p0, p1 - p0, ltmax, col0, ldsc, c->scores, c->btck, scorethld,
+  if (cth_launch_dp(&c->q.d, qidx, lq, &c->db.d, p0, p1 - p0, ltmax, col0, ldsc, c->scores + CTH_SCORE_PAD, c->btck, scorethld,
                     (cth_dpres*)c->dpout, rows ? c->grow : nullptr, c->st))
     return -1;
   CTH_HIP_CHECK(hipStreamSynchronize(c->st));
@@ -327,7 +324,7 @@ extern "C" int cth_phase2_block(cth_ctx* c, int qidx, int p0, int p1, float scor
   double* d_out = (double*)(((uintptr_t)(d_hist + 641 * (size_t)np2) + 15) & ~(uintptr_t)15);
   CTH_HIP_CHECK(hipMemcpyAsync(d_abs, abs_.data(), sizeof(int) * np2, hipMemcpyHostToDevice, c->st));
   CTH_HIP_CHECK(hipMemcpyAsync(d_rel, rel.data(), sizeof(int) * np2, hipMemcpyHostToDevice, c->st));
-  if (cth_launch_stats(&c->q.d, qidx, &c->db.d, p0, col0, ldsc, c->scores, d_abs, d_rel, (const cth_dpres*)c->dpout,
+  if (cth_launch_stats(&c->q.d, qidx, &c->db.d, p0, col0, ldsc, c->scores + CTH_SCORE_PAD, d_abs, d_rel, (const cth_dpres*)c->dpout,
                        np2, searchspace, ssemodel, d_hist, d_out, c->st))
     return -1;
   CTH_HIP_CHECK(hipStreamSynchronize(c->st));
@@ -367,7 +364,7 @@ extern "C" int cth_map_block(cth_ctx* c, int qidx, int p0, int p1, const int32_t
   if (ncols > (1ll << 30)) { cth_set_error("map_block: too many columns"); return -1; }
   const int64_t ldsc = (ncols + 63) / 64 * 64;
   const size_t need = sizeof(float) * (size_t)lq * ldsc;
-  if (cth_ctx_reserve(c, (void**)&c->scores, &c->cap_scores, need)) return -1;
+  if (cth_ctx_reserve(c, (void**)&c->scores, &c->cap_scores, need + 2 * CTH_SCORE_PAD * sizeof(float))) return -1;
   if (cth_ctx_reserve(c, (void**)&c->mods, &c->cap_mods, need)) return -1;
   if (cth_ctx_reserve(c, (void**)&c->mapbuf, &c->cap_mapbuf, need)) return -1;
   if (cth_ctx_reserve(c, (void**)&c->btck, &c->cap_btck, (size_t)lq * ldsc)) return -1;
@@ -378,12 +375,12 @@ extern "C" int cth_map_block(cth_ctx* c, int qidx, int p0, int p1, const int32_t
   cth_mapjob* d_jobs = (cth_mapjob*)(d_zrow + (size_t)njobs * lq);
   cth_mapres* d_res = (cth_mapres*)(((uintptr_t)(d_jobs + njobs) + 15) & ~(uintptr_t)15);
   CTH_HIP_CHECK(hipMemcpyAsync(d_jobs, jobs.data(), sizeof(cth_mapjob) * njobs, hipMemcpyHostToDevice, c->st));
-  if (cth_launch_score(&c->q.d, c->q.ddoff, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores, c->mods, 0,
+  if (cth_launch_score(&c->q.d, c->q.ddoff, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores + CTH_SCORE_PAD, c->mods, 0,
                        ddms_of(c, qidx, p0, p1), c->st))
     return -1;
   const size_t rows = cth_map_row_bytes(njobs, ltmax);
   if (rows && cth_ctx_reserve(c, (void**)&c->grow, &c->cap_grow, rows)) return -1;
-  if (cth_launch_map(&c->q.d, qidx, lq, &c->db.d, d_jobs, njobs, ltmax, col0, ldsc, c->scores, c->mods,
+  if (cth_launch_map(&c->q.d, qidx, lq, &c->db.d, d_jobs, njobs, ltmax, col0, ldsc, c->scores + CTH_SCORE_PAD, c->mods,
                      (float*)c->mapbuf, c->btck, d_zrow, minpp, nullptr, lq + ltmax, d_res, rows ? c->grow : nullptr,
                      c->st))
     return -1;

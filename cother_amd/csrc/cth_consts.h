@@ -15,17 +15,16 @@
 #define CTH_DDSTRIDE  128   // bytes per position of the distance list in HBM (n + 99 values + 0xff pad)
 #define CTH_PROSCALE 10000  // libpro/srcpro/PMProfileModel.h:58 ReadWriteScale
 #define CTH_MAXCOLUMNS 50000  // liblib/mylimits.h:50 MAXCOLUMNS: longest profile the readers accept
-// longest profile whose DP/MAP stripe boundary rows (5 floats per column)
+// longest profile whose MAP stripe boundary rows (5 floats per column)
 // fit one workgroup's 160 KiB of LDS; longer ones keep them in global memory
 #define CTH_LDS_ROW_MAX 8192
-// the phase-1 DP keeps the reference's buffer of maxima (value and cell per
-// column) next to its five boundary rows: 28 bytes per column in LDS
+// longest profile of a database that the batched search covers
 #define CTH_DP_LDS_ROW_MAX 5824
-// the per-query phase-1 DP keeps those rows in global memory from this
-// length on: a workgroup of one wavefront with 28 bytes of LDS per column
-// leaves most of a CU's SIMDs idle for long profiles
+// the phase-1 DP keeps its boundary rows and the reference's buffer of maxima
+// (28 bytes per column) in global memory from this profile length on: the
+// LDS holds them beside the transition rings of eight wavefronts up to here
 #ifndef CTH_DP_GLOBAL_FROM
-#define CTH_DP_GLOBAL_FROM 1536
+#define CTH_DP_GLOBAL_FROM 4096
 #endif
 
 // transition order (cudp/CuBatchDP_com.h:87-96)

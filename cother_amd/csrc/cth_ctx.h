@@ -4,18 +4,14 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
-#include <mutex>
 
 #include "cth_dev.h"
 #include "cth_devdb.h"
 #include "cth_tables.h"
 
-// an autotuned launch shape of the batched search, per batch shape
-struct cth_btune {
-  uint64_t key;
-  int dp_grid, small_grid;
-  float ms;  // the chosen phase-1 DP pass's time when tuned
-};
+// floats in front of and behind a context's score buffer: the DP sweeps read
+// up to 8 floats to either side of the matrix
+#define CTH_SCORE_PAD 64
 
 struct cth_ctx {
   int device;
@@ -37,16 +33,11 @@ struct cth_ctx {
   // batched search uses a fifth)
   hipEvent_t ev[5]; int has_ev; int nbev;
   // batched search (batch.hip): cell buffers and tables of a batch, the
-  // captured graph of the last batch shape and the tuned grid sizes
+  // captured graph of the last batch shape
   void* bcells; size_t cap_bcells;
   void* bsmall; size_t cap_bsmall;
   hipGraphExec_t bgraph; int has_bgraph; uint64_t bkey[12];
   int64_t nbgraph_captures, nbgraph_replays;
-  // tuned grid sizes; a shared context reads and adds to its parent's
-  // table (under the parent's tune_mu), so the slots of a serving loop tune
-  // each class of shapes once between them
-  cth_btune btune[32]; int nbtune;
-  std::mutex tune_mu;
   // a context made by cth_ctx_create_shared reads its parent's tables,
   // queries and database and frees only its own stream and scratch
   int borrowed;

@@ -17,6 +17,7 @@
 
 struct cth_dpset {
   int32_t nprof;
+  int32_t finite;          // CTH_SET_* (what the upload found in the values)
   int64_t npos;
   int64_t ld;              // padded leading dimension of position fields
   int64_t ldtr;            // padded leading dimension of transition fields (npos + nprof)
@@ -37,6 +38,18 @@ struct cth_dpset {
 };
 
 #define CTH_DD_MISSING 21
+
+// What an upload finds in a set's values.  CTH_SET_FINITE: frequencies in
+// [0, 1.5], backgrounds in [0, 4], SS probabilities in [0, 1], transitions
+// within +-1e6; CTH_SET_BKG: every background at least 2^-14.  Scores of two
+// finite sets, one with backgrounds, are finite or -inf (log-odds quotients
+// of at most 1.5^2 2^15, which FP16 holds too, and no 0/0), so no step of the
+// DPs over them gives a NaN.
+#define CTH_SET_FINITE 1
+#define CTH_SET_BKG 2
+static inline bool cth_finite_scores(const cth_dpset* q, const cth_dpset* db) {
+  return (q->finite & db->finite & CTH_SET_FINITE) && ((q->finite | db->finite) & CTH_SET_BKG);
+}
 
 #define CTH_HIP_CHECK(expr)                                                        \
   do {                                                                             \

@@ -45,8 +45,12 @@ __device__ __forceinline__ int flow_write_column(int x0, int tx, int lt) {
 // may read and write any memory can neither be crossed by a store nor, being
 // convergent, be duplicated into the branches.  The fence keeps the
 // memory-model ordering; a wavefront's LDS accesses execute in issue order.
+// kGlobal: the buffer is in global memory (a fence of LDS accesses alone
+// does not wait for the score loads in flight).
+template <bool kGlobal = true>
 __device__ __forceinline__ void flow_phase() {
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+  if constexpr (kGlobal) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+  else __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup", "local");
   asm volatile("" ::: "memory");
 }
 

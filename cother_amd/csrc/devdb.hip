@@ -39,6 +39,37 @@ int up_fields(void** dst, const float* src, int nf, int64_t n, int64_t ld) {
   return 0;
 }
 
+// bad[0]: some value outside CTH_SET_FINITE's ranges; bad[1]: some background below CTH_SET_BKG's
+__global__ __launch_bounds__(256) void k_check_values(cth_dpset d, int* bad) {
+  const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = gridDim.x * (int64_t)blockDim.x;
+  bool out = false, small = false;
+  auto within = [](float v, float a, float b) { return a <= v && v <= b; };
+  for (int64_t i = i0; i < d.npos; i += step) {
+    for (int a = 0; a < CTH_NAA; a++) out |= !within(d.trg[a * d.ld + i], 0.0f, 1.5f);
+    for (int a = 0; a < CTH_NSS; a++) out |= !within(d.ss[a * d.ld + i], 0.0f, 1.0f);
+  }
+  for (int64_t i = i0; i < d.npos + d.nprof; i += step)
+    for (int a = 0; a < CTH_NTRN; a++) out |= !within(d.trn[a * d.ldtr + i], -1e6f, 1e6f);
+  for (int64_t i = i0; i < (int64_t)d.nprof * CTH_NAA; i += step) {
+    out |= !within(d.bkg[i], 0.0f, 4.0f);
+    small |= !(d.bkg[i] >= 0x1p-14f);
+  }
+  if (out) bad[0] = 1;
+  if (small) bad[1] = 1;
+}
+
+// d.finite of an uploaded set; flags: two zeroed ints on the device
+int check_values(cth_dpset& d, int* flags) {
+  int h[2] = {0, 0};
+  const int64_t blocks = (d.npos + d.nprof + 255) / 256;
+  hipLaunchKernelGGL(k_check_values, dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(blocks, 2048))), dim3(256),
+                     0, 0, d, flags);
+  CTH_HIP_CHECK(hipGetLastError());
+  CTH_HIP_CHECK(hipMemcpy(h, flags, sizeof h, hipMemcpyDeviceToHost));
+  d.finite = (h[0] ? 0 : CTH_SET_FINITE) | (h[1] ? 0 : CTH_SET_BKG);
+  return 0;
+}
+
 }  // namespace
 
 int cth_devset_has_ddms(const cth_devset* s, int p0, int p1) {
@@ -136,6 +167,8 @@ extern "C" int cth_devset_upload(const cth_pset* h, cth_devset* s) {
     memcpy(s->h_len, h->len, sizeof(int32_t) * h->nprof);
     memcpy(s->h_dist, h->dist, sizeof(int64_t) * h->nprof);
   }
+  // (the zeroed 256 bytes behind the lengths hold the flags)
+  if (!rc) rc = check_values(d, (int*)d.len + np);
   if (rc) { cth_devset_free(s); return -1; }
   return 0;
 }

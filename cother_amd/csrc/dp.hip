@@ -1,29 +1,21 @@
 // dp.hip: phase-1 profile-profile DP with traceback, and its finalisation.
 //
-// k_dp computes, for one template profile per wavefront, the five-state
+// k_dp computes, for one template profile per workgroup, the five-state
 // local DP of ExecDP_Btck_Unroll32x (cudp/CuBatchDP_init_btck.cu:65-494)
-// over the whole Lq x Lt matrix.  MI355X layout: the 64 lanes of a
-// wavefront own 64 consecutive query rows (a stripe) and sweep the
-// anti-diagonals of the stripe; each step a lane takes its upper
-// neighbour's state (and the template column's transitions) from lane-1 by a
-// DPP wave_shr:1 move, so the wavefront advances one anti-diagonal per step
-// with no LDS round trip.  The bottom row of a stripe is kept in LDS for the
-// next stripe (in a global-memory row of the wavefront's own for profiles
-// longer than CTH_DP_GLOBAL_FROM positions in the per-query search, whose
-// five rows and buffer of maxima would leave a CU one or two single-wavefront
-// workgroups in LDS, and over CTH_DP_LDS_ROW_MAX, the LDS capacity, in the
-// batched search; the row of column x is read at step x + 31 and
-// overwritten at step x + 95 of the same wavefront, so one row serves both
-// stripes as in LDS).  Cell values
-// equal the reference's: rows start at column -1-(q mod 32) with zero
-// boundaries, rows q = 0 mod 32 see zeros above at
-// negative columns, rows q = 31 mod 32 see zeros left and upper-left at
-// column 0, out-of-range transitions are log(0) = -32768 and cells
-// outside the valid area score -9 -- the boundaries the reference's 32x32
-// oblique blocks produce.  The maximum and its cell are the ones the
-// reference's per-column buffer of maxima yields (dp_pair below), so equal
-// maxima resolve as there, and for templates under 32 positions the rows
-// whose block-end column lies before the matrix drop out as there.
+// over the whole Lq x Lt matrix, as the stripe sweep of cth_sweep.h: the 64
+// lanes of a wavefront own 64 consecutive query rows and sweep the
+// anti-diagonals of the stripe; each step a lane takes its upper neighbour's
+// state from lane-1 by a DPP wave_shr:1 move, and the stripes of a pair run
+// on wavefronts of one workgroup.  Cell values and the maximum with its cell
+// equal the reference's (dp_pair below).
+//
+// Bound by VALU issue (dp_pair: ~40 instructions per step in ~26 issue
+// slots).  Measured against one wavefront per pair with the boundary tests
+// and the transitions' lane-to-lane moves in every step (~190 VALU): first
+// pass of 128,000 pairs of 99 x 231 positions 16.6 -> 5.7 ms; a query of 2000
+// positions against 130 templates of 1000-3000, whose rows were in global
+// memory, 177 -> 5.9 ms for both passes; 250 positions against 4000 templates
+// (median 220) 4.6 -> 0.92 ms.
 //
 // k_dpfin restates FinalizeDPPro (cudp/CuBatchDP_final.cu:61-292): pass
 // test against the score threshold, traceback from the maximum, correlation
@@ -32,37 +24,168 @@
 // and begin coordinates.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cstring>
+
 #include "cth_batch.h"
 #include "cth_flow.h"
 #include "cth_dev.h"
 #include "cth_dp.h"
+#include "cth_sweep.h"
 
 namespace {
 
 constexpr float kLog0 = CTH_LOG0;
+// transitions of the columns past the profile: no path through them reaches
+// a positive match state, however large the maximum so far
+constexpr float kPast = -1e30f;
 
-__device__ __forceinline__ float dpp_shr1(float old_lane0, float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old_lane0),
-                                                               __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, false));
+// LDS of one workgroup of W wavefronts: each wavefront's transition ring and,
+// where the boundary rows are in global memory, its stages of 32 columns of
+// the row above (read) and of its own bottom row (written); else the pair's
+// boundary row of lt + 33 columns (MM, MI, IM, DN as float4, ND) and the
+// buffer of maxima (value and cell per column).
+constexpr int kStage = 32;
+__host__ __device__ constexpr size_t dp_wave_lds(bool grow) { return kRingBytes + (grow ? 2 * kStage * 20 : 0); }
+__host__ __device__ constexpr size_t dp_row_lds(int lt, bool grow) {
+  return grow ? 0 : (size_t)20 * (lt + 33) + (size_t)8 * lt;
 }
 
-__device__ __forceinline__ float mx(float a, float b) { return a < b ? b : a; }
-
-__device__ __forceinline__ int corner_maxlen(int lq, int lt) {
-  int m = (int)rintf(CTH_CORNERPRC * (float)(lq > lt ? lq : lt));
-  return m > CTH_MAXCORNER ? CTH_MAXCORNER : m;
+// the max the recursion takes.  kSel: the reference's select a < b ? b : a,
+// whose result differs from the hardware's max only for NaN operands (and in
+// the sign of a zero, which no result depends on); the hardware's max runs
+// when neither set can give a NaN (cth_dpset.tame)
+template <bool kSel>
+__device__ __forceinline__ float mx(float a, float b) {
+  if constexpr (kSel) return a < b ? b : a;
+  else return __builtin_fmaxf(a, b);
 }
 
-__device__ __forceinline__ bool in_valid_area(int lq, int lt, int edge, int y, int x) {
-  const bool corners = (lq <= y + edge && x <= edge + y - lq) || (lt - edge + y <= x && y < edge);
-  return !corners && 0 <= y && y < lq && 0 <= x && x < lt;
+// the state of a lane: its last column's cells, and what the diagonal
+// predecessors (the row above's cells of the column before) contribute, aMM
+// and aMI with the row's MM transition added already
+struct dp_state {
+  float cMM, cMI, cIM, cDN, cND;
+  float aMM, aMI, pIM, pDN, pND;
+};
+
+// One step (one cell per lane) with the row's transitions qt, the column's T0
+// and T1, the score S and the row above's b0, b1 for lane 0.  Sums are taken
+// in the reference's order; max(a, b) + c stands for max(a + c, b + c), which
+// is the same number (rounding is monotone), except for kSel, where a NaN
+// could tell them apart.
+template <bool kTrace, bool kSel>
+__device__ __forceinline__ int dp_step(dp_state& d, const float* qt, const float4& T0, const float4& T1, float S,
+                                       const float4& b0, float b1) {
+  const float uMM = dpp_shr1(b0.x, d.cMM), uMI = dpp_shr1(b0.y, d.cMI), uIM = dpp_shr1(b0.z, d.cIM);
+  const float uDN = dpp_shr1(b0.w, d.cDN), uND = dpp_shr1(b1, d.cND);
+  float nMM, nIM;
+  if constexpr (kSel) {
+    float v = d.aMI + T0.z;
+    v = mx<kSel>(v, d.pIM + qt[CTH_IM] + T0.x);
+    v = mx<kSel>(v, d.pDN + qt[CTH_DM] + T0.x);
+    v = mx<kSel>(v, d.pND + qt[CTH_MM] + T1.y);
+    v = mx<kSel>(v, d.aMM + T0.x);
+    nMM = mx<kSel>(v + S, 0.0f);
+    nIM = mx<kSel>(d.cMM + qt[CTH_MI] + T0.x, d.cIM + qt[CTH_II] + T0.x);
+  } else {
+    const float m1 = mx<kSel>(mx<kSel>(d.aMM, d.pIM + qt[CTH_IM]), d.pDN + qt[CTH_DM]) + T0.x;
+    const float v = mx<kSel>(mx<kSel>(m1, d.aMI + T0.z), d.pND + qt[CTH_MM] + T1.y);
+    nMM = mx<kSel>(v + S, 0.0f);
+    nIM = mx<kSel>(d.cMM + qt[CTH_MI], d.cIM + qt[CTH_II]) + T0.x;
+  }
+  d.aMM = uMM + qt[CTH_MM];
+  d.aMI = uMI + qt[CTH_MM];
+  const float nMI = mx<kSel>(d.aMM + T0.y, d.aMI + T0.w);
+  const float nDN = mx<kSel>(uMM + qt[CTH_MD], uDN + qt[CTH_DD]);
+  const float nND = mx<kSel>(d.cMM + T1.x, d.cND + T1.z);
+  int bk = 0;
+  if constexpr (kTrace) {
+    float m = nMM;
+    bk = nMM != 0.0f ? CTH_BT_DIAG : CTH_BT_STOP;
+    if (m < nMI) { m = nMI; bk = CTH_BT_UP; }
+    if (m < nIM) { m = nIM; bk = CTH_BT_LEFT; }
+    if (m < nDN) { m = nDN; bk = CTH_BT_UP; }
+    if (m < nND) { m = nND; bk = CTH_BT_LEFT; }
+  }
+  d.cMM = nMM; d.cMI = nMI; d.cIM = nIM; d.cDN = nDN; d.cND = nND;
+  d.pIM = uIM; d.pDN = uDN; d.pND = uND;
+  return bk;
 }
 
-// The DP of query qp against template profile p, whose scores begin at
-// scores[colp] (row stride ldsc); traceback bytes to btck at the same offsets
-// (NULL: none); bot: [7][lt] (LDS or global): the stripe boundary rows [5]
-// and the reference's buffer of maxima, values and cells.  The maximum and
-// its cell follow that buffer (see below) and reach every lane.
+// eight consecutive columns of a lane's score row, two dword-aligned 16-byte
+// loads.  Every lane reads its own row, so a load touches a cache line per
+// lane, and fewer, wider loads take the texture path and L1 far fewer
+// requests.  The loads are not guarded: the buffer is readable 8 floats to
+// either side, and what lies outside the profile is replaced at its use.
+struct score8 {
+  float v[8];
+};
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ score8 score_load8(const float* at) {
+  const float4u a = *reinterpret_cast<const float4u*>(at), b = *reinterpret_cast<const float4u*>(at + 4);
+  return {{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
+}
+
+// Store lane 63's cells of step j to its bottom row in LDS (outA, outB: byte
+// offsets of step 0's column): the lanes are chosen by exec inside one asm
+// block, because a branch around the stores would keep the compiler from
+// issuing the next step's LDS reads ahead of them (LDS accesses execute in
+// issue order, so its own waits stay sufficient).  mask: 1 << 63, or 0 where
+// no column is stored.
+__device__ __forceinline__ void store_bottom(uint32_t outA, uint32_t outB, uint64_t mask, const dp_state& d) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const f4 v = {d.cMM, d.cMI, d.cIM, d.cDN};
+  asm volatile(
+      "s_mov_b64 exec, %4\n\t"
+      "ds_write_b128 %0, %2\n\t"
+      "ds_write_b32 %1, %3\n\t"
+      "s_mov_b64 exec, -1"
+      :
+      : "v"(outA), "v"(outB), "v"(v), "v"(d.cND), "s"(mask));
+}
+
+// Eight steps, j0 .. j0+7 of a phase.  ring: the lane's column of step j0;
+// inA, inB: the row above from that step's column of lane 0; outA, outB: the
+// bottom row's columns, stored by lane 63 (mask); crel: the column of
+// step j0 relative to the row's first valid one, span: the last valid one
+// relative to it.  kFix: scores outside the valid columns are -9 (cells of
+// the ignored corners and outside the matrix, CuBatchDP_init_btck.cu:245).
+// mv, ms: the lane's running maximum and the step that set it (kSel: at
+// columns c + j below clt only, an infinite state passes any transition).
+template <bool kTrace, bool kSel, bool kFix>
+__device__ __forceinline__ void dp_steps8(dp_state& d, const float* qt, int j0, const float4* __restrict__ ring,
+                                          const float4* __restrict__ inA, const float* __restrict__ inB,
+                                          uint32_t outA, uint32_t outB, uint64_t mask, int crel,
+                                          uint32_t span, int c, uint32_t clt, const score8& sc, float& mv, int& ms,
+                                          uint32_t* bk) {
+  if constexpr (kTrace) bk[0] = bk[1] = 0;
+  int ml = -1;
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const float4 T0 = ring[j], T1 = ring[kRingCols + j];
+    const float4 b0 = inA[j];
+    const float b1 = inB[j];
+    float S = sc.v[j];
+    if constexpr (kFix) S = (uint32_t)(crel + j) <= span ? S : CTH_OUTSCORE;
+    const int b = dp_step<kTrace, kSel>(d, qt, T0, T1, S, b0, b1);
+    if constexpr (kTrace) bk[j >> 2] |= (uint32_t)b << (8 * (j & 3));
+    bool up = mv < d.cMM;
+    if constexpr (kSel) up = up && (uint32_t)(c + j) < clt;
+    ml = up ? j : ml;
+    mv = up ? d.cMM : mv;
+    store_bottom(outA + 16 * j, outB + 4 * j, mask, d);
+  }
+  ms = ml >= 0 ? j0 + ml : ms;
+}
+
+// The DP of query qp against template profile p on a workgroup of W
+// wavefronts, whose scores begin at scores[colp] (row stride ldsc);
+// traceback bytes to btck at the same offsets (kTrace).  lds: the
+// workgroup's dynamic LDS (W dp_wave_lds + dp_row_lds bytes); grow: 7 x lt
+// floats of global memory for the boundary row and the buffer of maxima
+// (kGlobalRow).  The maximum and its cell follow the reference's buffer (see
+// below); valid in every lane of wavefront 0.
 //
 // The reference (ExecDP_Btck_Unroll32x, cudp/CuBatchDP_init_btck.cu:246-263,
 // 328, 436-464) computes 32x32 oblique blocks; thread tx of a block starting
@@ -74,245 +197,236 @@ __device__ __forceinline__ bool in_valid_area(int lq, int lt, int edge, int y, i
 // covers the end; block row 0 overwrites, later ones keep the buffer's
 // value unless it is smaller).  FinalizeDPPro (cudp/CuBatchDP_final.cu:
 // 100-142) reduces the last 64 columns.  Here lane l of stripe s is row
-// 64s+l of block row 2s + l/32 with tx = 31 - l%32, and it reaches column c at
-// step c + l + 32: every lane's blocks start at steps = 31 and end at steps
-// = 30 (mod 32).  At a block end the lower half-wavefront writes before the
-// upper one (its block row's blocks run two launches ahead, so where the
-// right-edge writes of both meet a column, the lower one's comes first);
-// every buffer column then sees its block rows' writes and reads in the
-// reference's order.  Lanes past the query's end take part as the
-// reference's threads of those rows do.
+// 64s+l of block row 2s + l/32 with tx = 31 - l%32; its blocks start and end
+// with the phases, x0 = 32(k-1) - (32 for the upper half-wavefront) in phase
+// k.  At a block end the lower half-wavefront writes before the upper one
+// (its block row's blocks run two launches ahead, so where the right-edge
+// writes of both meet a column, the lower one's comes first); every buffer
+// column then sees its block rows' writes and reads in the reference's
+// order.  Lanes past the query's end take part as the reference's threads of
+// those rows do.
+//
+// Cells outside the matrix: the reference's rows start at column -1-(q mod
+// 32) with zero states, which is where lane l's phase 0 (lower half) or 1
+// (upper half) starts; rows q = 31 mod 32 see zeros left and upper-left at
+// column 0, the first column of lane 31's phase 1 and lane 63's phase 2; rows
+// q = 0 mod 32 see zeros above at negative columns, which are the zeroed
+// states of lane 31 at that point.  So the states are zeroed at three phase
+// starts, and the steps need no tests.  What lanes compute past the
+// profile's end stays out of the maxima (kPast) and reaches no cell inside.
+//
+// Cost: 18 adds (two issue together), 7 max, 5 DPP moves and 3 instructions
+// for the maximum per step, against ~190 VALU with the boundary tests,
+// transitions handed from lane to lane, selects for max and score selection
+// in every step.
+template <bool kTrace, bool kGlobalRow, bool kSel>
 __device__ __forceinline__ void dp_pair(const cth_dpset& q, int qp, const cth_dpset& db, int p, int64_t colp,
                                         int64_t ldsc, const float* __restrict__ scores, uint8_t* __restrict__ btck,
-                                        float* bot, float& best_out, uint32_t& bestxy_out) {
-  const int lane = threadIdx.x;
+                                        float4* lds, float* grow, int W, float& best_out, uint32_t& bestxy_out) {
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lq = q.len[qp], lt = db.len[p];
   const int64_t qb = q.dist[qp] + qp;      // query transition vector 0
   const int64_t tb = db.dist[p] + p;       // template transition vector 0
   const int edge = corner_maxlen(lq, lt);
-  const int ltmax = lt;  // row stride of bot (the launch reserves 7 x its longest profile per wavefront)
-  float* const bmv = bot + 5 * ltmax;
-  uint32_t* const bmc = reinterpret_cast<uint32_t*>(bot + 6 * ltmax);
-  const int nstripes = (lq + 63) >> 6;
-  const int c0 = -1 - (lane & 31);
+  const int ns = (lq + 63) >> 6, P = sweep_phases(lt);
   const int hi = lane & 32;           // 32 for the upper half-wavefront
   const int tx = 31 - (lane & 31);    // the reference's thread in its block
-  for (int s = 0; s < nstripes; s++) {
-    const int y = (s << 6) + lane;
-    const bool rowok = y < lq;
-    const int band = 2 * s + (hi >> 5);     // block row of this lane
-    const int yb = 32 * band + 31;          // its last query row
-    const bool bandok = 32 * band < lq;     // the block row takes part
-    float mv = 0.0f;                        // the lane's running maximum
-    uint32_t mc = 0;                        // and its cell
-    float qt[CTH_NTRN];
-    if (rowok) {
-      qt[CTH_MM] = q.trn[CTH_MM * q.ldtr + qb + y];
-      qt[CTH_MI] = q.trn[CTH_MI * q.ldtr + qb + y + 1];
-      qt[CTH_MD] = q.trn[CTH_MD * q.ldtr + qb + y];
-      qt[CTH_IM] = q.trn[CTH_IM * q.ldtr + qb + y];
-      qt[CTH_II] = q.trn[CTH_II * q.ldtr + qb + y + 1];
-      qt[CTH_DM] = q.trn[CTH_DM * q.ldtr + qb + y];
-      qt[CTH_DD] = q.trn[CTH_DD * q.ldtr + qb + y];
-    } else {
-#pragma unroll
-      for (int i = 0; i < CTH_NTRN; i++) qt[i] = kLog0;
+  float4* const wl = lds + w * (dp_wave_lds(kGlobalRow) / 16);
+  float4* const ring = wl;
+  // the pair's row and buffer: column c of the row at index c + 1 (index 0,
+  // column -1, stays zero)
+  float4* const rowA = kGlobalRow ? nullptr : lds + W * (dp_wave_lds(false) / 16);
+  float* const rowB = reinterpret_cast<float*>(rowA + (lt + 33));
+  float* const bmv = kGlobalRow ? grow + 5 * (int64_t)lt : rowB + (lt + 33);
+  uint32_t* const bmc = reinterpret_cast<uint32_t*>(bmv + lt);
+  // stages of the global row
+  float4* const sinA = wl + kRingBytes / 16;
+  float* const sinB = reinterpret_cast<float*>(sinA + kStage);
+  float4* const soutA = sinA + kStage + kStage / 4;
+  float* const soutB = reinterpret_cast<float*>(soutA + kStage);
+  // the first stripe's row above: zeros
+  if constexpr (!kGlobalRow) {
+    for (int k = threadIdx.x; k < lt + 33; k += 64 * W) {
+      rowA[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      rowB[k] = 0.0f;
     }
-    // wait for the query transitions here, once per stripe: a wait inside
-    // the step loop would also wait for the prefetches issued in it
-#pragma unroll
-    for (int i = 0; i < CTH_NTRN; i++) asm volatile("" ::"v"(qt[i]));
-    float cMM = 0, cMI = 0, cIM = 0, cDN = 0, cND = 0;     // state of this lane's last column
-    float pMM = 0, pMI = 0, pIM = 0, pDN = 0, pND = 0;     // up-state received last step (= diagonal now)
-    float dt[CTH_NTRN];
-#pragma unroll
-    for (int i = 0; i < CTH_NTRN; i++) dt[i] = kLog0;
-    // Loads run ahead of their use (the step itself is a few hundred cycles
-    // of dependent arithmetic): the template column's transitions and the
-    // previous stripe's bottom row one step ahead, this lane's score two
-    // steps ahead.  Step t uses template column t - 32 and lane column
-    // t - lane - 32.
-    float ntn[CTH_NTRN], bn[5];
-    auto load_col = [&](int cu, float* nt, float* b) {
-      if (0 <= cu && cu < lt) {
-        nt[CTH_MM] = db.trn[CTH_MM * db.ldtr + tb + cu];
-        nt[CTH_MI] = db.trn[CTH_MI * db.ldtr + tb + cu + 1];
-        nt[CTH_MD] = db.trn[CTH_MD * db.ldtr + tb + cu];
-        nt[CTH_IM] = db.trn[CTH_IM * db.ldtr + tb + cu];
-        nt[CTH_II] = db.trn[CTH_II * db.ldtr + tb + cu + 1];
-        nt[CTH_DM] = db.trn[CTH_DM * db.ldtr + tb + cu];
-        nt[CTH_DD] = db.trn[CTH_DD * db.ldtr + tb + cu];
-      } else {
-#pragma unroll
-        for (int i = 0; i < CTH_NTRN; i++) nt[i] = kLog0;
+    lds_barrier();
+  }
+  // a zero in a vector register: LDS addresses built on it are not rebuilt
+  // from scalar registers at every access
+  int vzero;
+  asm("v_mov_b32 %0, 0" : "=v"(vzero));
+  const int G = sweep_start(ns - 1, W, P) + P;
+  // this wavefront's current stripe
+  int s = w, gs = sweep_start(w, W, P);
+  float qt[CTH_NTRN];
+  dp_state d;
+  float mv = 0.0f;
+  uint32_t mc = 0;
+  int y = 0, lo = 0, hc = 0;
+  const float* srow = scores;
+  score8 nxt{};
+  for (int g = 0; g < G; g++) {
+    const int k = g - gs;
+    if (k >= 0 && s < ns) {
+      const int cf = 32 * k - 1 - lane;  // the lane's first column of the phase
+      const int band = 2 * s + (hi >> 5);   // block row of this lane
+      const int yb = 32 * band + 31;        // its last query row
+      const bool bandok = 32 * band < lq;   // the block row takes part
+      if (k == 0) {
+        y = (s << 6) + lane;
+        const bool rowok = y < lq;
+        valid_columns(lq, lt, edge, y, lo, hc);
+        if (hc < lo) lo = hc = 1 << 30;                  // no valid column
+        if (!rowok) { lo = -(1 << 30); hc = 1 << 30; }  // what its cells hold reaches nothing
+        const int64_t at = qb + (rowok ? y : 0);
+        qt[CTH_MM] = q.trn[CTH_MM * q.ldtr + at];
+        qt[CTH_MI] = q.trn[CTH_MI * q.ldtr + at + 1];
+        qt[CTH_MD] = q.trn[CTH_MD * q.ldtr + at];
+        qt[CTH_IM] = q.trn[CTH_IM * q.ldtr + at];
+        qt[CTH_II] = q.trn[CTH_II * q.ldtr + at + 1];
+        qt[CTH_DM] = q.trn[CTH_DM * q.ldtr + at];
+        qt[CTH_DD] = q.trn[CTH_DD * q.ldtr + at];
+        srow = scores + (int64_t)(rowok ? y : lq - 1) * ldsc + colp;
+        nxt = score_load8(srow + max(cf, -8));
+        const ring_block r0 = ring_load(db, tb, lt, -64, kLog0, kPast), r1 = ring_load(db, tb, lt, -32, kLog0, kPast),
+                         r2 = ring_load(db, tb, lt, 0, kLog0, kPast);
+        ring_store(ring, -64, r0);
+        ring_store(ring, -32, r1);
+        ring_store(ring, 0, r2);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local");
+        mv = 0.0f;
+        mc = 0u;
       }
-      if (s > 0 && 0 <= cu && cu < lt) {
-        b[0] = bot[0 * ltmax + cu]; b[1] = bot[1 * ltmax + cu]; b[2] = bot[2 * ltmax + cu];
-        b[3] = bot[3 * ltmax + cu]; b[4] = bot[4 * ltmax + cu];
-      } else {
-        b[0] = b[1] = b[2] = b[3] = b[4] = 0.0f;
+      // zero states: at the stripe's start, and where the boundary rules ask
+      if (k < 3 && (k == 0 || lane >= (k == 1 ? 31 : 63))) {
+        d.cMM = d.cMI = d.cIM = d.cDN = d.cND = 0.0f;
+        d.aMM = d.aMI = 0.0f + qt[CTH_MM];
+        d.pIM = d.pDN = d.pND = 0.0f;
       }
-    };
-    // the raw score at lane column c (0 outside the profile; the valid-area
-    // test is applied where it is used)
-    const float* __restrict__ srow = scores + (int64_t)y * ldsc + colp;
-    auto load_sc = [&](int c) { return (rowok && 0 <= c && c < lt) ? srow[c] : 0.0f; };
-    // The scores come in groups of four columns per lane, group G of lane l
-    // being columns 4G - l .. 4G - l + 3: at step t every lane is at element
-    // (t - 32) mod 4 of group (t - 32) / 4, so the whole wavefront refills at
-    // once, one 16-byte load (dword-aligned) per lane every four steps instead
-    // of four 4-byte loads; each lane reads its own row, so a load touches a
-    // cache line per lane, and fewer, wider loads take the texture path and
-    // L1 far fewer requests per cell.  Groups reaching outside the profile
-    // load their columns one by one (0 outside).
-    typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
-    auto load_grp = [&](int G, float* v) {
-      const int cs = 4 * G - lane;
-      if (rowok && 0 <= cs && cs + 3 < lt) {
-        const float4u x = *reinterpret_cast<const float4u*>(srow + cs);
-        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-      } else {
-        v[0] = load_sc(cs); v[1] = load_sc(cs + 1); v[2] = load_sc(cs + 2); v[3] = load_sc(cs + 3);
+      // a block starts: seed from the buffer at the column before
+      const int x0 = 32 * (k - 1) - hi;
+      const bool blk = bandok && -32 <= x0 && x0 < lt;
+      if (blk) {
+        const int xs = x0 + tx - 1;
+        const bool in = 0 <= xs && xs < lt;
+        mv = in ? bmv[xs] : 0.0f;
+        mc = in ? bmc[xs] : 0u;
       }
-    };
-    // Steps 0..30 compute no cell (lane l's first cell, at column
-    // -1-(l mod 32), comes at step 31 or later), write nothing and leave the
-    // state as it starts (dt log 0, zero states; no block starts or ends
-    // there), so the sweep starts at step 31 with its loads issued for it.
-    // After lane 63's last column (step lt + 94) only the final block end
-    // (step 32 ceil(lt/32) + 94, the next step = 30 mod 32, with no block
-    // start before it) remains, so the sweep jumps there.
-    constexpr int t0 = 31;
-    load_col(t0 - 32, ntn, bn);
-    float grp[4], grpn[4];  // this step's group and the next
-    load_grp((t0 - 32) >> 2, grp);
-    load_grp(((t0 - 32) >> 2) + 1, grpn);
-    // the last block of the upper half ends at step 32 ceil(lt/32) + 94
-    const int nsteps = 32 * ((lt + 31) >> 5) + 95;
-    const int tlast = lt + 94;
-    for (int t = t0; t < nsteps; t = t < tlast ? t + 1 : (t < nsteps - 1 ? nsteps - 1 : nsteps)) {
-      const int c = t - lane - 32;
-      const int cu = t - 32;
-      if ((t & 31) == 31) {
-        // a block starts: seed from the buffer at the column before
-        const int x0 = t - 63 - hi;
-        if (bandok && -32 <= x0 && x0 < lt) {
-          const int xs = x0 + tx - 1;
-          if (0 <= xs && xs < lt) {
-            mv = bmv[xs];
-            mc = bmc[xs];
-          } else {
-            mv = 0.0f;
-            mc = 0u;
+      const float mv0 = mv;
+      int ms = -1;
+      // the next phase's transitions (in the ring after this phase's steps)
+      const ring_block nring = ring_load(db, tb, lt, 32 * k + 32, kLog0, kPast);
+      // the row above from lane 0's first column on, the bottom row from lane
+      // 63's (columns past the profile carry what no cell inside reads)
+      const float4* inA;
+      const float* inB;
+      uint32_t outA, outB;
+      const int kb = k < (lt >> 5) ? k : (lt >> 5);
+      if constexpr (kGlobalRow) {
+        if (lane < kStage) {
+          const int c = 32 * k - 1 + lane;
+          float v[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+          if (s > 0 && 0 <= c && c < lt) {
+#pragma unroll
+            for (int i = 0; i < 5; i++) v[i] = grow[(int64_t)i * lt + c];
+          }
+          sinA[lane] = make_float4(v[0], v[1], v[2], v[3]);
+          sinB[lane] = v[4];
+        }
+        inA = sinA + vzero; inB = sinB + vzero;
+        outA = lds_offset(soutA); outB = lds_offset(soutB);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup", "local");
+      } else {
+        inA = rowA + 32 * kb + vzero; inB = rowB + 32 * kb + vzero;
+        outA = lds_offset(rowA) + 16 * (32 * k - 63); outB = lds_offset(rowB) + 4 * (32 * k - 63);
+      }
+      const uint64_t mask = k >= 2 ? 1ull << 63 : 0ull;
+      const float4* const rg = ring + (cf & (kRing - 1));
+      const bool fix = __builtin_amdgcn_ballot_w64(cf < lo || cf + 31 > hc) != 0;
+      const int crel = cf - lo;
+      const uint32_t span = (uint32_t)(hc - lo);
+      for (int j0 = 0; j0 < 32 && 32 * k - 64 + j0 < lt; j0 += 8) {
+        const score8 cur = nxt;
+        nxt = score_load8(srow + max(-8, min(cf + j0 + 8, lt)));
+        uint32_t bk[2];
+        if (fix)
+          dp_steps8<kTrace, kSel, true>(d, qt, j0, rg + j0, inA + j0, inB + j0, outA + 16 * j0, outB + 4 * j0, mask, crel + j0,
+                                        span, cf + j0, (uint32_t)lt, cur, mv, ms, bk);
+        else
+          dp_steps8<kTrace, kSel, false>(d, qt, j0, rg + j0, inA + j0, inB + j0, outA + 16 * j0, outB + 4 * j0, mask, 0, 0u,
+                                         cf + j0, (uint32_t)lt, cur, mv, ms, bk);
+        if constexpr (kTrace) {
+          if (y < lq) {
+            const int c = cf + j0;
+            uint8_t* const at = btck + (int64_t)y * ldsc + colp + c;
+            if (0 <= c && c + 7 < lt) {
+              memcpy(at, bk, 8);
+            } else {
+#pragma unroll
+              for (int j = 0; j < 8; j++)
+                if (0 <= c + j && c + j < lt) at[j] = (uint8_t)(bk[j >> 2] >> (8 * (j & 3)));
+            }
           }
         }
       }
-      // this step's column data, then the loads for the steps after
-      float nt[CTH_NTRN], bcu[5];
-#pragma unroll
-      for (int i = 0; i < CTH_NTRN; i++) nt[i] = ntn[i];
-#pragma unroll
-      for (int i = 0; i < 5; i++) bcu[i] = bn[i];
-      const int e = (t - 32) & 3;
-      const float scv = e == 0 ? grp[0] : e == 1 ? grp[1] : e == 2 ? grp[2] : grp[3];
-      if (e == 3) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) grp[i] = grpn[i];
-        load_grp(((t - 32) >> 2) + 2, grpn);
+      // the asm stores are not counted by the compiler's waits
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+      // rows past the query's end computed on whatever lies there
+      if (y >= lq) mv = mv0;
+      else if (ms >= 0) mc = ((uint32_t)(cf + ms) << 16) | (uint32_t)y;
+      ring_store(ring, 32 * k + 32, nring);
+      // a block ends: write the buffer, the lower half-wavefront first
+      const int wc = flow_write_column(x0, tx, lt);
+      const bool wr = blk && flow_block_iters(x0, yb, lq, lt) >= 1 && 0 <= wc && wc < lt;
+      if (wr && hi == 0 && (band == 0 || bmv[wc] < mv)) {
+        bmv[wc] = mv;
+        bmc[wc] = mc;
       }
-      load_col(cu + 1, ntn, bn);
-      // template transitions: lane 0 takes column t-32, the others lane-1's
-#pragma unroll
-      for (int i = 0; i < CTH_NTRN; i++) dt[i] = dpp_shr1(nt[i], dt[i]);
-      // up state: lane 0 reads the previous stripe's bottom row (zero for the
-      // first stripe and for negative columns), the others take lane-1's
-      float uMM = dpp_shr1(bcu[0], cMM), uMI = dpp_shr1(bcu[1], cMI), uIM = dpp_shr1(bcu[2], cIM);
-      float uDN = dpp_shr1(bcu[3], cDN), uND = dpp_shr1(bcu[4], cND);
-      if ((lane & 31) == 0 && c < 0) { uMM = uMI = uIM = uDN = uND = 0.0f; }
-      if ((lane & 31) == 31 && c == 0) {  // thread 0 of the block at x = 0: zero left/diagonal
-        cMM = cMI = cIM = cDN = cND = 0.0f;
-        pMM = pMI = pIM = pDN = pND = 0.0f;
+      flow_phase<kGlobalRow>();
+      if (wr && hi != 0 && bmv[wc] < mv) {
+        bmv[wc] = mv;
+        bmc[wc] = mc;
       }
-      if (rowok && c0 <= c && c < lt) {
-        const float S = in_valid_area(lq, lt, edge, y, c) ? scv : CTH_OUTSCORE;
-        float v1, v2, m;
-        int bk;
-        v1 = pMI + qt[CTH_MM] + dt[CTH_IM];
-        v2 = pIM + qt[CTH_IM] + dt[CTH_MM];
-        v1 = mx(v1, v2);
-        v2 = pDN + qt[CTH_DM] + dt[CTH_MM];
-        v1 = mx(v1, v2);
-        v2 = pND + qt[CTH_MM] + dt[CTH_DM];
-        v1 = mx(v1, v2);
-        v2 = pMM + qt[CTH_MM] + dt[CTH_MM];
-        v1 = mx(v1, v2);
-        const float nMM = mx(v1 + S, 0.0f);
-        m = nMM;
-        bk = nMM != 0.0f ? CTH_BT_DIAG : CTH_BT_STOP;
-        v1 = uMM + qt[CTH_MM] + dt[CTH_MI];
-        v2 = uMI + qt[CTH_MM] + dt[CTH_II];
-        const float nMI = mx(v1, v2);
-        if (m < nMI) { m = nMI; bk = CTH_BT_UP; }
-        v1 = cMM + qt[CTH_MI] + dt[CTH_MM];
-        v2 = cIM + qt[CTH_II] + dt[CTH_MM];
-        const float nIM = mx(v1, v2);
-        if (m < nIM) { m = nIM; bk = CTH_BT_LEFT; }
-        v1 = uMM + qt[CTH_MD];
-        v2 = uDN + qt[CTH_DD];
-        const float nDN = mx(v1, v2);
-        if (m < nDN) { m = nDN; bk = CTH_BT_UP; }
-        v1 = cMM + dt[CTH_MD];
-        v2 = cND + dt[CTH_DD];
-        const float nND = mx(v1, v2);
-        if (m < nND) { m = nND; bk = CTH_BT_LEFT; }
-        cMM = nMM; cMI = nMI; cIM = nIM; cDN = nDN; cND = nND;
-        if (0 <= c) {
-          if (mv < nMM) { mv = nMM; mc = ((uint32_t)c << 16) | (uint32_t)y; }
-          if (btck) btck[(int64_t)y * ldsc + colp + c] = (uint8_t)bk;
+      if constexpr (kGlobalRow) {
+        const int c = 32 * k - 64 + lane;
+        if (lane < kStage && k >= 2 && c < lt) {
+          const float4 a = soutA[lane];
+          grow[c] = a.x;
+          grow[(int64_t)lt + c] = a.y;
+          grow[(int64_t)2 * lt + c] = a.z;
+          grow[(int64_t)3 * lt + c] = a.w;
+          grow[(int64_t)4 * lt + c] = soutB[lane];
         }
       }
-      pMM = uMM; pMI = uMI; pIM = uIM; pDN = uDN; pND = uND;
-      if (lane == 63 && 0 <= c && c < lt) {
-        bot[0 * ltmax + c] = cMM; bot[1 * ltmax + c] = cMI; bot[2 * ltmax + c] = cIM;
-        bot[3 * ltmax + c] = cDN; bot[4 * ltmax + c] = cND;
-      }
-      if ((t & 31) == 30) {
-        // a block ends: write the buffer, the lower half-wavefront first
-        const int x0 = t - 94 - hi;
-        const int w = flow_write_column(x0, tx, lt);
-        const bool wr = bandok && -32 <= x0 && x0 < lt && flow_block_iters(x0, yb, lq, lt) >= 1 && 0 <= w && w < lt;
-        if (wr && hi == 0 && (band == 0 || bmv[w] < mv)) {
-          bmv[w] = mv;
-          bmc[w] = mc;
-        }
-        flow_phase();
-        if (wr && hi != 0 && bmv[w] < mv) {
-          bmv[w] = mv;
-          bmc[w] = mc;
-        }
-        flow_phase();
+      if (k == P - 1) {
+        s += W;
+        gs = sweep_start(s, W, P);
       }
     }
-    __syncthreads();
+    if constexpr (kGlobalRow) __syncthreads();
+    else lds_barrier();
   }
   // FinalizeDPPro's reduction of the buffer's last 64 columns
-  flow_final(bmv, bmc, lt, best_out, bestxy_out);
+  if (w == 0) flow_final(bmv, bmc, lt, best_out, bestxy_out);
 }
 
-template <bool kGlobalRow>
-__global__ __launch_bounds__(64) void k_dp(cth_dpset q, int qp, cth_dpset db, int pbase,
-                                           const int* __restrict__ plist, int64_t col0, int64_t ldsc,
-                                           const float* __restrict__ scores, uint8_t* __restrict__ btck,
-                                           cth_dpres* __restrict__ res, float* __restrict__ grow,
-                                           int64_t growstride) {
-  // [7][lt]: bottom row of the previous stripe and the buffer of maxima, in
-  // LDS or in this wavefront's growstride floats of grow
-  extern __shared__ float lds_row[];
-  float* const bot = kGlobalRow ? grow + (int64_t)blockIdx.x * growstride : lds_row;
+// wavefronts of the largest workgroup
+constexpr int kMaxWaves = 8;
+
+template <bool kTrace, bool kGlobalRow, bool kSel>
+__global__ __launch_bounds__(64 * kMaxWaves) void k_dp(cth_dpset q, int qp, cth_dpset db, int pbase,
+                                                       const int* __restrict__ plist, int64_t col0, int64_t ldsc,
+                                                       const float* __restrict__ scores, uint8_t* __restrict__ btck,
+                                                       cth_dpres* __restrict__ res, float* __restrict__ grow,
+                                                       int64_t growstride) {
+  extern __shared__ float4 lds_dp[];
   const int p = plist ? plist[blockIdx.x] : pbase + blockIdx.x;
-  float best;
-  uint32_t bestxy;
-  dp_pair(q, qp, db, p, db.dist[p] - col0, ldsc, scores, btck, bot, best, bestxy);
+  float best = 0.0f;
+  uint32_t bestxy = 0;
+  dp_pair<kTrace, kGlobalRow, kSel>(q, qp, db, p, db.dist[p] - col0, ldsc, scores, btck, lds_dp,
+                                    kGlobalRow ? grow + (int64_t)blockIdx.x * growstride : nullptr,
+                                    (int)(blockDim.x >> 6), best, bestxy);
   if (threadIdx.x == 0) {
     res[blockIdx.x].maxsc = best;
     res[blockIdx.x].maxxy = bestxy;
@@ -320,40 +434,49 @@ __global__ __launch_bounds__(64) void k_dp(cth_dpset q, int qp, cth_dpset db, in
 }
 
 // Batched phase 1: a persistent grid works through n pairs (or the *count
-// pairs listed in list), each wavefront taking the next pair from the device
+// pairs listed in list), each workgroup taking the next pair from the device
 // counter next; pair pairs[i] of query bq[pairs[i].b] reads that query's
 // scores (and writes its traceback bytes) at the query's offset; res is per
 // pair.  Pairs come in the order given (longest first), so the longest DPs
 // start first.
 //
-// No branch in this loop depends on the lane: every lane takes part in the
-// fetch (lane 0 adds 1, the others 0, so lane 0's old value is the pair) and
-// every lane stores the wave-uniform maximum.  A fetch under
+// No branch in this loop depends on the lane: every lane of wavefront 0 takes
+// part in the fetch (lane 0 adds 1, the others 0, so lane 0's old value is
+// the pair) and the others read it from LDS.  A fetch under
 // `if (threadIdx.x == 0)` lets the compiler thread that loop-invariant branch
 // across the back edge, which leaves lanes 1..63 in a second copy of the loop
 // that never fetches again (they re-run the first pair forever).
-template <bool kTrace>
-__global__ __launch_bounds__(64) void k_dp_batch(cth_dpset q, cth_dpset db, const cth_bquery* __restrict__ bq,
-                                                 const cth_bpair* __restrict__ pairs, const int* __restrict__ list,
-                                                 const int* __restrict__ count, int n, int* __restrict__ next,
-                                                 int64_t ldsc, const float* __restrict__ scores,
-                                                 uint8_t* __restrict__ btck, cth_dpres* __restrict__ res) {
-  extern __shared__ float lds_row[];
+template <bool kTrace, bool kGlobalRow, bool kSel>
+__global__ __launch_bounds__(64 * kMaxWaves) void k_dp_batch(
+    cth_dpset q, cth_dpset db, const cth_bquery* __restrict__ bq, const cth_bpair* __restrict__ pairs,
+    const int* __restrict__ list, const int* __restrict__ count, int n, int* __restrict__ next, int64_t ldsc,
+    const float* __restrict__ scores, uint8_t* __restrict__ btck, cth_dpres* __restrict__ res,
+    float* __restrict__ grow, int64_t growstride) {
+  extern __shared__ float4 lds_dp[];
+  __shared__ int s_next;
   const int nj = count ? *count : n;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   for (;;) {
+    if (w == 0) s_next = __builtin_amdgcn_readfirstlane(atomicAdd(next, threadIdx.x == 0 ? 1 : 0));
+    __syncthreads();
     // uniform: scalar loads of the pair and query
-    const int k = __builtin_amdgcn_readfirstlane(atomicAdd(next, threadIdx.x == 0 ? 1 : 0));
+    const int k = __builtin_amdgcn_readfirstlane(s_next);
     if (k >= nj) break;
     const int i = list ? list[k] : k;
     const cth_bpair pr = pairs[i];
     const cth_bquery Q = bq[pr.b];
-    float best;
-    uint32_t bestxy;
-    dp_pair(q, Q.qp, db, pr.p, db.dist[pr.p], ldsc, scores + Q.off, kTrace ? btck + Q.off : nullptr, lds_row, best,
-            bestxy);
-    // the butterfly in dp_pair leaves the same maximum in every lane
-    res[i].maxsc = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, best)));
-    res[i].maxxy = (uint32_t)__builtin_amdgcn_readfirstlane((int)bestxy);
+    float best = 0.0f;
+    uint32_t bestxy = 0;
+    dp_pair<kTrace, kGlobalRow, kSel>(q, Q.qp, db, pr.p, db.dist[pr.p], ldsc, scores + Q.off,
+                                      kTrace ? btck + Q.off : nullptr, lds_dp,
+                                      kGlobalRow ? grow + (int64_t)blockIdx.x * growstride : nullptr,
+                                      (int)(blockDim.x >> 6), best, bestxy);
+    if (w == 0) {
+      // flow_final leaves the same maximum in every lane
+      res[i].maxsc = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, best)));
+      res[i].maxxy = (uint32_t)__builtin_amdgcn_readfirstlane((int)bestxy);
+    }
+    __syncthreads();
   }
 }
 
@@ -466,26 +589,68 @@ extern "C" size_t cth_dp_row_bytes(int np, int ltmax) {
   return ltmax > CTH_DP_GLOBAL_FROM ? sizeof(float) * 7 * (size_t)ltmax * (size_t)(np > 0 ? np : 0) : 0;
 }
 
-// Phase 1 for np profiles: p0 + k, or plist[k] (device array of absolute
-// indices) when plist is not NULL; res[k] receives profile k's record.
-// btck NULL: no traceback bytes (maximum and its coordinates only);
-// finalize: run the finalisation (needs btck).  grow: cth_dp_row_bytes(np,
-// ltmax) bytes of device memory when ltmax exceeds CTH_DP_GLOBAL_FROM (else
-// unused).
-extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, const cth_dpset* db, int p0, const int* plist, int np,
-                                  int ltmax, int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck,
+namespace {
+
+// Wavefronts per pair: one per stripe up to kMaxWaves.
+int dp_waves(int lq) { return std::max(1, std::min(kMaxWaves, (lq + 63) / 64)); }
+
+bool dp_select(const cth_dpset* q, const cth_dpset* db) { return !cth_finite_scores(q, db); }
+
+template <bool kTrace, bool kGlobalRow>
+void dp_launch(const cth_dpset* q, int qp, const cth_dpset* db, int p0, const int* plist, int np, int W, size_t lds,
+               int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck, cth_dpres* res, float* grow,
+               int64_t growstride, hipStream_t st) {
+  if (dp_select(q, db))
+    hipLaunchKernelGGL((k_dp<kTrace, kGlobalRow, true>), dim3(np), dim3(64 * W), lds, st, *q, qp, *db, p0, plist, col0,
+                       ldsc, scores, btck, res, grow, growstride);
+  else
+    hipLaunchKernelGGL((k_dp<kTrace, kGlobalRow, false>), dim3(np), dim3(64 * W), lds, st, *q, qp, *db, p0, plist, col0,
+                       ldsc, scores, btck, res, grow, growstride);
+}
+
+template <bool kTrace, bool kGlobalRow>
+void dp_launch_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq, const cth_bpair* pairs,
+                     const int* list, const int* count, int n, int* next, int W, size_t lds, int grid, int64_t ldsc,
+                     const float* scores, uint8_t* btck, cth_dpres* res, float* grow, int64_t growstride,
+                     hipStream_t st) {
+  if (dp_select(q, db))
+    hipLaunchKernelGGL((k_dp_batch<kTrace, kGlobalRow, true>), dim3(grid), dim3(64 * W), lds, st, *q, *db, bq, pairs,
+                       list, count, n, next, ldsc, scores, btck, res, grow, growstride);
+  else
+    hipLaunchKernelGGL((k_dp_batch<kTrace, kGlobalRow, false>), dim3(grid), dim3(64 * W), lds, st, *q, *db, bq, pairs,
+                       list, count, n, next, ldsc, scores, btck, res, grow, growstride);
+}
+
+}  // namespace
+
+// Phase 1 for np profiles (query qp of lq positions): p0 + k, or plist[k]
+// (device array of absolute indices) when plist is not NULL; res[k] receives
+// profile k's record.  scores: readable 8 floats to either side of its
+// [lq][ldsc].  btck NULL: no traceback bytes (maximum and its coordinates
+// only); finalize: run the finalisation (needs btck).  grow:
+// cth_dp_row_bytes(np, ltmax) bytes of device memory when ltmax exceeds
+// CTH_DP_GLOBAL_FROM (else unused).
+extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, const int* plist,
+                                  int np, int ltmax, int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck,
                                   float scorethld, int finalize, cth_dpres* res, float* grow, hipStream_t st) {
   if (np <= 0) return 0;
   if (finalize && !btck) { cth_set_error("dp: finalisation needs the traceback"); return -1; }
   if (ltmax > CTH_MAXCOLUMNS) { cth_set_error("dp: profile length %d over %d", ltmax, CTH_MAXCOLUMNS); return -1; }
-  if (ltmax > CTH_DP_GLOBAL_FROM) {
-    if (!grow) { cth_set_error("dp: profile length %d needs global boundary rows", ltmax); return -1; }
-    hipLaunchKernelGGL(k_dp<true>, dim3(np), dim3(64), 0, st, *q, qp, *db, p0, plist, col0, ldsc, scores, btck, res,
-                       grow, (int64_t)7 * ltmax);
+  const bool global = ltmax > CTH_DP_GLOBAL_FROM;
+  if (global && !grow) { cth_set_error("dp: profile length %d needs global boundary rows", ltmax); return -1; }
+  const int W = dp_waves(lq);
+  const size_t lds = W * dp_wave_lds(global) + dp_row_lds(ltmax, global);
+  const int64_t gs = (int64_t)7 * ltmax;
+  if (global) {
+    if (btck)
+      dp_launch<true, true>(q, qp, db, p0, plist, np, W, lds, col0, ldsc, scores, btck, res, grow, gs, st);
+    else
+      dp_launch<false, true>(q, qp, db, p0, plist, np, W, lds, col0, ldsc, scores, btck, res, grow, gs, st);
   } else {
-    const size_t lds = sizeof(float) * 7 * (size_t)(ltmax > 0 ? ltmax : 1);
-    hipLaunchKernelGGL(k_dp<false>, dim3(np), dim3(64), lds, st, *q, qp, *db, p0, plist, col0, ldsc, scores, btck,
-                       res, nullptr, (int64_t)0);
+    if (btck)
+      dp_launch<true, false>(q, qp, db, p0, plist, np, W, lds, col0, ldsc, scores, btck, res, nullptr, 0, st);
+    else
+      dp_launch<false, false>(q, qp, db, p0, plist, np, W, lds, col0, ldsc, scores, btck, res, nullptr, 0, st);
   }
   CTH_HIP_CHECK(hipGetLastError());
   if (finalize) {
@@ -495,31 +660,47 @@ extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, const cth_dpset* d
   return 0;
 }
 
-extern "C" int cth_launch_dp(const cth_dpset* q, int qp, const cth_dpset* db, int p0, int np, int ltmax,
+extern "C" int cth_launch_dp(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int np, int ltmax,
                              int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck, float scorethld,
                              cth_dpres* res, float* grow, hipStream_t st) {
-  return cth_launch_dp_list(q, qp, db, p0, nullptr, np, ltmax, col0, ldsc, scores, btck, scorethld, 1, res, grow, st);
+  return cth_launch_dp_list(q, qp, lq, db, p0, nullptr, np, ltmax, col0, ldsc, scores, btck, scorethld, 1, res, grow,
+                            st);
 }
 
-// Batched phase 1 (k_dp_batch) on a persistent grid of `grid` wavefronts:
-// the first pass over n pairs (list NULL, btck NULL), or the traceback pass
-// over the *count pairs of list followed by their finalisation (btck not
-// NULL).  next: a device counter that starts at zero.  Every profile of the
-// database fits the LDS row limit (the batched path keeps boundary rows in
-// LDS; ltmax is the database's longest profile).
+// Bytes of global boundary rows a batched launch of `grid` workgroups needs.
+extern "C" size_t cth_dp_batch_row_bytes(int grid, int ltmax) { return cth_dp_row_bytes(grid, ltmax); }
+
+// Batched phase 1 (k_dp_batch) on a persistent grid of `grid` workgroups of W
+// wavefronts: the first pass over n pairs (list NULL, btck NULL), or the
+// traceback pass over the *count pairs of list followed by their
+// finalisation (btck not NULL).  next: a device counter that starts at zero;
+// ltmax: the database's longest profile; scores as in cth_launch_dp_list;
+// grow: cth_dp_batch_row_bytes(grid, ltmax) bytes.
 extern "C" int cth_launch_dp_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq,
                                    const cth_bpair* pairs, const int* list, const int* count, int n, int* next,
                                    int ltmax, int64_t ldsc, const float* scores, uint8_t* btck, cth_dpres* res,
-                                   int grid, hipStream_t st) {
-  if (ltmax > CTH_DP_LDS_ROW_MAX) { cth_set_error("dp batch: profile length %d over the LDS row limit", ltmax); return -1; }
+                                   float* grow, int grid, int W, hipStream_t st) {
   if (grid < 1) return 0;
-  const size_t lds = sizeof(float) * 7 * (size_t)(ltmax > 0 ? ltmax : 1);
-  if (btck)
-    hipLaunchKernelGGL(k_dp_batch<true>, dim3(grid), dim3(64), lds, st, *q, *db, bq, pairs, list, count, n, next, ldsc,
-                       scores, btck, res);
-  else
-    hipLaunchKernelGGL(k_dp_batch<false>, dim3(grid), dim3(64), lds, st, *q, *db, bq, pairs, list, count, n, next, ldsc,
-                       scores, btck, res);
+  if (W < 1 || W > kMaxWaves) { cth_set_error("dp batch: %d wavefronts per pair", W); return -1; }
+  const bool global = ltmax > CTH_DP_GLOBAL_FROM;
+  if (global && !grow) { cth_set_error("dp batch: profile length %d needs global boundary rows", ltmax); return -1; }
+  const size_t lds = W * dp_wave_lds(global) + dp_row_lds(ltmax, global);
+  const int64_t gs = (int64_t)7 * ltmax;
+  if (global) {
+    if (btck)
+      dp_launch_batch<true, true>(q, db, bq, pairs, list, count, n, next, W, lds, grid, ldsc, scores, btck, res, grow,
+                                  gs, st);
+    else
+      dp_launch_batch<false, true>(q, db, bq, pairs, list, count, n, next, W, lds, grid, ldsc, scores, btck, res, grow,
+                                   gs, st);
+  } else {
+    if (btck)
+      dp_launch_batch<true, false>(q, db, bq, pairs, list, count, n, next, W, lds, grid, ldsc, scores, btck, res,
+                                   nullptr, 0, st);
+    else
+      dp_launch_batch<false, false>(q, db, bq, pairs, list, count, n, next, W, lds, grid, ldsc, scores, btck, res,
+                                    nullptr, 0, st);
+  }
   CTH_HIP_CHECK(hipGetLastError());
   if (btck && list) {
     hipLaunchKernelGGL(k_dpfin_batch, dim3(grid), dim3(64), 0, st, *db, bq, pairs, list, count, ldsc, scores, btck,

@@ -34,7 +34,7 @@
 extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, int qp, const cth_dpset* db, int64_t col0, int ncols,
                                 int64_t ldsc, const cth_tables* dtabs, int lq, float* scores, float* mods, int contraction,
                                 int ddms, hipStream_t st);
-extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, const cth_dpset* db, int p0, const int* plist, int np,
+extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, const int* plist, int np,
                                   int ltmax, int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck,
                                   float scorethld, int finalize, cth_dpres* res, float* grow, hipStream_t st);
 extern "C" size_t cth_dp_row_bytes(int np, int ltmax);
@@ -160,11 +160,12 @@ struct chunk_bufs {
   int chunk(int qi, int lq, int ltchunk, int64_t ldsc, int np, bool map) {
     const size_t cells = (size_t)lq * (size_t)ldsc;
     if (!fixed) {
-      if (cth_ctx_reserve(c, (void**)&c->scores, &c->cap_scores, 4 * cells)) return -1;
+      // (the phase-1 DP reads up to 8 floats to either side of the scores)
+      if (cth_ctx_reserve(c, (void**)&c->scores, &c->cap_scores, 4 * cells + 2 * CTH_SCORE_PAD * sizeof(float))) return -1;
       if (cth_ctx_reserve(c, (void**)&c->mods, &c->cap_mods, 4 * cells)) return -1;
       if (cth_ctx_reserve(c, (void**)&c->btck, &c->cap_btck, cells)) return -1;
       if (cth_ctx_reserve(c, (void**)&c->dpout, &c->cap_dpout, sizeof(cth_dpres) * (size_t)np)) return -1;
-      scores = c->scores; mods = c->mods; btck = c->btck; dpout = (cth_dpres*)c->dpout;
+      scores = c->scores + CTH_SCORE_PAD; mods = c->mods; btck = c->btck; dpout = (cth_dpres*)c->dpout;
       mapbuf = nullptr;
       return 0;
     }
@@ -177,10 +178,11 @@ struct chunk_bufs {
     }
     size_t o = 0;
     auto take = [&](size_t n) { uint8_t* p = fixed + o; o += up(n); return p; };
+    // (records first: the phase-1 DP reads up to 8 floats to either side of the scores)
+    dpout = (cth_dpres*)take(sizeof(cth_dpres) * (size_t)np);
     scores = (float*)take(4 * cells);
     mods = (float*)take(4 * cells);
     btck = take(cells);
-    dpout = (cth_dpres*)take(sizeof(cth_dpres) * (size_t)np);
     mapbuf = map ? (float*)take(4 * cells) : nullptr;
     work_off = o;
     return 0;
@@ -368,7 +370,7 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
         }
         for (int a2 = a; a2 < b; a2 += nb) {
           const int b2 = std::min(b, a2 + nb);
-          if (cth_launch_dp_list(&c->q.d, qi, &db.d, a2, nullptr, b2 - a2, lg, col0, ldsc, scores, nullptr, scorethld,
+          if (cth_launch_dp_list(&c->q.d, qi, lq, &db.d, a2, nullptr, b2 - a2, lg, col0, ldsc, scores, nullptr, scorethld,
                                  0, dpout + (a2 - p0), grow, c->st))
             return -1;
         }
@@ -421,11 +423,11 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
         float* grow = nl ? (float*)(((uintptr_t)(d_res2 + nc) + 255) & ~(uintptr_t)255) : nullptr;
         CTH_HIP_CHECK(hipMemcpyAsync(d_cand, cand_abs.data(), sizeof(int) * nc, hipMemcpyHostToDevice, c->st));
         if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[1], c->st));
-        if (cth_launch_dp_list(&c->q.d, qi, &db.d, p0, d_cand, ns, ltc, col0, ldsc, scores, btck, scorethld, 1,
+        if (cth_launch_dp_list(&c->q.d, qi, lq, &db.d, p0, d_cand, ns, ltc, col0, ldsc, scores, btck, scorethld, 1,
                                d_res2, nullptr, c->st))
           return -1;
         for (int j = 0; j < nl; j += nbl)
-          if (cth_launch_dp_list(&c->q.d, qi, &db.d, p0, d_cand + ns + j, std::min(nbl, nl - j), ltl, col0, ldsc,
+          if (cth_launch_dp_list(&c->q.d, qi, lq, &db.d, p0, d_cand + ns + j, std::min(nbl, nl - j), ltl, col0, ldsc,
                                  scores, btck, scorethld, 1, d_res2 + ns + j, grow, c->st))
             return -1;
         if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[2], c->st));

@@ -271,8 +271,7 @@ int cth_search_noalloc(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, c
  * that runs each stage once over all its (query, profile) pairs in
  * persistent launches, with the next stage's pairs selected on the device,
  * and one synchronisation per batch; the launches are captured as a HIP
- * graph and replayed while the batch shape stays the same, and the
- * persistent grid sizes are autotuned per batch shape on its first run.
+ * graph and replayed while the batch shape stays the same.
  * Results (hits, their order, alignment rows) equal cth_search's.  Covers
  * the FP32 contraction and databases whose profiles have at most 5824
  * positions; other calls, and queries whose buffers alone exceed the budget,
