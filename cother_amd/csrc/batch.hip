@@ -62,7 +62,7 @@ extern "C" int cth_launch_map_batch(const cth_dpset* q, const cth_dpset* db, con
                                     const cth_bpair* pairs, const int* list, const int* count, int ltmax, int lqmax,
                                     int64_t ldsc, const float* scores, const float* mods, float* post, uint8_t* btck,
                                     const double* stats, double* zrow, float minpp, char* alnout, int rowcap,
-                                    cth_mapres* res, int grid, hipStream_t st);
+                                    cth_mapres* res, int grid, int W, hipStream_t st);
 
 namespace {
 
@@ -255,7 +255,7 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
     if (opt->do_map &&
         cth_launch_map_batch(&c->q.d, &db.d, L.bq, L.pairs, L.hitl, L.ctr + kCtrHits, ltmax, P.lqmax, ldsc, L.scores,
                              L.mods, L.post, L.btck, L.stats, L.zrow, opt->minpp > 0.0f ? opt->minpp : CTH_MINPP,
-                             L.alnout, rowcap, L.mres, std::min(S.small_grid, npairs), st))
+                             L.alnout, rowcap, L.mres, std::min(S.small_grid, npairs), S.trace_waves, st))
       return -1;
     hipLaunchKernelGGL(k_gather_hits, dim3(sel_grid), dim3(256), 0, st, L.bq, L.pairs, L.res, L.stats, L.mres,
                        opt->do_map, L.hitl, L.ctr + kCtrHits, L.hits);

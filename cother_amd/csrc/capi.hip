@@ -365,8 +365,8 @@ extern "C" int cth_map_block(cth_ctx* c, int qidx, int p0, int p1, const int32_t
   const int64_t ldsc = (ncols + 63) / 64 * 64;
   const size_t need = sizeof(float) * (size_t)lq * ldsc;
   if (cth_ctx_reserve(c, (void**)&c->scores, &c->cap_scores, need + 2 * CTH_SCORE_PAD * sizeof(float))) return -1;
-  if (cth_ctx_reserve(c, (void**)&c->mods, &c->cap_mods, need)) return -1;
-  if (cth_ctx_reserve(c, (void**)&c->mapbuf, &c->cap_mapbuf, need)) return -1;
+  if (cth_ctx_reserve(c, (void**)&c->mods, &c->cap_mods, need + 2 * CTH_SCORE_PAD * sizeof(float))) return -1;
+  if (cth_ctx_reserve(c, (void**)&c->mapbuf, &c->cap_mapbuf, need + 2 * CTH_SCORE_PAD * sizeof(float))) return -1;
   if (cth_ctx_reserve(c, (void**)&c->btck, &c->cap_btck, (size_t)lq * ldsc)) return -1;
   const size_t wneed = sizeof(double) * (size_t)njobs * lq + sizeof(cth_mapjob) * njobs +
                        sizeof(cth_mapres) * njobs + 512;
@@ -375,13 +375,13 @@ extern "C" int cth_map_block(cth_ctx* c, int qidx, int p0, int p1, const int32_t
   cth_mapjob* d_jobs = (cth_mapjob*)(d_zrow + (size_t)njobs * lq);
   cth_mapres* d_res = (cth_mapres*)(((uintptr_t)(d_jobs + njobs) + 15) & ~(uintptr_t)15);
   CTH_HIP_CHECK(hipMemcpyAsync(d_jobs, jobs.data(), sizeof(cth_mapjob) * njobs, hipMemcpyHostToDevice, c->st));
-  if (cth_launch_score(&c->q.d, c->q.ddoff, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores + CTH_SCORE_PAD, c->mods, 0,
+  if (cth_launch_score(&c->q.d, c->q.ddoff, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores + CTH_SCORE_PAD, c->mods + CTH_SCORE_PAD, 0,
                        ddms_of(c, qidx, p0, p1), c->st))
     return -1;
   const size_t rows = cth_map_row_bytes(njobs, ltmax);
   if (rows && cth_ctx_reserve(c, (void**)&c->grow, &c->cap_grow, rows)) return -1;
-  if (cth_launch_map(&c->q.d, qidx, lq, &c->db.d, d_jobs, njobs, ltmax, col0, ldsc, c->scores + CTH_SCORE_PAD, c->mods,
-                     (float*)c->mapbuf, c->btck, d_zrow, minpp, nullptr, lq + ltmax, d_res, rows ? c->grow : nullptr,
+  if (cth_launch_map(&c->q.d, qidx, lq, &c->db.d, d_jobs, njobs, ltmax, col0, ldsc, c->scores + CTH_SCORE_PAD, c->mods + CTH_SCORE_PAD,
+                     (float*)c->mapbuf + CTH_SCORE_PAD, c->btck, d_zrow, minpp, nullptr, lq + ltmax, d_res, rows ? c->grow : nullptr,
                      c->st))
     return -1;
   CTH_HIP_CHECK(hipMemcpyAsync(res, d_res, sizeof(cth_mapres) * njobs, hipMemcpyDeviceToHost, c->st));

@@ -15,9 +15,10 @@
 #define CTH_DDSTRIDE  128   // bytes per position of the distance list in HBM (n + 99 values + 0xff pad)
 #define CTH_PROSCALE 10000  // libpro/srcpro/PMProfileModel.h:58 ReadWriteScale
 #define CTH_MAXCOLUMNS 50000  // liblib/mylimits.h:50 MAXCOLUMNS: longest profile the readers accept
-// longest profile whose MAP stripe boundary rows (5 floats per column)
-// fit one workgroup's 160 KiB of LDS; longer ones keep them in global memory
-#define CTH_LDS_ROW_MAX 8192
+// longest profile whose MAP stripe boundary rows (5 floats per column) fit one
+// workgroup's 160 KiB of LDS beside the transition rings of eight wavefronts;
+// longer ones keep them in global memory
+#define CTH_LDS_ROW_MAX 6000
 // longest profile of a database that the batched search covers
 #define CTH_DP_LDS_ROW_MAX 5824
 // the phase-1 DP keeps its boundary rows and the reference's buffer of maxima

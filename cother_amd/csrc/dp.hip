@@ -341,7 +341,7 @@ __device__ __forceinline__ void dp_pair(const cth_dpset& q, int qp, const cth_dp
         inA = rowA + 32 * kb + vzero; inB = rowB + 32 * kb + vzero;
         outA = lds_offset(rowA) + 16 * (32 * k - 63); outB = lds_offset(rowB) + 4 * (32 * k - 63);
       }
-      const uint64_t mask = k >= 2 ? 1ull << 63 : 0ull;
+      const uint64_t mask = __builtin_amdgcn_readfirstlane(k) >= 2 ? 1ull << 63 : 0ull;  // (scalar)
       const float4* const rg = ring + (cf & (kRing - 1));
       const bool fix = __builtin_amdgcn_ballot_w64(cf < lo || cf + 31 > hc) != 0;
       const int crel = cf - lo;

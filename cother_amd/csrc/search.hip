@@ -160,12 +160,12 @@ struct chunk_bufs {
   int chunk(int qi, int lq, int ltchunk, int64_t ldsc, int np, bool map) {
     const size_t cells = (size_t)lq * (size_t)ldsc;
     if (!fixed) {
-      // (the phase-1 DP reads up to 8 floats to either side of the scores)
+      // (the DP sweeps read up to 8 floats to either side of their matrices)
       if (cth_ctx_reserve(c, (void**)&c->scores, &c->cap_scores, 4 * cells + 2 * CTH_SCORE_PAD * sizeof(float))) return -1;
-      if (cth_ctx_reserve(c, (void**)&c->mods, &c->cap_mods, 4 * cells)) return -1;
+      if (cth_ctx_reserve(c, (void**)&c->mods, &c->cap_mods, 4 * cells + 2 * CTH_SCORE_PAD * sizeof(float))) return -1;
       if (cth_ctx_reserve(c, (void**)&c->btck, &c->cap_btck, cells)) return -1;
       if (cth_ctx_reserve(c, (void**)&c->dpout, &c->cap_dpout, sizeof(cth_dpres) * (size_t)np)) return -1;
-      scores = c->scores + CTH_SCORE_PAD; mods = c->mods; btck = c->btck; dpout = (cth_dpres*)c->dpout;
+      scores = c->scores + CTH_SCORE_PAD; mods = c->mods + CTH_SCORE_PAD; btck = c->btck; dpout = (cth_dpres*)c->dpout;
       mapbuf = nullptr;
       return 0;
     }
@@ -178,7 +178,7 @@ struct chunk_bufs {
     }
     size_t o = 0;
     auto take = [&](size_t n) { uint8_t* p = fixed + o; o += up(n); return p; };
-    // (records first: the phase-1 DP reads up to 8 floats to either side of the scores)
+    // (records first: the DP sweeps read up to 8 floats to either side of their matrices)
     dpout = (cth_dpres*)take(sizeof(cth_dpres) * (size_t)np);
     scores = (float*)take(4 * cells);
     mods = (float*)take(4 * cells);
@@ -194,9 +194,10 @@ struct chunk_bufs {
       if (!mapbuf) cth_set_error("%s: no MAP buffer in this chunk's layout", who);
       return mapbuf;
     }
-    if (cth_ctx_reserve(c, (void**)&c->mapbuf, &c->cap_mapbuf, sizeof(float) * (size_t)lq * (size_t)ldsc))
+    if (cth_ctx_reserve(c, (void**)&c->mapbuf, &c->cap_mapbuf,
+                        sizeof(float) * ((size_t)lq * (size_t)ldsc + 2 * CTH_SCORE_PAD)))
       return nullptr;
-    return mapbuf = c->mapbuf;
+    return mapbuf = c->mapbuf + CTH_SCORE_PAD;
   }
 
   // How many profiles of one launch get global boundary rows of per_item
