@@ -287,7 +287,7 @@ extern "C" int cth_phase1_block(cth_ctx* c, int qidx, int p0, int p1, float scor
   return 0;
 }
 
-extern "C" int cth_launch_stats(const cth_dpset* q, int qp, const cth_dpset* db, int p0, int64_t col0, int64_t ldsc,
+extern "C" int cth_launch_stats(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int64_t col0, int64_t ldsc,
                                 const float* scores, const int* plist_abs, const int* plist_rel,
                                 const cth_dpres* dpres, int np2, double searchspace, int ssemodel, int* hist,
                                 double* out, hipStream_t st);
@@ -315,7 +315,6 @@ extern "C" int cth_phase2_block(cth_ctx* c, int qidx, int p0, int p1, float scor
   const int64_t col0 = c->db.h_dist[p0];
   const int64_t ncols = c->db.h_dist[p1 - 1] + c->db.h_len[p1 - 1] - col0;
   const int64_t ldsc = (ncols + 63) / 64 * 64;
-  (void)lq;
   const size_t need = sizeof(int) * 2 * np2 + sizeof(int) * 641 * (size_t)np2 + sizeof(double) * 10 * (size_t)np2 + 256;
   if (cth_ctx_reserve(c, &c->work, &c->cap_work, need)) return -1;
   int* d_abs = (int*)c->work;
@@ -324,7 +323,7 @@ extern "C" int cth_phase2_block(cth_ctx* c, int qidx, int p0, int p1, float scor
   double* d_out = (double*)(((uintptr_t)(d_hist + 641 * (size_t)np2) + 15) & ~(uintptr_t)15);
   CTH_HIP_CHECK(hipMemcpyAsync(d_abs, abs_.data(), sizeof(int) * np2, hipMemcpyHostToDevice, c->st));
   CTH_HIP_CHECK(hipMemcpyAsync(d_rel, rel.data(), sizeof(int) * np2, hipMemcpyHostToDevice, c->st));
-  if (cth_launch_stats(&c->q.d, qidx, &c->db.d, p0, col0, ldsc, c->scores + CTH_SCORE_PAD, d_abs, d_rel, (const cth_dpres*)c->dpout,
+  if (cth_launch_stats(&c->q.d, qidx, lq, &c->db.d, p0, col0, ldsc, c->scores + CTH_SCORE_PAD, d_abs, d_rel, (const cth_dpres*)c->dpout,
                        np2, searchspace, ssemodel, d_hist, d_out, c->st))
     return -1;
   CTH_HIP_CHECK(hipStreamSynchronize(c->st));

@@ -39,7 +39,7 @@ extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_
                                   float scorethld, int finalize, cth_dpres* res, float* grow, hipStream_t st);
 extern "C" size_t cth_dp_row_bytes(int np, int ltmax);
 extern "C" size_t cth_map_row_bytes(int njobs, int ltmax);
-extern "C" int cth_launch_stats(const cth_dpset* q, int qp, const cth_dpset* db, int p0, int64_t col0, int64_t ldsc,
+extern "C" int cth_launch_stats(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int64_t col0, int64_t ldsc,
                                 const float* scores, const int* plist_abs, const int* plist_rel,
                                 const cth_dpres* dpres, int np2, double searchspace, int ssemodel, int* hist,
                                 double* out, hipStream_t st);
@@ -462,7 +462,7 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
         CTH_HIP_CHECK(hipMemcpyAsync(d_abs, abs_.data(), sizeof(int) * np2, hipMemcpyHostToDevice, c->st));
         CTH_HIP_CHECK(hipMemcpyAsync(d_rel, rel.data(), sizeof(int) * np2, hipMemcpyHostToDevice, c->st));
         if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[3], c->st));
-        if (cth_launch_stats(&c->q.d, qi, &db.d, p0, col0, ldsc, scores, d_abs, d_rel, dpout, np2, sspace,
+        if (cth_launch_stats(&c->q.d, qi, lq, &db.d, p0, col0, ldsc, scores, d_abs, d_rel, dpout, np2, sspace,
                              opt->ssemodel, d_hist, d_out, c->st))
           return -1;
         if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[0], c->st));

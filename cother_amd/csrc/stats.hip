@@ -1,23 +1,28 @@
 // stats.hip: alignment statistics and E-values for profiles passed to phase 2.
 //
-// k_hist  : one workgroup per passed profile builds the 641-bin histogram of
-//           rint(32*clamp(S,-10,10)) over the profile's Lq x Lt scores in LDS
-//           (integer counts; masked 'X' positions skipped), the work of
-//           CalcScoreProbsXuninfDynPlmProfile (cuss/CuBatchSS_dynplm.cu:134-182).
-// k_stats : one wavefront per passed profile computes in double precision the
+// k_hist  : the 641-bin histogram of rint(32*clamp(S,-10,10)) over each passed
+//           profile's Lq x Lt scores (integer counts; masked 'X' positions
+//           skipped), the work of CalcScoreProbsXuninfDynPlmProfile
+//           (cuss/CuBatchSS_dynplm.cu:134-182), rows over several workgroups
+//           where profiles are few.  Bound by the LDS atomics.
+// k_stats : one workgroup per passed profile computes in double precision the
 //           parameters of CalcStatParamsDynPlmProfile (cuss/CuBatchSS_dynplm.cu:
 //           193-430): expected score, min/max, lambda by Newton-Raphson with
 //           bisection, relative entropy, K by the sigma series on the
-//           reference's 21x32 score grid (the 672 grid cells of one iteration
-//           are spread over the 64 lanes; each iteration's P_j sum is reduced
-//           in grid order), then the SS18 E-value of
-//           CalcSignificanceSS18DynPlmProfile (cuss/CuBatchSS_dynplm.cu:447-580,
-//           cuss/CuBatchSS_SS18.cuh:119-453) with the two small networks of
-//           cuss/CuBatchSS_NN.cuh:37-202.  Special functions: log regularized
-//           incomplete beta and upper incomplete gamma by Lentz continued
-//           fractions and the lower-gamma series (Numerical Recipes 3rd ed.,
-//           6.2, 6.4), in double precision.
+//           reference's 21x32 score grid (the 672 grid cells spread over the
+//           threads, each sum a workgroup reduction in a fixed order), then
+//           the SS18 E-value of CalcSignificanceSS18DynPlmProfile
+//           (cuss/CuBatchSS_dynplm.cu:447-580, cuss/CuBatchSS_SS18.cuh:119-453)
+//           with the two small networks of cuss/CuBatchSS_NN.cuh:37-202.
+//           Special functions: log regularized incomplete beta and upper
+//           incomplete gamma by Lentz continued fractions and the lower-gamma
+//           series (Numerical Recipes 3rd ed., 6.2, 6.4), in double precision.
+// Both are latency: a search has a handful of passed profiles.  10 profiles of
+// a 250-position query: 1.24 -> 0.12 ms (sums by one lane and one workgroup
+// per histogram before); 3 of a 2000-position query 11.6 -> 0.14 ms.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "cth_batch.h"
 #include "cth_dev.h"
@@ -49,35 +54,70 @@ __constant__ float c_nnw[93] = {
     0.1f, 12.0f, 1.0f, 4.0f, 0.05f, 1.0f, 0.1f, 0.35f, 0.65f,
     0.6f, 16.0f, 1.0f, 12.0f, 0.3f, -1.7f, 0.1f, 0.45f, 0.65f};
 
-// The 641-bin score histogram of query qp against profile p (scores from
-// scores[colp], row stride ldsc) into the workgroup's LDS array h.
+constexpr int kThreads = 256, kWaves = kThreads / 64;
+// copies of the histogram, by lane: the scores of neighbouring cells fall
+// into few bins, and atomics of a wavefront on one LDS word serialise
+constexpr int kCopies = 4;
+
+// Adds the scores of query rows [y0, y1) of query qp against profile p
+// (scores from scores[colp], row stride ldsc) to the workgroup's histogram
+// copies h (kCopies x 641, zeroed), a row per wavefront at a time.
 __device__ __forceinline__ void hist_fill(const cth_dpset& q, int qp, const cth_dpset& db, int p, int64_t colp,
-                                          int64_t ldsc, const float* __restrict__ scores, int* h) {
-  const int lq = q.len[qp], lt = db.len[p];
+                                          int64_t ldsc, const float* __restrict__ scores, int y0, int y1, int* h) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lt = db.len[p];
   const char* qaa = q.aa + q.dist[qp];
   const char* taa = db.aa + db.dist[p];
-  for (int b = threadIdx.x; b < kNssc; b += blockDim.x) h[b] = 0;
-  __syncthreads();
-  const int64_t ncell = (int64_t)lq * lt;
-  for (int64_t c = threadIdx.x; c < ncell; c += blockDim.x) {
-    const int y = (int)(c / lt), x = (int)(c - (int64_t)y * lt);
-    if (qaa[y] == 'X' || taa[x] == 'X') continue;
-    float s = scores[(int64_t)y * ldsc + colp + x];
-    if (s < -10.0f) s = -10.0f;
-    else if (s > 10.0f) s = 10.0f;
-    atomicAdd(&h[(int)rintf(s * 32.0f) - kSscMin], 1);
+  int* const hl = h + (lane & (kCopies - 1));
+  for (int x0 = 0; x0 < lt; x0 += 256) {
+    // four columns per lane, their masked positions once per column block
+    bool use[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int x = x0 + 64 * i + lane;
+      use[i] = x < lt && taa[x] != 'X';
+    }
+    for (int y = y0 + w; y < y1; y += kWaves) {
+      if (qaa[y] == 'X') continue;
+      const float* const row = scores + (int64_t)y * ldsc + colp + x0 + lane;
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = use[i] ? row[64 * i] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        float s = v[i];
+        if (s < -10.0f) s = -10.0f;
+        else if (s > 10.0f) s = 10.0f;
+        if (use[i]) atomicAdd(&hl[((int)rintf(s * 32.0f) - kSscMin) * kCopies], 1);
+      }
+    }
   }
-  __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void k_hist(const cth_dpset q, int qp, const cth_dpset db, int p0, int64_t col0,
-                                              int64_t ldsc, const float* __restrict__ scores,
-                                              const int* __restrict__ plist, int* __restrict__ hist) {
-  __shared__ int h[kNssc];
+// workgroup (k, split) adds its share of profile k's rows to hist (zeroed)
+__global__ __launch_bounds__(kThreads) void k_hist(const cth_dpset q, int qp, const cth_dpset db, int64_t col0,
+                                                   int64_t ldsc, const float* __restrict__ scores,
+                                                   const int* __restrict__ plist, int* __restrict__ hist) {
+  __shared__ int h[kNssc * kCopies];
   const int k = blockIdx.x;
   const int p = plist[k];
-  hist_fill(q, qp, db, p, db.dist[p] - col0, ldsc, scores, h);
-  for (int b = threadIdx.x; b < kNssc; b += blockDim.x) hist[(int64_t)k * kNssc + b] = h[b];
+  const int lq = q.len[qp], ny = (lq + (int)gridDim.y - 1) / (int)gridDim.y;
+  const int y0 = (int)blockIdx.y * ny, y1 = min(lq, y0 + ny);
+  if (y0 >= y1) return;
+  for (int b = threadIdx.x; b < kNssc * kCopies; b += kThreads) h[b] = 0;
+  __syncthreads();
+  hist_fill(q, qp, db, p, db.dist[p] - col0, ldsc, scores, y0, y1, h);
+  __syncthreads();
+  for (int b = threadIdx.x; b < kNssc; b += kThreads) {
+    int n = 0;
+    for (int i = 0; i < kCopies; i++) n += h[b * kCopies + i];
+    if (n) atomicAdd(&hist[(int64_t)k * kNssc + b], n);
+  }
+}
+
+__global__ void k_hist_zero(int* hist, int64_t n) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += gridDim.x * (int64_t)blockDim.x)
+    hist[i] = 0;
 }
 
 __device__ void grid_bounds(int y, int* left, int* right) {
@@ -89,21 +129,61 @@ __device__ void grid_bounds(int y, int* left, int* right) {
   *left = l; *right = r;
 }
 
-__device__ void lambda_eq(const double* G, const int* left, double x, double mn, double mxs, double* f, double* df) {
+// The workgroup's sums (and extremes) of two doubles per thread, to every
+// thread: a butterfly in each wavefront, then the wavefronts in order.  red:
+// 2 kWaves doubles of LDS.
+__device__ __forceinline__ void block_sum2(double& a, double& b, double* red) {
+  for (int off = 32; off >= 1; off >>= 1) {
+    a += __shfl_xor(a, off);
+    b += __shfl_xor(b, off);
+  }
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) { red[2 * w] = a; red[2 * w + 1] = b; }
+  __syncthreads();
+  a = red[0]; b = red[1];
+  for (int k = 1; k < kWaves; k++) { a += red[2 * k]; b += red[2 * k + 1]; }
+  __syncthreads();
+}
+__device__ __forceinline__ void block_minmax(double& mn, double& mxs, double* red) {
+  for (int off = 32; off >= 1; off >>= 1) {
+    const double a = __shfl_xor(mn, off), b = __shfl_xor(mxs, off);
+    if (a < mn) mn = a;
+    if (b > mxs) mxs = b;
+  }
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) { red[2 * w] = mn; red[2 * w + 1] = mxs; }
+  __syncthreads();
+  for (int k = 0; k < kWaves; k++) {
+    if (red[2 * k] < mn) mn = red[2 * k];
+    if (red[2 * k + 1] > mxs) mxs = red[2 * k + 1];
+  }
+  __syncthreads();
+}
+
+// a thread's cells of the 21 x 32 grid: cell threadIdx.x + 256 i, its score
+// and probability
+constexpr int kCells = (kNSC * kScale + kThreads - 1) / kThreads;
+struct grid_cells {
+  double g[kCells];
+  double sc[kCells];
+};
+
+// the lambda equation and its derivative at x, to every thread
+__device__ void lambda_eq(const grid_cells& C, double x, double mn, double mxs, double* red, double* f, double* df) {
   double lf = 0.0, ldf = 0.0;
-  for (int y = 0; y < kNSC; y++)
-    for (int k = 0; k < kScale; k++) {
-      double sc = left[y] + k + kSscMin;
-      if (mn <= sc && sc <= mxs) {
-        sc -= mxs;
-        const double e = x * sc;
-        if (kLogSpMin < e) {
-          const double t = exp(e) * G[y * kScale + k];
-          lf += t;
-          ldf += t * sc;
-        }
+  for (int i = 0; i < kCells; i++) {
+    double sc = C.sc[i];
+    if (C.g[i] != 0.0 && mn <= sc && sc <= mxs) {
+      sc -= mxs;
+      const double e = x * sc;
+      if (kLogSpMin < e) {
+        const double t = exp(e) * C.g[i];
+        lf += t;
+        ldf += t * sc;
       }
     }
+  }
+  block_sum2(lf, ldf, red);
   const double e = x * -mxs;
   if (kLogSpMin < e) {
     const double t = exp(e);
@@ -114,17 +194,18 @@ __device__ void lambda_eq(const double* G, const int* left, double x, double mn,
   *df = ldf;
 }
 
-__device__ double find_lambda(const double* G, const int* left, double mn, double mxs) {
+// uniform over the workgroup: every thread follows the same sums
+__device__ double find_lambda(const grid_cells& C, double mn, double mxs, double* red) {
   const double x1 = 1.0e-5, x2 = 10.0, acc = 1.0e-4;
   double f, df, fl, dx, dxold, xh, xl, rts;
-  lambda_eq(G, left, x1, mn, mxs, &fl, &df);
-  lambda_eq(G, left, x2, mn, mxs, &f, &df);
+  lambda_eq(C, x1, mn, mxs, red, &fl, &df);
+  lambda_eq(C, x2, mn, mxs, red, &f, &df);
   if ((fl > 0.0 && f > 0.0) || (fl < 0.0 && f < 0.0)) return -1.0;
   if (fl < 0.0) { xl = x1; xh = x2; } else { xh = x1; xl = x2; }
   rts = 0.5 * (x1 + x2);
   dxold = fabs(x2 - x1);
   dx = dxold;
-  lambda_eq(G, left, rts, mn, mxs, &f, &df);
+  lambda_eq(C, rts, mn, mxs, red, &f, &df);
   int n;
   for (n = 0; n < 32; n++) {
     bool stop = false;
@@ -142,7 +223,7 @@ __device__ double find_lambda(const double* G, const int* left, double mn, doubl
     }
     if (fabs(dx) < acc) stop = true;
     if (stop) break;
-    lambda_eq(G, left, rts, mn, mxs, &f, &df);
+    lambda_eq(C, rts, mn, mxs, red, &f, &df);
     if (f < 0.0) xl = rts; else xh = rts;
   }
   return n == 32 ? -1.0 : rts;
@@ -324,70 +405,83 @@ __device__ void significance(int ssemodel, int lq, int lt, double qeno, double t
   out[2] = logexp;
 }
 
-// The statistics of one passed profile p (one wavefront): parameters from
-// its histogram hc, then the significance of its phase-1 record r, into the
-// CTH_STATS_NOUT doubles at o.
+// The statistics of one passed profile p (one workgroup): parameters from
+// its histogram (bin b the sum of hc[b * copies .. +copies)), then the
+// significance of its phase-1 record r, into the CTH_STATS_NOUT doubles at o.
+// The grid's cells are spread over the threads, each sum a workgroup
+// reduction in a fixed order: a serial chain in one lane (672 exponentials per
+// evaluation of the lambda equation, ~12 evaluations) took ~0.8 ms.
+template <int kHistCopies>
 __device__ __forceinline__ void stats_one(const cth_dpset& q, int qp, const cth_dpset& db, int p, const int* hc,
                                           double searchspace, int ssemodel, const cth_dpres& r, double* o) {
-  __shared__ double G[kNSC * kScale], NG[kNSC * kScale], PJ[kNSC * kScale];
+  __shared__ double G[kNSC * kScale], NG[kNSC * kScale];
   __shared__ double pu[kNSC];
-  __shared__ int left[kNSC];
-  __shared__ double sh[8];  // umn, umx, E, H, lambda, K, total
-  const int lane = threadIdx.x;
-  if (lane < kNSC) {
-    int l, r;
-    grid_bounds(lane, &l, &r);
-    left[lane] = l;
-    double cnt = 0.0;
-    for (int x = 0; x < kScale; x++) {
-      const double v = (l + x <= r) ? (double)hc[l + x] : 0.0;
-      G[lane * kScale + x] = v;
-      cnt += v;
+  __shared__ double red[2 * kWaves];
+  const int tid = threadIdx.x;
+  auto bin = [&](int b) {
+    int n = 0;
+    for (int i = 0; i < kHistCopies; i++) n += hc[b * kHistCopies + i];
+    return (double)n;
+  };
+  // counts (whole numbers: their sums are exact in any order)
+  grid_cells C;
+  for (int i = 0; i < kCells; i++) {
+    const int c = tid + kThreads * i, y = c / kScale, x = c - y * kScale;
+    C.g[i] = 0.0;
+    C.sc[i] = 0.0;
+    if (c < kNSC * kScale) {
+      int l, rr;
+      grid_bounds(y, &l, &rr);
+      C.sc[i] = l + x + kSscMin;
+      if (l + x <= rr) C.g[i] = bin(l + x);
     }
-    pu[lane] = cnt;
+    double n = C.g[i];
+    for (int off = 16; off >= 1; off >>= 1) n += __shfl_xor(n, off);
+    if (c < kNSC * kScale && x == 0) pu[y] = n;
   }
-  __syncthreads();
-  if (lane == 0) {
-    double total = 0.0;
-    for (int b = 0; b < kNssc; b++) total += (double)hc[b];
-    for (int y = 0; y < kNSC; y++) pu[y] = pu[y] / total;
-    for (int c = 0; c < kNSC * kScale; c++) G[c] = G[c] / total;
-    double E = 0.0, mn = 0.0, mxs = 0.0;
-    for (int y = 0; y < kNSC; y++)
-      for (int x = 0; x < kScale; x++) {
-        const double sc = left[y] + x + kSscMin;
-        E += sc * G[y * kScale + x];
-        const double v = G[y * kScale + x] ? sc : 0.0;
-        if (v < mn) mn = v;
-        if (v > mxs) mxs = v;
+  double total = 0.0, E = 0.0;
+  for (int b = tid; b < kNssc; b += kThreads) total += bin(b);
+  block_sum2(total, E, red);
+  for (int i = 0; i < kCells; i++) C.g[i] = C.g[i] / total;
+  if (tid < kNSC) pu[tid] = pu[tid] / total;
+  double mn = 0.0, mxs = 0.0, zero = 0.0;
+  E = 0.0;
+  for (int i = 0; i < kCells; i++) {
+    E += C.sc[i] * C.g[i];
+    const double v = C.g[i] ? C.sc[i] : 0.0;
+    if (v < mn) mn = v;
+    if (v > mxs) mxs = v;
+  }
+  block_sum2(E, zero, red);
+  block_minmax(mn, mxs, red);
+  double lambda = -1.0;
+  if (!(0.0 <= E || mxs <= 0.0)) lambda = find_lambda(C, mn, mxs, red);
+  double H = -1.0;
+  if (lambda > 0.0) {
+    H = 0.0;
+    for (int i = 0; i < kCells; i++) {
+      const double sc = C.sc[i];
+      if (C.g[i] != 0.0 && mn <= sc && sc <= mxs) {
+        const double yy = lambda * sc;
+        if (kLogSpMin < yy && yy < kLogSpMax - 3.0) H += exp(yy) * yy * C.g[i];
       }
-    double lambda = -1.0;
-    if (!(0.0 <= E || mxs <= 0.0)) lambda = find_lambda(G, left, mn, mxs);
-    double H = -1.0;
-    if (lambda > 0.0) {
-      H = 0.0;
-      for (int y = 0; y < kNSC; y++)
-        for (int x = 0; x < kScale; x++) {
-          const double sc = left[y] + x + kSscMin;
-          if (mn <= sc && sc <= mxs) {
-            const double yy = lambda * sc;
-            if (kLogSpMin < yy && yy < kLogSpMax - 3.0) H += exp(yy) * yy * G[y * kScale + x];
-          }
-        }
     }
-    for (int x = 0; x < kScale; x++) G[10 * kScale + x] = 1.0;
-    lambda *= kScale;
-    E /= kScale;
-    double umn = 0.0, umx = 0.0;
-    for (int y = 0; y < kNSC; y++) {
-      const double v = pu[y] ? (double)(y - 10) : 0.0;
-      if (v < umn) umn = v;
-      if (v > umx) umx = v;
-    }
-    sh[0] = umn; sh[1] = umx; sh[2] = E; sh[3] = H; sh[4] = lambda; sh[5] = -1.0;
+    zero = 0.0;
+    block_sum2(H, zero, red);
+  }
+  lambda *= kScale;
+  E /= kScale;
+  for (int i = 0; i < kCells; i++) {
+    const int c = tid + kThreads * i;
+    if (c < kNSC * kScale) G[c] = c / kScale == 10 ? 1.0 : C.g[i];
   }
   __syncthreads();
-  const double umn = sh[0], umx = sh[1], E = sh[2], H = sh[3], lambda = sh[4];
+  double umn = 0.0, umx = 0.0;
+  for (int y = 0; y < kNSC; y++) {
+    const double v = pu[y] ? (double)(y - 10) : 0.0;
+    if (v < umn) umn = v;
+    if (v > umx) umx = v;
+  }
   double K = -1.0;
   if (!(0.0 <= E || lambda <= 0.0 || H <= 0.0)) {
     if (umn == -1.0 && umx == 1.0) {
@@ -401,10 +495,13 @@ __device__ __forceinline__ void stats_one(const cth_dpset& q, int qp, const cth_
       double sigma = 0.0, Pj = 1.0;
       int minscore = minu, maxscore = maxu;
       for (int j = 1; j <= 32 && 1.0e-4 < Pj; j++) {
-        for (int c = lane; c < kNSC * kScale; c += 64) {
+        double sum = 0.0;
+        for (int ic = 0; ic < kCells; ic++) {
+          const int c = tid + kThreads * ic;
+          if (c >= kNSC * kScale) continue;
           const int y = c / kScale, x = c - y * kScale;
-          double pji = 0.0, pj = 0.0;
-          const int sc = left[y] + x + kSscMin;
+          double pji = 0.0;
+          const int sc = (int)C.sc[ic];
           if (minscore <= sc && sc <= maxscore && -32 <= sc && sc <= 32) {
             const double etols = sc < 0 ? lambda * (double)sc : 0.0;
             if (kLogSpMin < etols) {
@@ -421,21 +518,16 @@ __device__ __forceinline__ void stats_one(const cth_dpset& q, int qp, const cth_
                 }
                 pji += G[yy * kScale + xx] * pu[i + 10];
               }
-              pj = pji * exp(etols);
+              sum += pji * exp(etols);
             }
           }
           NG[c] = pji;
-          PJ[c] = pj;
         }
+        zero = 0.0;
+        block_sum2(sum, zero, red);
+        for (int c = tid; c < kNSC * kScale; c += kThreads) G[c] = NG[c];
         __syncthreads();
-        for (int c = lane; c < kNSC * kScale; c += 64) G[c] = NG[c];
-        if (lane == 0) {
-          double s = 0.0;
-          for (int c = 0; c < kNSC * kScale; c++) s += PJ[c];
-          sh[6] = s;
-        }
-        __syncthreads();
-        Pj = sh[6];
+        Pj = sum;
         sigma += Pj / j;
         minscore += minu;
         maxscore += maxu;
@@ -443,7 +535,7 @@ __device__ __forceinline__ void stats_one(const cth_dpset& q, int qp, const cth_
       K = lambda * exp(-2.0 * sigma) / (H * (1.0 - exp(-lambda)));
     }
   }
-  if (lane == 0) {
+  if (tid == 0) {
     double sig[4];
     significance(ssemodel, q.len[qp], db.len[p], (double)q.eno[qp], (double)db.eno[p], searchspace,
                  (double)r.score, (double)r.psts, lambda, K, sig);
@@ -453,35 +545,38 @@ __device__ __forceinline__ void stats_one(const cth_dpset& q, int qp, const cth_
   }
 }
 
-__global__ __launch_bounds__(64) void k_stats(const cth_dpset q, int qp, const cth_dpset db,
-                                              const int* __restrict__ plist, const int* __restrict__ prel,
-                                              const cth_dpres* __restrict__ dpres,
-                                              const int* __restrict__ hist, double searchspace, int ssemodel,
-                                              double* __restrict__ out) {
+__global__ __launch_bounds__(kThreads) void k_stats(const cth_dpset q, int qp, const cth_dpset db,
+                                                    const int* __restrict__ plist, const int* __restrict__ prel,
+                                                    const cth_dpres* __restrict__ dpres,
+                                                    const int* __restrict__ hist, double searchspace, int ssemodel,
+                                                    double* __restrict__ out) {
   const int k = blockIdx.x;
-  stats_one(q, qp, db, plist[k], hist + (int64_t)k * kNssc, searchspace, ssemodel, dpres[prel[k]],
-            out + (int64_t)k * CTH_STATS_NOUT);
+  stats_one<1>(q, qp, db, plist[k], hist + (int64_t)k * kNssc, searchspace, ssemodel, dpres[prel[k]],
+               out + (int64_t)k * CTH_STATS_NOUT);
 }
 
 // Batched statistics over the *count passed pairs listed in list
-// (persistent, one wavefront per pair at a time): histogram in LDS, then the
+// (persistent, one workgroup per pair at a time): histogram in LDS, then the
 // parameters and significance against the pair's query's search space; out
 // and dpres are per pair.
-__global__ __launch_bounds__(64) void k_stats_batch(const cth_dpset q, const cth_dpset db,
-                                                    const cth_bquery* __restrict__ bq,
-                                                    const cth_bpair* __restrict__ pairs, const int* __restrict__ list,
-                                                    const int* __restrict__ count, int64_t ldsc,
-                                                    const float* __restrict__ scores,
-                                                    const cth_dpres* __restrict__ dpres, int ssemodel,
-                                                    double* __restrict__ out) {
-  __shared__ int h[kNssc];
+__global__ __launch_bounds__(kThreads) void k_stats_batch(const cth_dpset q, const cth_dpset db,
+                                                          const cth_bquery* __restrict__ bq,
+                                                          const cth_bpair* __restrict__ pairs,
+                                                          const int* __restrict__ list, const int* __restrict__ count,
+                                                          int64_t ldsc, const float* __restrict__ scores,
+                                                          const cth_dpres* __restrict__ dpres, int ssemodel,
+                                                          double* __restrict__ out) {
+  __shared__ int h[kNssc * kCopies];
   const int nj = *count;
   for (int k = blockIdx.x; k < nj; k += gridDim.x) {
     const int i = list[k];
     const cth_bpair pr = pairs[i];
     const cth_bquery Q = bq[pr.b];
-    hist_fill(q, Q.qp, db, pr.p, db.dist[pr.p], ldsc, scores + Q.off, h);
-    stats_one(q, Q.qp, db, pr.p, h, Q.sspace, ssemodel, dpres[i], out + (int64_t)i * CTH_STATS_NOUT);
+    for (int b = threadIdx.x; b < kNssc * kCopies; b += kThreads) h[b] = 0;
+    __syncthreads();
+    hist_fill(q, Q.qp, db, pr.p, db.dist[pr.p], ldsc, scores + Q.off, 0, Q.lq, h);
+    __syncthreads();
+    stats_one<kCopies>(q, Q.qp, db, pr.p, h, Q.sspace, ssemodel, dpres[i], out + (int64_t)i * CTH_STATS_NOUT);
     __syncthreads();
   }
 }
@@ -491,29 +586,34 @@ __global__ __launch_bounds__(64) void k_stats_batch(const cth_dpset q, const cth
 // Statistics for the np2 passed profiles listed in plist (indices into the
 // launch's profile range, relative to p0 as the DP results are); hist is
 // scratch of np2*641 ints, out receives np2 x CTH_STATS_NOUT doubles.
-extern "C" int cth_launch_stats(const cth_dpset* q, int qp, const cth_dpset* db, int p0, int64_t col0, int64_t ldsc,
-                                const float* scores, const int* plist_abs, const int* plist_rel,
+extern "C" int cth_launch_stats(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int64_t col0,
+                                int64_t ldsc, const float* scores, const int* plist_abs, const int* plist_rel,
                                 const cth_dpres* dpres, int np2, double searchspace, int ssemodel, int* hist,
                                 double* out, hipStream_t st) {
   if (np2 <= 0) return 0;
   (void)p0;
-  hipLaunchKernelGGL(k_hist, dim3(np2), dim3(256), 0, st, *q, qp, *db, p0, col0, ldsc, scores, plist_abs, hist);
+  // few profiles: their rows over several workgroups each, at least 16 rows
+  // apiece, about four workgroups per compute unit
+  const int split = std::max(1, std::min(1024 / np2, (lq + 15) / 16));
+  const int64_t n = (int64_t)np2 * kNssc;
+  hipLaunchKernelGGL(k_hist_zero, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 1024)), dim3(256), 0, st, hist, n);
+  hipLaunchKernelGGL(k_hist, dim3(np2, split), dim3(kThreads), 0, st, *q, qp, *db, col0, ldsc, scores, plist_abs, hist);
   CTH_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(k_stats, dim3(np2), dim3(64), 0, st, *q, qp, *db, plist_abs, plist_rel, dpres, hist,
+  hipLaunchKernelGGL(k_stats, dim3(np2), dim3(kThreads), 0, st, *q, qp, *db, plist_abs, plist_rel, dpres, hist,
                      searchspace, ssemodel, out);
   CTH_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
 // Batched statistics (k_stats_batch) on a persistent grid of `grid`
-// wavefronts over the *count pairs of list; out: CTH_STATS_NOUT doubles per pair.
+// workgroups over the *count pairs of list; out: CTH_STATS_NOUT doubles per pair.
 extern "C" int cth_launch_stats_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq,
                                       const cth_bpair* pairs, const int* list, const int* count, int64_t ldsc,
                                       const float* scores, const cth_dpres* dpres, int ssemodel, double* out,
                                       int grid, hipStream_t st) {
   if (grid < 1) return 0;
-  hipLaunchKernelGGL(k_stats_batch, dim3(grid), dim3(64), 0, st, *q, *db, bq, pairs, list, count, ldsc, scores, dpres,
-                     ssemodel, out);
+  hipLaunchKernelGGL(k_stats_batch, dim3(grid), dim3(kThreads), 0, st, *q, *db, bq, pairs, list, count, ldsc, scores,
+                     dpres, ssemodel, out);
   CTH_HIP_CHECK(hipGetLastError());
   return 0;
 }
