@@ -45,10 +45,11 @@
 #include "cth_search.h"
 #include "cth_stats.h"
 
-extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, const cth_dpset* db, int ncols,
+extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, const float* qrec, const cth_dpset* db,
+                                      int ncols,
                                       int64_t ldsc, const cth_tables* dtabs, const cth_bytile* ytab, int nytiles,
-                                      const cth_bquery* bq, float* scores, float* mods, int ddms, hipStream_t st);
-extern "C" int cth_score_rows_per_tile(int ddms);
+                                      const cth_bquery* bq, float* scores, float* mods, int ddms, int tile, hipStream_t st);
+extern "C" int cth_score_tile_rows(int ddms, int64_t rows, int64_t ncols);
 extern "C" int cth_launch_dp_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq,
                                    const cth_bpair* pairs, const int* list, const int* count, int n, int* next,
                                    int ltmax, int64_t ldsc, const float* scores, uint8_t* btck, cth_dpres* res,
@@ -188,6 +189,7 @@ struct batch_plan {
   int64_t cells = 0;
   int lqmax = 0;
   int ddms = 1;                     // 0: no cell of the batch has a DDMS term
+  int tile = 0;                     // rows of the score kernel's tiles
 };
 
 // Grids of the persistent launches (workgroups) and wavefronts per pair of
@@ -225,8 +227,8 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
     if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[0], st));
     hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, st, L.ctr);
     CTH_HIP_CHECK(hipGetLastError());
-    if (cth_launch_score_batch(&c->q.d, c->q.ddoff, &db.d, (int)db.d.npos, ldsc, c->dtab, L.ytab, ntiles, L.bq,
-                               L.scores, L.mods, P.ddms, st))
+    if (cth_launch_score_batch(&c->q.d, c->q.ddoff, c->q.qrec, &db.d, (int)db.d.npos, ldsc, c->dtab, L.ytab, ntiles, L.bq,
+                               L.scores, L.mods, P.ddms, P.tile, st))
       return -1;
     if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[1], st));
     if (cth_launch_dp_batch(&c->q.d, &db.d, L.bq, L.pairs, nullptr, nullptr, npairs, L.ctr + kCtrNext1, ltmax, ldsc,
@@ -344,7 +346,7 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
   uint64_t alnused = 0;
   // batch-local index of each query of the current batch (for its hits)
   std::vector<int> local(c->q.d.nprof, -1);
-  const int rows4 = cth_score_rows_per_tile(1);
+  const int rows4 = cth_score_tile_rows(1, 0, 0);
   for (int qa = 0; qa < nq;) {
     // the batch: consecutive entries of the list whose buffers fit the
     // budget together
@@ -393,7 +395,9 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
     P.ddms = 0;
     if (cth_devset_has_ddms(&db, 0, nprof))
       for (int k = P.q0; k < P.q1 && !P.ddms; k++) P.ddms = cth_devset_has_ddms(&c->q, ql[k], ql[k] + 1);
-    const int rows = cth_score_rows_per_tile(P.ddms);
+    int64_t allrows = 0;
+    for (int k = P.q0; k < P.q1; k++) allrows += c->q.h_len[ql[k]];
+    const int rows = P.tile = cth_score_tile_rows(P.ddms, allrows, npos);
     for (int k = P.q0; k < P.q1; k++) {
       const int qi = ql[k];
       local[qi] = k - P.q0;
@@ -486,15 +490,15 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
     // (buffers and their layout, sizes, options, the uploaded sets)
     uint32_t mp;
     memcpy(&mp, &opt->minpp, sizeof mp);
-    uint64_t key[12] = {(uint64_t)(uintptr_t)c->bcells, (uint64_t)(uintptr_t)c->bsmall, (uint64_t)npairs,
-                        (uint64_t)P.ytab.size() | ((uint64_t)P.bq.size() << 32),
+    uint64_t key[14] = {(uint64_t)(uintptr_t)c->bcells, (uint64_t)(uintptr_t)c->bsmall, (uint64_t)npairs,
+                        (uint64_t)P.ytab.size() | ((uint64_t)P.bq.size() << 32), (uint64_t)P.tile,
                         (uint64_t)P.cells, (uint64_t)P.lqmax | ((uint64_t)rowcap << 32),
                         (uint64_t)S.dp_grid | ((uint64_t)S.small_grid << 32),
                         (uint64_t)opt->do_map | ((uint64_t)opt->ssemodel << 8) | ((uint64_t)(alnbytes != 0) << 17) |
                             ((uint64_t)P.ddms << 18) | ((uint64_t)S.dp_waves << 20) |
                             ((uint64_t)S.trace_waves << 24) | ((uint64_t)mp << 32),
                         fnv(&db.d, sizeof db.d), fnv(&c->q.d, sizeof c->q.d),
-                        (uint64_t)(uintptr_t)c->q.ddoff, (uint64_t)(uintptr_t)c->dtab};
+                        (uint64_t)(uintptr_t)c->q.ddoff, (uint64_t)(uintptr_t)c->q.qrec, (uint64_t)(uintptr_t)c->dtab};
     if (timing) {
       // stage events: the launches run eagerly
       if (capture_or_launch(c, P, L, opt, ldsc, ltmax, rowcap, S, false, true)) return -1;

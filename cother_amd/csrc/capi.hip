@@ -151,6 +151,8 @@ extern "C" int cth_ctx_shape(const cth_ctx* c, int* nqueries, const int32_t** ql
   return 0;
 }
 
+extern "C" int cth_make_query_records(const cth_dpset* q, const cth_tables* dtabs, float** rec);
+
 extern "C" int cth_upload_queries(cth_ctx* c, const cth_pset* qs) {
   if (c->borrowed) { cth_set_error("upload on a shared context"); return -1; }
   if (c->nshared > 0) { cth_set_error("upload while %d shared contexts read this one", c->nshared.load()); return -1; }
@@ -158,7 +160,10 @@ extern "C" int cth_upload_queries(cth_ctx* c, const cth_pset* qs) {
   cth_devset_free(&c->q);
   c->has_q = 0;
   if (cth_devset_upload(qs, &c->q)) return -1;
-  if (cth_devset_make_ddoff(qs, &c->q)) { cth_devset_free(&c->q); return -1; }
+  if (cth_devset_make_ddoff(qs, &c->q) || cth_make_query_records(&c->q.d, c->dtab, &c->q.qrec)) {
+    cth_devset_free(&c->q);
+    return -1;
+  }
   c->has_q = 1;
   return 0;
 }
@@ -202,7 +207,7 @@ extern "C" int cth_upload_queries_packed(cth_ctx* c, char* const* pmbeg, char* c
   return rc;
 }
 
-extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, int qp, const cth_dpset* db, int64_t col0, int ncols,
+extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, const float* qrec, int qp, const cth_dpset* db, int64_t col0, int ncols,
                                 int64_t ldsc, const cth_tables* dtabs, int lq, float* scores, float* mods, int contraction,
                                 int ddms, hipStream_t st);
 
@@ -229,7 +234,7 @@ extern "C" int cth_score_block_ex(cth_ctx* c, int qidx, int p0, int p1, int cont
   const size_t need = sizeof(float) * (size_t)lq * ldsc;
   if (cth_ctx_reserve(c, (void**)&c->scores, &c->cap_scores, need)) return -1;
   if (cth_ctx_reserve(c, (void**)&c->mods, &c->cap_mods, need)) return -1;
-  if (cth_launch_score(&c->q.d, c->q.ddoff, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores, c->mods,
+  if (cth_launch_score(&c->q.d, c->q.ddoff, c->q.qrec, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores, c->mods,
                        contraction, ddms_of(c, qidx, p0, p1), c->st))
     return -1;
   CTH_HIP_CHECK(hipStreamSynchronize(c->st));
@@ -271,7 +276,7 @@ extern "C" int cth_phase1_block(cth_ctx* c, int qidx, int p0, int p1, float scor
   if (cth_ctx_reserve(c, (void**)&c->mods, &c->cap_mods, need)) return -1;
   if (cth_ctx_reserve(c, (void**)&c->btck, &c->cap_btck, (size_t)lq * ldsc)) return -1;
   if (cth_ctx_reserve(c, (void**)&c->dpout, &c->cap_dpout, sizeof(cth_dpres) * (size_t)(p1 - p0))) return -1;
-  if (cth_launch_score(&c->q.d, c->q.ddoff, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores + CTH_SCORE_PAD, c->mods, 0,
+  if (cth_launch_score(&c->q.d, c->q.ddoff, c->q.qrec, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores + CTH_SCORE_PAD, c->mods, 0,
                        ddms_of(c, qidx, p0, p1), c->st))
     return -1;
   // boundary rows in global memory for profiles over the LDS row limit
@@ -374,7 +379,7 @@ extern "C" int cth_map_block(cth_ctx* c, int qidx, int p0, int p1, const int32_t
   cth_mapjob* d_jobs = (cth_mapjob*)(d_zrow + (size_t)njobs * lq);
   cth_mapres* d_res = (cth_mapres*)(((uintptr_t)(d_jobs + njobs) + 15) & ~(uintptr_t)15);
   CTH_HIP_CHECK(hipMemcpyAsync(d_jobs, jobs.data(), sizeof(cth_mapjob) * njobs, hipMemcpyHostToDevice, c->st));
-  if (cth_launch_score(&c->q.d, c->q.ddoff, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores + CTH_SCORE_PAD, c->mods + CTH_SCORE_PAD, 0,
+  if (cth_launch_score(&c->q.d, c->q.ddoff, c->q.qrec, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores + CTH_SCORE_PAD, c->mods + CTH_SCORE_PAD, 0,
                        ddms_of(c, qidx, p0, p1), c->st))
     return -1;
   const size_t rows = cth_map_row_bytes(njobs, ltmax);

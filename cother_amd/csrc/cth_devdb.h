@@ -10,6 +10,7 @@ struct cth_devset {
   int64_t* h_dist;    // host copy of profile offsets
   int32_t* ddoff;     // query sets: [npos][128] distance lists as score-table byte offsets
                       // (entry 0 = count, entry k = 22 * 4 * value k), staged by the score kernel
+  float* qrec;        // query sets: [npos][64] records of the plain score kernel (cth_make_query_records)
   int32_t* h_maxdd;   // host: per profile, its longest distance list (values)
 };
 

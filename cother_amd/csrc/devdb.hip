@@ -86,6 +86,7 @@ extern "C" void cth_devset_free(cth_devset* s) {
                   (void*)s->d.cvprior, (void*)s->d.cvnorm2, (void*)s->d.dd})
     if (p) (void)hipFree(p);
   if (s->ddoff) (void)hipFree(s->ddoff);
+  if (s->qrec) (void)hipFree(s->qrec);
   free(s->h_len);
   free(s->h_dist);
   free(s->h_maxdd);

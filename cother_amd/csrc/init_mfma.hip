@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void k_init_mfma(cth_dpset q, int qp, cth_dpse
 #pragma unroll
   for (int r = 0; r < 16; r++) {
     const int row = row0 + wr + 8 * (r >> 2) + kh + (r & 3);
-    if (row < lq) out[(int64_t)row * ldsc + col] = cth_logf(acc[r]) - CTH_INITSHIFT;
+    if (row < lq) out[(int64_t)row * ldsc + col] = cth_logf_dev(acc[r]) - CTH_INITSHIFT;
   }
 }
 

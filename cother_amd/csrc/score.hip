@@ -22,6 +22,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "cth_batch.h"
 #include "cth_dev.h"
 #include "cth_math.h"
@@ -480,16 +483,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 // nothing), with the same per-cell arithmetic as k_score's log-odds, SS and
 // CVS terms.  Without the DDMS scan the cell is a few hundred instructions
 // and k_score's 4-row tiles would re-read each template column's fields per
-// 4 rows; here a workgroup covers kPlainRows query rows (every fourth row
-// per wavefront) of 64 template columns, each lane holding its column's fields
-// in registers.  The workgroup's query rows are staged in LDS, one 48-float
-// record per row, and a wavefront reads its row by broadcast: its values
-// are vector operands (scalar-register operands would keep the FP32
-// arithmetic from dual-issuing) and a row costs no scalar loads or address
-// arithmetic.
-constexpr int kPlainRows = 64;
-constexpr int kQrec = 48;  // floats per staged query row
-constexpr int kQvals = 44; // 20 frequencies, 3 SS, 19 context-vector entries, norm^2, prior
+// 4 rows; here a workgroup covers a tile of query rows (every fourth row per
+// wavefront) of 64 template columns, each lane holding its column in
+// registers: frequencies, denominators and their reciprocals, context vector
+// (128 VGPRs, 4 wavefronts per SIMD).  A row's values are uniform and come by
+// scalar loads from the query's record (k_query_records).
+//
+// Bound by VALU issue: ~205 instructions a row, 39 of them single-rate (a
+// scalar operand keeps an instruction from issuing with another wavefront's).
+// With the rows staged in LDS and the frequencies and context vectors there
+// too, the LDS returned ~250 cycles of data per row and wavefront, four of
+// which share it: 2.7e9 cells took 22.0 ms, this form in 64-row tiles 20.5,
+// in tiles of the whole query 17.9, and with the scalar loads a part ahead
+// 15.2 (4 B + 4 B written per cell: 4.8 ms at the rate of a large copy).
+// Rows of a tile: the whole query up to kPlainRowsMax, so that the column's
+// setup (20 divisions, the loads) is paid once, unless the launch would have
+// fewer than kPlainFill workgroups; then shorter tiles, at least 16 rows.
+constexpr int kPlainRowsMax = 256, kPlainRowsMin = 16, kPlainFill = 2048;
 
 // a factor of a log-odds numerator the quotient correction below admits:
 // +0 or [2^-32, 2], compared on the bit pattern
@@ -498,33 +508,83 @@ __device__ __forceinline__ bool in_quot_range(float v) {
   return b == 0u || b - 0x2F800000u <= 0x10800000u;
 }
 
-// value v (0..kQvals-1) of the staged record of query position qi
-__device__ __forceinline__ float query_value(const cth_dpset& q, int v, int64_t qi) {
-  if (v < CTH_NAA) return q.trg[v * q.ld + qi];
-  if (v < CTH_NAA + CTH_NSS) return q.ss[(v - CTH_NAA) * q.ld + qi];
-  if (v < CTH_NAA + CTH_NSS + CTH_NCV) return q.cv[(v - CTH_NAA - CTH_NSS) * q.ld + qi];
-  return v == kQvals - 2 ? q.cvnorm2[qi] : q.cvprior[qi];
+// A query position's values as the plain kernel reads them
+struct query_record {
+  float trg[CTH_NAA];
+  float cv[CTH_NCV];
+  float normk;         // squared norm + 1 + kappa
+  float prior;
+  float ss[CTH_NSS];
+  float ssh;           // last SS probability + 0.1
+  int32_t ssrow[CTH_NSS];  // rows of the square SS table, as byte offsets
+  int32_t quot;        // frequencies within in_quot_range
+  float pad[64 - CTH_NAA - CTH_NCV - 10];
+};
+static_assert(sizeof(query_record) == 256, "query record");
+// the two parts of a record as scalar loads fetch them
+typedef float sv16 __attribute__((ext_vector_type(16), aligned(4)));
+typedef float sv8 __attribute__((ext_vector_type(8), aligned(4)));
+typedef float sv4 __attribute__((ext_vector_type(4), aligned(4)));
+struct row_trg {
+  sv16 a;
+  sv4 b;
+  __device__ __forceinline__ float at(int k) const { return k < 16 ? a[k] : b[k - 16]; }
+};
+struct row_tail {
+  sv16 a;  // context vector 0..15
+  sv8 b;   // 16..18, normk, prior, ss 0..2
+  sv4 c;   // ssh, ssrow 0..2
+  __device__ __forceinline__ float cv(int k) const { return k < 16 ? a[k] : b[k - 16]; }
+  __device__ __forceinline__ float normk() const { return b[3]; }
+  __device__ __forceinline__ float prior() const { return b[4]; }
+  __device__ __forceinline__ float ss(int k) const { return b[5 + k]; }
+  __device__ __forceinline__ float ssh() const { return c[0]; }
+  __device__ __forceinline__ uint32_t ssrow(int k) const {
+    const float v = c[1 + k];
+    return __builtin_bit_cast(uint32_t, v);
+  }
+};
+static_assert(offsetof(query_record, cv) == 80 && offsetof(query_record, normk) == 156 &&
+                  offsetof(query_record, prior) == 160 && offsetof(query_record, ss) == 164 &&
+                  offsetof(query_record, ssh) == 176 && offsetof(query_record, ssrow) == 180,
+              "query record parts");
+
+__global__ __launch_bounds__(256) void k_query_records(cth_dpset q, const cth_tables* __restrict__ tabs,
+                                                       query_record* __restrict__ rec) {
+  const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (i >= q.npos) return;
+  query_record r;
+  r.quot = 1;
+  for (int a = 0; a < CTH_NAA; a++) {
+    r.trg[a] = q.trg[a * q.ld + i];
+    r.quot &= in_quot_range(r.trg[a]) ? 1 : 0;
+  }
+  for (int k = 0; k < CTH_NCV; k++) r.cv[k] = q.cv[k * q.ld + i];
+  r.normk = q.cvnorm2[i] + 1.0f + tabs->cvkappa0inv;
+  r.prior = q.cvprior[i];
+  for (int k = 0; k < CTH_NSS; k++) {
+    r.ss[k] = q.ss[k * q.ld + i];
+    r.ssrow[k] = (k * 10 + (int)(r.ss[k] * 9.999f)) * 30 * (int)sizeof(float);
+  }
+  r.ssh = r.ss[CTH_NSS - 1] + 0.1f;
+  for (float& v : r.pad) v = 0.0f;
+  rec[i] = r;
 }
 
-template <bool kBatch = false>
-// Five wavefronts per SIMD (at most 96 VGPRs): the template frequencies are
-// read from LDS per row, so that the column's denominators and their
-// reciprocals fit in registers beside the row's values.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_score_plain(
-    cth_dpset q, int qp, cth_dpset db, int64_t col0, int ncols, int64_t ldsc, const cth_tables* __restrict__ tabs,
-    float* __restrict__ scores, float* __restrict__ mods, const cth_bytile* __restrict__ ytab = nullptr,
-    const cth_bquery* __restrict__ bq = nullptr) {
+// kPreInit, kBatch: as k_score's
+template <bool kPreInit, bool kBatch>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_score_plain(
+    cth_dpset q, const query_record* __restrict__ rec, int qp, cth_dpset db, int64_t col0, int ncols, int64_t ldsc,
+    const cth_tables* __restrict__ tabs, float* __restrict__ scores, float* __restrict__ mods, int tile,
+    const cth_bytile* __restrict__ ytab, const cth_bquery* __restrict__ bq) {
   // the SS table square (30 x 30, symmetric: entry r*30+c is ss_lookup(r, c)),
-  // so that a lookup is one index add
+  // so that a lookup is one index add; a row's lookups fall into ten
+  // neighbouring words, so the reads have no bank conflicts
   __shared__ float Lsq[30 * 30];
   __shared__ float Lcv[CTH_CVMAXCARD];
-  __shared__ float4 Ltcv[5][kCols];
-  __shared__ float4 Ltf[5][kCols];
-  __shared__ __align__(16) float Lq[kPlainRows][kQrec];
-  __shared__ int Lbad[kPlainRows];  // a row has a frequency outside in_quot_range
   const int tid = threadIdx.x;
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int row0 = blockIdx.y * kPlainRows;
+  int row0 = blockIdx.y * tile;
   if constexpr (kBatch) {
     const cth_bytile t = ytab[blockIdx.y];
     const cth_bquery Q = bq[t.b];
@@ -533,60 +593,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
     scores += Q.off;
     mods += Q.off;
   }
-  const int lq = q.len[qp];
+  const int row1 = min(q.len[qp], row0 + tile);
   const int64_t q0 = q.dist[qp];
   const int col = blockIdx.x * kCols + lane;
   const bool colin = col < ncols;
   for (int k = tid; k < 30 * 30; k += 256) Lsq[k] = ss_lookup(tabs->ss, k / 30, k % 30);
   for (int k = tid; k < tabs->cvcard; k += 256) Lcv[k] = tabs->cvvals[k];
-  if (tid < kPlainRows) Lbad[tid] = 0;
-  __syncthreads();
-
-  // the query rows, read along the rows (rows past the query's end as zeros)
-  for (int k = tid; k < kPlainRows * kQvals; k += 256) {
-    const int r = k % kPlainRows, v = k / kPlainRows;
-    const float x = row0 + r < lq ? query_value(q, v, q0 + row0 + r) : 0.0f;
-    Lq[r][v] = x;
-    if (v < CTH_NAA && !in_quot_range(x)) Lbad[r] = 1;
-  }
 
   // this lane's template column (lanes past the last column read column 0
   // and leave after the staging): frequencies and the log-odds denominators
   // (CuBatchScoreMatrix_Init.cu:129-144,173-185: 0.5 (bq(a) + bt(a)), per
   // query and template profile), SS probabilities and their table columns,
-  // context vector, its prior and squared norm.  The frequencies and the
-  // context vectors go to LDS, staged by wavefront 0 for the workgroup's 64
-  // columns, four values a lane per 16-byte slot.
+  // context vector, its prior and squared norm.
   const int64_t tj = col0 + (colin ? col : 0);
   const int tp = db.pro[tj];
-  float tf[CTH_NAA], den[CTH_NAA];
-#pragma unroll
-  for (int a = 0; a < CTH_NAA; a++) {
-    tf[a] = db.trg[a * db.ld + tj];
-    den[a] = 0.5f * (q.bkg[qp * CTH_NAA + a] + db.bkg[tp * CTH_NAA + a]);
-  }
-  if (w == 0) {
-#pragma unroll
-    for (int i = 0; i < 5; i++) {
-      float4 v;
-      v.x = db.cv[(4 * i) * db.ld + tj];
-      v.y = db.cv[(4 * i + 1) * db.ld + tj];
-      v.z = db.cv[(4 * i + 2) * db.ld + tj];
-      v.w = 4 * i + 3 < CTH_NCV ? db.cv[(4 * i + 3) * db.ld + tj] : 0.0f;
-      Ltcv[i][lane] = v;
-      Ltf[i][lane] = make_float4(tf[4 * i], tf[4 * i + 1], tf[4 * i + 2], tf[4 * i + 3]);
-    }
-  }
+  const float kap = tabs->cvkappa0inv, cvpow = tabs->cvpowernu0, cvcterm = tabs->cvcterm;
+  const int card = tabs->cvcard, cvshift = tabs->cvshift;
+  const float key0 = tabs->cvkeys[0], key1 = tabs->cvkeys[card - 1];
   float ts[CTH_NSS];
-  int tc[CTH_NSS];
+  uint32_t tc[CTH_NSS];
 #pragma unroll
   for (int j = 0; j < CTH_NSS; j++) {
     ts[j] = db.ss[j * db.ld + tj];
-    tc[j] = j * 10 + (int)(ts[j] * 9.999f);
+    tc[j] = 4u * (uint32_t)(j * 10 + (int)(ts[j] * 9.999f));
   }
-  const float kap = tabs->cvkappa0inv;
+  const float tsh = ts[CTH_NSS - 1] + 0.1f;
   const float tn = db.cvnorm2[tj] + 1.0f + kap;
   const float tprior = db.cvprior[tj];
+  float tcv[CTH_NCV];
+#pragma unroll
+  for (int i = 0; i < CTH_NCV; i++) tcv[i] = db.cv[i * db.ld + tj];
   // The log-odds quotients num / den[a] by Markstein's correction: with
   // y = RN(1 / den) (an IEEE division, once per lane), q0 = RN(num y),
   // r = fma(-den, q0, num) (exact) and q = RN(q0 + r y) equal RN(num / den)
@@ -594,112 +630,173 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
   // 34:111-119, 1990): here when den lies in [2^-30, 2^30] and both factors
   // of num are 0 or in [2^-32, 2].  A wavefront whose columns or query row
   // have an operand outside those ranges divides.
-  float y[CTH_NAA];
-  bool lane_ok = true;
+  float tf[CTH_NAA], den[CTH_NAA], y[CTH_NAA];
+  bool cols_ok = true;
+  if constexpr (!kPreInit) {
+    bool lane_ok = true;
 #pragma unroll
-  for (int a = 0; a < CTH_NAA; a++) {
-    y[a] = 1.0f / den[a];
-    lane_ok &= in_quot_range(tf[a]) && __builtin_bit_cast(uint32_t, den[a]) - 0x30800000u <= 0x1E000000u;
+    for (int a = 0; a < CTH_NAA; a++) {
+      tf[a] = db.trg[a * db.ld + tj];
+      den[a] = 0.5f * (q.bkg[qp * CTH_NAA + a] + db.bkg[tp * CTH_NAA + a]);
+      y[a] = 1.0f / den[a];
+      lane_ok &= in_quot_range(tf[a]) && __builtin_bit_cast(uint32_t, den[a]) - 0x30800000u <= 0x1E000000u;
+    }
+    cols_ok = __builtin_amdgcn_ballot_w64(!lane_ok) == 0;
   }
   __syncthreads();
   if (!colin) return;
-  const bool cols_ok = __builtin_amdgcn_ballot_w64(!lane_ok) == 0;
+  const char* const sq = reinterpret_cast<const char*>(Lsq);
 
-  for (int k = 0; k < kPlainRows / 4; k++) {
-    const int rl = k * 4 + w;  // rows interleaved over the wavefronts: partial tiles stay balanced
-    const int row = row0 + rl;
-    if (row >= lq) break;
-    const float* const R = Lq[rl];
-    // log-odds
-    float tfr[CTH_NAA];
-#pragma unroll
-    for (int i4 = 0; i4 < 5; i4++) {
-      const float4 v = Ltf[i4][lane];
-      tfr[4 * i4] = v.x;
-      tfr[4 * i4 + 1] = v.y;
-      tfr[4 * i4 + 2] = v.z;
-      tfr[4 * i4 + 3] = v.w;
-    }
-    float s = 0.0f;
-    if (cols_ok && __builtin_amdgcn_readfirstlane(Lbad[rl]) == 0) {
-#pragma unroll
-      for (int a = 0; a < CTH_NAA; a++) {
-        const float num = R[a] * tfr[a];
-        const float q0 = num * y[a];
-        s = s + fmaf(fmaf(-den[a], q0, num), y[a], q0);
+  // every row of the tile within the quotient correction's ranges
+  bool quot = cols_ok;
+  for (int r = row0; r < row1; r += 64)
+    quot = quot && __builtin_amdgcn_ballot_w64(r + lane < row1 && rec[q0 + min(r + lane, row1 - 1)].quot == 0) == 0;
+
+  // Rows in straight-line code, interleaved over the wavefronts so that
+  // partial tiles stay balanced.  The row's values are scalar loads issued
+  // well ahead of their use: the second part of its record while its log-odds
+  // are summed, the frequencies of the next row while this one's SS and
+  // context terms are.  The empty asm statements are where each part is
+  // waited for; without them the compiler moves the loads to their uses and
+  // waits four times per row.  The rare cells whose logarithms are not those
+  // of positive normal numbers make the wavefront take them again with the
+  // general function.  kQuot: log-odds by the quotient correction.
+  auto rows = [&](auto kQuot) {
+    int row = row0 + w;
+    if (row >= row1) return;
+    row_trg F{};
+    auto load_trg = [&](int r) {
+      if constexpr (!kPreInit) {
+        const query_record& Q = rec[q0 + r];
+        F.a = *reinterpret_cast<const sv16*>(&Q.trg[0]);
+        F.b = *reinterpret_cast<const sv4*>(&Q.trg[16]);
       }
-    } else {
+    };
+    load_trg(row);
+    if constexpr (!kPreInit) asm volatile("" : "+s"(F.a), "+s"(F.b));
+    for (; row < row1; row += 4) {
+      const query_record& Q = rec[q0 + row];
+      float* const out = scores + row * ldsc + col;
+      row_tail R;
+      R.a = *reinterpret_cast<const sv16*>(&Q.cv[0]);
+      R.b = *reinterpret_cast<const sv8*>(&Q.cv[16]);
+      R.c = *reinterpret_cast<const sv4*>(&Q.ssh);
+      __builtin_amdgcn_sched_barrier(0);
+      float s = 0.0f;
+      if constexpr (kPreInit) {
+        s = *out;
+      } else {
 #pragma unroll
-      for (int a = 0; a < CTH_NAA; a++) s = s + R[a] * tfr[a] / den[a];
-    }
-    s = cth_logf(s) - CTH_INITSHIFT;
-    // SS (CuBatchScoreMatrix_ssss.cuh:64-116)
-    float sss = 0.0f;
-#pragma unroll
-    for (int i = 0; i < CTH_NSS; i++) {
-      const float f1 = R[CTH_NAA + i];
-      const int r30 = (i * 10 + (int)(f1 * 9.999f)) * 30;
-#pragma unroll
-      for (int j = 0; j < CTH_NSS; j++) sss = fmaf(f1 * ts[j], Lsq[r30 + tc[j]], sss);
-    }
-    {
-      const float f1 = R[CTH_NAA + CTH_NSS - 1];
-      if (-99.f < sss) {
-        sss = fmaf((f1 + 0.1f) * (ts[CTH_NSS - 1] + 0.1f), 0.1111111f, sss);
-        sss -= CTH_SSSHIFT;
-        sss *= CTH_SSSWGT;
+        for (int a = 0; a < CTH_NAA; a++) {
+          const float num = F.at(a) * tf[a];
+          if constexpr (kQuot.value) {
+            const float q0 = num * y[a];
+            s = s + fmaf(fmaf(-den[a], q0, num), y[a], q0);
+          } else {
+            s = s + num / den[a];
+          }
+        }
       }
-    }
-    // CVS (CuBatchScoreMatrix_cvs2s.cuh:80-113)
-    float cvs = 0.0f;
+      asm volatile("" : "+s"(R.a), "+s"(R.b), "+s"(R.c));
+      load_trg(min(row + 4, row1 - 1));
+      __builtin_amdgcn_sched_barrier(0);
+      // SS (CuBatchScoreMatrix_ssss.cuh:64-116)
+      float sss = 0.0f;
 #pragma unroll
-    for (int i4 = 0; i4 < 5; i4++) {
-      const float4 v = Ltcv[i4][lane];
-      const float* const c = R + CTH_NAA + CTH_NSS + 4 * i4;
-      cvs = fmaf(c[0], v.x, cvs);
-      cvs = fmaf(c[1], v.y, cvs);
-      cvs = fmaf(c[2], v.z, cvs);
-      if (4 * i4 + 3 < CTH_NCV) cvs = fmaf(c[3], v.w, cvs);
+      for (int i = 0; i < CTH_NSS; i++) {
+#pragma unroll
+        for (int j = 0; j < CTH_NSS; j++)
+          sss = fmaf(R.ss(i) * ts[j], *reinterpret_cast<const float*>(sq + (R.ssrow(i) + tc[j])), sss);
+      }
+      {
+        float v = fmaf(R.ssh() * tsh, 0.1111111f, sss);
+        v -= CTH_SSSHIFT;
+        v *= CTH_SSSWGT;
+        sss = -99.f < sss ? v : sss;
+      }
+      // CVS (CuBatchScoreMatrix_cvs2s.cuh:80-113)
+      float cvs = 0.0f;
+#pragma unroll
+      for (int i = 0; i < CTH_NCV; i++) cvs = fmaf(R.cv(i), tcv[i], cvs);
+      cvs += kap;
+      cvs = fmaf(-cvs, cvs, R.normk() * tn);
+      const float prior = R.prior();
+      if constexpr (!kPreInit) asm volatile("" : "+s"(F.a), "+s"(F.b));
+      const bool odd = !cth_logf_ordinary(cvs) || (!kPreInit && !cth_logf_ordinary(s));
+      float lc = cth_logf_core(cvs);
+      float ls = kPreInit ? 0.0f : cth_logf_core(s);
+      if (__builtin_amdgcn_ballot_w64(odd) != 0) {
+        lc = cth_logf(cvs);
+        if (!kPreInit) ls = cth_logf(s);
+      }
+      if (!kPreInit) s = ls - CTH_INITSHIFT;
+      cvs = fmaf(cvpow, lc, cvcterm) - prior - tprior;
+      int at = cvshift + (int)rintf(2.0f * cvs);
+      at = key1 <= cvs ? card - 1 : at;
+      at = cvs <= key0 ? 0 : at;
+      cvs = Lcv[at] * CTH_CVSWGT;
+      const float sc = sss + cvs;
+      *out = s + sc;
+      mods[row * ldsc + col] = fmaf(-CTH_CVSSHIFT, CTH_CVSWGT, sc);
     }
-    cvs += kap;
-    {
-      const float a = (R[kQvals - 2] + 1.0f + kap) * tn;
-      cvs = fmaf(-cvs, cvs, a);
-      cvs = fmaf(tabs->cvpowernu0, cth_logf(cvs), tabs->cvcterm) - R[kQvals - 1] - tprior;
-      const int card = tabs->cvcard;
-      float v;
-      if (cvs <= tabs->cvkeys[0]) v = Lcv[0];
-      else if (tabs->cvkeys[card - 1] <= cvs) v = Lcv[card - 1];
-      else v = Lcv[tabs->cvshift + (int)rintf(2.0f * cvs)];
-      cvs = v * CTH_CVSWGT;
-    }
-    const float sc = sss + cvs;
-    s = s + sc;
-    scores[row * ldsc + col] = s;
-    mods[row * ldsc + col] = fmaf(-CTH_CVSSHIFT, CTH_CVSWGT, sc);
+  };
+  if (quot) rows(std::true_type{});
+  else rows(std::false_type{});
+}
+
+__global__ void k_selftest_logf(int* bad) {
+  // every significand at a few exponents, with lanes of one exponent together
+  const uint32_t m = blockIdx.x * 256 + threadIdx.x;
+  const int exps[] = {1, 64, 126, 127, 128, 200, 254};
+  for (int e : exps) {
+    const float x = __builtin_bit_cast(float, (uint32_t)e << 23 | m);
+    if (__builtin_bit_cast(uint32_t, cth_logf_dev(x)) != __builtin_bit_cast(uint32_t, cth_logf(x))) atomicAdd(bad, 1);
   }
+  // arguments outside the fast path, alone and beside ordinary ones
+  const uint32_t odd[] = {0u, 1u, 0x007fffffu, 0x7f800000u, 0x80000000u, 0xbf800000u, 0x3f800000u | m};
+  const float x = __builtin_bit_cast(float, odd[m % 7]);
+  if (__builtin_bit_cast(uint32_t, cth_logf_dev(x)) != __builtin_bit_cast(uint32_t, cth_logf(x))) atomicAdd(bad, 1);
 }
 
 }  // namespace
+
+// rows of one tile of the score kernel (ddms 0: of k_score_plain) where it
+// runs over `rows` query rows (all queries of a batch) and ncols columns
+extern "C" int cth_score_tile_rows(int ddms, int64_t rows, int64_t ncols) {
+  if (ddms) return kRows;
+  const int64_t cols = (ncols + kCols - 1) / kCols;
+  const int64_t fit = rows * cols / kPlainFill;  // rows per tile that leave kPlainFill workgroups
+  return (int)std::max<int64_t>(kPlainRowsMin, std::min<int64_t>({(rows + 3) / 4 * 4, fit / 4 * 4, kPlainRowsMax}));
+}
 
 // Launch the score stage for query profile qp against template positions
 // [col0, col0+ncols) of db; outputs are [Lq][ldsc].
 // contraction 0: the FP32 log-odds term of the reference; 1 / 2: the term
 // from the BF16 / FP16 matrix-core product (init_mfma.hip) first.  ddms 0:
 // no cell can have a DDMS term (the query's or every template's lists are
-// shorter than DSTSEGM), so the FP32 stage runs k_score_plain.
+// shorter than DSTSEGM), so k_score_plain runs.  qrec: the query set's
+// records (cth_make_query_records).
 extern "C" int cth_launch_init_mfma(const cth_dpset* q, int qp, const cth_dpset* db, int64_t col0, int ncols,
                                     int64_t ldsc, int lq, int prec, float* out, hipStream_t st);
-extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, int qp, const cth_dpset* db, int64_t col0,
+extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, const float* qrec, int qp, const cth_dpset* db, int64_t col0,
                                 int ncols, int64_t ldsc, const cth_tables* dtabs, int lq, float* scores, float* mods,
                                 int contraction, int ddms, hipStream_t st) {
   if (ncols <= 0 || lq <= 0) return 0;
   if (!qoff) { cth_set_error("score: query distance offsets not built"); return -1; }
   if (ldsc < ncols) { cth_set_error("score: ldsc %lld < ncols %d", (long long)ldsc, ncols); return -1; }
-  if (!ddms && !contraction) {
-    dim3 pgrid((ncols + kCols - 1) / kCols, (lq + kPlainRows - 1) / kPlainRows);
-    hipLaunchKernelGGL(k_score_plain<false>, pgrid, dim3(256), 0, st, *q, qp, *db, col0, ncols, ldsc, dtabs, scores,
-                       mods);
+  if (!ddms) {
+    if (!qrec) { cth_set_error("score: query records not built"); return -1; }
+    const query_record* const rec = reinterpret_cast<const query_record*>(qrec);
+    const int tile = cth_score_tile_rows(0, lq, ncols);
+    const dim3 pgrid((ncols + kCols - 1) / kCols, (lq + tile - 1) / tile);
+    if (contraction) {
+      if (cth_launch_init_mfma(q, qp, db, col0, ncols, ldsc, lq, contraction, scores, st)) return -1;
+      hipLaunchKernelGGL((k_score_plain<true, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
+                         dtabs, scores, mods, tile, nullptr, nullptr);
+    } else {
+      hipLaunchKernelGGL((k_score_plain<false, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
+                         dtabs, scores, mods, tile, nullptr, nullptr);
+    }
     CTH_HIP_CHECK(hipGetLastError());
     return 0;
   }
@@ -716,21 +813,24 @@ extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, int qp,
 }
 
 // The score stage of a batch of queries in one launch: nytiles row tiles
-// (ytab: query of the batch and first row, cth_score_rows_per_tile(ddms)
-// rows each) against the whole resident database (ncols positions from
+// (ytab: query of the batch and first row, `tile` rows each, as
+// cth_score_tile_rows gives them) against the whole resident database (ncols positions from
 // column 0); each query's scores and modular scores at its offset
 // (bq[].off, row stride ldsc); ddms 0 as in cth_launch_score.
-extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, const cth_dpset* db, int ncols,
+extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, const float* qrec, const cth_dpset* db,
+                                      int ncols,
                                       int64_t ldsc, const cth_tables* dtabs, const cth_bytile* ytab, int nytiles,
-                                      const cth_bquery* bq, float* scores, float* mods, int ddms, hipStream_t st) {
+                                      const cth_bquery* bq, float* scores, float* mods, int ddms, int tile, hipStream_t st) {
   if (ncols <= 0 || nytiles <= 0) return 0;
   if (!qoff) { cth_set_error("score batch: query distance offsets not built"); return -1; }
   if (ldsc < ncols) { cth_set_error("score batch: ldsc %lld < ncols %d", (long long)ldsc, ncols); return -1; }
   if (nytiles > 65535) { cth_set_error("score batch: %d row tiles (at most 65535)", nytiles); return -1; }
   dim3 grid((ncols + kCols - 1) / kCols, nytiles);
+  if (!ddms && !qrec) { cth_set_error("score batch: query records not built"); return -1; }
   if (!ddms)
-    hipLaunchKernelGGL((k_score_plain<true>), grid, dim3(256), 0, st, *q, 0, *db, (int64_t)0, ncols, ldsc, dtabs,
-                       scores, mods, ytab, bq);
+    hipLaunchKernelGGL((k_score_plain<false, true>), grid, dim3(256), 0, st, *q,
+                       reinterpret_cast<const query_record*>(qrec), 0, *db, (int64_t)0, ncols, ldsc, dtabs, scores,
+                       mods, tile, ytab, bq);
   else
     hipLaunchKernelGGL((k_score<false, true>), grid, dim3(256), 0, st, *q, 0, *db, (int64_t)0, ncols, ldsc, dtabs,
                        scores, mods, qoff, ytab, bq);
@@ -738,5 +838,28 @@ extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, c
   return 0;
 }
 
-// rows of one tile of the score kernel (ddms 0: of k_score_plain)
-extern "C" int cth_score_rows_per_tile(int ddms) { return ddms ? kRows : kPlainRows; }
+// The records of an uploaded query set that the plain kernel reads (256 bytes
+// per position), allocated here.
+extern "C" int cth_make_query_records(const cth_dpset* q, const cth_tables* dtabs, float** rec) {
+  *rec = nullptr;
+  const int64_t n = q->npos > 0 ? q->npos : 1;
+  CTH_HIP_CHECK(hipMalloc((void**)rec, (size_t)n * sizeof(query_record)));
+  hipLaunchKernelGGL(k_query_records, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, *q, dtabs,
+                     reinterpret_cast<query_record*>(*rec));
+  CTH_HIP_CHECK(hipGetLastError());
+  CTH_HIP_CHECK(hipStreamSynchronize(0));
+  return 0;
+}
+
+// Device check of cth_logf_dev against cth_logf over all significands:
+// *bad = number of differing results (0 expected).
+extern "C" int cth_selftest_logf(int* bad) {
+  int* d = nullptr;
+  CTH_HIP_CHECK(hipMalloc((void**)&d, sizeof(int)));
+  CTH_HIP_CHECK(hipMemset(d, 0, sizeof(int)));
+  hipLaunchKernelGGL(k_selftest_logf, dim3((1 << 23) / 256), dim3(256), 0, 0, d);
+  const bool ok = hipGetLastError() == hipSuccess && hipMemcpy(bad, d, sizeof(int), hipMemcpyDeviceToHost) == hipSuccess;
+  (void)hipFree(d);
+  if (!ok) { cth_set_error("selftest_logf: launch or copy failed"); return -1; }
+  return 0;
+}

@@ -31,7 +31,7 @@
 #include "cth_search.h"
 #include "cth_stats.h"
 
-extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, int qp, const cth_dpset* db, int64_t col0, int ncols,
+extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, const float* qrec, int qp, const cth_dpset* db, int64_t col0, int ncols,
                                 int64_t ldsc, const cth_tables* dtabs, int lq, float* scores, float* mods, int contraction,
                                 int ddms, hipStream_t st);
 extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, const int* plist, int np,
@@ -343,7 +343,7 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
       // no DDMS term anywhere in the chunk when the query's or every template's
       // distance lists are shorter than DSTSEGM
       const int ddms = cth_devset_has_ddms(&c->q, qi, qi + 1) && cth_devset_has_ddms(&db, p0, p1);
-      if (cth_launch_score(&c->q.d, c->q.ddoff, qi, &db.d, col0, (int)ncols, ldsc, c->dtab, lq, scores, mods,
+      if (cth_launch_score(&c->q.d, c->q.ddoff, c->q.qrec, qi, &db.d, col0, (int)ncols, ldsc, c->dtab, lq, scores, mods,
                            opt->contraction, ddms, c->st))
         return -1;
       if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[1], c->st));
