@@ -14,10 +14,14 @@
 // distance list is uniform across a wavefront and each lane walks its own
 // template list.  The 64 template lists (132-byte padded rows, conflict-free
 // byte reads) and the 22x22 pair-score table with its halved copy are staged
-// in LDS; a wavefront's query list is read by scalar loads, as pair-table
-// byte offsets.  The per-cell DDMS dynamic programme (the dominant cost,
-// ~2200 cell updates per score cell for full lists) runs from LDS, scalar
-// registers and vector registers.
+// in LDS with each wavefront's query list, as pair-table byte offsets.  The
+// per-cell DDMS dynamic programme (the dominant cost, ~2200 cell updates per
+// score cell for full lists) runs from LDS and vector registers.  It is bound
+// by VALU issue: by the counters 25,300 instructions a wavefront in 14,700
+// issue slots (11,100 instructions as the second of a pair), which fill its
+// time (8 wavefronts a SIMD).  233 Mcells of full lists: 97.8 ms with doubled sums (5 VALU a
+// cell with one move more) and a register updated by selects and branches,
+// 92.8 ms as it is.
 #include <float.h>
 
 #include <hip/hip_runtime.h>
@@ -35,13 +39,14 @@ constexpr int kRows = 4;        // query rows per workgroup (one per wavefront)
 constexpr int kCols = 64;       // template columns per workgroup (one per lane)
 constexpr int kListPitch = 132; // LDS bytes per template list
 
+constexpr float kSumScale = 0x1p-6f;  // of the distance-match sums (a segment's stays below 1)
 constexpr int kQlEntries = 112;  // query record entries the DDMS scan reads (0..111)
 
 struct ScoreLds {
   uint8_t tl[kCols * kListPitch];  // template lists, values scaled by 4 (table byte columns)
   int32_t ql[kRows][kQlEntries];   // each wavefront's query list as table byte offsets
-  float dms[22 * 22];
-  float dmsh[22 * 22];  // the pair scores halved (exact), right after dms
+  float dms[22 * 22];   // the pair scores times kSumScale
+  float dmsh[22 * 22];  // and halved (both exact), right after dms
   float ss[467];
   float cvvals[CTH_CVMAXCARD];
 };
@@ -70,62 +75,78 @@ constexpr uint32_t kMagic = 0x4b000000u;  // the bits of 2^23
 // entries that intersect nothing: begins 255, ends 0
 constexpr uint32_t kNoBeginN = kEndBias - (kMagic + 0x0007f8ffu), kNoEnd = kMagic + kEndBias;
 
-// whether segment s (begin sb, end se) intersects register entry c (nb, ce):
-// on the query or the template axis the byte-wise max of the begins is <=
-// the min of the ends (CuBatchScoreMatrix_ddms2s.cuh:141-153), i.e. (begin
-// <= end within each segment) ce >= sb and se >= cb
-__device__ __forceinline__ bool meets(uint32_t sb, uint32_t se, uint32_t nb, uint32_t ce) {
+// the AND that is zero when segment s (begin sb, end se) does not intersect
+// register entry c (nb, ce): on the query or the template axis the byte-wise
+// max of the begins is <= the min of the ends
+// (CuBatchScoreMatrix_ddms2s.cuh:141-153), i.e. (begin <= end within each
+// segment) ce >= sb and se >= cb
+__device__ __forceinline__ uint32_t overlap(uint32_t sb, uint32_t se, uint32_t nb, uint32_t ce) {
   // the three-input and as one instruction (left to itself the compiler
   // shares (ce - sb) & kEndBias between tests at the cost of an extra and)
-  return __builtin_amdgcn_bitop3_b32(ce - sb, se + nb, kEndBias, 0x80) != 0u;
+  return __builtin_amdgcn_bitop3_b32(ce - sb, se + nb, kEndBias, 0x80);
 }
 
-// RegisterMaxDDMScore (CuBatchScoreMatrix_ddms2s.cuh:168-261): keep the
-// three best segment scores m0 >= m1 >= m2 whose coordinates do not
-// intersect.  Called only for s >= max(m2, FLT_MIN).  The reference's three
-// cases, as selects on the two intersection tests with the current m0 and m1:
-//  s >= m0: s becomes m0; the old m0 stays (as m1) unless it intersects s,
-//           the old m1 stays (next) unless it intersects s, the old m2 drops;
+// Lane masks of the comparisons of the scan: as masks each comparison is made
+// once (as booleans the compiler repeats those whose negation is also used)
+// and their combinations are scalar.
+__device__ __forceinline__ uint64_t mask_ge(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 3); }
+__device__ __forceinline__ uint64_t mask_zero(uint32_t a) { return __builtin_amdgcn_uicmp(a, 0u, 32); }
+__device__ __forceinline__ bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// The three best segment scores m0 >= m1 >= m2 whose coordinates do not
+// intersect, m0's and m1's with their coordinates.  An empty entry holds
+// FLT_MIN: every comparison with a segment's sum (at least 2^-99) falls as
+// with 0, and in the final sum it vanishes beside a sum or the intercept.
+struct ddms_register {
+  float m0, m1, m2;
+  uint32_t nb0, ce0, nb1, ce1;
+};
+// RegisterMaxDDMScore (CuBatchScoreMatrix_ddms2s.cuh:168-261) for the lanes
+// whose segment s >= m2 (begin sb, end se) changes the register; masks: ge0
+// s >= m0, ge1 s >= m1, n0 and n1 s does not intersect m0, m1.  The
+// reference's three cases:
+//  s >= m0: s becomes m0; the old m0 becomes m1 and the old m1 m2 (dropped if
+//           it intersects s), unless the old m0 intersects s: then it drops,
+//           the old m1 stays m1 unless it intersects s, and m2 is empty;
 //  m1 <= s < m0, s not intersecting m0: s becomes m1, the old m1 becomes m2
 //           unless it intersects s;
 //  m2 <= s < m1, s intersecting neither m0 nor m1: s becomes m2.
-// Only m0's and m1's coordinates are ever tested, so m2's are not kept.  An
-// entry whose value is 0 may keep stale coordinates: every intersection test
-// with it only decides between two zeros, and no segment intersects the
-// initial entries (kNoBeginN, kNoEnd).  lt0: s < m0; i0, i1: whether s
-// intersects the current m0, m1.  The register changes only if
-// register_changes(); register_max is called only then.
-__device__ __forceinline__ bool register_changes(bool lt0, float m1, float s, bool i0, bool i1) {
-  return !lt0 | (!i0 & ((m1 <= s) | !i1));
-}
-__device__ __forceinline__ void register_max(float& m0, float& m1, float& m2, uint32_t& nb0, uint32_t& e0,
-                                             uint32_t& nb1, uint32_t& e1, float s, bool lt0, uint32_t sb,
-                                             uint32_t se, bool i0, bool i1) {
-  // one block per case, so that a wavefront runs only the cases its lanes
-  // have (most often only the first: the best segment growing)
-  if (!lt0) {
-    // s becomes m0
-    const float ym1 = i1 ? 0.0f : m1;
-    m2 = i0 ? 0.0f : ym1;
-    m1 = i0 ? ym1 : m0;
-    nb1 = i0 ? nb1 : nb0;
-    e1 = i0 ? e1 : e0;
-    m0 = s;
-    nb0 = kEndBias - sb;
-    e0 = se + kEndBias;
-    // new values rather than the candidate's registers, so that the join
-    // keeps m0 and its coordinates where they live without copies
-    asm("" : "+v"(m0), "+v"(nb0), "+v"(e0));
-  } else if (m1 <= s) {
-    // s becomes m1 (s does not intersect m0 when the register changes)
-    m2 = i1 ? 0.0f : m1;
-    m1 = s;
-    nb1 = kEndBias - sb;
-    e1 = se + kEndBias;
-  } else {
-    // s becomes m2 (s intersects neither m0 nor m1 when the register changes)
-    m2 = s;
-  }
+// So where s >= m0 the two change places, and what is left is inserted at m1
+// or not.  Only m0's and m1's coordinates are ever tested, so m2's are not
+// kept; an empty entry may keep stale coordinates (a test with it only
+// decides between two empty values), and no segment intersects the initial
+// ones (kNoBeginN, kNoEnd).
+//
+// One asm block whose assignments choose their lanes by exec: a move per
+// value where selects take up to two conditional moves, and no branches (a
+// branch around each case's few moves costs more than the moves).
+__device__ __forceinline__ void register_max(ddms_register& R, float s, uint32_t sb, uint32_t se, uint64_t ge0,
+                                             uint64_t ge1, uint64_t n0, uint64_t n1) {
+  uint32_t nb = kEndBias - sb, ce = se + kEndBias;
+  const float rest = in_mask(n1) ? R.m1 : FLT_MIN;
+  const uint64_t insert = (ge0 & n0) | (~ge0 & ge1), self = ge0 & ~n0, low = ~(ge0 | ge1);
+  uint64_t all;
+  asm volatile(
+      "s_mov_b64 %[all], exec\n\t"
+      "s_and_b64 exec, %[all], %[ge0]\n\t"
+      "v_swap_b32 %[s], %[m0]\n\t"
+      "v_swap_b32 %[nb], %[nb0]\n\t"
+      "v_swap_b32 %[ce], %[ce0]\n\t"
+      "s_and_b64 exec, %[all], %[insert]\n\t"
+      "v_mov_b32 %[m2], %[rest]\n\t"
+      "v_mov_b32 %[m1], %[s]\n\t"
+      "v_mov_b32 %[nb1], %[nb]\n\t"
+      "v_mov_b32 %[ce1], %[ce]\n\t"
+      "s_and_b64 exec, %[all], %[self]\n\t"
+      "v_mov_b32 %[m1], %[rest]\n\t"
+      "v_mov_b32 %[m2], 0x00800000\n\t"
+      "s_and_b64 exec, %[all], %[low]\n\t"
+      "v_mov_b32 %[m2], %[s]\n\t"
+      "s_mov_b64 exec, %[all]"
+      : [all] "=&s"(all), [s] "+v"(s), [nb] "+v"(nb), [ce] "+v"(ce), [m0] "+v"(R.m0), [m1] "+v"(R.m1),
+        [m2] "+v"(R.m2), [nb0] "+v"(R.nb0), [ce0] "+v"(R.ce0), [nb1] "+v"(R.nb1), [ce1] "+v"(R.ce1)
+      : [rest] "v"(rest), [ge0] "s"(ge0), [insert] "s"(insert), [self] "s"(self), [low] "s"(low)
+      : "scc");
 }
 
 // CalcDDMS2ScoreSMEMh2<2,true,2> (cusco/CuBatchScoreMatrix_ddms2s_h2.cuh:435-500):
@@ -134,39 +155,33 @@ __device__ __forceinline__ void register_max(float& m0, float& m1, float& m2, ui
 // are exact pair scores and cells 1 and 3 their means; per 4-cell step the
 // best qualifying segment (length >= DSTSEGM) goes to the top-3 register.
 //
-// The per-cell update in arithmetic that issues on the VALU's second
-// (add/mul) slot: compares, selects and min/max issue one per cycle, plain
-// FP32 adds, multiplies and fmas (source modifiers and clamp included) two.
-// The running sum is kept doubled, u = 2 segsco (exact), so that the next
-// sum is one fma.  Per cell, with x the cell's pair score (or, for the
-// interpolated cells, 0.5 (a + b): the reference's 0.5f * (a + b), exact),
-// dd = the segment's begin minus the cell index (an integer value, <= 0) and
-// big = 2^126:
+// What counts is the number of VALU instructions: the SIMD issues two per
+// slot, of two wavefronts, one of which has to be a plain FP32 add, multiply
+// or fma (source modifiers and clamp included), a u32 add, a logic op or a
+// move.  The sums are kept scaled by 2^-6 (an exact scaling: no value comes
+// near the denormals), which puts every segment's sum below 1 (at most 102
+// cells of at most 0.5), so that one add with the clamp modifier is
+// max(sum + x, 0) with the reference's one rounding.  Per cell, with x the
+// cell's scaled pair score (or, for the interpolated cells, 0.5 (a + b): the
+// reference's 0.5f * (a + b), exact), dd = the segment's begin minus the cell
+// index (an integer value, <= 0) and big = 2^126:
 //   nz   = clamp(u * big)          1 when the previous sum is > 0, else 0
-//                                  (positive sums of pair scores are far
-//                                  above 2^-126)
+//                                  (positive sums are far above 2^-126)
 //   dd   = fma(nz, dd, -nz)        dd - 1, or 0 where the segment restarts
-//   t    = fma(0.5, u, x)          segsco + x with the reference's one
-//                                  rounding (0.5 u is exact)
-//   u    = t + |t|                 2 max(t, 0), exact
+//   u    = clamp(u + x)
 //   cand = u * clamp(-dd - 4)      u if the segment has at least DSTSEGM = 6
 //                                  cells (dd <= -5), else 0
 // and the step's best is the max of its four candidates: the reference takes
 // a cell when its sum exceeds the best so far, i.e. the first cell reaching
 // the max.  The clamp at 0 differs from the reference's select only in the
 // sign of a zero sum, and a zero is never registered.  The top-3 register
-// holds doubled sums too (doubling commutes with every comparison and with
-// the rounding of the final sum, which is halved exactly).  It is entered
-// only when the step's best can displace its smallest entry:
-// scom >= max(m2, FLT_MIN) (positive sums are far above FLT_MIN, so this is
-// scom > 0 && scom >= m2; m2 is finite, so the max is the median of m2,
-// FLT_MIN and FLT_MAX, one instruction).
+// holds scaled sums too (scaling commutes with every comparison and with the
+// rounding of the final sum, which is scaled back exactly).
 #define CTH_DDMS_CELL(X, COUT)                                                \
   {                                                                           \
     const float nz = __builtin_amdgcn_fmed3f(u * big, 0.0f, 1.0f);            \
     dd = fmaf(nz, dd, -nz);                                                   \
-    const float t = fmaf(0.5f, u, X);                                         \
-    u = t + fabsf(t);                                                         \
+    u = __builtin_amdgcn_fmed3f(u + (X), 0.0f, 1.0f);                         \
     COUT = u * __builtin_amdgcn_fmed3f(-dd - 4.0f, 0.0f, 1.0f);               \
   }
 // one 4-cell step, cells K0+1..K0+4 relative to the base ib, with pair
@@ -176,15 +191,15 @@ __device__ __forceinline__ void register_max(float& m0, float& m1, float& m2, ui
 // interpolated sum 0.5f * (a + b) is h(a) + h(b), halving being exact and
 // commuting with the rounding of the sum.  The begin and end of the step's
 // best are recovered only when it can be registered.  Three levels: the
-// step's best is a candidate when it reaches max(m2, FLT_MIN) (m2 is zero
-// most of the time: a growing best segment drops it); a candidate whose
-// segment already meets m0 with its end at the step's first cell and that
-// scores below m0 is dropped after one intersection test, before its end cell
-// is selected (most candidates are of this kind: segments of neighbouring
-// diagonals through the same region); the rest take the full test, and the
-// update runs for a wavefront only when one of its lanes really changes its
-// register.  The empty asm statements keep the candidate's packed words in
-// registers: without them the compiler folds their sums into each test as
+// step's best is a candidate when it reaches m2 (empty most of the time: a
+// growing best segment drops it); a candidate whose segment already meets m0
+// with its end at the step's first cell and that scores below m0 is dropped
+// after one intersection test, before its end cell is selected (most
+// candidates are of this kind: segments of neighbouring diagonals through
+// the same region); the rest take the full test, and the update runs for a
+// wavefront only when one of its lanes really changes its register.  The
+// empty asm statements keep the candidate's packed words in registers:
+// without them the compiler folds their sums into each test as
 // scalar-operand adds, which issue one per cycle.
 #define CTH_DDMS_4CELL(H0, A2, H2, A4, H4, FB)                                \
   {                                                                           \
@@ -195,7 +210,7 @@ __device__ __forceinline__ void register_max(float& m0, float& m1, float& m2, ui
     CTH_DDMS_CELL(H2 + H4, cd3)                                               \
     CTH_DDMS_CELL(A4, cd4)                                                    \
     const float scom = fmaxf(fmaxf(cd1, cd2), fmaxf(cd3, cd4));               \
-    if (scom >= m2f) {                                                        \
+    if (in_mask(mask_ge(scom, R.m2))) {                                       \
       /* the step's first cell on both axes, packed (with kMagic) */          \
       const uint32_t base = __float_as_uint(FB);                              \
       /* begin: the candidate's segment has DSTSEGM or more cells at a cell   \
@@ -206,13 +221,13 @@ __device__ __forceinline__ void register_max(float& m0, float& m1, float& m2, ui
       /* the end lies in cells 1..4 and an intersection, once there, stays as \
          the end grows: a segment that meets m0 ending at cell 1 meets it at  \
          its end, and below m0 it cannot change the register */               \
-      const bool lt0 = scom < m0;                                             \
-      if (!(meets(sb, base, nb0, ce0) && lt0)) {                              \
+      const uint64_t ge0 = mask_ge(scom, R.m0);                               \
+      if (in_mask(ge0 | mask_zero(overlap(sb, base, R.nb0, R.ce0)))) {        \
         /* end: the first of cells 1..4 reaching scom, the cell k + 1 after   \
            the first, as 2^23 + first cell + k (1 + 2^11); n_k = 1 where cell \
-           k is below scom and 0 at scom (scom >= cd_k, and sums of the pair  \
-           scores are multiples of 2^-99, so a difference is 0 or scaled by   \
-           2^100 at least 2), so k = n1 (1 + n2 (1 + n3)):                    \
+           k is below scom and 0 at scom (scom >= cd_k, and the scaled sums   \
+           are multiples of 2^-105, so a difference is 0 or scaled by 2^120   \
+           at least 1), so k = n1 (1 + n2 (1 + n3)):                          \
            fmas that dual-issue, where compares and selects do not */         \
         const float sbig = scom * big2;                                       \
         const float n1 = __builtin_amdgcn_fmed3f(fmaf(cd1, -big2, sbig), 0.0f, 1.0f); \
@@ -220,15 +235,37 @@ __device__ __forceinline__ void register_max(float& m0, float& m1, float& m2, ui
         const float n3 = __builtin_amdgcn_fmed3f(fmaf(cd3, -big2, sbig), 0.0f, 1.0f); \
         uint32_t se = __float_as_uint(fmaf(n1, fmaf(n2, fmaf(n3, packf, packf), packf), FB)); \
         asm("" : "+v"(se));                                                   \
-        const bool i0 = meets(sb, se, nb0, ce0);                              \
-        const bool i1 = meets(sb, se, nb1, ce1);                              \
-        if (register_changes(lt0, m1, scom, i0, i1)) {                        \
-          register_max(m0, m1, m2, nb0, ce0, nb1, ce1, scom, lt0, sb, se, i0, \
-                       i1);                                                   \
-          m2f = __builtin_amdgcn_fmed3f(m2, FLT_MIN, FLT_MAX);                \
-        }                                                                     \
+        const uint64_t free0 = mask_zero(overlap(sb, se, R.nb0, R.ce0));      \
+        const uint64_t free1 = mask_zero(overlap(sb, se, R.nb1, R.ce1));      \
+        const uint64_t ge1 = mask_ge(scom, R.m1);                             \
+        if (in_mask(ge0 | (free0 & (ge1 | free1))))                           \
+          register_max(R, scom, sb, se, ge0, ge1, free0, free1);              \
       }                                                                       \
     }                                                                         \
+  }
+// eight cells (two steps); the pair scores of the step after are loaded one
+// step ahead (lists are padded).  GUARD: whether the second step is due.
+#define CTH_DDMS_8CELL(GUARD)                                                 \
+  {                                                                           \
+    const int q6 = lds_i32(lds, qo + 24), q8 = lds_i32(lds, qo + 32);         \
+    const int t6 = lds_u8(lds, to + 6), t8 = lds_u8(lds, to + 8);             \
+    const float n2 = pair(lds, q6, t6), nh2 = pairh(lds, q6, t6);             \
+    const float n4 = pair(lds, q8, t8), nh4 = pairh(lds, q8, t8);             \
+    CTH_DDMS_4CELL(h0, s2, h2, s4, h4, fb)                                    \
+    const int q10 = lds_i32(lds, qo + 40), q12 = lds_i32(lds, qo + 48);       \
+    const int t10 = lds_u8(lds, to + 10), t12 = lds_u8(lds, to + 12);         \
+    const float p2 = pair(lds, q10, t10), ph2 = pairh(lds, q10, t10);         \
+    const float p4 = pair(lds, q12, t12), ph4 = pairh(lds, q12, t12);         \
+    if (GUARD) CTH_DDMS_4CELL(h4, n2, nh2, n4, nh4, fb + 4.0f * kPackF)       \
+    fb += 8.0f * kPackF;                                                      \
+    qo += 32;                                                                 \
+    to += 8;                                                                  \
+    asm("" : "+v"(qo), "+v"(to));                                             \
+    h0 = nh4;                                                                 \
+    s2 = p2;                                                                  \
+    h2 = ph2;                                                                 \
+    s4 = p4;                                                                  \
+    h4 = ph4;                                                                 \
   }
 
 // The scan reads everything from the workgroup's LDS block by byte offsets
@@ -249,104 +286,59 @@ __device__ __forceinline__ float pairh(const char* lds, int qb, int tv) {
 
 // lds: the workgroup's block; qr: byte offset of the wavefront's query list
 // (int32 table byte offsets, entry 0 = the list length); tr: byte offset of
-// the lane's template list (byte 0 = length, then values times 4)
-__device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr) {
-  const int len1 = lds_i32(lds, qr), len2 = lds_u8(lds, tr);
+// the lane's template list (byte 0 = length, then values times 4); lmin,
+// lmax: the shortest and the longest template list of the wavefront
+__device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int lmin, int lmax) {
+  const int len1 = __builtin_amdgcn_readfirstlane(lds_i32(lds, qr)), len2 = lds_u8(lds, tr);
   if (len1 < CTH_DSTSEGM || len2 < CTH_DSTSEGM) return 0.0f;
-  float m0 = 0.0f, m1 = 0.0f, m2 = 0.0f, m2f = FLT_MIN;
-  uint32_t nb0 = kNoBeginN, ce0 = kNoEnd, nb1 = kNoBeginN, ce1 = kNoEnd;
-  // 2^126, 1 + 2^11 and 2^100 in vector registers: as scalar operands they
+  ddms_register R{FLT_MIN, FLT_MIN, FLT_MIN, kNoBeginN, kNoEnd, kNoBeginN, kNoEnd};
+  // 2^126, 1 + 2^11 and 2^120 in vector registers: as scalar operands they
   // would keep the multiplies and fmas off the second issue slot
   float big, packf, big2;
   asm("v_mov_b32 %0, 0x7e800000" : "=v"(big));
-  asm("v_mov_b32 %0, 0x71800000" : "=v"(big2));  // 2^100
+  asm("v_mov_b32 %0, 0x7b800000" : "=v"(big2));  // 2^120
   asm("v_mov_b32 %0, %1" : "=v"(packf) : "i"(__builtin_bit_cast(uint32_t, kPackF)));
-  // upper part: diagonal j pairs query index i with template index j + i
-  for (int j = len2 >> 2; 0 <= j; j -= 2) {
-    const int iend = min(len1, len2 - j);
-    // byte offsets of query entry 1 and template entry j + 1, advanced by
-    // one iteration (8 entries) at a time in vector registers
-    int qo = qr + 4, to = tr + 1 + j;
+  // the diagonals: upper ones j = len2>>2 .. 0 pair query index i with
+  // template index j + i, lower ones i = len1>>2 .. 1 query index i + j with
+  // template index j
+  const int upper = (lmax >> 3) + 1, lower = ((len1 >> 2) + 1) >> 1;
+  for (int k = 0; k < upper + lower; k++) {
+    const int i = k < upper ? 0 : (len1 >> 2) - 2 * (k - upper);
+    const int j = k < upper ? (len2 >> 2) - 2 * k : 0;
+    if (j < 0) continue;
+    const int n = min(len1 - i, len2 - j);  // cells of the diagonal
+    // cells that every lane's diagonal has (len - (len >> 2) grows with len):
+    // their steps are taken without a test of the lane's end
+    const int full = min(len1 - i, k < upper ? lmin - (lmin >> 2) + 2 * k : lmin);
+    // byte offsets of the diagonal's first query and template entries,
+    // advanced by one iteration (8 entries) at a time in vector registers
+    int qo = qr + 4 * (1 + i), to = tr + 1 + j;
     const float s0 = pair(lds, lds_i32(lds, qo), lds_u8(lds, to));
-    float u = s0 + fabsf(s0);  // 2 max(s0, 0)
+    float u = __builtin_amdgcn_fmed3f(s0, 0.0f, 1.0f);  // max(s0, 0)
     float dd = 0.0f;
-    // 2^23 + the packed coordinates of cell 1 (query 1, template j + 1)
-    float fb = __uint_as_float(kMagic + kPack + ((uint32_t)j << 11));
+    // 2^23 + the packed coordinates of cell 1 (query i + 1, template j + 1)
+    float fb = __uint_as_float(kMagic + kPack + (uint32_t)i + ((uint32_t)j << 11));
     float h0 = pairh(lds, lds_i32(lds, qo), lds_u8(lds, to));
     float s2 = pair(lds, lds_i32(lds, qo + 8), lds_u8(lds, to + 2)),
           h2 = pairh(lds, lds_i32(lds, qo + 8), lds_u8(lds, to + 2));
     float s4 = pair(lds, lds_i32(lds, qo + 16), lds_u8(lds, to + 4)),
           h4 = pairh(lds, lds_i32(lds, qo + 16), lds_u8(lds, to + 4));
-    for (int ib = 0; ib < iend; ib += 8) {
-      // two steps per iteration; the pair scores of the step after are loaded
-      // one step ahead (lists are padded)
-      const int q6 = lds_i32(lds, qo + 24), q8 = lds_i32(lds, qo + 32);
-      const int t6 = lds_u8(lds, to + 6), t8 = lds_u8(lds, to + 8);
-      const float n2 = pair(lds, q6, t6), nh2 = pairh(lds, q6, t6);
-      const float n4 = pair(lds, q8, t8), nh4 = pairh(lds, q8, t8);
-      CTH_DDMS_4CELL(h0, s2, h2, s4, h4, fb)
-      const int q10 = lds_i32(lds, qo + 40), q12 = lds_i32(lds, qo + 48);
-      const int t10 = lds_u8(lds, to + 10), t12 = lds_u8(lds, to + 12);
-      const float p2 = pair(lds, q10, t10), ph2 = pairh(lds, q10, t10);
-      const float p4 = pair(lds, q12, t12), ph4 = pairh(lds, q12, t12);
-      if (ib + 4 < iend) CTH_DDMS_4CELL(h4, n2, nh2, n4, nh4, fb + 4.0f * kPackF)
-      fb += 8.0f * kPackF;
-      qo += 32;
-      to += 8;
-      asm("" : "+v"(qo), "+v"(to));
-      h0 = nh4;
-      s2 = p2;
-      h2 = ph2;
-      s4 = p4;
-      h4 = ph4;
-    }
-  }
-  // lower part: diagonal i pairs query index i + j with template index j
-  for (int i = len1 >> 2; 0 < i; i -= 2) {
-    const int jend = min(len2, len1 - i);
-    int qo = qr + 4 * (1 + i), to = tr + 1;
-    const float s0 = pair(lds, lds_i32(lds, qo), lds_u8(lds, to));
-    float u = s0 + fabsf(s0);  // 2 max(s0, 0)
-    float dd = 0.0f;
-    // 2^23 + the packed coordinates of cell 1 (query i + 1, template 1)
-    float fb = __uint_as_float(kMagic + kPack + (uint32_t)i);
-    float h0 = pairh(lds, lds_i32(lds, qo), lds_u8(lds, to));
-    float s2 = pair(lds, lds_i32(lds, qo + 8), lds_u8(lds, to + 2)),
-          h2 = pairh(lds, lds_i32(lds, qo + 8), lds_u8(lds, to + 2));
-    float s4 = pair(lds, lds_i32(lds, qo + 16), lds_u8(lds, to + 4)),
-          h4 = pairh(lds, lds_i32(lds, qo + 16), lds_u8(lds, to + 4));
-    for (int ib = 0; ib < jend; ib += 8) {
-      const int q6 = lds_i32(lds, qo + 24), q8 = lds_i32(lds, qo + 32);
-      const int t6 = lds_u8(lds, to + 6), t8 = lds_u8(lds, to + 8);
-      const float n2 = pair(lds, q6, t6), nh2 = pairh(lds, q6, t6);
-      const float n4 = pair(lds, q8, t8), nh4 = pairh(lds, q8, t8);
-      CTH_DDMS_4CELL(h0, s2, h2, s4, h4, fb)
-      const int q10 = lds_i32(lds, qo + 40), q12 = lds_i32(lds, qo + 48);
-      const int t10 = lds_u8(lds, to + 10), t12 = lds_u8(lds, to + 12);
-      const float p2 = pair(lds, q10, t10), ph2 = pairh(lds, q10, t10);
-      const float p4 = pair(lds, q12, t12), ph4 = pairh(lds, q12, t12);
-      if (ib + 4 < jend) CTH_DDMS_4CELL(h4, n2, nh2, n4, nh4, fb + 4.0f * kPackF)
-      fb += 8.0f * kPackF;
-      qo += 32;
-      to += 8;
-      asm("" : "+v"(qo), "+v"(to));
-      h0 = nh4;
-      s2 = p2;
-      h2 = ph2;
-      s4 = p4;
-      h4 = ph4;
-    }
+    asm("" : "+v"(qo), "+v"(to));
+    int ib = 0;
+    for (; ib + 4 < full; ib += 8) CTH_DDMS_8CELL(true)
+    for (; ib < n; ib += 8) CTH_DDMS_8CELL(ib + 4 < n)
   }
   float s = 0.0f;
-  s += m0;
-  s += m1;
-  s += m2;
-  s *= 0.5f;  // the register holds doubled sums
+  s += R.m0;
+  s += R.m1;
+  s += R.m2;
+  s *= 1.0f / kSumScale;  // the register holds scaled sums
   s = fmaf(CTH_DDMS_SLOPE * CTH_DDMS_SCALE, s, CTH_DDMS_ICEPT);
   return s * CTH_DDMSWGT;
 }
 #undef CTH_DDMS_CELL
 #undef CTH_DDMS_4CELL
+#undef CTH_DDMS_8CELL
 
 // kPreInit: the log-odds term is already in scores (the reduced-precision
 // contraction of init_mfma.hip); otherwise it is computed here in FP32.
@@ -377,8 +369,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 
   // stage tables
   for (int k = tid; k < 22 * 22; k += 256) {
-    L.dms[k] = tabs->dms[k];
-    L.dmsh[k] = 0.5f * tabs->dms[k];
+    L.dms[k] = kSumScale * tabs->dms[k];
+    L.dmsh[k] = 0.5f * kSumScale * tabs->dms[k];
   }
   for (int k = tid; k < 467; k += 256) L.ss[k] = tabs->ss[k];
   for (int k = tid; k < tabs->cvcard; k += 256) L.cvvals[k] = tabs->cvvals[k];
@@ -401,11 +393,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
     for (int k = lane; k < kQlEntries; k += 64) L.ql[w][k] = qsrc[k];
   }
   __syncthreads();
-  if (row >= lq || col >= ncols) return;
 
   // DDMS first, while nothing else is live
+  int lmin = L.tl[lane * kListPitch], lmax = lmin;
+  if (lmin < CTH_DSTSEGM) lmin = CTH_MAXDST;  // such lanes take no step
+  for (int o = 32; o >= 1; o >>= 1) {
+    lmin = min(lmin, __shfl_xor(lmin, o));
+    lmax = max(lmax, __shfl_xor(lmax, o));
+  }
+  if (row >= lq || col >= ncols) return;
   const float d = ddms_cell(reinterpret_cast<const char*>(&L), (int)offsetof(ScoreLds, ql) + w * kQlEntries * 4,
-                            lane * kListPitch);
+                            lane * kListPitch, __builtin_amdgcn_readfirstlane(lmin),
+                            __builtin_amdgcn_readfirstlane(lmax));
 
   const int64_t qi = q0 + row;
   const int64_t tj = col0 + col;

@@ -187,12 +187,14 @@ extern "C" int cth_tables_load(const char* envdir, cth_tables* t) {
       }
       t->dms[a * 22 + b] = v;
     }
-  // the score kernel's DDMS scan tells a positive running sum from zero, and
-  // two sums apart, by scaling with 2^126 and 2^100 and clamping to [0, 1]:
-  // exact when every nonzero pair score is at least 2^-75 in magnitude (all
-  // sums of such scores and of their halves are then multiples of 2^-99);
-  // these entries are multiples of 2^-48, the smallest nonzero near 2^-25
+  // the score kernel's DDMS scan keeps its sums times 2^-6 and clamps them to
+  // [0, 1]: exact when no pair score exceeds 0.5 (a diagonal has at most 102
+  // cells).  It tells a positive sum from zero, and two sums apart, by
+  // scaling with 2^126 and 2^120 and clamping: exact when every nonzero pair
+  // score is at least 2^-75 in magnitude (all sums of such scores and of
+  // their halves are then multiples of 2^-99, of 2^-105 scaled); these
+  // entries are multiples of 2^-48, the smallest nonzero near 2^-25
   for (float v : t->dms)
-    if (v != 0.0f && fabsf(v) < 0x1p-75f) return 200;
+    if ((v != 0.0f && fabsf(v) < 0x1p-75f) || v > 0.5f) return 200;
   return 0;
 }
