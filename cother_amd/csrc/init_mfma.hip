@@ -11,53 +11,22 @@
 // FP16) and multiplied on the MFMA units with FP32 accumulation, K = 20
 // padded to 32 with zeros; the logarithm stays FP32.  The score kernel then
 // adds the secondary-structure, context-vector and DDMS terms to it
-// unchanged.  The FP32 path (the default) does not use this kernel.
+// unchanged.  Where no cell has a DDMS term the plain score kernel forms the
+// product itself (score.hip); the FP32 path (the default) uses neither.
 //
 // Tile: a workgroup of four wavefronts computes 64 query rows x 64 template
 // columns; each wavefront one 32 x 32 block with two
-// v_mfma_f32_32x32x16 (bf16 / f16) steps over K.  Operand layout of the 32x32x16
-// instruction (lane l, 64 lanes): A holds row l%32, k = 8*(l/32) + 0..7; B
-// holds column l%32, the same k; the 16 accumulators of lane l hold column
-// l%32, rows 8*(r/4) + 4*(l/32) + r%4 for r = 0..15 (checked on the device by
-// cth_selftest_mfma).
+// v_mfma_f32_32x32x16 (bf16 / f16) steps over K.
 #include <hip/hip_runtime.h>
 
 #include "cth_dev.h"
 #include "cth_math.h"
+#include "cth_mfma.h"
 
 namespace {
 
-typedef short v8s __attribute__((ext_vector_type(8)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-
 constexpr int kTile = 64;
 constexpr int kK = 32;
-
-// FP32 -> BF16, round to nearest even (the operands are finite and >= 0)
-__device__ __forceinline__ uint16_t to_bf16(float x) {
-  uint32_t u = __float_as_uint(x);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-
-__device__ __forceinline__ uint16_t to_f16(float x) {
-  const _Float16 h = (_Float16)x;
-  return *reinterpret_cast<const uint16_t*>(&h);
-}
-
-template <int kPrec>  // 1: BF16, 2: FP16; a, b: 8 consecutive k of the lane's row / column
-__device__ __forceinline__ v16f mfma(const uint16_t* a, const uint16_t* b, v16f acc) {
-  const v8s av = *reinterpret_cast<const v8s*>(a);
-  const v8s bv = *reinterpret_cast<const v8s*>(b);
-  if constexpr (kPrec == 1)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, av), __builtin_bit_cast(v8bf, bv), acc,
-                                                   0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, av), __builtin_bit_cast(v8h, bv), acc, 0,
-                                                  0, 0);
-}
 
 template <int kPrec>
 __global__ __launch_bounds__(256) void k_init_mfma(cth_dpset q, int qp, cth_dpset db, int64_t col0, int ncols,
@@ -83,8 +52,8 @@ __global__ __launch_bounds__(256) void k_init_mfma(cth_dpset q, int qp, cth_dpse
         vb = db.trg[k * db.ld + tj] / (0.5f * (bq[k] + db.bkg[tp * CTH_NAA + k]));
       }
     }
-    A[r][k] = kPrec == 1 ? to_bf16(va) : to_f16(va);
-    B[r][k] = kPrec == 1 ? to_bf16(vb) : to_f16(vb);
+    A[r][k] = mfma_operand<kPrec>(va);
+    B[r][k] = mfma_operand<kPrec>(vb);
   }
   __syncthreads();
   const int wr = (w >> 1) * 32, wc = (w & 1) * 32;
@@ -93,7 +62,9 @@ __global__ __launch_bounds__(256) void k_init_mfma(cth_dpset q, int qp, cth_dpse
   const int l32 = lane & 31, kh = (lane >> 5) * 4, ko = (lane >> 5) * 8;
   v16f acc = {};
 #pragma unroll
-  for (int kb = 0; kb < kK; kb += 16) acc = mfma<kPrec>(&A[wr + l32][kb + ko], &B[wc + l32][kb + ko], acc);
+  for (int kb = 0; kb < kK; kb += 16) 
+    acc = mfma<kPrec>(*reinterpret_cast<const v8s*>(&A[wr + l32][kb + ko]),
+                      *reinterpret_cast<const v8s*>(&B[wc + l32][kb + ko]), acc);
   const int col = c0 + wc + l32;
   if (col >= ncols) return;
 #pragma unroll
@@ -112,13 +83,13 @@ template <int kPrec>
 __global__ void k_selftest_mfma(float* out, int h) {
   const int lane = threadIdx.x;
   const int l32 = lane & 31, ko = (lane >> 5) * 8;
-  __align__(16) uint16_t a[8], b[8];
+  v8s a, b;
   for (int k = 0; k < 8; k++) {
     const int kk = ko + k;
     const float av = (l32 == kk) ? 1.0f : 0.0f;
     const float bv = (kk >> 3) == h ? (float)(32 * (kk - 8 * h) + l32) : 0.0f;
-    a[k] = kPrec == 1 ? to_bf16(av) : to_f16(av);
-    b[k] = kPrec == 1 ? to_bf16(bv) : to_f16(bv);
+    a[k] = (short)mfma_operand<kPrec>(av);
+    b[k] = (short)mfma_operand<kPrec>(bv);
   }
   v16f acc = {};
   acc = mfma<kPrec>(a, b, acc);

@@ -32,6 +32,7 @@
 #include "cth_batch.h"
 #include "cth_dev.h"
 #include "cth_math.h"
+#include "cth_mfma.h"
 
 namespace {
 
@@ -498,6 +499,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 // Rows of a tile: the whole query up to kPlainRowsMax, so that the column's
 // setup (20 divisions, the loads) is paid once, unless the launch would have
 // fewer than kPlainFill workgroups; then shorter tiles, at least 16 rows.
+constexpr int kProdPitch = 40;  // of a column's product operands, in entries
 constexpr int kPlainRowsMax = 256, kPlainRowsMin = 16, kPlainFill = 2048;
 
 // a factor of a log-odds numerator the quotient correction below admits:
@@ -570,8 +572,16 @@ __global__ __launch_bounds__(256) void k_query_records(cth_dpset q, const cth_ta
   rec[i] = r;
 }
 
-// kPreInit, kBatch: as k_score's
-template <bool kPreInit, bool kBatch>
+// kBatch: as k_score's.  kPrec 1, 2: the log-odds sum from the BF16 / FP16
+// product on the matrix cores (as k_init_mfma forms it), 0: in FP32.
+//
+// The product's tile is 32 of the wavefront's rows x its 64 columns, two
+// 32 x 32 blocks; it goes through the wavefront's own LDS block to one column
+// per lane.  Against the product by k_init_mfma, whose 64 x 64 tiles divide
+// each column's frequencies again and whose logarithms are written and read
+// back (4 B + 4 B a cell), the score stage of 142 Mcells takes 0.51 ms instead
+// of 0.76.
+template <int kPrec, bool kBatch>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_score_plain(
     cth_dpset q, const query_record* __restrict__ rec, int qp, cth_dpset db, int64_t col0, int ncols, int64_t ldsc,
     const cth_tables* __restrict__ tabs, float* __restrict__ scores, float* __restrict__ mods, int tile,
@@ -581,6 +591,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   // neighbouring words, so the reads have no bank conflicts
   __shared__ float Lsq[30 * 30];
   __shared__ float Lcv[CTH_CVMAXCARD];
+  // the product's column operands (rows of 80 bytes: aligned 16-byte reads,
+  // spread over the banks), then each wavefront's 32 x 64 sums
+  __shared__ __align__(16) float Lp[kPrec ? 4 * 32 * 64 : 1];
   const int tid = threadIdx.x;
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   int row0 = blockIdx.y * tile;
@@ -631,7 +644,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   // have an operand outside those ranges divides.
   float tf[CTH_NAA], den[CTH_NAA], y[CTH_NAA];
   bool cols_ok = true;
-  if constexpr (!kPreInit) {
+  v8s pb[2][2];  // the product's column operands of this lane
+  if constexpr (!kPrec) {
     bool lane_ok = true;
 #pragma unroll
     for (int a = 0; a < CTH_NAA; a++) {
@@ -641,15 +655,56 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
       lane_ok &= in_quot_range(tf[a]) && __builtin_bit_cast(uint32_t, den[a]) - 0x30800000u <= 0x1E000000u;
     }
     cols_ok = __builtin_amdgcn_ballot_w64(!lane_ok) == 0;
+    __syncthreads();
+    if (!colin) return;
+  } else {
+    // each wavefront divides 5 of the 20 frequencies of the 64 columns and
+    // clears 3 of the 12 entries that pad K to 32.  Lanes past the last
+    // column stay: the product takes all 64.
+    uint16_t* const B = reinterpret_cast<uint16_t*>(Lp) + lane * kProdPitch;
+    for (int k = 5 * w; k < 5 * w + 5; k++)
+      B[k] = mfma_operand<kPrec>(db.trg[k * db.ld + tj] /
+                                 (0.5f * (q.bkg[qp * CTH_NAA + k] + db.bkg[tp * CTH_NAA + k])));
+    for (int k = CTH_NAA + 3 * w; k < CTH_NAA + 3 * w + 3; k++) B[k] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+      for (int kb = 0; kb < 2; kb++)
+        pb[c][kb] = *reinterpret_cast<const v8s*>(reinterpret_cast<const uint16_t*>(Lp) +
+                                                  (32 * c + (lane & 31)) * kProdPitch + 16 * kb + 8 * (lane >> 5));
+    __syncthreads();
   }
-  __syncthreads();
-  if (!colin) return;
   const char* const sq = reinterpret_cast<const char*>(Lsq);
 
   // every row of the tile within the quotient correction's ranges
   bool quot = cols_ok;
   for (int r = row0; r < row1; r += 64)
     quot = quot && __builtin_amdgcn_ballot_w64(r + lane < row1 && rec[q0 + min(r + lane, row1 - 1)].quot == 0) == 0;
+
+  // the sums of 32 of the wavefront's rows from `row` on (rows past the tile's
+  // end repeat the last)
+  float* const sums = &Lp[kPrec ? w * 32 * 64 : 0];
+  auto product = [&](int row) {
+    const float* const f = rec[q0 + min(row + 4 * (lane & 31), row1 - 1)].trg;
+    const bool low = lane < 32;
+    v8s a0, a1;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      a0[k] = (short)mfma_operand<kPrec>(f[(low ? 0 : 8) + k]);
+      a1[k] = k < 4 && low ? (short)mfma_operand<kPrec>(f[16 + (k & 3)]) : 0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      v16f acc = {};
+      acc = mfma<kPrec>(a0, pb[c][0], acc);
+      acc = mfma<kPrec>(a1, pb[c][1], acc);
+#pragma unroll
+      for (int r = 0; r < 16; r++) sums[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * 64 + 32 * c + (lane & 31)] = acc[r];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
 
   // Rows in straight-line code, interleaved over the wavefronts so that
   // partial tiles stay balanced.  The row's values are scalar loads issued
@@ -665,15 +720,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     if (row >= row1) return;
     row_trg F{};
     auto load_trg = [&](int r) {
-      if constexpr (!kPreInit) {
+      if constexpr (!kPrec) {
         const query_record& Q = rec[q0 + r];
         F.a = *reinterpret_cast<const sv16*>(&Q.trg[0]);
         F.b = *reinterpret_cast<const sv4*>(&Q.trg[16]);
       }
     };
     load_trg(row);
-    if constexpr (!kPreInit) asm volatile("" : "+s"(F.a), "+s"(F.b));
+    if constexpr (!kPrec) asm volatile("" : "+s"(F.a), "+s"(F.b));
     for (; row < row1; row += 4) {
+      if constexpr (kPrec != 0) {
+        if (((row - row0) & 127) < 4) product(row);
+      }
       const query_record& Q = rec[q0 + row];
       float* const out = scores + row * ldsc + col;
       row_tail R;
@@ -682,8 +740,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
       R.c = *reinterpret_cast<const sv4*>(&Q.ssh);
       __builtin_amdgcn_sched_barrier(0);
       float s = 0.0f;
-      if constexpr (kPreInit) {
-        s = *out;
+      if constexpr (kPrec != 0) {
+        s = sums[((row - row0) >> 2 & 31) * 64 + lane];
       } else {
 #pragma unroll
         for (int a = 0; a < CTH_NAA; a++) {
@@ -720,23 +778,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
       cvs += kap;
       cvs = fmaf(-cvs, cvs, R.normk() * tn);
       const float prior = R.prior();
-      if constexpr (!kPreInit) asm volatile("" : "+s"(F.a), "+s"(F.b));
-      const bool odd = !cth_logf_ordinary(cvs) || (!kPreInit && !cth_logf_ordinary(s));
+      if constexpr (!kPrec) asm volatile("" : "+s"(F.a), "+s"(F.b));
+      const bool odd = !cth_logf_ordinary(cvs) || !cth_logf_ordinary(s);
       float lc = cth_logf_core(cvs);
-      float ls = kPreInit ? 0.0f : cth_logf_core(s);
+      float ls = cth_logf_core(s);
       if (__builtin_amdgcn_ballot_w64(odd) != 0) {
         lc = cth_logf(cvs);
-        if (!kPreInit) ls = cth_logf(s);
+        ls = cth_logf(s);
       }
-      if (!kPreInit) s = ls - CTH_INITSHIFT;
+      s = ls - CTH_INITSHIFT;
       cvs = fmaf(cvpow, lc, cvcterm) - prior - tprior;
       int at = cvshift + (int)rintf(2.0f * cvs);
       at = key1 <= cvs ? card - 1 : at;
       at = cvs <= key0 ? 0 : at;
       cvs = Lcv[at] * CTH_CVSWGT;
       const float sc = sss + cvs;
-      *out = s + sc;
-      mods[row * ldsc + col] = fmaf(-CTH_CVSSHIFT, CTH_CVSWGT, sc);
+      if (!kPrec || colin) {
+        *out = s + sc;
+        mods[row * ldsc + col] = fmaf(-CTH_CVSSHIFT, CTH_CVSWGT, sc);
+      }
     }
   };
   if (quot) rows(std::true_type{});
@@ -771,7 +831,8 @@ extern "C" int cth_score_tile_rows(int ddms, int64_t rows, int64_t ncols) {
 // Launch the score stage for query profile qp against template positions
 // [col0, col0+ncols) of db; outputs are [Lq][ldsc].
 // contraction 0: the FP32 log-odds term of the reference; 1 / 2: the term
-// from the BF16 / FP16 matrix-core product (init_mfma.hip) first.  ddms 0:
+// from the BF16 / FP16 matrix-core product (before k_score by
+// init_mfma.hip, within k_score_plain).  ddms 0:
 // no cell can have a DDMS term (the query's or every template's lists are
 // shorter than DSTSEGM), so k_score_plain runs.  qrec: the query set's
 // records (cth_make_query_records).
@@ -788,12 +849,18 @@ extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, const f
     const query_record* const rec = reinterpret_cast<const query_record*>(qrec);
     const int tile = cth_score_tile_rows(0, lq, ncols);
     const dim3 pgrid((ncols + kCols - 1) / kCols, (lq + tile - 1) / tile);
-    if (contraction) {
-      if (cth_launch_init_mfma(q, qp, db, col0, ncols, ldsc, lq, contraction, scores, st)) return -1;
-      hipLaunchKernelGGL((k_score_plain<true, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
+    if (contraction < 0 || contraction > 2) {
+      cth_set_error("score: contraction %d (0 FP32, 1 BF16, 2 FP16)", contraction);
+      return -1;
+    }
+    if (contraction == 1) {
+      hipLaunchKernelGGL((k_score_plain<1, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
+                         dtabs, scores, mods, tile, nullptr, nullptr);
+    } else if (contraction == 2) {
+      hipLaunchKernelGGL((k_score_plain<2, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
                          dtabs, scores, mods, tile, nullptr, nullptr);
     } else {
-      hipLaunchKernelGGL((k_score_plain<false, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
+      hipLaunchKernelGGL((k_score_plain<0, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
                          dtabs, scores, mods, tile, nullptr, nullptr);
     }
     CTH_HIP_CHECK(hipGetLastError());
@@ -827,7 +894,7 @@ extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, c
   dim3 grid((ncols + kCols - 1) / kCols, nytiles);
   if (!ddms && !qrec) { cth_set_error("score batch: query records not built"); return -1; }
   if (!ddms)
-    hipLaunchKernelGGL((k_score_plain<false, true>), grid, dim3(256), 0, st, *q,
+    hipLaunchKernelGGL((k_score_plain<0, true>), grid, dim3(256), 0, st, *q,
                        reinterpret_cast<const query_record*>(qrec), 0, *db, (int64_t)0, ncols, ldsc, dtabs, scores,
                        mods, tile, ytab, bq);
   else

@@ -52,3 +52,24 @@ def test_contraction_route_equals_the_general_kernel(ctx, contraction):
     n = plain.npos
     for a, b in zip(got["plain"], got["mixed"]):
         assert (a.view(np.int32) == b[:, :n].view(np.int32)).all()
+
+
+@pytest.mark.parametrize("contraction", [1, 2])
+@pytest.mark.parametrize("lq,lts", [(1, (1,)), (5, (63, 2)), (33, (64,)), (128, (65,)), (129, (31, 33)), (300, (7, 90))])
+def test_product_tiles_equal_the_general_kernel(ctx, contraction, lq, lts):
+    """The product within the plain kernel at the edges of its tiles (32 of a
+    wavefront's rows by 64 columns, 256 rows a workgroup) against the product
+    before the general kernel: bit for bit, as both form the same sums."""
+    q = cother_amd.synth(1, 2, lmin=lq, lmax=lq, dist_mode=0, sort_desc=0, seed=1330 + lq)
+    plain = cother_amd.concat([cother_amd.synth(1, 2, lmin=lt, lmax=lt, dist_mode=2, sort_desc=0, seed=1340 + lt)
+                               for lt in lts])
+    mixed = cother_amd.concat([plain, cother_amd.synth(1, 2, lmin=50, lmax=50, dist_mode=1, seed=1341)])
+    set_informative_cv(q, 4)
+    q.field("trg")[:, lq // 2] = 0.0  # a row whose sums are zero
+    ctx.upload_queries(q)
+    ctx.upload_db(plain)
+    got = ctx.score_block(0, 0, plain.nprof, contraction)
+    ctx.upload_db(mixed)
+    want = ctx.score_block(0, 0, mixed.nprof, contraction)
+    for a, b in zip(got, want):
+        assert (a.view(np.int32) == b[:, :plain.npos].view(np.int32)).all()
