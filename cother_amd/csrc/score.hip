@@ -494,8 +494,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 // With the rows staged in LDS and the frequencies and context vectors there
 // too, the LDS returned ~250 cycles of data per row and wavefront, four of
 // which share it: 2.7e9 cells took 22.0 ms, this form in 64-row tiles 20.5,
-// in tiles of the whole query 17.9, and with the scalar loads a part ahead
-// 15.2 (4 B + 4 B written per cell: 4.8 ms at the rate of a large copy).
+// in tiles of the whole query 17.9, with the scalar loads a part ahead 15.2,
+// and with all of a column's and the table's loads under way before the first
+// is waited for 14.2 (4 B + 4 B written per cell: 4.8 ms at the rate of a
+// large copy).  The context-vector products on the matrix cores
+// (v_mfma_f32_16x16x1, the same fma chain bit for bit) take as many VALU
+// instructions for 16 of a wavefront's ~24 rows as they save: 14.9.
 // Rows of a tile: the whole query up to kPlainRowsMax, so that the column's
 // setup (20 divisions, the loads) is paid once, unless the launch would have
 // fewer than kPlainFill workgroups; then shorter tiles, at least 16 rows.
@@ -609,8 +613,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   const int64_t q0 = q.dist[qp];
   const int col = blockIdx.x * kCols + lane;
   const bool colin = col < ncols;
-  for (int k = tid; k < 30 * 30; k += 256) Lsq[k] = ss_lookup(tabs->ss, k / 30, k % 30);
-  for (int k = tid; k < tabs->cvcard; k += 256) Lcv[k] = tabs->cvvals[k];
+  // the tables, stored after the column's loads are on their way
+  float sqv[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const int e = min(tid + 256 * k, 30 * 30 - 1);
+    sqv[k] = ss_lookup(tabs->ss, e / 30, e % 30);
+  }
 
   // this lane's template column (lanes past the last column read column 0
   // and leave after the staging): frequencies and the log-odds denominators
@@ -635,6 +644,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   float tcv[CTH_NCV];
 #pragma unroll
   for (int i = 0; i < CTH_NCV; i++) tcv[i] = db.cv[i * db.ld + tj];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (tid + 256 * k < 30 * 30) Lsq[tid + 256 * k] = sqv[k];
+  for (int k = tid; k < tabs->cvcard; k += 256) Lcv[k] = tabs->cvvals[k];
   // The log-odds quotients num / den[a] by Markstein's correction: with
   // y = RN(1 / den) (an IEEE division, once per lane), q0 = RN(num y),
   // r = fma(-den, q0, num) (exact) and q = RN(q0 + r y) equal RN(num / den)
@@ -646,11 +659,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   bool cols_ok = true;
   v8s pb[2][2];  // the product's column operands of this lane
   if constexpr (!kPrec) {
-    bool lane_ok = true;
+    // all loads first: left to itself the compiler loads an operand and waits
+    // for it 20 times
+    float bt[CTH_NAA], bqa[CTH_NAA];
 #pragma unroll
     for (int a = 0; a < CTH_NAA; a++) {
       tf[a] = db.trg[a * db.ld + tj];
-      den[a] = 0.5f * (q.bkg[qp * CTH_NAA + a] + db.bkg[tp * CTH_NAA + a]);
+      bt[a] = db.bkg[tp * CTH_NAA + a];
+      bqa[a] = q.bkg[qp * CTH_NAA + a];
+    }
+#pragma unroll
+    for (int a = 0; a < CTH_NAA; a++) asm volatile("" : "+v"(tf[a]), "+v"(bt[a]), "+s"(bqa[a]));
+    bool lane_ok = true;
+#pragma unroll
+    for (int a = 0; a < CTH_NAA; a++) {
+      den[a] = 0.5f * (bqa[a] + bt[a]);
       y[a] = 1.0f / den[a];
       lane_ok &= in_quot_range(tf[a]) && __builtin_bit_cast(uint32_t, den[a]) - 0x30800000u <= 0x1E000000u;
     }
