@@ -32,6 +32,7 @@
 #include "cth_dev.h"
 #include "cth_dp.h"
 #include "cth_sweep.h"
+#include "cth_trace.h"
 
 namespace {
 
@@ -480,46 +481,32 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_dp_batch(
   }
 }
 
-// FinalizeDPPro for one profile (lane 0): pass test against scorethld,
+// FinalizeDPPro for one profile, by a wavefront: pass test against scorethld,
 // traceback from the maximum, correlation bonus, signed square root,
-// positive-score count and begin coordinates into r.
+// positive-score count and begin coordinates into r (in every lane).  The
+// bonus takes the path's scores 32 at a time, v[n] (((v[n-4] + v[n-3]) +
+// v[n-2]) + v[n-1]) summed by an xor butterfly.
 __device__ __forceinline__ void dpfin_pair(const cth_dpset& db, int p, int64_t colp, int64_t ldsc, const float* __restrict__ scores,
-                           const uint8_t* __restrict__ btck, float scorethld, cth_dpres& r, float* cache,
-                           float* tree) {
+                           const uint8_t* __restrict__ btck, float scorethld, cth_dpres& r, uint32_t* tile) {
   r.passed = 0; r.score = 0.0f; r.psts = 0; r.beg = 0;
   if (r.maxsc <= scorethld) return;
+  const int lane = threadIdx.x & 63;
   int x = (int)(r.maxxy >> 16), y = (int)(r.maxxy & 0xffff);
   int psts = 0;
-  for (int k = 0; k < 36; k++) cache[k] = 0.0f;
-  float sum = 0.0f;
-  int bt = CTH_BT_DIAG;
-  while (bt != CTH_BT_STOP) {
-    for (int k = 0; k < 4; k++) cache[k] = cache[32 + k];
-    int ndx;
-    for (ndx = 4; ndx < 36;) {
-      if (x < 0 || y < 0) { bt = CTH_BT_STOP; break; }
-      const int64_t a = (int64_t)y * ldsc + colp + x;
-      bt = btck[a];
-      if (bt == CTH_BT_STOP) break;
-      if (bt == CTH_BT_UP) { y--; continue; }
-      if (bt == CTH_BT_LEFT) { x--; continue; }
-      const float v = scores[a];
-      cache[ndx] = v;
-      if (v > 0.0f) psts++;
-      x--; y--;
-      ndx++;
+  float sum = 0.0f, last = 0.0f;  // last: the 32 scores before
+  trace_walk<32, true>(btck + colp, ldsc, x, y, tile, [&](int cnt, int px, int py, int) {
+    const float v = lane < cnt ? scores[(int64_t)py * ldsc + colp + px] : 0.0f;
+    psts += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v > 0.0f));
+    float before[4];
+    for (int j = 1; j <= 4; j++) {
+      const float here = __shfl(v, lane - j & 31), prev = __shfl(last, lane - j & 31);
+      before[j - 1] = lane >= j ? here : prev;
     }
-    for (int l = 0; l < 32; l++)
-      tree[l] = (ndx <= l + 4) ? 0.0f
-                               : cache[l + 4] * (((cache[l] + cache[l + 1]) + cache[l + 2]) + cache[l + 3]);
-    // xor butterfly (offsets 16,8,4,2,1); lane 0's value
-    for (int off = 16; off >= 1; off >>= 1) {
-      float nt[32];
-      for (int l = 0; l < 32; l++) nt[l] = tree[l] + tree[l ^ off];
-      for (int l = 0; l < 32; l++) tree[l] = nt[l];
-    }
-    sum += tree[0];
-  }
+    float t = lane < cnt ? v * (((before[3] + before[2]) + before[1]) + before[0]) : 0.0f;
+    for (int off = 16; off >= 1; off >>= 1) t += __shfl_xor(t, off);
+    sum += __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, t)));
+    last = v;
+  });
   sum *= 0.5f;
   sum = sum < 0.0f ? -sqrtf(-sum) : sqrtf(sum);
   const float score = r.maxsc + sum;
@@ -529,18 +516,16 @@ __device__ __forceinline__ void dpfin_pair(const cth_dpset& db, int p, int64_t c
   r.passed = scorethld < score ? 1 : 0;
 }
 
-// lane 0 of each wavefront finalises one profile
+// one wavefront per profile
 __global__ __launch_bounds__(64) void k_dpfin(cth_dpset db, int pbase, const int* __restrict__ plist, int64_t col0,
                                               int64_t ldsc, const float* __restrict__ scores,
                                               const uint8_t* __restrict__ btck, float scorethld,
                                               cth_dpres* __restrict__ res) {
-  __shared__ float cache[36];
-  __shared__ float tree[32];
-  if (threadIdx.x != 0) return;
+  __shared__ uint32_t tile[kTraceTileBytes / 4];
   const int p = plist ? plist[blockIdx.x] : pbase + blockIdx.x;
   cth_dpres r = res[blockIdx.x];
-  dpfin_pair(db, p, db.dist[p] - col0, ldsc, scores, btck, scorethld, r, cache, tree);
-  res[blockIdx.x] = r;
+  dpfin_pair(db, p, db.dist[p] - col0, ldsc, scores, btck, scorethld, r, tile);
+  if (threadIdx.x == 0) res[blockIdx.x] = r;
 }
 
 // Batched finalisation over the *count pairs listed in list (persistent,
@@ -550,17 +535,15 @@ __global__ __launch_bounds__(64) void k_dpfin_batch(cth_dpset db, const cth_bque
                                                     const int* __restrict__ count, int64_t ldsc,
                                                     const float* __restrict__ scores,
                                                     const uint8_t* __restrict__ btck, cth_dpres* __restrict__ res) {
-  __shared__ float cache[36];
-  __shared__ float tree[32];
-  if (threadIdx.x != 0) return;
+  __shared__ uint32_t tile[kTraceTileBytes / 4];
   const int nj = *count;
   for (int k = blockIdx.x; k < nj; k += gridDim.x) {
     const int i = list[k];
     const cth_bpair pr = pairs[i];
     const cth_bquery Q = bq[pr.b];
     cth_dpres r = res[i];
-    dpfin_pair(db, pr.p, db.dist[pr.p], ldsc, scores + Q.off, btck + Q.off, Q.scorethld, r, cache, tree);
-    res[i] = r;
+    dpfin_pair(db, pr.p, db.dist[pr.p], ldsc, scores + Q.off, btck + Q.off, Q.scorethld, r, tile);
+    if (threadIdx.x == 0) res[i] = r;
   }
 }
 

@@ -41,6 +41,7 @@
 #include "cth_stats.h"
 #include "cth_math.h"
 #include "cth_sweep.h"
+#include "cth_trace.h"
 
 namespace {
 
@@ -48,6 +49,7 @@ constexpr float kLP0 = -99.0f;
 constexpr int NT = CTH_NTRN;
 constexpr int kMaxWaves = 8;
 constexpr int kStage = 32;
+static_assert(kTraceTileBytes <= kRingBytes, "the traceback's tile takes a wavefront's ring");
 
 __device__ __forceinline__ float dpp_shl1(float old_lane63, float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old_lane63),
@@ -702,42 +704,41 @@ __device__ __forceinline__ void map_align_one(const cth_dpset& q, int qp, const 
 __device__ __forceinline__ void map_fin_one(const cth_dpset& q, int qp, const cth_dpset& db, int p, int64_t colp,
                                             int64_t ldsc, const float* __restrict__ scores,
                                             const uint8_t* __restrict__ btck, char* __restrict__ o, int rowcap,
-                                            cth_mapres& r) {
+                                            uint32_t* tile, cth_mapres& r) {
   const char* qaa = q.aa + q.dist[qp];
   const char* taa = db.aa + db.dist[p];
   const char* qss = q.sss + q.dist[qp];
   const char* tss = db.sss + db.dist[p];
   const bool qssok = qss[0] != 0, tssok = tss[0] != 0;
   const uint32_t xx = (0.0f < r.maxsc) ? r.end : 0u;
+  const int lane = threadIdx.x & 63;
   int y = (int)(xx & 0xffff), x = (int)(xx >> 16);
   int idts = 0, psts = 0, gaps = 0, n = 0;
-  while (x >= 0 && y >= 0) {
-    const int64_t a = (int64_t)y * ldsc + colp + x;
-    const int b = btck[a];
-    if (b == CTH_BT_STOP) break;
-    char cq, cm, ct, sq = ' ', st = ' ';
-    if (b == CTH_BT_UP) {
-      gaps++; cq = qaa[y]; ct = '-'; cm = ' ';
-      if (qssok) sq = qss[y];
-      y--;
-    } else if (b == CTH_BT_LEFT) {
-      gaps++; cq = '-'; ct = taa[x]; cm = ' ';
-      if (tssok) st = tss[x];
-      x--;
-    } else {
-      cq = qaa[y]; ct = taa[x];
-      if (qssok) sq = qss[y];
-      if (tssok) st = tss[x];
-      if (cq == ct) { cm = cq; idts++; }
-      else if (scores[a] > 0.0f) { cm = '+'; psts++; }
-      else cm = ' ';
-      x--; y--;
+  trace_walk<64, false>(btck + colp, ldsc, x, y, tile, [&](int cnt, int px, int py, int b) {
+    const bool in = lane < cnt, up = b == CTH_BT_UP, left = b == CTH_BT_LEFT;
+    char cq = '-', cm = ' ', ct = '-', sq = ' ', st = ' ';
+    float v = 0.0f;
+    if (in && !left) {
+      cq = qaa[py];
+      if (qssok) sq = qss[py];
     }
-    if (o && n < rowcap) {
-      o[n] = cq; o[rowcap + n] = cm; o[2 * rowcap + n] = ct; o[3 * rowcap + n] = sq; o[4 * rowcap + n] = st;
+    if (in && !up) {
+      ct = taa[px];
+      if (tssok) st = tss[px];
     }
-    n++;
-  }
+    const bool diag = in && !up && !left;
+    if (diag) v = scores[(int64_t)py * ldsc + colp + px];
+    const bool ident = diag && cq == ct, pos = diag && !ident && v > 0.0f;
+    cm = ident ? cq : pos ? '+' : ' ';
+    idts += __builtin_popcountll(__builtin_amdgcn_ballot_w64(ident));
+    psts += __builtin_popcountll(__builtin_amdgcn_ballot_w64(pos));
+    gaps += __builtin_popcountll(__builtin_amdgcn_ballot_w64(in && !diag));
+    const int k = n + lane;
+    if (o && in && k < rowcap) {
+      o[k] = cq; o[rowcap + k] = cm; o[2 * rowcap + k] = ct; o[3 * rowcap + k] = sq; o[4 * rowcap + k] = st;
+    }
+    n += cnt;
+  });
   r.end = xx;
   r.beg = ((uint32_t)(x + 1) << 16) | (uint32_t)(y + 1);
   r.idnts = idts;
@@ -783,12 +784,13 @@ __device__ __forceinline__ void map_pair(const cth_dpset& q, int qp, const cth_d
   uint32_t mapxy = 0;
   map_align_one<kGlobalRow>(q, qp, db, p, colp, ldsc, post, btck, minpp, logz, L, W, mapsc, mapxy);
   __syncthreads();  // the traceback bytes are in memory
-  if (threadIdx.x == 0) {
+  if (w == 0) {
     r.maxlog = maxlog;
     r.logz = logz;
-    r.maxsc = mapsc;
-    r.end = mapxy;
-    map_fin_one(q, qp, db, p, colp, ldsc, scores, btck, o, rowcap, r);
+    // lane 0's, uniform for the walk
+    r.maxsc = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, mapsc)));
+    r.end = (uint32_t)__builtin_amdgcn_readfirstlane((int)mapxy);
+    map_fin_one(q, qp, db, p, colp, ldsc, scores, btck, o, rowcap, reinterpret_cast<uint32_t*>(lds), r);
   }
 }
 
