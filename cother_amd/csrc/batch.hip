@@ -346,7 +346,6 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
   uint64_t alnused = 0;
   // batch-local index of each query of the current batch (for its hits)
   std::vector<int> local(c->q.d.nprof, -1);
-  const int rows4 = cth_score_tile_rows(1, 0, 0);
   for (int qa = 0; qa < nq;) {
     // the batch: consecutive entries of the list whose buffers fit the
     // budget together
@@ -358,8 +357,8 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
     while (qb < nq) {
       const int lq = c->q.h_len[ql[qb]];
       const size_t qbytes = (size_t)lq * (size_t)ldsc * bytes_per_cell;
-      // row tiles of the 4-row score kernel (the plain kernel's taller tiles are fewer)
-      const int qt = (lq + rows4 - 1) / rows4;
+      // row tiles of its score kernels, the most any choice of them has
+      const int qt = (lq + CTH_DDMS_TILE - 1) / CTH_DDMS_TILE * (CTH_DDMS_TILE / CTH_SCORE_TILE_MIN);
       if (qb > qa && (bytes + qbytes > budget || tiles + qt > 65535)) break;
       bytes += qbytes;
       tiles += qt;
@@ -390,8 +389,8 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
       continue;
     }
     // no DDMS term in the batch when the database's or every query's
-    // distance lists are shorter than DSTSEGM: the plain score kernel and
-    // its taller row tiles
+    // distance lists are shorter than DSTSEGM: the plain score kernel alone
+    // and row tiles by its own rule
     P.ddms = 0;
     if (cth_devset_has_ddms(&db, 0, nprof))
       for (int k = P.q0; k < P.q1 && !P.ddms; k++) P.ddms = cth_devset_has_ddms(&c->q, ql[k], ql[k] + 1);

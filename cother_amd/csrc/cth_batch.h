@@ -22,7 +22,11 @@ struct cth_bpair {
   int32_t p;
 };
 
-// one row tile of the batched score kernel: batch-local query and its first row
+// rows of the score kernels' row tiles: those of a batch with distance terms,
+// and the fewest of any kernel
+constexpr int CTH_DDMS_TILE = 64, CTH_SCORE_TILE_MIN = 16;
+
+// one row tile of the batched score kernels: batch-local query and its first row
 struct cth_bytile {
   int32_t b;
   int32_t row0;

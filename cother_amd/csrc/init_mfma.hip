@@ -28,52 +28,6 @@ namespace {
 constexpr int kTile = 64;
 constexpr int kK = 32;
 
-template <int kPrec>
-__global__ __launch_bounds__(256) void k_init_mfma(cth_dpset q, int qp, cth_dpset db, int64_t col0, int ncols,
-                                                   int64_t ldsc, int lq, float* __restrict__ out) {
-  // +8: rows of 80 bytes, 16-byte aligned for the 8-element operand reads,
-  // spread over the LDS banks
-  __shared__ __align__(16) uint16_t A[kTile][kK + 8];
-  __shared__ __align__(16) uint16_t B[kTile][kK + 8];
-  __shared__ float bq[CTH_NAA];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int row0 = blockIdx.y * kTile, c0 = blockIdx.x * kTile;
-  const int64_t q0 = q.dist[qp];
-  if (tid < CTH_NAA) bq[tid] = q.bkg[qp * CTH_NAA + tid];
-  __syncthreads();
-  for (int e = tid; e < kTile * kK; e += 256) {
-    const int r = e / kK, k = e % kK;
-    float va = 0.0f, vb = 0.0f;
-    if (k < CTH_NAA) {
-      if (row0 + r < lq) va = q.trg[k * q.ld + q0 + row0 + r];
-      if (c0 + r < ncols) {
-        const int64_t tj = col0 + c0 + r;
-        const int tp = db.pro[tj];
-        vb = db.trg[k * db.ld + tj] / (0.5f * (bq[k] + db.bkg[tp * CTH_NAA + k]));
-      }
-    }
-    A[r][k] = mfma_operand<kPrec>(va);
-    B[r][k] = mfma_operand<kPrec>(vb);
-  }
-  __syncthreads();
-  const int wr = (w >> 1) * 32, wc = (w & 1) * 32;
-  // operands: row / column l32, k = kb + 8 (lane / 32) + 0..7; accumulators:
-  // rows 8 (r / 4) + 4 (lane / 32) + r % 4
-  const int l32 = lane & 31, kh = (lane >> 5) * 4, ko = (lane >> 5) * 8;
-  v16f acc = {};
-#pragma unroll
-  for (int kb = 0; kb < kK; kb += 16) 
-    acc = mfma<kPrec>(*reinterpret_cast<const v8s*>(&A[wr + l32][kb + ko]),
-                      *reinterpret_cast<const v8s*>(&B[wc + l32][kb + ko]), acc);
-  const int col = c0 + wc + l32;
-  if (col >= ncols) return;
-#pragma unroll
-  for (int r = 0; r < 16; r++) {
-    const int row = row0 + wr + 8 * (r >> 2) + kh + (r & 3);
-    if (row < lq) out[(int64_t)row * ldsc + col] = cth_logf_dev(acc[r]) - CTH_INITSHIFT;
-  }
-}
-
 // Lane layout check of the 32x32x16 instructions: A = I (32 x 16 block of
 // the identity), B[k][c] = 32 (k - 8 h) + c for k in [8 h, 8 h + 8) and 0
 // elsewhere (h = 0, 1; every value below 256, exact in BF16), so
@@ -97,18 +51,6 @@ __global__ void k_selftest_mfma(float* out, int h) {
 }
 
 }  // namespace
-
-extern "C" int cth_launch_init_mfma(const cth_dpset* q, int qp, const cth_dpset* db, int64_t col0, int ncols,
-                                    int64_t ldsc, int lq, int prec, float* out, hipStream_t st) {
-  if (ncols <= 0 || lq <= 0) return 0;
-  if (prec != 1 && prec != 2) { cth_set_error("init_mfma: precision %d (1 BF16, 2 FP16)", prec); return -1; }
-  if (ldsc < ncols) { cth_set_error("init_mfma: ldsc %lld < ncols %d", (long long)ldsc, ncols); return -1; }
-  dim3 grid((ncols + kTile - 1) / kTile, (lq + kTile - 1) / kTile);
-  if (prec == 1) hipLaunchKernelGGL(k_init_mfma<1>, grid, dim3(256), 0, st, *q, qp, *db, col0, ncols, ldsc, lq, out);
-  else hipLaunchKernelGGL(k_init_mfma<2>, grid, dim3(256), 0, st, *q, qp, *db, col0, ncols, ldsc, lq, out);
-  CTH_HIP_CHECK(hipGetLastError());
-  return 0;
-}
 
 // Device check of the MFMA lane layout assumed above: 0 when every
 // accumulator holds the expected element (for both precisions).

@@ -1,7 +1,7 @@
 // score.hip: the score-matrix stage on gfx950.
 //
-// One kernel computes, for a query profile against a contiguous range of
-// template positions, every cell of
+// For a query profile against a contiguous range of template positions, every
+// cell of
 //   S[i,j]   = Init + (SS + CVS) + DDMS
 //   mod[i,j] = (SS + CVS - 0.5*CVSWGT) + (DDMS - 0.2*DDMSWGT)
 // in the order the reference's three kernels accumulate them
@@ -9,19 +9,10 @@
 // CalcSM_SSSS_CVS2S_SMEMUnroll2x_2 adds SS+CVS and writes mod,
 // CalcSM_DDMS2S_SMEMUnroll2x_h2 adds DDMS to both when it is non-zero).
 //
-// Tiling: a workgroup of 256 lanes covers 4 query rows x 64 template
-// columns; wave w owns query row w and lane l column l, so the query's
-// distance list is uniform across a wavefront and each lane walks its own
-// template list.  The 64 template lists (132-byte padded rows, conflict-free
-// byte reads) and the 22x22 pair-score table with its halved copy are staged
-// in LDS with each wavefront's query list, as pair-table byte offsets.  The
-// per-cell DDMS dynamic programme (the dominant cost, ~2200 cell updates per
-// score cell for full lists) runs from LDS and vector registers.  It is bound
-// by VALU issue: by the counters 25,300 instructions a wavefront in 14,700
-// issue slots (11,100 instructions as the second of a pair), which fill its
-// time (8 wavefronts a SIMD).  233 Mcells of full lists: 97.8 ms with doubled sums (5 VALU a
-// cell with one move more) and a register updated by selects and branches,
-// 92.8 ms as it is.
+// k_score_plain writes all but the distance-match term; where a cell can have
+// one, k_score_ddms adds it to both matrices afterwards (the order of the
+// sums is the reference's, and the 16 bytes a cell that pass through memory
+// once more are nothing beside the scan's time).
 #include <float.h>
 
 #include <hip/hip_runtime.h>
@@ -36,20 +27,20 @@
 
 namespace {
 
-constexpr int kRows = 4;        // query rows per workgroup (one per wavefront)
-constexpr int kCols = 64;       // template columns per workgroup (one per lane)
-constexpr int kListPitch = 132; // LDS bytes per template list
+constexpr int kCols = 64;  // template columns per workgroup of the plain kernel (one per lane)
 
+// The distance-match scan's workgroup: kDRows query rows x kDCols template
+// columns, one cell per lane.
+constexpr int kDThreads = 512, kDRows = 16, kDCols = kDThreads / kDRows;
+constexpr int kListPitch = 132;  // LDS bytes per template list
+constexpr int kQlEntries = 112;  // query record entries the scan reads (0..111)
+constexpr int kQlPitch = 113;    // LDS words per query list: rows fall on different banks
 constexpr float kSumScale = 0x1p-6f;  // of the distance-match sums (a segment's stays below 1)
-constexpr int kQlEntries = 112;  // query record entries the DDMS scan reads (0..111)
 
-struct ScoreLds {
-  uint8_t tl[kCols * kListPitch];  // template lists, values scaled by 4 (table byte columns)
-  int32_t ql[kRows][kQlEntries];   // each wavefront's query list as table byte offsets
-  float dms[22 * 22];   // the pair scores times kSumScale
-  float dmsh[22 * 22];  // and halved (both exact), right after dms
-  float ss[467];
-  float cvvals[CTH_CVMAXCARD];
+struct DdmsLds {
+  uint8_t tl[kDCols * kListPitch];  // template lists, values scaled by 4 (table byte columns)
+  int32_t ql[kDRows * kQlPitch];    // query lists as table byte offsets
+  float dms[22 * 22];               // the pair scores times kSumScale
 };
 
 __device__ __forceinline__ float ss_lookup(const float* ss, int row, int col) {
@@ -163,13 +154,14 @@ __device__ __forceinline__ void register_max(ddms_register& R, float s, uint32_t
 // near the denormals), which puts every segment's sum below 1 (at most 102
 // cells of at most 0.5), so that one add with the clamp modifier is
 // max(sum + x, 0) with the reference's one rounding.  Per cell, with x the
-// cell's scaled pair score (or, for the interpolated cells, 0.5 (a + b): the
-// reference's 0.5f * (a + b), exact), dd = the segment's begin minus the cell
-// index (an integer value, <= 0) and big = 2^126:
+// cell's scaled pair score (or, for the interpolated cells, 0.5 (a + b),
+// whose halving is exact and joins the sum in one fma), dd = the segment's
+// begin minus the cell index (an integer value, <= 0) and big = 2^126:
 //   nz   = clamp(u * big)          1 when the previous sum is > 0, else 0
 //                                  (positive sums are far above 2^-126)
 //   dd   = fma(nz, dd, -nz)        dd - 1, or 0 where the segment restarts
 //   u    = clamp(u + x)
+// and, where some lane of the wavefront can have a candidate in the step,
 //   cand = u * clamp(-dd - 4)      u if the segment has at least DSTSEGM = 6
 //                                  cells (dd <= -5), else 0
 // and the step's best is the max of its four candidates: the reference takes
@@ -178,19 +170,16 @@ __device__ __forceinline__ void register_max(ddms_register& R, float s, uint32_t
 // sign of a zero sum, and a zero is never registered.  The top-3 register
 // holds scaled sums too (scaling commutes with every comparison and with the
 // rounding of the final sum, which is scaled back exactly).
-#define CTH_DDMS_CELL(X, COUT)                                                \
-  {                                                                           \
-    const float nz = __builtin_amdgcn_fmed3f(u * big, 0.0f, 1.0f);            \
-    dd = fmaf(nz, dd, -nz);                                                   \
-    u = __builtin_amdgcn_fmed3f(u + (X), 0.0f, 1.0f);                         \
-    COUT = u * __builtin_amdgcn_fmed3f(-dd - 4.0f, 0.0f, 1.0f);               \
-  }
-// one 4-cell step, cells K0+1..K0+4 relative to the base ib, with pair
-// scores A2, A4 (cells K0+2 and K0+4) and the halves H0, H2, H4 of those of
-// cells K0 (the previous step's last cell), K0+2 and K0+4, and FB the float
-// 2^23 + the packed coordinates of cell K0+1 on both axes: the reference's
-// interpolated sum 0.5f * (a + b) is h(a) + h(b), halving being exact and
-// commuting with the rounding of the sum.  The begin and end of the step's
+#define CTH_DDMS_CELL(U, DD, SUM, UOUT, DDOUT)                                \
+  const float nz##UOUT = __builtin_amdgcn_fmed3f((U) * big, 0.0f, 1.0f);      \
+  const float DDOUT = fmaf(nz##UOUT, DD, -nz##UOUT);                          \
+  const float UOUT = __builtin_amdgcn_fmed3f(SUM, 0.0f, 1.0f);
+// one 4-cell step, cells K0+1..K0+4 relative to the base ib, with the pair
+// scores S0, S2, S4 of cells K0 (the previous step's last cell), K0+2 and
+// K0+4, and FB the float 2^23 + the packed coordinates of cell K0+1 on both
+// axes.  A candidate's segment has 6 cells or more at a cell of the step, so
+// at least 3 at its first (dd1 <= -2): where no lane's has, the step ends
+// there.  The begin and end of the step's
 // best are recovered only when it can be registered.  Three levels: the
 // step's best is a candidate when it reaches m2 (empty most of the time: a
 // growing best segment drops it); a candidate whose segment already meets m0
@@ -202,14 +191,20 @@ __device__ __forceinline__ void register_max(ddms_register& R, float s, uint32_t
 // empty asm statements keep the candidate's packed words in registers:
 // without them the compiler folds their sums into each test as
 // scalar-operand adds, which issue one per cycle.
-#define CTH_DDMS_4CELL(H0, A2, H2, A4, H4, FB)                                \
+#define CTH_DDMS_4CELL(S0, S2, S4, FB)                                        \
   {                                                                           \
-    float cd1, cd2, cd3, cd4;                                                 \
-    CTH_DDMS_CELL(H0 + H2, cd1)                                               \
-    const float dd1 = dd;                                                     \
-    CTH_DDMS_CELL(A2, cd2)                                                    \
-    CTH_DDMS_CELL(H2 + H4, cd3)                                               \
-    CTH_DDMS_CELL(A4, cd4)                                                    \
+    const float t1 = S0 + S2, t3 = S2 + S4;                                   \
+    CTH_DDMS_CELL(u, dd, fmaf(t1, 0.5f, u), u1, dd1)                          \
+    CTH_DDMS_CELL(u1, dd1, u1 + S2, u2, dd2)                                  \
+    CTH_DDMS_CELL(u2, dd2, fmaf(t3, 0.5f, u2), u3, dd3)                       \
+    CTH_DDMS_CELL(u3, dd3, u3 + S4, u4, dd4)                                  \
+    u = u4;                                                                   \
+    dd = dd4;                                                                 \
+    if (in_mask(mask_ge(-2.0f, dd1))) {                                       \
+    const float cd1 = u1 * __builtin_amdgcn_fmed3f(-dd1 - 4.0f, 0.0f, 1.0f);  \
+    const float cd2 = u2 * __builtin_amdgcn_fmed3f(-dd2 - 4.0f, 0.0f, 1.0f);  \
+    const float cd3 = u3 * __builtin_amdgcn_fmed3f(-dd3 - 4.0f, 0.0f, 1.0f);  \
+    const float cd4 = u4 * __builtin_amdgcn_fmed3f(-dd4 - 4.0f, 0.0f, 1.0f);  \
     const float scom = fmaxf(fmaxf(cd1, cd2), fmaxf(cd3, cd4));               \
     if (in_mask(mask_ge(scom, R.m2))) {                                       \
       /* the step's first cell on both axes, packed (with kMagic) */          \
@@ -243,55 +238,50 @@ __device__ __forceinline__ void register_max(ddms_register& R, float s, uint32_t
           register_max(R, scom, sb, se, ge0, ge1, free0, free1);              \
       }                                                                       \
     }                                                                         \
+    }                                                                         \
   }
 // eight cells (two steps); the pair scores of the step after are loaded one
 // step ahead (lists are padded).  GUARD: whether the second step is due.
 #define CTH_DDMS_8CELL(GUARD)                                                 \
   {                                                                           \
-    const int q6 = lds_i32(lds, qo + 24), q8 = lds_i32(lds, qo + 32);         \
-    const int t6 = lds_u8(lds, to + 6), t8 = lds_u8(lds, to + 8);             \
-    const float n2 = pair(lds, q6, t6), nh2 = pairh(lds, q6, t6);             \
-    const float n4 = pair(lds, q8, t8), nh4 = pairh(lds, q8, t8);             \
-    CTH_DDMS_4CELL(h0, s2, h2, s4, h4, fb)                                    \
-    const int q10 = lds_i32(lds, qo + 40), q12 = lds_i32(lds, qo + 48);       \
-    const int t10 = lds_u8(lds, to + 10), t12 = lds_u8(lds, to + 12);         \
-    const float p2 = pair(lds, q10, t10), ph2 = pairh(lds, q10, t10);         \
-    const float p4 = pair(lds, q12, t12), ph4 = pairh(lds, q12, t12);         \
-    if (GUARD) CTH_DDMS_4CELL(h4, n2, nh2, n4, nh4, fb + 4.0f * kPackF)       \
+    const float n2 = pair(lds, lds_i32(lds, qo + 24), lds_u8(lds, to + 6));   \
+    const float n4 = pair(lds, lds_i32(lds, qo + 32), lds_u8(lds, to + 8));   \
+    CTH_DDMS_4CELL(s0, s2, s4, fb)                                            \
+    const float p2 = pair(lds, lds_i32(lds, qo + 40), lds_u8(lds, to + 10));  \
+    const float p4 = pair(lds, lds_i32(lds, qo + 48), lds_u8(lds, to + 12));  \
+    if (GUARD) CTH_DDMS_4CELL(s4, n2, n4, fb + 4.0f * kPackF)                 \
     fb += 8.0f * kPackF;                                                      \
     qo += 32;                                                                 \
     to += 8;                                                                  \
     asm("" : "+v"(qo), "+v"(to));                                             \
-    h0 = nh4;                                                                 \
+    s0 = n4;                                                                  \
     s2 = p2;                                                                  \
-    h2 = ph2;                                                                 \
     s4 = p4;                                                                  \
-    h4 = ph4;                                                                 \
   }
 
 // The scan reads everything from the workgroup's LDS block by byte offsets
 // held in vector registers, so that each table address is one vector add
 // (which dual-issues) and the rest is the instruction's immediate offset.
-// kDms, kDmsh: the pair-score table and its halves in the block
-constexpr int kDms = (int)offsetof(ScoreLds, dms), kDmsh = (int)offsetof(ScoreLds, dmsh);
+// kDms: the pair-score table in the block
+constexpr int kDms = (int)offsetof(DdmsLds, dms);
 __device__ __forceinline__ int lds_i32(const char* lds, int off) { return *reinterpret_cast<const int32_t*>(lds + off); }
 __device__ __forceinline__ int lds_u8(const char* lds, int off) { return *reinterpret_cast<const uint8_t*>(lds + off); }
 // the pair score of list values whose table byte offsets are qb (query,
-// d1*88) and tv (template, d2*4): dmsT[d1][d2], and its half
+// d1*88) and tv (template, d2*4): dmsT[d1][d2]
 __device__ __forceinline__ float pair(const char* lds, int qb, int tv) {
   return *reinterpret_cast<const float*>(lds + kDms + qb + tv);
 }
-__device__ __forceinline__ float pairh(const char* lds, int qb, int tv) {
-  return *reinterpret_cast<const float*>(lds + kDmsh + qb + tv);
-}
 
-// lds: the workgroup's block; qr: byte offset of the wavefront's query list
-// (int32 table byte offsets, entry 0 = the list length); tr: byte offset of
-// the lane's template list (byte 0 = length, then values times 4); lmin,
-// lmax: the shortest and the longest template list of the wavefront
-__device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int lmin, int lmax) {
-  const int len1 = __builtin_amdgcn_readfirstlane(lds_i32(lds, qr)), len2 = lds_u8(lds, tr);
-  if (len1 < CTH_DSTSEGM || len2 < CTH_DSTSEGM) return 0.0f;
+// The shortest and the longest list of the wavefront's cells on each axis
+// (of the cells whose lists both reach DSTSEGM).
+struct ddms_lens {
+  int qmin, qmax, tmin, tmax;
+};
+
+// lds: the workgroup's block; qr: byte offset of the lane's query list (int32
+// table byte offsets after entry 0); tr: byte offset of its template list
+// (values times 4 after byte 0); len1, len2: their lengths, at least DSTSEGM
+__device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int len1, int len2, const ddms_lens& n) {
   ddms_register R{FLT_MIN, FLT_MIN, FLT_MIN, kNoBeginN, kNoEnd, kNoBeginN, kNoEnd};
   // 2^126, 1 + 2^11 and 2^120 in vector registers: as scalar operands they
   // would keep the multiplies and fmas off the second issue slot
@@ -302,32 +292,30 @@ __device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int 
   // the diagonals: upper ones j = len2>>2 .. 0 pair query index i with
   // template index j + i, lower ones i = len1>>2 .. 1 query index i + j with
   // template index j
-  const int upper = (lmax >> 3) + 1, lower = ((len1 >> 2) + 1) >> 1;
+  const int upper = (n.tmax >> 3) + 1, lower = ((n.qmax >> 2) + 1) >> 1;
   for (int k = 0; k < upper + lower; k++) {
     const int i = k < upper ? 0 : (len1 >> 2) - 2 * (k - upper);
     const int j = k < upper ? (len2 >> 2) - 2 * k : 0;
-    if (j < 0) continue;
-    const int n = min(len1 - i, len2 - j);  // cells of the diagonal
+    if (k < upper ? j < 0 : i < 1) continue;
+    const int cells = min(len1 - i, len2 - j);  // of the diagonal
     // cells that every lane's diagonal has (len - (len >> 2) grows with len):
     // their steps are taken without a test of the lane's end
-    const int full = min(len1 - i, k < upper ? lmin - (lmin >> 2) + 2 * k : lmin);
+    const int full = k < upper ? min(n.qmin, n.tmin - (n.tmin >> 2) + 2 * k)
+                               : min(n.qmin - (n.qmin >> 2) + 2 * (k - upper), n.tmin);
     // byte offsets of the diagonal's first query and template entries,
     // advanced by one iteration (8 entries) at a time in vector registers
     int qo = qr + 4 * (1 + i), to = tr + 1 + j;
-    const float s0 = pair(lds, lds_i32(lds, qo), lds_u8(lds, to));
+    float s0 = pair(lds, lds_i32(lds, qo), lds_u8(lds, to));
     float u = __builtin_amdgcn_fmed3f(s0, 0.0f, 1.0f);  // max(s0, 0)
     float dd = 0.0f;
     // 2^23 + the packed coordinates of cell 1 (query i + 1, template j + 1)
     float fb = __uint_as_float(kMagic + kPack + (uint32_t)i + ((uint32_t)j << 11));
-    float h0 = pairh(lds, lds_i32(lds, qo), lds_u8(lds, to));
-    float s2 = pair(lds, lds_i32(lds, qo + 8), lds_u8(lds, to + 2)),
-          h2 = pairh(lds, lds_i32(lds, qo + 8), lds_u8(lds, to + 2));
-    float s4 = pair(lds, lds_i32(lds, qo + 16), lds_u8(lds, to + 4)),
-          h4 = pairh(lds, lds_i32(lds, qo + 16), lds_u8(lds, to + 4));
+    float s2 = pair(lds, lds_i32(lds, qo + 8), lds_u8(lds, to + 2));
+    float s4 = pair(lds, lds_i32(lds, qo + 16), lds_u8(lds, to + 4));
     asm("" : "+v"(qo), "+v"(to));
     int ib = 0;
     for (; ib + 4 < full; ib += 8) CTH_DDMS_8CELL(true)
-    for (; ib < n; ib += 8) CTH_DDMS_8CELL(ib + 4 < n)
+    for (; ib < cells; ib += 8) CTH_DDMS_8CELL(ib + 4 < cells)
   }
   float s = 0.0f;
   s += R.m0;
@@ -341,153 +329,90 @@ __device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int 
 #undef CTH_DDMS_4CELL
 #undef CTH_DDMS_8CELL
 
-// kPreInit: the log-odds term is already in scores (the reduced-precision
-// contraction of init_mfma.hip); otherwise it is computed here in FP32.
-// kBatch: the row tiles of several queries in one launch, blockIdx.y indexing
-// ytab (query of the batch and first row), each query's blocks at its offset.
-template <bool kPreInit, bool kBatch = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_score(cth_dpset q, int qp, cth_dpset db, int64_t col0, int ncols,
-                                               int64_t ldsc, const cth_tables* __restrict__ tabs,
-                                               float* __restrict__ scores, float* __restrict__ mods,
-                                               const int32_t* __restrict__ qoff,
-                                               const cth_bytile* __restrict__ ytab = nullptr,
-                                               const cth_bquery* __restrict__ bq = nullptr) {
-  __shared__ ScoreLds L;
+// Adds the distance-match term to the matrices that k_score_plain wrote.
+//
+// A wavefront covers kDRows query rows x 64 / kDRows template columns (each
+// lane a cell with its own two lists; in a tile of fewer rows more columns).
+// The register code of a step runs when any of the wavefront's lanes needs
+// it, and the lists of neighbouring positions are alike, on the query's side
+// most of all: replayed with the synthetic lists, a step reaches the
+// candidate test in 75% of a 1 x 64 wavefront's steps, 42% of an 8 x 8's and
+// 37% of a 16 x 4's, and changes a register in 31, 23 and 21%.
+// kBatch: the row tiles of several queries in one launch, ytab[blockIdx.y /
+// ysplit] giving query and first row of ysplit tiles of kDRows rows.
+template <bool kBatch>
+__global__ __launch_bounds__(kDThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_score_ddms(
+    cth_dpset q, int qp, cth_dpset db, int64_t col0, int ncols, int64_t ldsc, const cth_tables* __restrict__ tabs,
+    float* __restrict__ scores, float* __restrict__ mods, const int32_t* __restrict__ qoff,
+    const cth_bytile* __restrict__ ytab, int ysplit, const cth_bquery* __restrict__ bq) {
+  __shared__ DdmsLds L;
   const int tid = threadIdx.x;
-  const int lane = tid & 63, w = tid >> 6;
-  int row = blockIdx.y * kRows + w;
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int row0 = blockIdx.y * kDRows;
   if constexpr (kBatch) {
-    const cth_bytile t = ytab[blockIdx.y];
+    const cth_bytile t = ytab[blockIdx.y / ysplit];
     const cth_bquery Q = bq[t.b];
     qp = Q.qp;
-    row = t.row0 + w;
+    row0 = t.row0 + (int)(blockIdx.y % ysplit) * kDRows;
     scores += Q.off;
     mods += Q.off;
   }
-  const int lq = q.len[qp];
-  const int64_t q0 = q.dist[qp];
-  const int col = blockIdx.x * kCols + lane;
-
-  // stage tables
-  for (int k = tid; k < 22 * 22; k += 256) {
-    L.dms[k] = kSumScale * tabs->dms[k];
-    L.dmsh[k] = 0.5f * kSumScale * tabs->dms[k];
-  }
-  for (int k = tid; k < 467; k += 256) L.ss[k] = tabs->ss[k];
-  for (int k = tid; k < tabs->cvcard; k += 256) L.cvvals[k] = tabs->cvvals[k];
-  // stage 64 template lists (32 dwords each), values (<= 21) times 4: the
-  // pair table's byte column; the length byte stays
-  for (int k = tid; k < kCols * 32; k += 256) {
+  const int rows = min(kDRows, q.len[qp] - row0);
+  if (rows <= 0) return;
+  const int64_t q0 = q.dist[qp] + row0;
+  const int c0 = blockIdx.x * kDCols;
+  for (int k = tid; k < 22 * 22; k += kDThreads) L.dms[k] = kSumScale * tabs->dms[k];
+  // template lists (32 dwords each), values (<= 21) times 4: the pair table's
+  // byte column; the length byte stays
+  for (int k = tid; k < kDCols * 32; k += kDThreads) {
     const int c = k >> 5, d = k & 31;
-    const int cc = blockIdx.x * kCols + c;
-    uint32_t v = 0x15151515u;  // padding value 21
-    if (cc < ncols) v = reinterpret_cast<const uint32_t*>(db.dd + (size_t)(col0 + cc) * CTH_DDSTRIDE)[d];
-    if (cc >= ncols && d == 0) v = 0x15151500u;  // empty list
+    uint32_t v = 0x15151500u;  // (an empty list's first dword)
+    if (c0 + c < ncols) v = reinterpret_cast<const uint32_t*>(db.dd + (size_t)(col0 + c0 + c) * CTH_DDSTRIDE)[d];
     v = d == 0 ? (v & 0xffu) | ((v & 0xffffff00u) << 2) : v << 2;
     *reinterpret_cast<uint32_t*>(&L.tl[c * kListPitch + d * 4]) = v;
   }
-  // each wavefront's query list (table byte offsets; rows past the query
-  // stage its last row, whose results are not stored)
-  {
-    const int rr = min(row, lq - 1);
-    const int32_t* qsrc = qoff + (size_t)(q0 + rr) * CTH_DDSTRIDE;
-    for (int k = lane; k < kQlEntries; k += 64) L.ql[w][k] = qsrc[k];
+  for (int k = tid; k < rows * 128; k += kDThreads) {
+    const int r = k >> 7, e = k & 127;
+    if (e < kQlEntries) L.ql[r * kQlPitch + e] = qoff[(size_t)(q0 + r) * CTH_DDSTRIDE + e];
   }
   __syncthreads();
 
-  // DDMS first, while nothing else is live
-  int lmin = L.tl[lane * kListPitch], lmax = lmin;
-  if (lmin < CTH_DSTSEGM) lmin = CTH_MAXDST;  // such lanes take no step
+  // rows of the wavefront's cells: the tile's, up to a power of two
+  // (at least two: 64 / 2 columns are the tile's)
+  static_assert(kDCols == 32 && kDRows <= 64, "a wavefront's columns lie within the tile");
+  const int tqs = rows > 2 ? 32 - __builtin_clz(rows - 1) : 1;
+  const int r = lane >> (6 - tqs), c = (w << (6 - tqs)) + (lane & (63 >> tqs));
+  if ((w << (6 - tqs)) >= kDCols) return;
+  const char* const lds = reinterpret_cast<const char*>(&L);
+  const int qr = (int)offsetof(DdmsLds, ql) + 4 * kQlPitch * min(r, rows - 1), tr = kListPitch * c;
+  const int len1 = lds_i32(lds, qr), len2 = lds_u8(lds, tr);
+  const bool on = r < rows && c0 + c < ncols && len1 >= CTH_DSTSEGM && len2 >= CTH_DSTSEGM;
+  ddms_lens n{on ? len1 : CTH_MAXDST, on ? len1 : 0, on ? len2 : CTH_MAXDST, on ? len2 : 0};
   for (int o = 32; o >= 1; o >>= 1) {
-    lmin = min(lmin, __shfl_xor(lmin, o));
-    lmax = max(lmax, __shfl_xor(lmax, o));
+    n.qmin = min(n.qmin, __shfl_xor(n.qmin, o));
+    n.qmax = max(n.qmax, __shfl_xor(n.qmax, o));
+    n.tmin = min(n.tmin, __shfl_xor(n.tmin, o));
+    n.tmax = max(n.tmax, __shfl_xor(n.tmax, o));
   }
-  if (row >= lq || col >= ncols) return;
-  const float d = ddms_cell(reinterpret_cast<const char*>(&L), (int)offsetof(ScoreLds, ql) + w * kQlEntries * 4,
-                            lane * kListPitch, __builtin_amdgcn_readfirstlane(lmin),
-                            __builtin_amdgcn_readfirstlane(lmax));
-
-  const int64_t qi = q0 + row;
-  const int64_t tj = col0 + col;
-  const int tp = db.pro[tj];
-
-  // Init: log-odds (CuBatchScoreMatrix_Init.cu:129-144,173-185)
-  float s = 0.0f;
-  if constexpr (kPreInit) {
-    s = scores[row * ldsc + col];
-  } else {
-  #pragma unroll
-    for (int a = 0; a < CTH_NAA; a++) {
-      const float f1 = q.trg[a * q.ld + qi];
-      const float f2 = q.bkg[qp * CTH_NAA + a];
-      const float num = f1 * db.trg[a * db.ld + tj];
-      const float den = 0.5f * (f2 + db.bkg[tp * CTH_NAA + a]);
-      s = s + num / den;
-    }
-    s = cth_logf(s) - CTH_INITSHIFT;
-  }
-
-  // SS (CuBatchScoreMatrix_ssss.cuh:64-116)
-  float sss = 0.0f;
-#pragma unroll
-  for (int i = 0; i < CTH_NSS; i++) {
-    const float f1 = q.ss[i * q.ld + qi];
-    const int r = i * 10 + (int)(f1 * 9.999f);
-#pragma unroll
-    for (int j = 0; j < CTH_NSS; j++) {
-      const float f2 = db.ss[j * db.ld + tj];
-      const int c = j * 10 + (int)(f2 * 9.999f);
-      sss = fmaf(f1 * f2, ss_lookup(L.ss, r, c), sss);
-    }
-  }
-  {
-    const float f1 = q.ss[(CTH_NSS - 1) * q.ld + qi];
-    if (-99.f < sss) {
-      const float f2 = db.ss[(CTH_NSS - 1) * db.ld + tj];
-      sss = fmaf((f1 + 0.1f) * (f2 + 0.1f), 0.1111111f, sss);
-      sss -= CTH_SSSHIFT;
-      sss *= CTH_SSSWGT;
-    }
-  }
-  // CVS (CuBatchScoreMatrix_cvs2s.cuh:80-113)
-  float cvs = 0.0f;
-#pragma unroll
-  for (int i = 0; i < CTH_NCV; i++) cvs = fmaf(q.cv[i * q.ld + qi], db.cv[i * db.ld + tj], cvs);
-  const float kap = tabs->cvkappa0inv;
-  cvs += kap;
-  {
-    const float a = (q.cvnorm2[qi] + 1.0f + kap) * (db.cvnorm2[tj] + 1.0f + kap);
-    cvs = fmaf(-cvs, cvs, a);
-    cvs = fmaf(tabs->cvpowernu0, cth_logf(cvs), tabs->cvcterm) - q.cvprior[qi] - db.cvprior[tj];
-    const int card = tabs->cvcard;
-    float v;
-    if (cvs <= tabs->cvkeys[0]) v = L.cvvals[0];
-    else if (tabs->cvkeys[card - 1] <= cvs) v = L.cvvals[card - 1];
-    else v = L.cvvals[tabs->cvshift + (int)rintf(2.0f * cvs)];
-    cvs = v * CTH_CVSWGT;
-  }
-  const float sc = sss + cvs;
-  s = s + sc;
-  float ms = fmaf(-CTH_CVSSHIFT, CTH_CVSWGT, sc);
-
+  if (!on) return;
+  n.qmin = __builtin_amdgcn_readfirstlane(n.qmin);
+  n.qmax = __builtin_amdgcn_readfirstlane(n.qmax);
+  n.tmin = __builtin_amdgcn_readfirstlane(n.tmin);
+  n.tmax = __builtin_amdgcn_readfirstlane(n.tmax);
+  const float d = ddms_cell(lds, qr, tr, len1, len2, n);
   if (d != 0.0f) {
-    s = s + d;
-    ms = ms + fmaf(-CTH_DDMSSHIFT, CTH_DDMSWGT, d);
+    const int64_t at = (int64_t)(row0 + r) * ldsc + c0 + c;
+    scores[at] = scores[at] + d;
+    mods[at] = mods[at] + fmaf(-CTH_DDMSSHIFT, CTH_DDMSWGT, d);
   }
-  scores[row * ldsc + col] = s;
-  mods[row * ldsc + col] = ms;
 }
 
-// The score stage where no cell can have a DDMS term (every query or every
-// template list shorter than DSTSEGM: ddms_cell returns 0 and k_score adds
-// nothing), with the same per-cell arithmetic as k_score's log-odds, SS and
-// CVS terms.  Without the DDMS scan the cell is a few hundred instructions
-// and k_score's 4-row tiles would re-read each template column's fields per
-// 4 rows; here a workgroup covers a tile of query rows (every fourth row per
-// wavefront) of 64 template columns, each lane holding its column in
-// registers: frequencies, denominators and their reciprocals, context vector
-// (128 VGPRs, 4 wavefronts per SIMD).  A row's values are uniform and come by
-// scalar loads from the query's record (k_query_records).
+// The score matrices without the DDMS term.  A workgroup covers a tile of
+// query rows (every fourth row per wavefront) of 64 template columns, each
+// lane holding its column in registers: frequencies, denominators and their
+// reciprocals, context vector (128 VGPRs, 4 wavefronts per SIMD).  A row's
+// values are uniform and come by scalar loads from the query's record
+// (k_query_records).
 //
 // Bound by VALU issue: ~205 instructions a row, 39 of them single-rate (a
 // scalar operand keeps an instruction from issuing with another wavefront's).
@@ -576,8 +501,9 @@ __global__ __launch_bounds__(256) void k_query_records(cth_dpset q, const cth_ta
   rec[i] = r;
 }
 
-// kBatch: as k_score's.  kPrec 1, 2: the log-odds sum from the BF16 / FP16
-// product on the matrix cores (as k_init_mfma forms it), 0: in FP32.
+// kBatch: as k_score_ddms's (ytab[blockIdx.y] a tile of `tile` rows).
+// kPrec 1, 2: the log-odds sum from the BF16 / FP16 product on the matrix
+// cores, 0: in FP32.
 //
 // The product's tile is 32 of the wavefront's rows x its 64 columns, two
 // 32 x 32 blocks; it goes through the wavefront's own LDS block to one column
@@ -842,87 +768,79 @@ __global__ void k_selftest_logf(int* bad) {
 
 }  // namespace
 
-// rows of one tile of the score kernel (ddms 0: of k_score_plain) where it
-// runs over `rows` query rows (all queries of a batch) and ncols columns
+// Rows of one tile of k_score_plain over `rows` query rows (all queries of a
+// batch) and ncols columns.  A batch with DDMS terms (ddms) runs both kernels
+// over one table of tiles, so they are CTH_DDMS_TILE rows there, a multiple
+// of kDRows; the plain kernel's share of its time is small.
 extern "C" int cth_score_tile_rows(int ddms, int64_t rows, int64_t ncols) {
-  if (ddms) return kRows;
+  if (ddms) return CTH_DDMS_TILE;
   const int64_t cols = (ncols + kCols - 1) / kCols;
   const int64_t fit = rows * cols / kPlainFill;  // rows per tile that leave kPlainFill workgroups
   return (int)std::max<int64_t>(kPlainRowsMin, std::min<int64_t>({(rows + 3) / 4 * 4, fit / 4 * 4, kPlainRowsMax}));
 }
+static_assert(CTH_DDMS_TILE % kDRows == 0 && kDRows >= CTH_SCORE_TILE_MIN && kPlainRowsMin >= CTH_SCORE_TILE_MIN,
+              "row tiles");
 
 // Launch the score stage for query profile qp against template positions
 // [col0, col0+ncols) of db; outputs are [Lq][ldsc].
 // contraction 0: the FP32 log-odds term of the reference; 1 / 2: the term
-// from the BF16 / FP16 matrix-core product (before k_score by
-// init_mfma.hip, within k_score_plain).  ddms 0:
-// no cell can have a DDMS term (the query's or every template's lists are
-// shorter than DSTSEGM), so k_score_plain runs.  qrec: the query set's
-// records (cth_make_query_records).
-extern "C" int cth_launch_init_mfma(const cth_dpset* q, int qp, const cth_dpset* db, int64_t col0, int ncols,
-                                    int64_t ldsc, int lq, int prec, float* out, hipStream_t st);
+// from the BF16 / FP16 matrix-core product.  ddms 0: no cell can have a DDMS
+// term (the query's or every template's lists are shorter than DSTSEGM).
+// qrec: the query set's records (cth_make_query_records).
 extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, const float* qrec, int qp, const cth_dpset* db, int64_t col0,
                                 int ncols, int64_t ldsc, const cth_tables* dtabs, int lq, float* scores, float* mods,
                                 int contraction, int ddms, hipStream_t st) {
   if (ncols <= 0 || lq <= 0) return 0;
-  if (!qoff) { cth_set_error("score: query distance offsets not built"); return -1; }
+  if (!qoff || !qrec) { cth_set_error("score: query distance offsets or records not built"); return -1; }
   if (ldsc < ncols) { cth_set_error("score: ldsc %lld < ncols %d", (long long)ldsc, ncols); return -1; }
-  if (!ddms) {
-    if (!qrec) { cth_set_error("score: query records not built"); return -1; }
-    const query_record* const rec = reinterpret_cast<const query_record*>(qrec);
-    const int tile = cth_score_tile_rows(0, lq, ncols);
-    const dim3 pgrid((ncols + kCols - 1) / kCols, (lq + tile - 1) / tile);
-    if (contraction < 0 || contraction > 2) {
-      cth_set_error("score: contraction %d (0 FP32, 1 BF16, 2 FP16)", contraction);
-      return -1;
-    }
-    if (contraction == 1) {
-      hipLaunchKernelGGL((k_score_plain<1, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
-                         dtabs, scores, mods, tile, nullptr, nullptr);
-    } else if (contraction == 2) {
-      hipLaunchKernelGGL((k_score_plain<2, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
-                         dtabs, scores, mods, tile, nullptr, nullptr);
-    } else {
-      hipLaunchKernelGGL((k_score_plain<0, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
-                         dtabs, scores, mods, tile, nullptr, nullptr);
-    }
-    CTH_HIP_CHECK(hipGetLastError());
-    return 0;
+  if (contraction < 0 || contraction > 2) {
+    cth_set_error("score: contraction %d (0 FP32, 1 BF16, 2 FP16)", contraction);
+    return -1;
   }
-  dim3 grid((ncols + kCols - 1) / kCols, (lq + kRows - 1) / kRows);
-  if (contraction) {
-    if (cth_launch_init_mfma(q, qp, db, col0, ncols, ldsc, lq, contraction, scores, st)) return -1;
-    hipLaunchKernelGGL(k_score<true>, grid, dim3(256), 0, st, *q, qp, *db, col0, ncols, ldsc, dtabs, scores, mods, qoff);
+  const query_record* const rec = reinterpret_cast<const query_record*>(qrec);
+  const int tile = cth_score_tile_rows(0, lq, ncols);
+  const dim3 pgrid((ncols + kCols - 1) / kCols, (lq + tile - 1) / tile);
+  if (contraction == 1) {
+    hipLaunchKernelGGL((k_score_plain<1, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
+                       dtabs, scores, mods, tile, nullptr, nullptr);
+  } else if (contraction == 2) {
+    hipLaunchKernelGGL((k_score_plain<2, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
+                       dtabs, scores, mods, tile, nullptr, nullptr);
   } else {
-    hipLaunchKernelGGL(k_score<false>, grid, dim3(256), 0, st, *q, qp, *db, col0, ncols, ldsc, dtabs, scores, mods,
-                       qoff);
+    hipLaunchKernelGGL((k_score_plain<0, false>), pgrid, dim3(256), 0, st, *q, rec, qp, *db, col0, ncols, ldsc,
+                       dtabs, scores, mods, tile, nullptr, nullptr);
   }
+  CTH_HIP_CHECK(hipGetLastError());
+  if (!ddms) return 0;
+  hipLaunchKernelGGL(k_score_ddms<false>, dim3((ncols + kDCols - 1) / kDCols, (lq + kDRows - 1) / kDRows),
+                     dim3(kDThreads), 0, st, *q, qp, *db, col0, ncols, ldsc, dtabs, scores, mods, qoff, nullptr, 1,
+                     nullptr);
   CTH_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
-// The score stage of a batch of queries in one launch: nytiles row tiles
-// (ytab: query of the batch and first row, `tile` rows each, as
-// cth_score_tile_rows gives them) against the whole resident database (ncols positions from
-// column 0); each query's scores and modular scores at its offset
-// (bq[].off, row stride ldsc); ddms 0 as in cth_launch_score.
+// The score stage of a batch of queries: nytiles row tiles (ytab: query of
+// the batch and first row, `tile` rows each, as cth_score_tile_rows gives
+// them) against the whole resident database (ncols positions from column 0);
+// each query's scores and modular scores at its offset (bq[].off, row stride
+// ldsc); ddms 0 as in cth_launch_score.
 extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, const float* qrec, const cth_dpset* db,
                                       int ncols,
                                       int64_t ldsc, const cth_tables* dtabs, const cth_bytile* ytab, int nytiles,
                                       const cth_bquery* bq, float* scores, float* mods, int ddms, int tile, hipStream_t st) {
   if (ncols <= 0 || nytiles <= 0) return 0;
-  if (!qoff) { cth_set_error("score batch: query distance offsets not built"); return -1; }
+  if (!qoff || !qrec) { cth_set_error("score batch: query distance offsets or records not built"); return -1; }
   if (ldsc < ncols) { cth_set_error("score batch: ldsc %lld < ncols %d", (long long)ldsc, ncols); return -1; }
-  if (nytiles > 65535) { cth_set_error("score batch: %d row tiles (at most 65535)", nytiles); return -1; }
-  dim3 grid((ncols + kCols - 1) / kCols, nytiles);
-  if (!ddms && !qrec) { cth_set_error("score batch: query records not built"); return -1; }
-  if (!ddms)
-    hipLaunchKernelGGL((k_score_plain<0, true>), grid, dim3(256), 0, st, *q,
-                       reinterpret_cast<const query_record*>(qrec), 0, *db, (int64_t)0, ncols, ldsc, dtabs, scores,
-                       mods, tile, ytab, bq);
-  else
-    hipLaunchKernelGGL((k_score<false, true>), grid, dim3(256), 0, st, *q, 0, *db, (int64_t)0, ncols, ldsc, dtabs,
-                       scores, mods, qoff, ytab, bq);
+  const int ysplit = ddms ? tile / kDRows : 1;
+  if (ddms && tile % kDRows) { cth_set_error("score batch: row tiles of %d", tile); return -1; }
+  if ((int64_t)nytiles * ysplit > 65535) { cth_set_error("score batch: %d row tiles", nytiles); return -1; }
+  hipLaunchKernelGGL((k_score_plain<0, true>), dim3((ncols + kCols - 1) / kCols, nytiles), dim3(256), 0, st, *q,
+                     reinterpret_cast<const query_record*>(qrec), 0, *db, (int64_t)0, ncols, ldsc, dtabs, scores,
+                     mods, tile, ytab, bq);
+  CTH_HIP_CHECK(hipGetLastError());
+  if (!ddms) return 0;
+  hipLaunchKernelGGL(k_score_ddms<true>, dim3((ncols + kDCols - 1) / kDCols, nytiles * ysplit), dim3(kDThreads), 0, st,
+                     *q, 0, *db, (int64_t)0, ncols, ldsc, dtabs, scores, mods, qoff, ytab, ysplit, bq);
   CTH_HIP_CHECK(hipGetLastError());
   return 0;
 }
