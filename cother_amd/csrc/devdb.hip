@@ -176,7 +176,9 @@ extern "C" int cth_devset_upload(const cth_pset* h, cth_devset* s) {
 
 // The query set's distance lists as byte offsets into the 22 x 22 pair-score
 // table (value v -> row v, 22 floats per row), one 128-entry record per
-// position, so the score kernel adds the template value's column directly.
+// position, so the score kernel adds the template value's column directly:
+// entry k in the low half-word, entry k + 2 (the scan's next) in the high one;
+// record entry 0 is the length.
 extern "C" int cth_devset_make_ddoff(const cth_pset* h, cth_devset* s) {
   const int64_t n = h->npos;
   std::vector<int32_t> buf((size_t)std::max<int64_t>(n, 1) * CTH_DDSTRIDE);
@@ -188,6 +190,7 @@ extern "C" int cth_devset_make_ddoff(const cth_pset* h, cth_devset* s) {
       const uint8_t v = r[k];
       const int c = v == 255 ? CTH_DD_MISSING : (v < CTH_DMS_MAXDST ? v : CTH_DMS_MAXDST);
       o[k] = c * 22 * (int)sizeof(float);
+      if (k > 2) o[k - 2] |= o[k] << 16;
     }
   }
   if (s->ddoff) (void)hipFree(s->ddoff);

@@ -29,18 +29,24 @@ namespace {
 
 constexpr int kCols = 64;  // template columns per workgroup of the plain kernel (one per lane)
 
-// The distance-match scan's workgroup: kDRows query rows x kDCols template
-// columns, one cell per lane.
-constexpr int kDThreads = 512, kDRows = 16, kDCols = kDThreads / kDRows;
-constexpr int kListPitch = 132;  // LDS bytes per template list
-constexpr int kQlEntries = 112;  // query record entries the scan reads (0..111)
-constexpr int kQlPitch = 113;    // LDS words per query list: rows fall on different banks
+// The distance-match scan's workgroup: 256 cells, one per lane, as 32, 16 or
+// 8 query rows (the fewest that hold the tile's) x 8, 16 or 32 template
+// columns, whose lists are in LDS (eight workgroups a compute unit).
+constexpr int kDThreads = 256, kDRows = 32, kDRowsMin = 8;
+constexpr int kDColsMin = kDThreads / kDRows;
+constexpr int kDLists = kDRows + kDColsMin;
+static_assert(kDRowsMin + kDThreads / kDRowsMin <= kDLists, "lists of the lowest tile");
+constexpr int kListEntries = 112;  // entries of a list the scan reads (0..111)
+constexpr int kListPitch = 4 * 113;  // LDS bytes per list: lists fall on different banks
 constexpr float kSumScale = 0x1p-6f;  // of the distance-match sums (a segment's stays below 1)
 
 struct DdmsLds {
-  uint8_t tl[kDCols * kListPitch];  // template lists, values scaled by 4 (table byte columns)
-  int32_t ql[kDRows * kQlPitch];    // query lists as table byte offsets
-  float dms[22 * 22];               // the pair scores times kSumScale
+  // Lists as the pair table's byte rows (query lists, first) and byte columns
+  // (template lists), a word per entry: the entry in the low half-word, the
+  // one after next, with which the scan takes it, in the high one.  Entry 0
+  // is the length.
+  uint8_t list[kDLists * kListPitch];
+  float dms[22 * 22];  // the pair scores times kSumScale
 };
 
 __device__ __forceinline__ float ss_lookup(const float* ss, int row, int col) {
@@ -82,6 +88,7 @@ __device__ __forceinline__ uint32_t overlap(uint32_t sb, uint32_t se, uint32_t n
 // once (as booleans the compiler repeats those whose negation is also used)
 // and their combinations are scalar.
 __device__ __forceinline__ uint64_t mask_ge(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 3); }
+__device__ __forceinline__ uint64_t mask_gt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 2); }
 __device__ __forceinline__ uint64_t mask_zero(uint32_t a) { return __builtin_amdgcn_uicmp(a, 0u, 32); }
 __device__ __forceinline__ bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
@@ -177,10 +184,11 @@ __device__ __forceinline__ void register_max(ddms_register& R, float s, uint32_t
 // one 4-cell step, cells K0+1..K0+4 relative to the base ib, with the pair
 // scores S0, S2, S4 of cells K0 (the previous step's last cell), K0+2 and
 // K0+4, and FB the float 2^23 + the packed coordinates of cell K0+1 on both
-// axes.  A candidate's segment has 6 cells or more at a cell of the step, so
-// at least 3 at its first (dd1 <= -2): where no lane's has, the step ends
-// there.  The begin and end of the step's
-// best are recovered only when it can be registered.  Three levels: the
+// axes.  Where no lane has a sum or a positive score in the step every sum
+// stays 0 (and dd, which then counts for nothing, as it is).  A candidate's
+// segment has 6 cells or more at a cell of the step, so at least 3 at its
+// first (dd1 <= -2): where no lane's has, the step ends there.  The begin and
+// end of the step's best are recovered only when it can be registered.  Three levels: the
 // step's best is a candidate when it reaches m2 (empty most of the time: a
 // growing best segment drops it); a candidate whose segment already meets m0
 // with its end at the step's first cell and that scores below m0 is dropped
@@ -192,7 +200,7 @@ __device__ __forceinline__ void register_max(ddms_register& R, float s, uint32_t
 // without them the compiler folds their sums into each test as
 // scalar-operand adds, which issue one per cycle.
 #define CTH_DDMS_4CELL(S0, S2, S4, FB)                                        \
-  {                                                                           \
+  if (mask_gt(fmaxf(fmaxf(u, S2), S4), 0.0f) != 0) {                          \
     const float t1 = S0 + S2, t3 = S2 + S4;                                   \
     CTH_DDMS_CELL(u, dd, fmaf(t1, 0.5f, u), u1, dd1)                          \
     CTH_DDMS_CELL(u1, dd1, u1 + S2, u2, dd2)                                  \
@@ -200,7 +208,7 @@ __device__ __forceinline__ void register_max(ddms_register& R, float s, uint32_t
     CTH_DDMS_CELL(u3, dd3, u3 + S4, u4, dd4)                                  \
     u = u4;                                                                   \
     dd = dd4;                                                                 \
-    if (in_mask(mask_ge(-2.0f, dd1))) {                                       \
+    if (mask_ge(-2.0f, dd1) != 0) {                                           \
     const float cd1 = u1 * __builtin_amdgcn_fmed3f(-dd1 - 4.0f, 0.0f, 1.0f);  \
     const float cd2 = u2 * __builtin_amdgcn_fmed3f(-dd2 - 4.0f, 0.0f, 1.0f);  \
     const float cd3 = u3 * __builtin_amdgcn_fmed3f(-dd3 - 4.0f, 0.0f, 1.0f);  \
@@ -240,36 +248,36 @@ __device__ __forceinline__ void register_max(ddms_register& R, float s, uint32_t
     }                                                                         \
     }                                                                         \
   }
-// eight cells (two steps); the pair scores of the step after are loaded one
-// step ahead (lists are padded).  GUARD: whether the second step is due.
-#define CTH_DDMS_8CELL(GUARD)                                                 \
+// eight cells (two steps) from entry O on; the pair scores of the step after
+// are loaded one step ahead (lists are padded).  GUARD: whether the second
+// step is due.
+#define CTH_DDMS_8CELL(O, GUARD)                                              \
   {                                                                           \
-    const float n2 = pair(lds, lds_i32(lds, qo + 24), lds_u8(lds, to + 6));   \
-    const float n4 = pair(lds, lds_i32(lds, qo + 32), lds_u8(lds, to + 8));   \
-    CTH_DDMS_4CELL(s0, s2, s4, fb)                                            \
-    const float p2 = pair(lds, lds_i32(lds, qo + 40), lds_u8(lds, to + 10));  \
-    const float p4 = pair(lds, lds_i32(lds, qo + 48), lds_u8(lds, to + 12));  \
-    if (GUARD) CTH_DDMS_4CELL(s4, n2, n4, fb + 4.0f * kPackF)                 \
-    fb += 8.0f * kPackF;                                                      \
-    qo += 32;                                                                 \
-    to += 8;                                                                  \
-    asm("" : "+v"(qo), "+v"(to));                                             \
+    const uint32_t a6 = lds_u32(lds, qo + 4 * (O + 6)) + lds_u32(lds, to + 4 * (O + 6)); \
+    const float n2 = pair(lds, a6 & low), n4 = pair(lds, a6 >> 16);           \
+    CTH_DDMS_4CELL(s0, s2, s4, O ? fb + O * kPackF : fb)                      \
+    const uint32_t a10 = lds_u32(lds, qo + 4 * (O + 10)) + lds_u32(lds, to + 4 * (O + 10)); \
+    const float p2 = pair(lds, a10 & low), p4 = pair(lds, a10 >> 16);         \
+    if (GUARD) CTH_DDMS_4CELL(s4, n2, n4, fb + (O + 4) * kPackF)              \
     s0 = n4;                                                                  \
     s2 = p2;                                                                  \
     s4 = p4;                                                                  \
   }
+#define CTH_DDMS_ADVANCE(N)                                                   \
+  fb += N * kPackF;                                                           \
+  qo += 4 * N;                                                                \
+  to += 4 * N;                                                                \
+  asm("" : "+v"(qo), "+v"(to));
 
 // The scan reads everything from the workgroup's LDS block by byte offsets
-// held in vector registers, so that each table address is one vector add
-// (which dual-issues) and the rest is the instruction's immediate offset.
-// kDms: the pair-score table in the block
+// held in vector registers.  One add of two list words gives the table
+// offsets of two pairs.  kDms: the pair-score table in the block
 constexpr int kDms = (int)offsetof(DdmsLds, dms);
-__device__ __forceinline__ int lds_i32(const char* lds, int off) { return *reinterpret_cast<const int32_t*>(lds + off); }
-__device__ __forceinline__ int lds_u8(const char* lds, int off) { return *reinterpret_cast<const uint8_t*>(lds + off); }
-// the pair score of list values whose table byte offsets are qb (query,
-// d1*88) and tv (template, d2*4): dmsT[d1][d2]
-__device__ __forceinline__ float pair(const char* lds, int qb, int tv) {
-  return *reinterpret_cast<const float*>(lds + kDms + qb + tv);
+__device__ __forceinline__ uint32_t lds_u32(const char* lds, int off) {
+  return *reinterpret_cast<const uint32_t*>(lds + off);
+}
+__device__ __forceinline__ float pair(const char* lds, uint32_t off) {
+  return *reinterpret_cast<const float*>(lds + kDms + off);
 }
 
 // The shortest and the longest list of the wavefront's cells on each axis
@@ -278,16 +286,18 @@ struct ddms_lens {
   int qmin, qmax, tmin, tmax;
 };
 
-// lds: the workgroup's block; qr: byte offset of the lane's query list (int32
-// table byte offsets after entry 0); tr: byte offset of its template list
-// (values times 4 after byte 0); len1, len2: their lengths, at least DSTSEGM
+// lds: the workgroup's block; qr, tr: byte offsets of the lane's query and
+// template lists; len1, len2: their lengths, at least DSTSEGM
 __device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int len1, int len2, const ddms_lens& n) {
   ddms_register R{FLT_MIN, FLT_MIN, FLT_MIN, kNoBeginN, kNoEnd, kNoBeginN, kNoEnd};
   // 2^126, 1 + 2^11 and 2^120 in vector registers: as scalar operands they
-  // would keep the multiplies and fmas off the second issue slot
+  // would keep the multiplies and fmas off the second issue slot (the
+  // half-word mask the ands)
   float big, packf, big2;
   asm("v_mov_b32 %0, 0x7e800000" : "=v"(big));
   asm("v_mov_b32 %0, 0x7b800000" : "=v"(big2));  // 2^120
+  uint32_t low;
+  asm("v_mov_b32 %0, 0xffff" : "=v"(low));
   asm("v_mov_b32 %0, %1" : "=v"(packf) : "i"(__builtin_bit_cast(uint32_t, kPackF)));
   // the diagonals: upper ones j = len2>>2 .. 0 pair query index i with
   // template index j + i, lower ones i = len1>>2 .. 1 query index i + j with
@@ -304,18 +314,24 @@ __device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int 
                                : min(n.qmin - (n.qmin >> 2) + 2 * (k - upper), n.tmin);
     // byte offsets of the diagonal's first query and template entries,
     // advanced by one iteration (8 entries) at a time in vector registers
-    int qo = qr + 4 * (1 + i), to = tr + 1 + j;
-    float s0 = pair(lds, lds_i32(lds, qo), lds_u8(lds, to));
+    int qo = qr + 4 * (1 + i), to = tr + 4 * (1 + j);
+    const uint32_t a0 = lds_u32(lds, qo) + lds_u32(lds, to), a4 = lds_u32(lds, qo + 16) + lds_u32(lds, to + 16);
+    float s0 = pair(lds, a0 & low), s2 = pair(lds, a0 >> 16), s4 = pair(lds, a4 & low);
     float u = __builtin_amdgcn_fmed3f(s0, 0.0f, 1.0f);  // max(s0, 0)
     float dd = 0.0f;
     // 2^23 + the packed coordinates of cell 1 (query i + 1, template j + 1)
     float fb = __uint_as_float(kMagic + kPack + (uint32_t)i + ((uint32_t)j << 11));
-    float s2 = pair(lds, lds_i32(lds, qo + 8), lds_u8(lds, to + 2));
-    float s4 = pair(lds, lds_i32(lds, qo + 16), lds_u8(lds, to + 4));
     asm("" : "+v"(qo), "+v"(to));
     int ib = 0;
-    for (; ib + 4 < full; ib += 8) CTH_DDMS_8CELL(true)
-    for (; ib < cells; ib += 8) CTH_DDMS_8CELL(ib + 4 < cells)
+    for (; ib + 12 < full; ib += 16) {
+      CTH_DDMS_8CELL(0, true)
+      CTH_DDMS_8CELL(8, true)
+      CTH_DDMS_ADVANCE(16)
+    }
+    for (; ib < cells; ib += 8) {
+      CTH_DDMS_8CELL(0, ib + 4 < cells)
+      CTH_DDMS_ADVANCE(8)
+    }
   }
   float s = 0.0f;
   s += R.m0;
@@ -328,16 +344,31 @@ __device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int 
 #undef CTH_DDMS_CELL
 #undef CTH_DDMS_4CELL
 #undef CTH_DDMS_8CELL
+#undef CTH_DDMS_ADVANCE
 
 // Adds the distance-match term to the matrices that k_score_plain wrote.
 //
-// A wavefront covers kDRows query rows x 64 / kDRows template columns (each
-// lane a cell with its own two lists; in a tile of fewer rows more columns).
-// The register code of a step runs when any of the wavefront's lanes needs
-// it, and the lists of neighbouring positions are alike, on the query's side
-// most of all: replayed with the synthetic lists, a step reaches the
-// candidate test in 75% of a 1 x 64 wavefront's steps, 42% of an 8 x 8's and
-// 37% of a 16 x 4's, and changes a register in 31, 23 and 21%.
+// A wavefront covers 32 query rows x 2 template columns, each lane a cell with
+// its own two lists (a tile of fewer rows, as many as the next power of two
+// and more columns).  A part of a step runs when any of the wavefront's lanes
+// needs it, and the lists of neighbouring positions are alike, on the query's
+// side most of all.  Replayed with the synthetic lists, of a wavefront's steps
+// as 1 x 64, 8 x 8, 16 x 4 and 32 x 2 cells
+//   86, 55, 49, 47%  have a sum or a positive score,
+//   75, 42, 37, 34%  reach the candidate test,
+//   31, 23, 21, 20%  change a register;
+// 64 x 1 would be 43, 31 and 19%, but its query lists take the LDS of eight
+// workgroups.
+//
+// Bound by VALU issue: by the counters 15,600 instructions a wavefront in 9,500
+// issue slots of its 9,800 cycles (1 x 64 cells with every step's arithmetic
+// taken: 25,300 in 14,700).  The score stage of 250 positions against 4000
+// templates (median 220) takes 62.0 ms; with 16 x 4 cells, lists read an entry
+// at a time and no test for a step without sums 73.4, with 16 rows and words
+// of two 16-bit entries added by SDWA (which issue alone) 68.4.  Workgroups of
+// 512 lanes: 67.0 against 65.9 (a wavefront's place waits for the seven others).
+// Tiles of the fewest rows that hold a query's last ones: 40 positions against
+// 6000 templates 5.05 ms, with 32 x 8 tiles alone 6.4.
 // kBatch: the row tiles of several queries in one launch, ytab[blockIdx.y /
 // ysplit] giving query and first row of ysplit tiles of kDRows rows.
 template <bool kBatch>
@@ -359,33 +390,46 @@ __global__ __launch_bounds__(kDThreads) __attribute__((amdgpu_waves_per_eu(8, 8)
   }
   const int rows = min(kDRows, q.len[qp] - row0);
   if (rows <= 0) return;
+  // rows of a wavefront's cells, as a shift (a wavefront's columns lie within
+  // the tile's), and the tile's columns; workgroups past the last one leave
+  const int tqs = max(6 - __builtin_ctz(kDThreads / kDRowsMin), rows > 1 ? 32 - __builtin_clz(rows - 1) : 0);
+  const int cols = kDThreads >> max(tqs, __builtin_ctz(kDRowsMin));
+  const int c0 = blockIdx.x * cols;
+  if (c0 >= ncols) return;
   const int64_t q0 = q.dist[qp] + row0;
-  const int c0 = blockIdx.x * kDCols;
   for (int k = tid; k < 22 * 22; k += kDThreads) L.dms[k] = kSumScale * tabs->dms[k];
-  // template lists (32 dwords each), values (<= 21) times 4: the pair table's
-  // byte column; the length byte stays
-  for (int k = tid; k < kDCols * 32; k += kDThreads) {
-    const int c = k >> 5, d = k & 31;
-    uint32_t v = 0x15151500u;  // (an empty list's first dword)
-    if (c0 + c < ncols) v = reinterpret_cast<const uint32_t*>(db.dd + (size_t)(col0 + c0 + c) * CTH_DDSTRIDE)[d];
-    v = d == 0 ? (v & 0xffu) | ((v & 0xffffff00u) << 2) : v << 2;
-    *reinterpret_cast<uint32_t*>(&L.tl[c * kListPitch + d * 4]) = v;
-  }
   for (int k = tid; k < rows * 128; k += kDThreads) {
     const int r = k >> 7, e = k & 127;
-    if (e < kQlEntries) L.ql[r * kQlPitch + e] = qoff[(size_t)(q0 + r) * CTH_DDSTRIDE + e];
+    if (e < kListEntries)
+      *reinterpret_cast<int32_t*>(&L.list[r * kListPitch + 4 * e]) = qoff[(size_t)(q0 + r) * CTH_DDSTRIDE + e];
+  }
+  // template values (<= 21) times 4; the length byte stays
+  const int t0 = rows * kListPitch;
+  for (int k = tid; k < cols * 32; k += kDThreads) {
+    const int c = k >> 5, d = k & 31;
+    if (d >= kListEntries / 4) continue;
+    uint32_t v = 0, v1 = 0;  // (an empty list)
+    if (c0 + c < ncols) {
+      const uint32_t* const src = reinterpret_cast<const uint32_t*>(db.dd + (size_t)(col0 + c0 + c) * CTH_DDSTRIDE);
+      v = src[d];
+      v1 = src[d + 1];
+    }
+    v = d == 0 ? (v & 0xffu) | ((v & 0xffffff00u) << 2) : v << 2;
+    v1 <<= 2;
+    uint32_t* const dst = reinterpret_cast<uint32_t*>(&L.list[t0 + c * kListPitch + 16 * d]);
+    // bytes 0 and 2, 1 and 3, 2 and 4, 3 and 5
+    dst[0] = __builtin_amdgcn_perm(v1, v, 0x0c020c00u);
+    dst[1] = __builtin_amdgcn_perm(v1, v, 0x0c030c01u);
+    dst[2] = __builtin_amdgcn_perm(v1, v, 0x0c040c02u);
+    dst[3] = __builtin_amdgcn_perm(v1, v, 0x0c050c03u);
   }
   __syncthreads();
 
-  // rows of the wavefront's cells: the tile's, up to a power of two
-  // (at least two: 64 / 2 columns are the tile's)
-  static_assert(kDCols == 32 && kDRows <= 64, "a wavefront's columns lie within the tile");
-  const int tqs = rows > 2 ? 32 - __builtin_clz(rows - 1) : 1;
   const int r = lane >> (6 - tqs), c = (w << (6 - tqs)) + (lane & (63 >> tqs));
-  if ((w << (6 - tqs)) >= kDCols) return;
+  if ((w << (6 - tqs)) >= cols) return;
   const char* const lds = reinterpret_cast<const char*>(&L);
-  const int qr = (int)offsetof(DdmsLds, ql) + 4 * kQlPitch * min(r, rows - 1), tr = kListPitch * c;
-  const int len1 = lds_i32(lds, qr), len2 = lds_u8(lds, tr);
+  const int qr = kListPitch * min(r, rows - 1), tr = t0 + kListPitch * c;
+  const int len1 = (int)(lds_u32(lds, qr) & 0xff), len2 = (int)(lds_u32(lds, tr) & 0xff);
   const bool on = r < rows && c0 + c < ncols && len1 >= CTH_DSTSEGM && len2 >= CTH_DSTSEGM;
   ddms_lens n{on ? len1 : CTH_MAXDST, on ? len1 : 0, on ? len2 : CTH_MAXDST, on ? len2 : 0};
   for (int o = 32; o >= 1; o >>= 1) {
@@ -812,7 +856,7 @@ extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, const f
   }
   CTH_HIP_CHECK(hipGetLastError());
   if (!ddms) return 0;
-  hipLaunchKernelGGL(k_score_ddms<false>, dim3((ncols + kDCols - 1) / kDCols, (lq + kDRows - 1) / kDRows),
+  hipLaunchKernelGGL(k_score_ddms<false>, dim3((ncols + kDColsMin - 1) / kDColsMin, (lq + kDRows - 1) / kDRows),
                      dim3(kDThreads), 0, st, *q, qp, *db, col0, ncols, ldsc, dtabs, scores, mods, qoff, nullptr, 1,
                      nullptr);
   CTH_HIP_CHECK(hipGetLastError());
@@ -839,7 +883,7 @@ extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, c
                      mods, tile, ytab, bq);
   CTH_HIP_CHECK(hipGetLastError());
   if (!ddms) return 0;
-  hipLaunchKernelGGL(k_score_ddms<true>, dim3((ncols + kDCols - 1) / kDCols, nytiles * ysplit), dim3(kDThreads), 0, st,
+  hipLaunchKernelGGL(k_score_ddms<true>, dim3((ncols + kDColsMin - 1) / kDColsMin, nytiles * ysplit), dim3(kDThreads), 0, st,
                      *q, 0, *db, (int64_t)0, ncols, ldsc, dtabs, scores, mods, qoff, ytab, ysplit, bq);
   CTH_HIP_CHECK(hipGetLastError());
   return 0;
