@@ -1,20 +1,19 @@
 // batch.hip: the batched search -- many queries against the resident
 // database in one pass of fused, persistent launches.
 //
-// cth_search runs the pipeline query by query and chunk by chunk, with the
-// host choosing the next stage's profiles after each stage (four
-// synchronisations per chunk).  For a batch of queries whose buffers fit the
-// memory budget together, cth_search_batch instead runs every stage once
-// over all (query, profile) pairs of the batch, and decides on the device
-// which pairs go on to the next stage:
+// cth_search runs the pipeline query by query and chunk by chunk.  For a batch
+// of queries whose buffers fit the memory budget together, cth_search_batch
+// instead runs every stage once over all (query, profile) pairs of the batch,
+// and decides on the device which pairs go on to the next stage (as cth_search
+// does for a chunk of the database, cth_chunk_finish below):
 //   1. scores of every query of the batch (one launch, row tiles of all
 //      queries);
 //   2. phase-1 DP of every pair without traceback (persistent wavefronts
 //      taking pairs, longest first, from a device counter);
 //   3. pairs over their query's score threshold -> list (device compaction);
 //   4. DP with traceback and finalisation of the listed pairs (persistent);
-//   5. passed pairs -> list; their statistics (histogram in LDS, then the
-//      parameters and E-value; persistent);
+//   5. passed pairs -> list; their statistics (histogram, then the parameters
+//      and E-value; persistent);
 //   6. pairs within their query's E-value threshold -> list; MAP forward,
 //      backward, MAP DP and traceback of each in one persistent kernel;
 //   7. the hit records of the listed pairs gathered into one array.
@@ -57,8 +56,8 @@ extern "C" int cth_launch_dp_batch(const cth_dpset* q, const cth_dpset* db, cons
 extern "C" size_t cth_dp_batch_row_bytes(int grid, int ltmax);
 extern "C" int cth_launch_stats_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq,
                                       const cth_bpair* pairs, const int* list, const int* count, int64_t ldsc,
-                                      const float* scores, const cth_dpres* dpres, int ssemodel, double* out,
-                                      int grid, hipStream_t st);
+                                      const float* scores, const cth_dpres* dpres, int ssemodel, int lqmax, int* hist,
+                                      int cap, double* out, int grid, hipStream_t st);
 extern "C" int cth_launch_map_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq,
                                     const cth_bpair* pairs, const int* list, const int* count, int ltmax, int lqmax,
                                     int64_t ldsc, const float* scores, const float* mods, float* post, uint8_t* btck,
@@ -75,9 +74,12 @@ __global__ void k_batch_reset(int* ctr) {
 
 // Pairs whose phase-1 maximum exceeds their query's score threshold go to
 // the traceback pass (the only ones FinalizeDPPro traces back,
-// cudp/CuBatchDP_final.cu:144); the others get an empty record.
+// cudp/CuBatchDP_final.cu:144); the others get an empty record.  On the way the
+// statistics' histograms are cleared.
 __global__ void k_select_cand(const cth_bquery* __restrict__ bq, const cth_bpair* __restrict__ pairs, int npairs,
-                              cth_dpres* __restrict__ res, int* __restrict__ list, int* __restrict__ count) {
+                              cth_dpres* __restrict__ res, int* __restrict__ list, int* __restrict__ count,
+                              int* __restrict__ hist, int nhist) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nhist; i += gridDim.x * blockDim.x) hist[i] = 0;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < npairs; i += gridDim.x * blockDim.x) {
     cth_dpres r = res[i];
     if (bq[pairs[i].b].scorethld < r.maxsc) {
@@ -163,6 +165,11 @@ double now_ms() {
 
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
 
+// Pairs whose histograms k_hist_batch splits over workgroups: with more there
+// is a workgroup for each anyway.
+constexpr int kHistCap = 512;
+int hist_ints(int npairs) { return std::min(npairs, kHistCap) * 641; }
+
 // FNV-1a over the bytes of a plain struct
 uint64_t fnv(const void* p, size_t n) {
   uint64_t h = 1469598103934665603ull;
@@ -177,7 +184,7 @@ struct batch_layout {
   float* scores; float* mods; float* post; uint8_t* btck;
   // small
   cth_bquery* bq; cth_bytile* ytab; cth_bpair* pairs; cth_dpres* res; double* stats; cth_mapres* mres;
-  int* cand; int* passed; int* hitl; int* ctr; double* zrow; cth_hit* hits; char* alnout; float* grow;
+  int* cand; int* passed; int* hitl; int* hist; int* ctr; double* zrow; cth_hit* hits; char* alnout; float* grow;
 };
 
 // One batch's description on the host.
@@ -236,8 +243,8 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
                             S.dp_waves, st))
       return -1;
     const int sel_grid = std::max(1, std::min(1024, (npairs + 255) / 256));
-    hipLaunchKernelGGL(k_select_cand, dim3(sel_grid), dim3(256), 0, st, L.bq, L.pairs, npairs, L.res, L.cand,
-                       L.ctr + kCtrCand);
+    hipLaunchKernelGGL(k_select_cand, dim3(std::max(sel_grid, hist_ints(npairs) / 4096)), dim3(256), 0, st, L.bq, L.pairs, npairs, L.res, L.cand,
+                       L.ctr + kCtrCand, L.hist, hist_ints(npairs));
     CTH_HIP_CHECK(hipGetLastError());
     if (cth_launch_dp_batch(&c->q.d, &db.d, L.bq, L.pairs, L.cand, L.ctr + kCtrCand, 0, L.ctr + kCtrNext2, ltmax,
                             ldsc, L.scores, L.btck, L.res, L.grow, std::min(S.small_grid, npairs),
@@ -248,7 +255,8 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
     CTH_HIP_CHECK(hipGetLastError());
     if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[2], st));
     if (cth_launch_stats_batch(&c->q.d, &db.d, L.bq, L.pairs, L.passed, L.ctr + kCtrPassed, ldsc, L.scores, L.res,
-                               opt->ssemodel, L.stats, std::min(S.small_grid, npairs), st))
+                               opt->ssemodel, P.lqmax, L.hist, std::min(npairs, kHistCap), L.stats,
+                               std::min(S.small_grid, npairs), st))
       return -1;
     hipLaunchKernelGGL(k_select_hits, dim3(sel_grid), dim3(256), 0, st, L.bq, L.pairs, L.stats, L.passed,
                        L.ctr + kCtrPassed, L.hitl, L.ctr + kCtrHits);
@@ -280,7 +288,120 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
   return rc;
 }
 
+// A chunk's tables and counters, as the batched kernels read them: pair i is
+// the chunk's profile i of query 0.
+__global__ void k_chunk_tables(cth_bquery Q, int p0, int np, cth_bquery* __restrict__ bq,
+                               cth_bpair* __restrict__ pairs, int* __restrict__ ctr) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < np) pairs[i] = cth_bpair{0, p0 + i};
+  if (i < kNCtr) ctr[i] = 0;
+  if (i == 0) *bq = Q;
+}
+
+// hit records that come back with the counters
+constexpr int kFirstHits = 128;
+
+struct chunk_layout {
+  cth_bquery* bq; cth_bpair* pairs; double* stats; cth_mapres* mres; int* cand; int* passed; int* hitl; int* hist;
+  double* zrow; int* ctr; cth_hit* hits; char* alnout;
+  size_t bytes;
+};
+chunk_layout chunk_lay(const cth_chunk& k, int ncu, void* base) {
+  chunk_layout L;
+  size_t o = 0;
+  auto take = [&](size_t n) { void* p = (uint8_t*)base + o; o += up256(n); return p; };
+  const size_t np = (size_t)k.np;
+  L.bq = (cth_bquery*)take(sizeof(cth_bquery));
+  L.pairs = (cth_bpair*)take(sizeof(cth_bpair) * np);
+  L.stats = (double*)take(sizeof(double) * CTH_STATS_NOUT * np);
+  L.mres = (cth_mapres*)take(sizeof(cth_mapres) * np);
+  L.cand = (int*)take(sizeof(int) * np);
+  L.passed = (int*)take(sizeof(int) * np);
+  L.hitl = (int*)take(sizeof(int) * np);
+  L.hist = (int*)take(sizeof(int) * hist_ints(k.np));
+  L.zrow = (double*)take(sizeof(double) * std::min<size_t>(np, 4 * ncu) * k.lq);
+  L.ctr = (int*)take(sizeof(int) * 64);  // (the hit records follow at 256 bytes)
+  L.hits = (cth_hit*)take(sizeof(cth_hit) * np);
+  L.alnout = k.rows ? (char*)take(np * 5 * (size_t)(k.lq + k.ltmax)) : nullptr;
+  L.bytes = o;
+  return L;
+}
+
 }  // namespace
+
+size_t cth_chunk_work_bytes(const cth_chunk& k, int ncu) { return chunk_lay(k, ncu, nullptr).bytes; }
+
+// The stages after a chunk's first DP pass, chosen and run on the device as
+// the batched search does: one synchronisation, where the host's choice of the
+// next stage's profiles took four with copies of all records between them
+// (0.2-0.45 ms of a search).
+int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt, int ncu, void* work, hipEvent_t* ev,
+                     cth_chunk_hits& out) {
+  hipStream_t st = c->st;
+  const cth_dpset *q = &c->q.d, *db = &c->db.d;
+  const chunk_layout L = chunk_lay(k, ncu, work);
+  if (!c->h_pin) {
+    const size_t n = 256 + sizeof(cth_hit) * kFirstHits;
+    CTH_HIP_CHECK(hipHostMalloc(&c->h_pin, n));
+    c->cap_pin = n;
+  }
+  cth_bquery Q{};
+  Q.qp = k.qi;
+  Q.lq = k.lq;
+  Q.off = -k.col0;
+  Q.scorethld = k.scorethld;
+  Q.logethld = k.logethld;
+  Q.sspace = k.sspace;
+  const int W = std::min(8, std::max(1, (k.lq + 63) / 64));
+  const int grid = std::min(4 * ncu, k.np), sel = std::max(1, std::min(1024, (k.np + 255) / 256));
+  hipLaunchKernelGGL(k_chunk_tables, dim3((k.np + 255) / 256), dim3(256), 0, st, Q, k.p0, k.np, L.bq, L.pairs, L.ctr);
+  hipLaunchKernelGGL(k_select_cand, dim3(std::max(sel, hist_ints(k.np) / 4096)), dim3(256), 0, st, L.bq, L.pairs, k.np, k.res, L.cand, L.ctr + kCtrCand,
+                     L.hist, hist_ints(k.np));
+  CTH_HIP_CHECK(hipGetLastError());
+  if (cth_launch_dp_batch(q, db, L.bq, L.pairs, L.cand, L.ctr + kCtrCand, 0, L.ctr + kCtrNext2, k.ltmax, k.ldsc,
+                          k.scores, k.btck, k.res, nullptr, grid, W, st))
+    return -1;
+  hipLaunchKernelGGL(k_select_passed, dim3(sel), dim3(256), 0, st, k.res, L.cand, L.ctr + kCtrCand, L.passed,
+                     L.ctr + kCtrPassed);
+  CTH_HIP_CHECK(hipGetLastError());
+  if (ev) CTH_HIP_CHECK(hipEventRecord(ev[0], st));
+  if (cth_launch_stats_batch(q, db, L.bq, L.pairs, L.passed, L.ctr + kCtrPassed, k.ldsc, k.scores, k.res,
+                             opt->ssemodel, k.lq, L.hist, std::min(k.np, kHistCap), L.stats, grid, st))
+    return -1;
+  hipLaunchKernelGGL(k_select_hits, dim3(sel), dim3(256), 0, st, L.bq, L.pairs, L.stats, L.passed,
+                     L.ctr + kCtrPassed, L.hitl, L.ctr + kCtrHits);
+  CTH_HIP_CHECK(hipGetLastError());
+  if (ev) CTH_HIP_CHECK(hipEventRecord(ev[1], st));
+  out.rowcap = k.lq + k.ltmax;
+  if (opt->do_map &&
+      cth_launch_map_batch(q, db, L.bq, L.pairs, L.hitl, L.ctr + kCtrHits, k.ltmax, k.lq, k.ldsc, k.scores, k.mods,
+                           k.post, k.btck, L.stats, L.zrow, opt->minpp > 0.0f ? opt->minpp : CTH_MINPP, L.alnout,
+                           out.rowcap, L.mres, grid, W, st))
+    return -1;
+  hipLaunchKernelGGL(k_gather_hits, dim3(sel), dim3(256), 0, st, L.bq, L.pairs, k.res, L.stats, L.mres, opt->do_map,
+                     L.hitl, L.ctr + kCtrHits, L.hits);
+  CTH_HIP_CHECK(hipGetLastError());
+  if (ev) CTH_HIP_CHECK(hipEventRecord(ev[2], st));
+  const int first = std::min(k.np, kFirstHits);
+  CTH_HIP_CHECK(hipMemcpyAsync(c->h_pin, L.ctr, 256 + sizeof(cth_hit) * first, hipMemcpyDeviceToHost, st));
+  CTH_HIP_CHECK(hipStreamSynchronize(st));
+  const int* const ctr = (const int*)c->h_pin;
+  const int nb = ctr[kCtrHits];
+  out.npassed = ctr[kCtrPassed];
+  out.hits.resize(nb);
+  out.rows.clear();
+  if (nb) memcpy(out.hits.data(), (const uint8_t*)c->h_pin + 256, sizeof(cth_hit) * std::min(nb, first));
+  if (nb > first)
+    CTH_HIP_CHECK(hipMemcpyAsync(out.hits.data() + first, L.hits + first, sizeof(cth_hit) * (nb - first),
+                                 hipMemcpyDeviceToHost, st));
+  if (nb && L.alnout && opt->do_map) {
+    out.rows.resize((size_t)nb * 5 * out.rowcap);
+    CTH_HIP_CHECK(hipMemcpyAsync(out.rows.data(), L.alnout, out.rows.size(), hipMemcpyDeviceToHost, st));
+  }
+  if (nb > first || !out.rows.empty()) CTH_HIP_CHECK(hipStreamSynchronize(st));
+  std::sort(out.hits.begin(), out.hits.end(), [](const cth_hit& a, const cth_hit& b) { return a.profile < b.profile; });
+  return 0;
+}
 
 namespace {
 
@@ -449,7 +570,7 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
                           up256(sizeof(cth_bpair) * npairs) + up256(sizeof(cth_dpres) * npairs) +
                           up256(sizeof(double) * CTH_STATS_NOUT * npairs) + up256(sizeof(cth_mapres) * npairs) +
                           3 * up256(sizeof(int) * npairs) + up256(sizeof(int) * kNCtr) +
-                          up256(sizeof(double) * (size_t)small_max * P.lqmax) + up256(sizeof(cth_hit) * npairs) +
+                          up256(sizeof(int) * hist_ints(npairs)) + up256(sizeof(double) * (size_t)small_max * P.lqmax) + up256(sizeof(cth_hit) * npairs) +
                           up256(alnbytes) + up256(growbytes);
     if (cth_ctx_reserve(c, &c->bcells, &c->cap_bcells, cbytes)) return -1;
     if (cth_ctx_reserve(c, &c->bsmall, &c->cap_bsmall, sbytes)) return -1;
@@ -474,6 +595,7 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
       L.passed = (int*)takes(sizeof(int) * npairs);
       L.hitl = (int*)takes(sizeof(int) * npairs);
       L.ctr = (int*)takes(sizeof(int) * kNCtr);
+      L.hist = (int*)takes(sizeof(int) * hist_ints(npairs));
       L.zrow = (double*)takes(sizeof(double) * (size_t)small_max * P.lqmax);
       L.hits = (cth_hit*)takes(sizeof(cth_hit) * npairs);
       L.alnout = alnbytes ? (char*)takes(alnbytes) : nullptr;

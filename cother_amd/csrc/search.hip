@@ -5,15 +5,18 @@
 // resident database whose score buffers fit the memory budget, the score
 // matrix, phase-1 DP and its finalisation run on the context's stream; the
 // passed profiles of the chunk then get their statistics (and, with MAP
-// enabled, the MAP alignment stage).  Host work is limited to the score
+// enabled, the MAP alignment stage).  The device chooses each stage's profiles
+// (cth_chunk_finish, batch.hip), or the host after each stage where profiles
+// need boundary rows in global memory or no device memory may be allocated.
+// Other host work is limited to the score
 // threshold (JobDispatcher::CalculateScoreThreshold,
 // cualn/JobDispatcher.cpp:806-860), the search-space length adjustment
 // (AbstractScoreMatrix::ComputeLengthAdjustment,
-// libpro/srcsco/AbstractScoreMatrix.cpp:303-395), the passed-profile lists and
-// the final hit ordering.
+// libpro/srcsco/AbstractScoreMatrix.cpp:303-395) and the final hit ordering.
 //
-// Deterministic by construction: passed profiles are taken in database order
-// (the reference appends them in atomic order, cudp/CuBatchDP_final.cu:260-264)
+// Deterministic by construction: a profile's records do not depend on the
+// order in which profiles pass (the reference appends them in atomic order,
+// cudp/CuBatchDP_final.cu:260-264), alignment rows are stored in database order
 // and hits are sorted by (log E-value, database index) (the reference's sort is
 // unstable, cupro/CuBatchProcessingFinalizer.cpp:289-292).
 #include <hip/hip_runtime.h>
@@ -284,6 +287,22 @@ extern "C" int cth_search_opts_check(const cth_search_opts* opt, const char* who
 
 namespace {
 
+// Append a hit's five rows of alnlen letters each, in reading order, to the
+// caller's buffer (src: in traceback order, rowcap letters apart).
+int append_rows(const cth_search_opts* opt, const char* src, size_t rowcap, cth_hit& h, uint64_t* used,
+                const char* who) {
+  const size_t n = (size_t)h.alnlen;
+  if (*used + 5 * n > opt->alncap) {
+    cth_set_error("%s: alignment buffer full (%llu bytes)", who, (unsigned long long)opt->alncap);
+    return -1;
+  }
+  h.alnoff = *used;
+  for (int r = 0; r < 5; r++)
+    for (size_t m = 0; m < n; m++) opt->alnbuf[*used + r * n + m] = src[r * rowcap + n - 1 - m];
+  *used += 5 * n;
+  return 0;
+}
+
 // The whole per-query pipeline; its per-chunk device buffers come from bufs.
 int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* hits, int maxhits, int* nhits,
                cth_search_stats* stats, chunk_bufs& bufs) {
@@ -307,6 +326,12 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
     for (int k = 0; k < 4; k++) CTH_HIP_CHECK(hipEventCreate(&c->ev[k]));
     c->has_ev = 1;
   }
+  if (timing && c->nbev < 5) {
+    CTH_HIP_CHECK(hipEventCreate(&c->ev[4]));
+    c->nbev = 5;
+  }
+  int ncu = 0;
+  CTH_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
   int nh = 0;
   uint64_t alnused = 0;
   cth_search_stats st{};
@@ -375,6 +400,45 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
                                  0, dpout + (a2 - p0), grow, c->st))
             return -1;
         }
+      }
+      // the rest on the device, unless the buffers are fixed, profiles need
+      // boundary rows in global memory (sized for the candidates), or the
+      // alignment rows of all profiles would be more than kRowsCap
+      constexpr size_t kRowsCap = (size_t)256 << 20;
+      cth_chunk k{qi, lq, p0, p1 - p0, ltchunk, col0, ldsc, scorethld, logethld, sspace, scores, mods, nullptr, btck,
+                  dpout, opt->alnbuf && opt->do_map ? 1 : 0};
+      if (!bufs.fixed && ltchunk <= CTH_DP_GLOBAL_FROM &&
+          (!k.rows || (size_t)k.np * 5 * (size_t)(lq + ltchunk) <= kRowsCap)) {
+        if (opt->do_map && !(k.post = bufs.map_buffer(lq, ldsc))) return -1;
+        void* const work = bufs.work(cth_chunk_work_bytes(k, ncu));
+        if (!work) return -1;
+        cth_chunk_hits got;
+        if (cth_chunk_finish(c, k, opt, ncu, work, timing ? c->ev + 2 : nullptr, got)) return -1;
+        if (timing) {
+          float ms[4];
+          for (int e = 0; e < 4; e++) CTH_HIP_CHECK(hipEventElapsedTime(&ms[e], c->ev[e], c->ev[e + 1]));
+          st.ms_k_score += ms[0];
+          st.ms_k_dp += ms[1];
+          st.ms_k_stats += ms[2];
+          st.ms_k_map += ms[3];
+        }
+        st.ms_phase1 += now_ms() - t0;
+        st.cells += (double)lq * (double)ncols;
+        st.npassed += got.npassed;
+        st.nchunks += 1;
+        for (cth_hit& h : got.hits) {
+          if (opt->do_map) st.map_cells += (double)lq * (double)db.h_len[h.profile];
+          if (opt->do_map && h.alnlen < 1) continue;
+          if (nh >= maxhits) { cth_set_error("%s: hit buffer full (%d)", who, maxhits); return -1; }
+          const size_t slot = (size_t)h.alnoff;
+          h.alnoff = 0;
+          if (k.rows &&
+              append_rows(opt, got.rows.data() + slot * 5 * (size_t)got.rowcap, (size_t)got.rowcap, h, &alnused, who))
+            return -1;
+          hits[nh++] = h;
+        }
+        p0 = p1;
+        continue;
       }
       if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[2], c->st));
       std::vector<cth_dpres> res(p1 - p0);
@@ -582,17 +646,7 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
           h.pstvs_map = mres[k].psts;
           h.mapscore = mres[k].maxsc;
           if (opt->alnbuf) {
-            // five rows of alnlen letters each, in reading order
-            const size_t n = (size_t)mres[k].alnlen;
-            if (alnused + 5 * n > opt->alncap) {
-              cth_set_error("%s: alignment buffer full (%llu bytes)", who, (unsigned long long)opt->alncap);
-              return -1;
-            }
-            h.alnoff = alnused;
-            const char* src = hrows.data() + k * 5 * (size_t)rowcap;
-            for (int r = 0; r < 5; r++)
-              for (size_t m = 0; m < n; m++) opt->alnbuf[alnused + r * n + m] = src[r * (size_t)rowcap + n - 1 - m];
-            alnused += 5 * n;
+            if (append_rows(opt, hrows.data() + k * 5 * (size_t)rowcap, (size_t)rowcap, h, &alnused, who)) return -1;
           }
         }
       }

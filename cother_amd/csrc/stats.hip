@@ -555,16 +555,51 @@ __global__ __launch_bounds__(kThreads) void k_stats(const cth_dpset q, int qp, c
                out + (int64_t)k * CTH_STATS_NOUT);
 }
 
+// Histograms of the *count passed pairs listed in list into hist (zeroed, one
+// per list slot), where they are at most cap: rows over workgroups as in
+// cth_launch_stats.  More pairs leave theirs to k_stats_batch.
+__global__ __launch_bounds__(kThreads) void k_hist_batch(const cth_dpset q, const cth_dpset db,
+                                                         const cth_bquery* __restrict__ bq,
+                                                         const cth_bpair* __restrict__ pairs,
+                                                         const int* __restrict__ list, const int* __restrict__ count,
+                                                         int64_t ldsc, const float* __restrict__ scores, int lqmax,
+                                                         int* __restrict__ hist, int cap) {
+  __shared__ int h[kNssc * kCopies];
+  const int nj = *count;
+  if (nj < 1 || nj > cap) return;
+  const int split = max(1, min(1024 / nj, (lqmax + 15) / 16));
+  for (int u = blockIdx.x; u < nj * split; u += gridDim.x) {
+    const int k = u / split;
+    const cth_bpair pr = pairs[list[k]];
+    const cth_bquery Q = bq[pr.b];
+    const int ny = (Q.lq + split - 1) / split;
+    const int y0 = (u - k * split) * ny, y1 = min(Q.lq, y0 + ny);
+    if (y0 >= y1) continue;
+    for (int b = threadIdx.x; b < kNssc * kCopies; b += kThreads) h[b] = 0;
+    __syncthreads();
+    hist_fill(q, Q.qp, db, pr.p, db.dist[pr.p], ldsc, scores + Q.off, y0, y1, h);
+    __syncthreads();
+    for (int b = threadIdx.x; b < kNssc; b += kThreads) {
+      int n = 0;
+      for (int i = 0; i < kCopies; i++) n += h[b * kCopies + i];
+      if (n) atomicAdd(&hist[(int64_t)k * kNssc + b], n);
+    }
+    __syncthreads();
+  }
+}
+
 // Batched statistics over the *count passed pairs listed in list
-// (persistent, one workgroup per pair at a time): histogram in LDS, then the
-// parameters and significance against the pair's query's search space; out
-// and dpres are per pair.
+// (persistent, one workgroup per pair at a time): its histogram from
+// k_hist_batch, or in LDS where those are more than cap, then the parameters
+// and significance against the pair's query's search space; out and dpres are
+// per pair.
 __global__ __launch_bounds__(kThreads) void k_stats_batch(const cth_dpset q, const cth_dpset db,
                                                           const cth_bquery* __restrict__ bq,
                                                           const cth_bpair* __restrict__ pairs,
                                                           const int* __restrict__ list, const int* __restrict__ count,
                                                           int64_t ldsc, const float* __restrict__ scores,
                                                           const cth_dpres* __restrict__ dpres, int ssemodel,
+                                                          const int* __restrict__ hist, int cap,
                                                           double* __restrict__ out) {
   __shared__ int h[kNssc * kCopies];
   const int nj = *count;
@@ -572,10 +607,13 @@ __global__ __launch_bounds__(kThreads) void k_stats_batch(const cth_dpset q, con
     const int i = list[k];
     const cth_bpair pr = pairs[i];
     const cth_bquery Q = bq[pr.b];
-    for (int b = threadIdx.x; b < kNssc * kCopies; b += kThreads) h[b] = 0;
+    for (int b = threadIdx.x; b < kNssc * kCopies; b += kThreads)
+      h[b] = nj <= cap && b % kCopies == 0 ? hist[(int64_t)k * kNssc + b / kCopies] : 0;
     __syncthreads();
-    hist_fill(q, Q.qp, db, pr.p, db.dist[pr.p], ldsc, scores + Q.off, 0, Q.lq, h);
-    __syncthreads();
+    if (nj > cap) {
+      hist_fill(q, Q.qp, db, pr.p, db.dist[pr.p], ldsc, scores + Q.off, 0, Q.lq, h);
+      __syncthreads();
+    }
     stats_one<kCopies>(q, Q.qp, db, pr.p, h, Q.sspace, ssemodel, dpres[i], out + (int64_t)i * CTH_STATS_NOUT);
     __syncthreads();
   }
@@ -605,15 +643,19 @@ extern "C" int cth_launch_stats(const cth_dpset* q, int qp, int lq, const cth_dp
   return 0;
 }
 
-// Batched statistics (k_stats_batch) on a persistent grid of `grid`
-// workgroups over the *count pairs of list; out: CTH_STATS_NOUT doubles per pair.
+// Batched statistics (k_hist_batch, k_stats_batch) on a persistent grid of
+// `grid` workgroups over the *count pairs of list; hist: cap x 641 zeroed ints;
+// lqmax: the longest query; out: CTH_STATS_NOUT doubles per pair.
 extern "C" int cth_launch_stats_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq,
                                       const cth_bpair* pairs, const int* list, const int* count, int64_t ldsc,
-                                      const float* scores, const cth_dpres* dpres, int ssemodel, double* out,
-                                      int grid, hipStream_t st) {
+                                      const float* scores, const cth_dpres* dpres, int ssemodel, int lqmax, int* hist,
+                                      int cap, double* out, int grid, hipStream_t st) {
   if (grid < 1) return 0;
+  hipLaunchKernelGGL(k_hist_batch, dim3(1024), dim3(kThreads), 0, st, *q, *db, bq, pairs, list, count, ldsc, scores,
+                     lqmax, hist, cap);
+  CTH_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(k_stats_batch, dim3(grid), dim3(kThreads), 0, st, *q, *db, bq, pairs, list, count, ldsc, scores,
-                     dpres, ssemodel, out);
+                     dpres, ssemodel, hist, cap, out);
   CTH_HIP_CHECK(hipGetLastError());
   return 0;
 }
