@@ -618,6 +618,7 @@ extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_
                                   float scorethld, int finalize, cth_dpres* res, float* grow, hipStream_t st) {
   if (np <= 0) return 0;
   if (finalize && !btck) { cth_set_error("dp: finalisation needs the traceback"); return -1; }
+  if (finalize && ldsc % 4) { cth_set_error("dp: rows of %lld traceback bytes", (long long)ldsc); return -1; }
   if (ltmax > CTH_MAXCOLUMNS) { cth_set_error("dp: profile length %d over %d", ltmax, CTH_MAXCOLUMNS); return -1; }
   const bool global = ltmax > CTH_DP_GLOBAL_FROM;
   if (global && !grow) { cth_set_error("dp: profile length %d needs global boundary rows", ltmax); return -1; }
@@ -665,6 +666,7 @@ extern "C" int cth_launch_dp_batch(const cth_dpset* q, const cth_dpset* db, cons
                                    float* grow, int grid, int W, hipStream_t st) {
   if (grid < 1) return 0;
   if (W < 1 || W > kMaxWaves) { cth_set_error("dp batch: %d wavefronts per pair", W); return -1; }
+  if (btck && ldsc % 4) { cth_set_error("dp batch: rows of %lld traceback bytes", (long long)ldsc); return -1; }
   const bool global = ltmax > CTH_DP_GLOBAL_FROM;
   if (global && !grow) { cth_set_error("dp batch: profile length %d needs global boundary rows", ltmax); return -1; }
   const size_t lds = W * dp_wave_lds(global) + dp_row_lds(ltmax, global);

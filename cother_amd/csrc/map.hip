@@ -882,6 +882,7 @@ extern "C" int cth_launch_map(const cth_dpset* q, int qp, int lq, const cth_dpse
                               char* alnout, int rowcap, cth_mapres* res, float* grow, hipStream_t st) {
   if (njobs <= 0) return 0;
   if (ltmax > CTH_MAXCOLUMNS) { cth_set_error("map: profile length %d over %d", ltmax, CTH_MAXCOLUMNS); return -1; }
+  if (ldsc % 4) { cth_set_error("map: rows of %lld traceback bytes", (long long)ldsc); return -1; }
   if (alnout && rowcap < lq + ltmax) { cth_set_error("map: row capacity %d < %d", rowcap, lq + ltmax); return -1; }
   const bool global = ltmax > CTH_LDS_ROW_MAX;
   if (global && !grow) { cth_set_error("map: profile length %d needs global boundary rows", ltmax); return -1; }
@@ -914,6 +915,7 @@ extern "C" int cth_launch_map_batch(const cth_dpset* q, const cth_dpset* db, con
                                     const double* stats, double* zrow, float minpp, char* alnout, int rowcap,
                                     cth_mapres* res, int grid, int W, hipStream_t st) {
   if (ltmax > CTH_LDS_ROW_MAX) { cth_set_error("map batch: profile length %d over the LDS row limit", ltmax); return -1; }
+  if (ldsc % 4) { cth_set_error("map batch: rows of %lld traceback bytes", (long long)ldsc); return -1; }
   if (W < 1 || W > kMaxWaves) { cth_set_error("map batch: %d wavefronts per pair", W); return -1; }
   if (grid < 1) return 0;
   const size_t lds = W * map_wave_lds(false) + map_row_lds(ltmax, false);

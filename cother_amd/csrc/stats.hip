@@ -129,14 +129,35 @@ __device__ void grid_bounds(int y, int* left, int* right) {
   *left = l; *right = r;
 }
 
+// v with the lanes moved by a DPP control (lanes without a source: 0)
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, kCtrl, kRowMask, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), kCtrl, kRowMask, 0xf, false);
+  return v + __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+// The wavefront's sum of v, in every lane: within rows of 16 lanes, then over
+// the rows, in the DPP moves' fixed order (a shuffle waits for the LDS).
+__device__ __forceinline__ double wave_sum(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15, :31
+  v = dpp_add<0x143, 0xc>(v);
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, 63);
+  const uint32_t hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
 // The workgroup's sums (and extremes) of two doubles per thread, to every
-// thread: a butterfly in each wavefront, then the wavefronts in order.  red:
+// thread: a sum in each wavefront, then the wavefronts in order.  red:
 // 2 kWaves doubles of LDS.
 __device__ __forceinline__ void block_sum2(double& a, double& b, double* red) {
-  for (int off = 32; off >= 1; off >>= 1) {
-    a += __shfl_xor(a, off);
-    b += __shfl_xor(b, off);
-  }
+  a = wave_sum(a);
+  b = wave_sum(b);
   const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) { red[2 * w] = a; red[2 * w + 1] = b; }
   __syncthreads();
@@ -313,12 +334,50 @@ constexpr double kSS18MinScale = (double)0.1f, kSS18Log001 = (double)-4.60517018
                  kSS18NbdProb = (double)0.757213f, kSS18EbmDfo2 = (double)1.346206f,
                  kSS18EbmC = (double)1.485656f;
 
-// significance of one alignment, out = [lmbdest, kest, logE, logEpA]: SSEMODEL
-// 0 observed statistics, 1 and 2 the SS18 model and its variant
-__device__ void significance(int ssemodel, int lq, int lt, double qeno, double teno, double searchspace, double score,
-                             double psts, double lambda, double K, double* out) {
-  const double lref = CTH_UNGAP_LAMBDA, kref = CTH_UNGAP_K, lg = CTH_GAPPED_LAMBDA, kg = CTH_GAPPED_K;
+// The significance of one alignment in parts that do not wait for each other:
+// what follows from the profiles and the positives alone, what follows from
+// lambda, and the rest.
+struct sig_parts {
+  double emu, logpp;  // network of the effective lengths; positives' log p-value
+  double lmu, lsc;    // networks of lambda
+};
+
+// emu and logpp (SS18; PredictEVDParametersSS18, cuss/CuBatchSS_SS18.cuh:119-233)
+__device__ void sig_profiles(int lq, int lt, double qeno, double teno, double psts, sig_parts& S) {
   const double ln1k = 6.90775527898213681510242167860;
+  double in[4];
+  double e1 = qeno, e2 = teno;
+  int n1 = lq, n2 = lt;
+  if (e1 < e2) { double t = e1; e1 = e2; e2 = t; int u = n1; n1 = n2; n2 = u; }
+  else if (e1 == e2 && n1 < n2) { int u = n1; n1 = n2; n2 = u; }
+  in[0] = (double)0.05f * e1; in[1] = log((double)n1) / ln1k;
+  in[2] = (double)0.05f * e2; in[3] = log((double)n2) / ln1k;
+  S.emu = nn_out(in, c_nnw, 30.0);
+  const double l1l2 = (double)(float)((uint32_t)lq * (uint32_t)lt);
+  const double lp = l1l2 < 625.0 ? 625.0 : l1l2;
+  const double pn = rint(100000.0 * psts / pow(lp, 1.5));
+  S.logpp = lbetainc(pn + 1.0, kSS18NbdShape, kSS18NbdProb);
+}
+
+// lmu and lsc
+__device__ void sig_lambda(int lq, int lt, double lambda, sig_parts& S) {
+  const double ln1k = 6.90775527898213681510242167860;
+  double in[4];
+  double lm = rint(lambda * 10.0) / 10.0;
+  if (lm <= 0.0) lm = 0.1;
+  if (10.0 < lm) lm = 10.0;
+  int n1 = lq, n2 = lt;
+  if (n1 < n2) { int u = n1; n1 = n2; n2 = u; }
+  in[0] = (double)0.2f * lm; in[1] = log((double)n1) / ln1k; in[2] = log((double)n2) / ln1k; in[3] = 0.0;
+  S.lmu = nn_out(in, c_nnw + 25, 30.0);
+  S.lsc = nn_out(in, c_nnw + 50, 5.0);
+}
+
+// out = [lmbdest, kest, logE, logEpA]: SSEMODEL 0 observed statistics (S not
+// used), 1 and 2 the SS18 model and its variant
+__device__ void significance(int ssemodel, int lq, int lt, double searchspace, double score, double lambda, double K,
+                             const sig_parts& S, double* out) {
+  const double lref = CTH_UNGAP_LAMBDA, kref = CTH_UNGAP_K, lg = CTH_GAPPED_LAMBDA, kg = CTH_GAPPED_K;
   out[0] = 0.0; out[1] = 0.0;
   if (0.0 < lambda) out[0] = lambda * (lg / lref);
   if (0.0 < K) out[1] = K * (kg / kref);
@@ -332,27 +391,7 @@ __device__ void significance(int ssemodel, int lq, int lt, double qeno, double t
     out[2] = log(kg * searchspace) - lg * score;
     return;
   }
-  // PredictEVDParametersSS18 (cuss/CuBatchSS_SS18.cuh:119-233)
-  double in[4];
-  {
-    double e1 = qeno, e2 = teno;
-    int n1 = lq, n2 = lt;
-    if (e1 < e2) { double t = e1; e1 = e2; e2 = t; int u = n1; n1 = n2; n2 = u; }
-    else if (e1 == e2 && n1 < n2) { int u = n1; n1 = n2; n2 = u; }
-    in[0] = (double)0.05f * e1; in[1] = log((double)n1) / ln1k;
-    in[2] = (double)0.05f * e2; in[3] = log((double)n2) / ln1k;
-  }
-  double emu = nn_out(in, c_nnw, 30.0);
-  {
-    double lm = rint(lambda * 10.0) / 10.0;
-    if (lm <= 0.0) lm = 0.1;
-    if (10.0 < lm) lm = 10.0;
-    int n1 = lq, n2 = lt;
-    if (n1 < n2) { int u = n1; n1 = n2; n2 = u; }
-    in[0] = (double)0.2f * lm; in[1] = log((double)n1) / ln1k; in[2] = log((double)n2) / ln1k; in[3] = 0.0;
-  }
-  double lmu = nn_out(in, c_nnw + 25, 30.0);
-  double lsc = nn_out(in, c_nnw + 50, 5.0);
+  double emu = S.emu, lmu = S.lmu, lsc = S.lsc;
   const float* adj = ssemodel == 2 ? c_nnw + 84 : c_nnw + 75;
   if (emu < 3.0) emu = 3.0;
   if (lmu < 3.0) lmu = 3.0;
@@ -391,10 +430,7 @@ __device__ void significance(int ssemodel, int lq, int lt, double qeno, double t
       else logp = log(1.0 - exp(-t));
     }
   }
-  const double lp = l1l2 < 625.0 ? 625.0 : l1l2;
-  const double pn = rint(100000.0 * psts / pow(lp, 1.5));
-  const double logpp = lbetainc(pn + 1.0, kSS18NbdShape, kSS18NbdProb);
-  logp = lgammaincq(kSS18EbmDfo2, (-logp - logpp) / kSS18EbmC);
+  logp = lgammaincq(kSS18EbmDfo2, (-logp - S.logpp) / kSS18EbmC);
   logexp = logp;
   if (kSS18Log001 <= logp) {
     const double p = exp(logp);
@@ -403,6 +439,70 @@ __device__ void significance(int ssemodel, int lq, int lt, double qeno, double t
   }
   logexp += log(searchspace / l1l2);
   out[2] = logexp;
+}
+
+// The sigma series of K (cuss/CuBatchSS_K.cuh) by one wavefront: the sum over j
+// of P_j / j for unscaled scores minu..maxu of probabilities pu, lambda.  A
+// cell's next value is the sum over i of G[c - i] pu[i], the grid's rows being
+// 32 scores apart and its cells consecutive.  Only cells of scores within +-32
+// get values, 66 consecutive ones: a lane's two are in registers with their
+// weights exp(lambda min(score, 0)), and the values in LDS need no barriers.
+// G: the grid at the start, which this overwrites around those cells.
+//
+// 32 turns over all 672 cells on the workgroup, its barriers and shuffles, took
+// 61 us of a profile's 92.
+__device__ double sigma_series(int minu, int maxu, double lambda, double* G, const double* pu) {
+  constexpr int kFirst = 10 * kScale - 17, kActive = 66;  // scores -32..16 and 16..32
+  const int lane = threadIdx.x & 63, range = maxu - minu + 1;
+  int cell[2], sc[2];
+  double weight[2];
+  bool on[2];
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    const int k = min(lane + 64 * s, kActive - 1);
+    cell[s] = kFirst + k;
+    sc[s] = k < 49 ? k - 32 : k - 33;
+    const double e = sc[s] < 0 ? lambda * (double)sc[s] : 0.0;
+    on[s] = lane + 64 * s < kActive && kLogSpMin < e;
+    weight[s] = exp(e);
+  }
+  double sigma = 0.0, Pj = 1.0;
+  int minscore = minu, maxscore = maxu;
+  for (int j = 1; j <= 32 && 1.0e-4 < Pj; j++) {
+    int lo[2], hi[2];
+    double v[2] = {0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      lo[s] = maxscore - sc[s] < range ? maxu - (maxscore - sc[s]) : minu;
+      hi[s] = sc[s] - minscore < range ? minu + (sc[s] - minscore) : maxu;
+      if (!(on[s] && minscore <= sc[s] && sc[s] <= maxscore)) hi[s] = lo[s] - 1;
+    }
+    for (int i = minu; i <= maxu; i += 4) {
+      double g[2][4], p[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        p[u] = pu[min(i + u + 10, kNSC - 1)];
+        g[0][u] = G[cell[0] - i - u];
+        g[1][u] = G[cell[1] - i - u];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+          if (lo[s] <= i + u && i + u <= hi[s]) v[s] += g[s][u] * p[u];
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (j == 1 && lane < 13) G[kFirst - 1 - lane] = G[kFirst + kActive + lane] = 0.0;
+    G[cell[0]] = v[0];
+    if (lane + 64 < kActive) G[cell[1]] = v[1];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    Pj = wave_sum(v[0] * weight[0] + v[1] * weight[1]);
+    sigma += Pj / j;
+    minscore += minu;
+    maxscore += maxu;
+  }
+  return sigma;
 }
 
 // The statistics of one passed profile p (one workgroup): parameters from
@@ -414,10 +514,12 @@ __device__ void significance(int ssemodel, int lq, int lt, double qeno, double t
 template <int kHistCopies>
 __device__ __forceinline__ void stats_one(const cth_dpset& q, int qp, const cth_dpset& db, int p, const int* hc,
                                           double searchspace, int ssemodel, const cth_dpres& r, double* o) {
-  __shared__ double G[kNSC * kScale], NG[kNSC * kScale];
+  __shared__ double G[kNSC * kScale];
   __shared__ double pu[kNSC];
   __shared__ double red[2 * kWaves];
-  const int tid = threadIdx.x;
+  __shared__ sig_parts S;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lq = q.len[qp], lt = db.len[p];
   auto bin = [&](int b) {
     int n = 0;
     for (int i = 0; i < kHistCopies; i++) n += hc[b * kHistCopies + i];
@@ -482,8 +584,9 @@ __device__ __forceinline__ void stats_one(const cth_dpset& q, int qp, const cth_
     if (v < umn) umn = v;
     if (v > umx) umx = v;
   }
+  // K on wavefront 0, meanwhile the significance's independent parts on two others
   double K = -1.0;
-  if (!(0.0 <= E || lambda <= 0.0 || H <= 0.0)) {
+  if (w == 0 && !(0.0 <= E || lambda <= 0.0 || H <= 0.0)) {
     if (umn == -1.0 && umx == 1.0) {
       const double a = pu[9], b = pu[11];
       K = (a - b) * (a - b) / a;
@@ -491,54 +594,18 @@ __device__ __forceinline__ void stats_one(const cth_dpset& q, int qp, const cth_
       if (umx != 1.0) K = lambda / H * (1.0 - exp(-lambda)) * (E * E);
       else K = H / lambda * (1.0 - exp(-lambda));
     } else {
-      const int minu = (int)umn, maxu = (int)umx, range = (int)(umx - umn + 1.0);
-      double sigma = 0.0, Pj = 1.0;
-      int minscore = minu, maxscore = maxu;
-      for (int j = 1; j <= 32 && 1.0e-4 < Pj; j++) {
-        double sum = 0.0;
-        for (int ic = 0; ic < kCells; ic++) {
-          const int c = tid + kThreads * ic;
-          if (c >= kNSC * kScale) continue;
-          const int y = c / kScale, x = c - y * kScale;
-          double pji = 0.0;
-          const int sc = (int)C.sc[ic];
-          if (minscore <= sc && sc <= maxscore && -32 <= sc && sc <= 32) {
-            const double etols = sc < 0 ? lambda * (double)sc : 0.0;
-            if (kLogSpMin < etols) {
-              const int mnu = (maxscore - sc < range) ? maxu - (maxscore - sc) : minu;
-              const int mxu = (sc - minscore < range) ? minu + (sc - minscore) : maxu;
-              for (int i = mnu; i <= mxu; i++) {
-                int yy = y, xx = x - i;
-                if (kScale <= xx) {
-                  xx -= kScale;
-                  if (yy + 1 < kNSC) yy++; else continue;
-                } else if (xx < 0) {
-                  xx += kScale;
-                  if (0 < yy) yy--; else continue;
-                }
-                pji += G[yy * kScale + xx] * pu[i + 10];
-              }
-              sum += pji * exp(etols);
-            }
-          }
-          NG[c] = pji;
-        }
-        zero = 0.0;
-        block_sum2(sum, zero, red);
-        for (int c = tid; c < kNSC * kScale; c += kThreads) G[c] = NG[c];
-        __syncthreads();
-        Pj = sum;
-        sigma += Pj / j;
-        minscore += minu;
-        maxscore += maxu;
-      }
+      const double sigma = sigma_series((int)umn, (int)umx, lambda, G, pu);
       K = lambda * exp(-2.0 * sigma) / (H * (1.0 - exp(-lambda)));
     }
   }
+  if (ssemodel != 0 && (tid & 63) == 0) {
+    if (w == 1) sig_profiles(lq, lt, (double)q.eno[qp], (double)db.eno[p], (double)r.psts, S);
+    if (w == 2) sig_lambda(lq, lt, lambda, S);
+  }
+  __syncthreads();
   if (tid == 0) {
     double sig[4];
-    significance(ssemodel, q.len[qp], db.len[p], (double)q.eno[qp], (double)db.eno[p], searchspace,
-                 (double)r.score, (double)r.psts, lambda, K, sig);
+    significance(ssemodel, lq, lt, searchspace, (double)r.score, lambda, K, S, sig);
     o[CTH_ST_LMBDEST] = sig[0]; o[CTH_ST_KEST] = sig[1]; o[CTH_ST_LOGE] = sig[2]; o[CTH_ST_LOGEPA] = sig[3];
     o[CTH_ST_MIN] = umn; o[CTH_ST_MAX] = umx; o[CTH_ST_E] = E; o[CTH_ST_H] = H;
     o[CTH_ST_LMBD] = lambda; o[CTH_ST_K] = K;
