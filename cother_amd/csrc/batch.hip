@@ -62,7 +62,9 @@ extern "C" int cth_launch_map_batch(const cth_dpset* q, const cth_dpset* db, con
                                     const cth_bpair* pairs, const int* list, const int* count, int ltmax, int lqmax,
                                     int64_t ldsc, const float* scores, const float* mods, float* post, uint8_t* btck,
                                     const double* stats, double* zrow, float minpp, char* alnout, int rowcap,
-                                    cth_mapres* res, int grid, int W, hipStream_t st);
+                                    cth_mapres* res, int grid, int W, int nsplit, float* back, hipStream_t st);
+extern "C" int cth_map_split(int lq, int ltmax, int npairs);
+extern "C" size_t cth_map_split_bytes(int lq, int ltmax, int n);
 
 namespace {
 
@@ -184,7 +186,7 @@ struct batch_layout {
   float* scores; float* mods; float* post; uint8_t* btck;
   // small
   cth_bquery* bq; cth_bytile* ytab; cth_bpair* pairs; cth_dpres* res; double* stats; cth_mapres* mres;
-  int* cand; int* passed; int* hitl; int* hist; int* ctr; double* zrow; cth_hit* hits; char* alnout; float* grow;
+  int* cand; int* passed; int* hitl; int* hist; int* ctr; double* zrow; cth_hit* hits; char* alnout; float* grow; float* back;
 };
 
 // One batch's description on the host.
@@ -202,7 +204,7 @@ struct batch_plan {
 // Grids of the persistent launches (workgroups) and wavefronts per pair of
 // the two DP passes.
 struct launch_shape {
-  int dp_grid, dp_waves, small_grid, trace_waves;
+  int dp_grid, dp_waves, small_grid, map_grid, trace_waves;
 };
 
 // One wavefront per pair where the pairs fill the chip (128,000 pairs of 99 x
@@ -219,6 +221,7 @@ launch_shape choose_shape(int ncu, int npairs, int lqmax, int ltmax) {
   S.trace_waves = stripes;
   S.dp_grid = ncu * (ltmax > CTH_DP_GLOBAL_FROM ? 8 : 16);
   S.small_grid = ncu * 4;
+  S.map_grid = ncu * 16;  // (2000 pairs of 130 positions: 2.85 ms with four per unit, 2.1 with one per pair)
   return S;
 }
 
@@ -265,7 +268,8 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
     if (opt->do_map &&
         cth_launch_map_batch(&c->q.d, &db.d, L.bq, L.pairs, L.hitl, L.ctr + kCtrHits, ltmax, P.lqmax, ldsc, L.scores,
                              L.mods, L.post, L.btck, L.stats, L.zrow, opt->minpp > 0.0f ? opt->minpp : CTH_MINPP,
-                             L.alnout, rowcap, L.mres, std::min(S.small_grid, npairs), S.trace_waves, st))
+                             L.alnout, rowcap, L.mres, std::min(S.map_grid, npairs), S.trace_waves,
+                             cth_map_split(P.lqmax, ltmax, npairs), L.back, st))
       return -1;
     hipLaunchKernelGGL(k_gather_hits, dim3(sel_grid), dim3(256), 0, st, L.bq, L.pairs, L.res, L.stats, L.mres,
                        opt->do_map, L.hitl, L.ctr + kCtrHits, L.hits);
@@ -300,10 +304,13 @@ __global__ void k_chunk_tables(cth_bquery Q, int p0, int np, cth_bquery* __restr
 
 // hit records that come back with the counters
 constexpr int kFirstHits = 128;
+// the MAP stage's workgroups per compute unit, as choose_shape's
+constexpr int kChunkMapGrid = 16;
 
 struct chunk_layout {
   cth_bquery* bq; cth_bpair* pairs; double* stats; cth_mapres* mres; int* cand; int* passed; int* hitl; int* hist;
-  double* zrow; int* ctr; cth_hit* hits; char* alnout;
+  double* zrow; int* ctr; cth_hit* hits; char* alnout; float* back;
+  int nsplit;
   size_t bytes;
 };
 chunk_layout chunk_lay(const cth_chunk& k, int ncu, void* base) {
@@ -319,10 +326,12 @@ chunk_layout chunk_lay(const cth_chunk& k, int ncu, void* base) {
   L.passed = (int*)take(sizeof(int) * np);
   L.hitl = (int*)take(sizeof(int) * np);
   L.hist = (int*)take(sizeof(int) * hist_ints(k.np));
-  L.zrow = (double*)take(sizeof(double) * std::min<size_t>(np, 4 * ncu) * k.lq);
+  L.zrow = (double*)take(sizeof(double) * std::min<size_t>(np, kChunkMapGrid * ncu) * k.lq);
   L.ctr = (int*)take(sizeof(int) * 64);  // (the hit records follow at 256 bytes)
   L.hits = (cth_hit*)take(sizeof(cth_hit) * np);
   L.alnout = k.rows ? (char*)take(np * 5 * (size_t)(k.lq + k.ltmax)) : nullptr;
+  L.nsplit = k.post ? cth_map_split(k.lq, k.ltmax, k.np) : 0;
+  L.back = (float*)take(cth_map_split_bytes(k.lq, k.ltmax, L.nsplit));
   L.bytes = o;
   return L;
 }
@@ -376,7 +385,7 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
   if (opt->do_map &&
       cth_launch_map_batch(q, db, L.bq, L.pairs, L.hitl, L.ctr + kCtrHits, k.ltmax, k.lq, k.ldsc, k.scores, k.mods,
                            k.post, k.btck, L.stats, L.zrow, opt->minpp > 0.0f ? opt->minpp : CTH_MINPP, L.alnout,
-                           out.rowcap, L.mres, grid, W, st))
+                           out.rowcap, L.mres, std::min(kChunkMapGrid * ncu, k.np), W, L.nsplit, L.back, st))
     return -1;
   hipLaunchKernelGGL(k_gather_hits, dim3(sel), dim3(256), 0, st, L.bq, L.pairs, k.res, L.stats, L.mres, opt->do_map,
                      L.hitl, L.ctr + kCtrHits, L.hits);
@@ -564,6 +573,8 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
     const size_t cells = (size_t)P.cells;
     const size_t cbytes = up256(4 * cells) * (opt->do_map ? 3 : 2) + up256(cells);
     const int small_max = std::max(1, std::min(npairs, ncu * 32));
+    const size_t backbytes =
+        opt->do_map ? cth_map_split_bytes(P.lqmax, ltmax, cth_map_split(P.lqmax, ltmax, npairs)) : 0;
     const launch_shape S = choose_shape(ncu, npairs, P.lqmax, ltmax);
     const size_t growbytes = cth_dp_batch_row_bytes(std::min(npairs, std::max(S.dp_grid, S.small_grid)), ltmax);
     const size_t sbytes = up256(sizeof(cth_bquery) * P.bq.size()) + up256(sizeof(cth_bytile) * P.ytab.size()) +
@@ -571,7 +582,7 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
                           up256(sizeof(double) * CTH_STATS_NOUT * npairs) + up256(sizeof(cth_mapres) * npairs) +
                           3 * up256(sizeof(int) * npairs) + up256(sizeof(int) * kNCtr) +
                           up256(sizeof(int) * hist_ints(npairs)) + up256(sizeof(double) * (size_t)small_max * P.lqmax) + up256(sizeof(cth_hit) * npairs) +
-                          up256(alnbytes) + up256(growbytes);
+                          up256(alnbytes) + up256(growbytes) + up256(backbytes);
     if (cth_ctx_reserve(c, &c->bcells, &c->cap_bcells, cbytes)) return -1;
     if (cth_ctx_reserve(c, &c->bsmall, &c->cap_bsmall, sbytes)) return -1;
     batch_layout L{};
@@ -600,6 +611,7 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
       L.hits = (cth_hit*)takes(sizeof(cth_hit) * npairs);
       L.alnout = alnbytes ? (char*)takes(alnbytes) : nullptr;
       L.grow = growbytes ? (float*)takes(growbytes) : nullptr;
+      L.back = backbytes ? (float*)takes(backbytes) : nullptr;
     }
     // the batch's tables (outside the graph: a replayed graph reads the current ones)
     CTH_HIP_CHECK(hipMemcpyAsync(L.bq, P.bq.data(), sizeof(cth_bquery) * P.bq.size(), hipMemcpyHostToDevice, c->st));

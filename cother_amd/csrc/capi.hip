@@ -362,7 +362,9 @@ extern "C" int cth_phase2_block(cth_ctx* c, int qidx, int p0, int p1, float scor
 extern "C" int cth_launch_map(const cth_dpset* q, int qp, int lq, const cth_dpset* db, const cth_mapjob* jobs,
                               int njobs, int ltmax, int64_t col0, int64_t ldsc, const float* scores,
                               const float* mods, float* post, uint8_t* btck, double* zrow, float minpp,
-                              char* alnout, int rowcap, cth_mapres* res, float* grow, hipStream_t st);
+                              char* alnout, int rowcap, cth_mapres* res, float* grow, float* back, hipStream_t st);
+extern "C" int cth_map_split(int lq, int ltmax, int npairs);
+extern "C" size_t cth_map_split_bytes(int lq, int ltmax, int n);
 
 // Score matrix of query qidx against template profiles [p0,p1), then the MAP
 // stage for njobs of them (absolute indices profiles[], log pair E-values
@@ -397,7 +399,9 @@ extern "C" int cth_map_block(cth_ctx* c, int qidx, int p0, int p1, const int32_t
   if (cth_ctx_reserve(c, (void**)&c->btck, &c->cap_btck, (size_t)lq * ldsc)) return -1;
   const size_t wneed = sizeof(double) * (size_t)njobs * lq + sizeof(cth_mapjob) * njobs +
                        sizeof(cth_mapres) * njobs + 512;
-  if (cth_ctx_reserve(c, &c->work, &c->cap_work, wneed)) return -1;
+  // (backward values of their own where the jobs are few)
+  const size_t split = cth_map_split(lq, ltmax, njobs) == njobs ? cth_map_split_bytes(lq, ltmax, njobs) : 0;
+  if (cth_ctx_reserve(c, &c->work, &c->cap_work, wneed + split)) return -1;
   double* d_zrow = (double*)c->work;
   cth_mapjob* d_jobs = (cth_mapjob*)(d_zrow + (size_t)njobs * lq);
   cth_mapres* d_res = (cth_mapres*)(((uintptr_t)(d_jobs + njobs) + 15) & ~(uintptr_t)15);
@@ -409,7 +413,7 @@ extern "C" int cth_map_block(cth_ctx* c, int qidx, int p0, int p1, const int32_t
   if (rows && cth_ctx_reserve(c, (void**)&c->grow, &c->cap_grow, rows)) return -1;
   if (cth_launch_map(&c->q.d, qidx, lq, &c->db.d, d_jobs, njobs, ltmax, col0, ldsc, c->scores + CTH_SCORE_PAD, c->mods + CTH_SCORE_PAD,
                      (float*)c->mapbuf + CTH_SCORE_PAD, c->btck, d_zrow, minpp, nullptr, lq + ltmax, d_res, rows ? c->grow : nullptr,
-                     c->st))
+                     split ? (float*)(((uintptr_t)(d_res + njobs) + 255) & ~(uintptr_t)255) : nullptr, c->st))
     return -1;
   CTH_HIP_CHECK(hipMemcpyAsync(res, d_res, sizeof(cth_mapres) * njobs, hipMemcpyDeviceToHost, c->st));
   CTH_HIP_CHECK(hipStreamSynchronize(c->st));

@@ -49,7 +49,7 @@ extern "C" int cth_launch_stats(const cth_dpset* q, int qp, int lq, const cth_dp
 extern "C" int cth_launch_map(const cth_dpset* q, int qp, int lq, const cth_dpset* db, const cth_mapjob* jobs,
                               int njobs, int ltmax, int64_t col0, int64_t ldsc, const float* scores,
                               const float* mods, float* post, uint8_t* btck, double* zrow, float minpp,
-                              char* alnout, int rowcap, cth_mapres* res, float* grow, hipStream_t st);
+                              char* alnout, int rowcap, cth_mapres* res, float* grow, float* back, hipStream_t st);
 
 namespace {
 
@@ -582,13 +582,13 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
         if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[3], c->st));
         const float minpp = opt->minpp > 0.0f ? opt->minpp : CTH_MINPP;
         if (cth_launch_map(&c->q.d, qi, lq, &db.d, d_jobs, nms, ltms, col0, ldsc, scores, mods, post, btck, d_zrow,
-                           minpp, d_aln, rowcap, d_res, nullptr, c->st))
+                           minpp, d_aln, rowcap, d_res, nullptr, nullptr, c->st))
           return -1;
         for (int j = nms; j < nj; j += nbm) {
           const int n = std::min(nbm, nj - j);
           if (cth_launch_map(&c->q.d, qi, lq, &db.d, d_jobs + j, n, ltm, col0, ldsc, scores, mods, post, btck,
                              d_zrow + (size_t)j * lq, minpp, d_aln ? d_aln + (size_t)j * 5 * rowcap : nullptr, rowcap,
-                             d_res + j, grow, c->st))
+                             d_res + j, grow, nullptr, c->st))
             return -1;
         }
         if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[0], c->st));
