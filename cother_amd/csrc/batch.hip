@@ -93,12 +93,14 @@ __global__ void k_select_cand(const cth_bquery* __restrict__ bq, const cth_bpair
   }
 }
 
-// passed pairs of the traceback pass -> list
+// passed pairs of the traceback pass -> list; that pass took the *ncand pairs of
+// cand, or (null) all npairs
 __global__ void k_select_passed(const cth_dpres* __restrict__ res, const int* __restrict__ cand,
-                                const int* __restrict__ ncand, int* __restrict__ list, int* __restrict__ count) {
-  const int n = *ncand;
+                                const int* __restrict__ ncand, int npairs, int* __restrict__ list,
+                                int* __restrict__ count) {
+  const int n = cand ? *ncand : npairs;
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-    const int i = cand[k];
+    const int i = cand ? cand[k] : k;
     if (res[i].passed) list[atomicAdd(count, 1)] = i;
   }
 }
@@ -253,8 +255,8 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
                             ldsc, L.scores, L.btck, L.res, L.grow, std::min(S.small_grid, npairs),
                             S.trace_waves, st))
       return -1;
-    hipLaunchKernelGGL(k_select_passed, dim3(sel_grid), dim3(256), 0, st, L.res, L.cand, L.ctr + kCtrCand, L.passed,
-                       L.ctr + kCtrPassed);
+    hipLaunchKernelGGL(k_select_passed, dim3(sel_grid), dim3(256), 0, st, L.res, L.cand, L.ctr + kCtrCand, npairs,
+                       L.passed, L.ctr + kCtrPassed);
     CTH_HIP_CHECK(hipGetLastError());
     if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[2], st));
     if (cth_launch_stats_batch(&c->q.d, &db.d, L.bq, L.pairs, L.passed, L.ctr + kCtrPassed, ldsc, L.scores, L.res,
@@ -293,10 +295,12 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
 }
 
 // A chunk's tables and counters, as the batched kernels read them: pair i is
-// the chunk's profile i of query 0.
+// the chunk's profile i of query 0; and the statistics' histograms cleared.
 __global__ void k_chunk_tables(cth_bquery Q, int p0, int np, cth_bquery* __restrict__ bq,
-                               cth_bpair* __restrict__ pairs, int* __restrict__ ctr) {
+                               cth_bpair* __restrict__ pairs, int* __restrict__ ctr, int* __restrict__ hist,
+                               int nhist) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  for (int k = i; k < nhist; k += gridDim.x * blockDim.x) hist[k] = 0;
   if (i < np) pairs[i] = cth_bpair{0, p0 + i};
   if (i < kNCtr) ctr[i] = 0;
   if (i == 0) *bq = Q;
@@ -363,15 +367,20 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
   Q.sspace = k.sspace;
   const int W = std::min(8, std::max(1, (k.lq + 63) / 64));
   const int grid = std::min(4 * ncu, k.np), sel = std::max(1, std::min(1024, (k.np + 255) / 256));
-  hipLaunchKernelGGL(k_chunk_tables, dim3((k.np + 255) / 256), dim3(256), 0, st, Q, k.p0, k.np, L.bq, L.pairs, L.ctr);
-  hipLaunchKernelGGL(k_select_cand, dim3(std::max(sel, hist_ints(k.np) / 4096)), dim3(256), 0, st, L.bq, L.pairs, k.np, k.res, L.cand, L.ctr + kCtrCand,
-                     L.hist, hist_ints(k.np));
+  const int nhist = hist_ints(k.np);
+  hipLaunchKernelGGL(k_chunk_tables, dim3(std::max((k.np + 255) / 256, nhist / 4096)), dim3(256), 0, st, Q, k.p0, k.np,
+                     L.bq, L.pairs, L.ctr, L.hist, nhist);
   CTH_HIP_CHECK(hipGetLastError());
-  if (cth_launch_dp_batch(q, db, L.bq, L.pairs, L.cand, L.ctr + kCtrCand, 0, L.ctr + kCtrNext2, k.ltmax, k.ldsc,
-                          k.scores, k.btck, k.res, nullptr, grid, W, st))
-    return -1;
-  hipLaunchKernelGGL(k_select_passed, dim3(sel), dim3(256), 0, st, k.res, L.cand, L.ctr + kCtrCand, L.passed,
-                     L.ctr + kCtrPassed);
+  if (!k.traced) {
+    hipLaunchKernelGGL(k_select_cand, dim3(sel), dim3(256), 0, st, L.bq, L.pairs, k.np, k.res, L.cand,
+                       L.ctr + kCtrCand, nullptr, 0);
+    CTH_HIP_CHECK(hipGetLastError());
+    if (cth_launch_dp_batch(q, db, L.bq, L.pairs, L.cand, L.ctr + kCtrCand, 0, L.ctr + kCtrNext2, k.ltmax, k.ldsc,
+                            k.scores, k.btck, k.res, nullptr, grid, W, st))
+      return -1;
+  }
+  hipLaunchKernelGGL(k_select_passed, dim3(sel), dim3(256), 0, st, k.res, k.traced ? nullptr : L.cand,
+                     L.ctr + kCtrCand, k.np, L.passed, L.ctr + kCtrPassed);
   CTH_HIP_CHECK(hipGetLastError());
   if (ev) CTH_HIP_CHECK(hipEventRecord(ev[0], st));
   if (cth_launch_stats_batch(q, db, L.bq, L.pairs, L.passed, L.ctr + kCtrPassed, k.ldsc, k.scores, k.res,

@@ -27,7 +27,8 @@ struct cth_chunk {
   float* post;
   uint8_t* btck;
   cth_dpres* res;
-  int rows;  // alignment rows wanted
+  int rows;    // alignment rows wanted
+  int traced;  // the first pass left traceback bytes and finalised records
 };
 // What the rest of its pipeline leaves: the hit records in profile order (their
 // alnoff a slot of rows, 5 x rowcap letters each), before those without an

@@ -372,18 +372,39 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
                            opt->contraction, ddms, c->st))
         return -1;
       if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[1], c->st));
+      // the stages after the first DP pass on the device, unless the buffers are
+      // fixed, profiles need boundary rows in global memory (sized for the
+      // candidates), or the alignment rows of all profiles would be more than
+      // kRowsCap
+      constexpr size_t kRowsCap = (size_t)256 << 20;
+      const int np = p1 - p0;
+      cth_chunk k{qi, lq, p0, np, ltchunk, col0, ldsc, scorethld, logethld, sspace, scores, mods, nullptr, btck,
+                  dpout, opt->alnbuf && opt->do_map ? 1 : 0, 0};
+      const bool ondevice = !bufs.fixed && ltchunk <= CTH_DP_GLOBAL_FROM &&
+                            (!k.rows || (size_t)np * 5 * (size_t)(lq + ltchunk) <= kRowsCap);
       // phase 1 in two passes: the DP of every profile without traceback,
       // then, for the profiles whose maximum exceeds the score threshold (the
       // only ones FinalizeDPPro traces back, cudp/CuBatchDP_final.cu:144),
-      // the same DP with traceback and the finalisation.  The first pass runs
-      // in groups of consecutive profiles, each launch reserving LDS for its
-      // own longest profile, so that groups of shorter profiles (databases
-      // are sorted by length) run more wavefronts per CU.
+      // the same DP with traceback and the finalisation.  Where every profile
+      // has a compute unit to itself one pass with traceback takes no longer
+      // than the second would (61 positions against 96 templates: 50 us
+      // instead of 30 + 50).
+      // The first pass runs in groups of consecutive profiles, each launch
+      // reserving LDS for its own longest profile (databases are sorted by
+      // length).  A launch ends with few profiles in flight, so groups are
+      // small only where the LDS of long profiles leaves few workgroups a
+      // compute unit: 165 positions against 6000 templates of up to 830 0.69 ms
+      // in one launch, 0.78 in groups of 2048; of up to 1500, uniform, 2.43 and
+      // 2.31.
       // Profiles longer than CTH_DP_GLOBAL_FROM keep their stripe boundary rows
       // in the work area, in launches of as many profiles as their rows fit.
-      constexpr int kDpGroup = 2048;
-      for (int a = p0; a < p1; a += kDpGroup) {
-        const int b = std::min(p1, a + kDpGroup);
+      k.traced = ondevice && np <= ncu;
+      if (k.traced && cth_launch_dp_list(&c->q.d, qi, lq, &db.d, p0, nullptr, np, ltchunk, col0, ldsc, scores, btck,
+                                         scorethld, 1, dpout, nullptr, c->st))
+        return -1;
+      constexpr int kDpGroup = 16384, kDpGroupLong = 2048, kDpLong = 1024;
+      for (int a = k.traced ? p1 : p0, b; a < p1; a = b) {
+        b = std::min(p1, a + (db.h_len[a] > kDpLong ? kDpGroupLong : kDpGroup));
         int lg = 0;
         for (int p = a; p < b; p++) lg = std::max(lg, db.h_len[p]);
         int nb = b - a;
@@ -401,14 +422,7 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
             return -1;
         }
       }
-      // the rest on the device, unless the buffers are fixed, profiles need
-      // boundary rows in global memory (sized for the candidates), or the
-      // alignment rows of all profiles would be more than kRowsCap
-      constexpr size_t kRowsCap = (size_t)256 << 20;
-      cth_chunk k{qi, lq, p0, p1 - p0, ltchunk, col0, ldsc, scorethld, logethld, sspace, scores, mods, nullptr, btck,
-                  dpout, opt->alnbuf && opt->do_map ? 1 : 0};
-      if (!bufs.fixed && ltchunk <= CTH_DP_GLOBAL_FROM &&
-          (!k.rows || (size_t)k.np * 5 * (size_t)(lq + ltchunk) <= kRowsCap)) {
+      if (ondevice) {
         if (opt->do_map && !(k.post = bufs.map_buffer(lq, ldsc))) return -1;
         void* const work = bufs.work(cth_chunk_work_bytes(k, ncu));
         if (!work) return -1;
