@@ -249,8 +249,8 @@ extern "C" int cth_score_block(cth_ctx* c, int qidx, int p0, int p1, float* h_sc
   return cth_score_block_ex(c, qidx, p0, p1, 0, h_scores, h_mods);
 }
 
-extern "C" int cth_launch_dp(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int np, int ltmax,
-                             int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck, float scorethld,
+extern "C" int cth_launch_dp(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int np, int ltmean,
+                             int ltmax, int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck, float scorethld,
                              cth_dpres* res, float* grow, hipStream_t st);
 extern "C" size_t cth_dp_row_bytes(int np, int ltmax);
 extern "C" size_t cth_map_row_bytes(int njobs, int ltmax);
@@ -297,7 +297,7 @@ extern "C" int cth_phase1_block(cth_ctx* c, int qidx, int p0, int p1, float scor
   // boundary rows in global memory for profiles over the LDS row limit
   const size_t rows = cth_dp_row_bytes(p1 - p0, ltmax);
   if (rows && cth_ctx_reserve(c, (void**)&c->grow, &c->cap_grow, rows)) return -1;
-  if (cth_launch_dp(&c->q.d, qidx, lq, &c->db.d, p0, p1 - p0, ltmax, col0, ldsc, c->scores + CTH_SCORE_PAD, c->btck, scorethld,
+  if (cth_launch_dp(&c->q.d, qidx, lq, &c->db.d, p0, p1 - p0, (int)(ncols / (p1 - p0)), ltmax, col0, ldsc, c->scores + CTH_SCORE_PAD, c->btck, scorethld,
                     (cth_dpres*)c->dpout, rows ? c->grow : nullptr, c->st))
     return -1;
   CTH_HIP_CHECK(hipStreamSynchronize(c->st));

@@ -27,7 +27,7 @@ constexpr int kSweepLag = 3;
 __host__ __device__ __forceinline__ int sweep_phases(int lt) { return ((lt + 31) >> 5) + 2; }
 
 // the phase of the pair's schedule in which stripe s starts
-__device__ __forceinline__ int sweep_start(int s, int W, int P) {
+__host__ __device__ __forceinline__ int sweep_start(int s, int W, int P) {
   const int round = s / W, period = P > kSweepLag * W ? P : kSweepLag * W;
   return round * period + (s - round * W) * kSweepLag;
 }

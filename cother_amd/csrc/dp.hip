@@ -574,8 +574,39 @@ extern "C" size_t cth_dp_row_bytes(int np, int ltmax) {
 
 namespace {
 
-// Wavefronts per pair: one per stripe up to kMaxWaves.
-int dp_waves(int lq) { return std::max(1, std::min(kMaxWaves, (lq + 63) / 64)); }
+// Wavefronts per pair of np pairs of queries of lq positions and profiles of
+// ltmean positions on average, ltmax at most.  One per stripe gives the
+// shortest schedule of a pair (the phases until its last stripe ends), which is
+// what few pairs take: 600 positions against 1300 templates 0.69 ms with eight,
+// 0.82 with three.  But from a third of a stripe's phases on a wavefront waits
+// for the stripe above, and it takes registers and LDS from other pairs.
+// Taken is the number of phases that is least for all pairs: a compute unit's
+// share over those that fit it, plus half as many again as the longest pair's,
+// which few others accompany and which start first (databases are sorted).  372
+// positions against 1500 templates (235 on average, up to 700), with
+// traceback: 0.72 ms with three or four, 1.19 with six; 600 against 6000
+// without: 2.0 with three, 2.8 with eight.  Five to seven where there are more
+// stripes load the four SIMDs unevenly (800 against 3000: 2.17 ms, with eight
+// 1.77, with three 1.36).
+int dp_waves(int lq, int ltmean, int ltmax, int np, bool global, bool trace) {
+  constexpr int kCUs = 256;
+  constexpr size_t kUnitLds = (size_t)160 << 10;
+  const int unit = trace ? 12 : 16;  // wavefronts a compute unit holds, by their registers
+  const int ns = std::max(1, (lq + 63) / 64), most = std::min(kMaxWaves, ns);
+  auto schedule = [&](int W, int lt) { return sweep_start(ns - 1, W, sweep_phases(lt)) + sweep_phases(lt); };
+  int best = most;
+  double least = 0.0;
+  for (int W = most; W >= 1; W = std::min(W - 1, 4)) {
+    const size_t lds = W * dp_wave_lds(global) + dp_row_lds(ltmax, global);
+    const int fit = std::max(1, std::min((int)(kUnitLds / lds), unit / W));
+    const double t = (double)np / (kCUs * fit) * schedule(W, ltmean) + 1.5 * schedule(W, ltmax);
+    if (W == most || t < least) {
+      least = t;
+      best = W;
+    }
+  }
+  return best;
+}
 
 bool dp_select(const cth_dpset* q, const cth_dpset* db) { return !cth_finite_scores(q, db); }
 
@@ -607,22 +638,24 @@ void dp_launch_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* 
 }  // namespace
 
 // Phase 1 for np profiles (query qp of lq positions): p0 + k, or plist[k]
-// (device array of absolute indices) when plist is not NULL; res[k] receives
+// (device array of absolute indices) when plist is not NULL, of at most ltmax
+// positions and about ltmean on average; res[k] receives
 // profile k's record.  scores: readable 8 floats to either side of its
 // [lq][ldsc].  btck NULL: no traceback bytes (maximum and its coordinates
 // only); finalize: run the finalisation (needs btck).  grow:
 // cth_dp_row_bytes(np, ltmax) bytes of device memory when ltmax exceeds
 // CTH_DP_GLOBAL_FROM (else unused).
 extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, const int* plist,
-                                  int np, int ltmax, int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck,
-                                  float scorethld, int finalize, cth_dpres* res, float* grow, hipStream_t st) {
+                                  int np, int ltmean, int ltmax, int64_t col0, int64_t ldsc, const float* scores,
+                                  uint8_t* btck, float scorethld, int finalize, cth_dpres* res, float* grow,
+                                  hipStream_t st) {
   if (np <= 0) return 0;
   if (finalize && !btck) { cth_set_error("dp: finalisation needs the traceback"); return -1; }
   if (finalize && ldsc % 4) { cth_set_error("dp: rows of %lld traceback bytes", (long long)ldsc); return -1; }
   if (ltmax > CTH_MAXCOLUMNS) { cth_set_error("dp: profile length %d over %d", ltmax, CTH_MAXCOLUMNS); return -1; }
   const bool global = ltmax > CTH_DP_GLOBAL_FROM;
   if (global && !grow) { cth_set_error("dp: profile length %d needs global boundary rows", ltmax); return -1; }
-  const int W = dp_waves(lq);
+  const int W = dp_waves(lq, ltmean, ltmax, np, global, btck != nullptr);
   const size_t lds = W * dp_wave_lds(global) + dp_row_lds(ltmax, global);
   const int64_t gs = (int64_t)7 * ltmax;
   if (global) {
@@ -644,11 +677,11 @@ extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_
   return 0;
 }
 
-extern "C" int cth_launch_dp(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int np, int ltmax,
-                             int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck, float scorethld,
-                             cth_dpres* res, float* grow, hipStream_t st) {
-  return cth_launch_dp_list(q, qp, lq, db, p0, nullptr, np, ltmax, col0, ldsc, scores, btck, scorethld, 1, res, grow,
-                            st);
+extern "C" int cth_launch_dp(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int np, int ltmean,
+                             int ltmax, int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck,
+                             float scorethld, cth_dpres* res, float* grow, hipStream_t st) {
+  return cth_launch_dp_list(q, qp, lq, db, p0, nullptr, np, ltmean, ltmax, col0, ldsc, scores, btck, scorethld, 1, res,
+                            grow, st);
 }
 
 // Bytes of global boundary rows a batched launch of `grid` workgroups needs.

@@ -38,7 +38,7 @@ extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, const f
                                 int64_t ldsc, const cth_tables* dtabs, int lq, float* scores, float* mods, int contraction,
                                 int ddms, hipStream_t st);
 extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, const int* plist, int np,
-                                  int ltmax, int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck,
+                                  int ltmean, int ltmax, int64_t col0, int64_t ldsc, const float* scores, uint8_t* btck,
                                   float scorethld, int finalize, cth_dpres* res, float* grow, hipStream_t st);
 extern "C" size_t cth_dp_row_bytes(int np, int ltmax);
 extern "C" size_t cth_map_row_bytes(int njobs, int ltmax);
@@ -399,14 +399,18 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
       // Profiles longer than CTH_DP_GLOBAL_FROM keep their stripe boundary rows
       // in the work area, in launches of as many profiles as their rows fit.
       k.traced = ondevice && np <= ncu;
-      if (k.traced && cth_launch_dp_list(&c->q.d, qi, lq, &db.d, p0, nullptr, np, ltchunk, col0, ldsc, scores, btck,
-                                         scorethld, 1, dpout, nullptr, c->st))
+      if (k.traced && cth_launch_dp_list(&c->q.d, qi, lq, &db.d, p0, nullptr, np, (int)(ncols / np), ltchunk, col0,
+                                         ldsc, scores, btck, scorethld, 1, dpout, nullptr, c->st))
         return -1;
       constexpr int kDpGroup = 16384, kDpGroupLong = 2048, kDpLong = 1024;
       for (int a = k.traced ? p1 : p0, b; a < p1; a = b) {
         b = std::min(p1, a + (db.h_len[a] > kDpLong ? kDpGroupLong : kDpGroup));
         int lg = 0;
-        for (int p = a; p < b; p++) lg = std::max(lg, db.h_len[p]);
+        int64_t lsum = 0;
+        for (int p = a; p < b; p++) {
+          lg = std::max(lg, db.h_len[p]);
+          lsum += db.h_len[p];
+        }
         int nb = b - a;
         float* grow = nullptr;
         if (lg > CTH_DP_GLOBAL_FROM) {
@@ -417,8 +421,8 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
         }
         for (int a2 = a; a2 < b; a2 += nb) {
           const int b2 = std::min(b, a2 + nb);
-          if (cth_launch_dp_list(&c->q.d, qi, lq, &db.d, a2, nullptr, b2 - a2, lg, col0, ldsc, scores, nullptr, scorethld,
-                                 0, dpout + (a2 - p0), grow, c->st))
+          if (cth_launch_dp_list(&c->q.d, qi, lq, &db.d, a2, nullptr, b2 - a2, (int)(lsum / (b - a)), lg, col0, ldsc,
+                                 scores, nullptr, scorethld, 0, dpout + (a2 - p0), grow, c->st))
             return -1;
         }
       }
@@ -502,11 +506,11 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
         float* grow = nl ? (float*)(((uintptr_t)(d_res2 + nc) + 255) & ~(uintptr_t)255) : nullptr;
         CTH_HIP_CHECK(hipMemcpyAsync(d_cand, cand_abs.data(), sizeof(int) * nc, hipMemcpyHostToDevice, c->st));
         if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[1], c->st));
-        if (cth_launch_dp_list(&c->q.d, qi, lq, &db.d, p0, d_cand, ns, ltc, col0, ldsc, scores, btck, scorethld, 1,
+        if (cth_launch_dp_list(&c->q.d, qi, lq, &db.d, p0, d_cand, ns, ltc, ltc, col0, ldsc, scores, btck, scorethld, 1,
                                d_res2, nullptr, c->st))
           return -1;
         for (int j = 0; j < nl; j += nbl)
-          if (cth_launch_dp_list(&c->q.d, qi, lq, &db.d, p0, d_cand + ns + j, std::min(nbl, nl - j), ltl, col0, ldsc,
+          if (cth_launch_dp_list(&c->q.d, qi, lq, &db.d, p0, d_cand + ns + j, std::min(nbl, nl - j), ltl, ltl, col0, ldsc,
                                  scores, btck, scorethld, 1, d_res2 + ns + j, grow, c->st))
             return -1;
         if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[2], c->st));
