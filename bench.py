@@ -390,7 +390,7 @@ def main():
     roofline = {"bound": "valu", "achieved": round(achieved, 3), "peak": PEAK_VALU_FP32_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(achieved / PEAK_VALU_FP32_TFLOPS, 4),
                 "traffic": (bpc * cells_per_launch) if bpc is not None else None,
-                "kernel": "k_score", "avg_launch_ms": round(ms_score / max(nlaunch, 1.0), 3),
+                "kernel": "k_score_plain + k_score_ddms", "avg_launch_ms": round(ms_score / max(nlaunch, 1.0), 3),
                 "ops_per_launch": ops / max(nlaunch, 1.0)}
     serving = None
     if args.serve_requests > 0:

@@ -1,5 +1,5 @@
 // cth_mfma.h: operands and products of the reduced-precision contraction on
-// the matrix cores (precision 1: BF16, 2: FP16), shared by its kernels.
+// the matrix cores (precision 1: BF16, 2: FP16).
 //
 // v_mfma_f32_32x32x16 (lane l, 64 lanes): A holds row l%32, k = 8*(l/32) +
 // 0..7; B holds column l%32, the same k; the 16 accumulators of lane l hold

@@ -551,7 +551,7 @@ __global__ __launch_bounds__(256) void k_query_records(cth_dpset q, const cth_ta
 //
 // The product's tile is 32 of the wavefront's rows x its 64 columns, two
 // 32 x 32 blocks; it goes through the wavefront's own LDS block to one column
-// per lane.  Against the product by k_init_mfma, whose 64 x 64 tiles divide
+// per lane.  Against a product of its own kernel before, whose 64 x 64 tiles divide
 // each column's frequencies again and whose logarithms are written and read
 // back (4 B + 4 B a cell), the score stage of 142 Mcells takes 0.51 ms instead
 // of 0.76.

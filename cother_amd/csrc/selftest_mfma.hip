@@ -1,22 +1,6 @@
-// init_mfma.hip: the log-odds term of the score matrix as a product on the
-// matrix cores (the reduced-precision contraction variant).
-//
-// The reference sums the term per cell in FP32 (CalcSM_Init_SMEMUnroll2x,
-// cusco/CuBatchScoreMatrix_Init.cu:129-144,174-185):
-//   init[i][j] = log( sum_a q_i(a) t_j(a) / (0.5 (bq(a) + bt_p(j)(a))) ) - 0.002
-// which is a product of the query's target frequencies Q [Lq x 20] and the
-// template's weighted frequencies T' [ncols x 20], T'[j][a] = t_j(a) /
-// (0.5 (bq(a) + bt_p(j)(a))) (its weights depend on the query's background,
-// so T' is formed per launch).  Here both operands are rounded to BF16 (or
-// FP16) and multiplied on the MFMA units with FP32 accumulation, K = 20
-// padded to 32 with zeros; the logarithm stays FP32.  The score kernel then
-// adds the secondary-structure, context-vector and DDMS terms to it
-// unchanged.  Where no cell has a DDMS term the plain score kernel forms the
-// product itself (score.hip); the FP32 path (the default) uses neither.
-//
-// Tile: a workgroup of four wavefronts computes 64 query rows x 64 template
-// columns; each wavefront one 32 x 32 block with two
-// v_mfma_f32_32x32x16 (bf16 / f16) steps over K.
+// selftest_mfma.hip: device check of the matrix instructions' lane layout
+// (cth_mfma.h), on which the reduced-precision log-odds product of
+// k_score_plain (score.hip) relies.
 #include <hip/hip_runtime.h>
 
 #include "cth_dev.h"
@@ -24,9 +8,6 @@
 #include "cth_mfma.h"
 
 namespace {
-
-constexpr int kTile = 64;
-constexpr int kK = 32;
 
 // Lane layout check of the 32x32x16 instructions: A = I (32 x 16 block of
 // the identity), B[k][c] = 32 (k - 8 h) + c for k in [8 h, 8 h + 8) and 0
