@@ -4,7 +4,7 @@
 //           profile's Lq x Lt scores (integer counts; masked 'X' positions
 //           skipped), the work of CalcScoreProbsXuninfDynPlmProfile
 //           (cuss/CuBatchSS_dynplm.cu:134-182), rows over several workgroups
-//           where profiles are few.  Bound by the LDS atomics.
+//           where profiles are few.
 // k_stats : one workgroup per passed profile computes in double precision the
 //           parameters of CalcStatParamsDynPlmProfile (cuss/CuBatchSS_dynplm.cu:
 //           193-430): expected score, min/max, lambda by Newton-Raphson with
@@ -58,6 +58,10 @@ constexpr int kThreads = 256, kWaves = kThreads / 64;
 // copies of the histogram, by lane: the scores of neighbouring cells fall
 // into few bins, and atomics of a wavefront on one LDS word serialise
 constexpr int kCopies = 4;
+// rows of a wavefront whose scores are loaded together: with one at a time it
+// waited for every row's (1500 profiles of 372 x 235 cells 243 us instead of
+// 316; two or eight rows, and more copies, are alike)
+constexpr int kHistRows = 4;
 
 // Adds the scores of query rows [y0, y1) of query qp against profile p
 // (scores from scores[colp], row stride ldsc) to the workgroup's histogram
@@ -77,18 +81,26 @@ __device__ __forceinline__ void hist_fill(const cth_dpset& q, int qp, const cth_
       const int x = x0 + 64 * i + lane;
       use[i] = x < lt && taa[x] != 'X';
     }
-    for (int y = y0 + w; y < y1; y += kWaves) {
-      if (qaa[y] == 'X') continue;
-      const float* const row = scores + (int64_t)y * ldsc + colp + x0 + lane;
-      float v[4];
+    for (int y = y0 + w; y < y1; y += kHistRows * kWaves) {
+      float v[kHistRows][4];
+      bool in[kHistRows];
 #pragma unroll
-      for (int i = 0; i < 4; i++) v[i] = use[i] ? row[64 * i] : 0.0f;
+      for (int r = 0; r < kHistRows; r++) {
+        const int yr = min(y + r * kWaves, y1 - 1);
+        in[r] = y + r * kWaves < y1 && qaa[yr] != 'X';
+        const float* const row = scores + (int64_t)yr * ldsc + colp + x0 + lane;
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        float s = v[i];
-        if (s < -10.0f) s = -10.0f;
-        else if (s > 10.0f) s = 10.0f;
-        if (use[i]) atomicAdd(&hl[((int)rintf(s * 32.0f) - kSscMin) * kCopies], 1);
+        for (int i = 0; i < 4; i++) v[r][i] = use[i] ? row[64 * i] : 0.0f;
+      }
+#pragma unroll
+      for (int r = 0; r < kHistRows; r++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float s = v[r][i];
+          if (s < -10.0f) s = -10.0f;
+          else if (s > 10.0f) s = 10.0f;
+          if (in[r] && use[i]) atomicAdd(&hl[((int)rintf(s * 32.0f) - kSscMin) * kCopies], 1);
+        }
       }
     }
   }
