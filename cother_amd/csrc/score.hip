@@ -299,28 +299,15 @@ __device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int 
   uint32_t low;
   asm("v_mov_b32 %0, 0xffff" : "=v"(low));
   asm("v_mov_b32 %0, %1" : "=v"(packf) : "i"(__builtin_bit_cast(uint32_t, kPackF)));
-  // the diagonals: upper ones j = len2>>2 .. 0 pair query index i with
-  // template index j + i, lower ones i = len1>>2 .. 1 query index i + j with
-  // template index j
-  const int upper = (n.tmax >> 3) + 1, lower = ((n.qmax >> 2) + 1) >> 1;
-  for (int k = 0; k < upper + lower; k++) {
-    const int i = k < upper ? 0 : (len1 >> 2) - 2 * (k - upper);
-    const int j = k < upper ? (len2 >> 2) - 2 * k : 0;
-    if (k < upper ? j < 0 : i < 1) continue;
-    const int cells = min(len1 - i, len2 - j);  // of the diagonal
-    // cells that every lane's diagonal has (len - (len >> 2) grows with len):
-    // their steps are taken without a test of the lane's end
-    const int full = k < upper ? min(n.qmin, n.tmin - (n.tmin >> 2) + 2 * k)
-                               : min(n.qmin - (n.qmin >> 2) + 2 * (k - upper), n.tmin);
-    // byte offsets of the diagonal's first query and template entries,
-    // advanced by one iteration (8 entries) at a time in vector registers
-    int qo = qr + 4 * (1 + i), to = tr + 4 * (1 + j);
+  // a diagonal of `cells` cells from the entries at byte offsets qo and to on,
+  // `first` its cell 1 as 2^23 + packed coordinates; full: cells that every
+  // lane's diagonal has, whose steps are taken without a test of the lane's
+  // end.  The offsets advance by one iteration at a time in vector registers.
+  auto diagonal = [&](int qo, int to, uint32_t first, int cells, int full) {
     const uint32_t a0 = lds_u32(lds, qo) + lds_u32(lds, to), a4 = lds_u32(lds, qo + 16) + lds_u32(lds, to + 16);
     float s0 = pair(lds, a0 & low), s2 = pair(lds, a0 >> 16), s4 = pair(lds, a4 & low);
     float u = __builtin_amdgcn_fmed3f(s0, 0.0f, 1.0f);  // max(s0, 0)
-    float dd = 0.0f;
-    // 2^23 + the packed coordinates of cell 1 (query i + 1, template j + 1)
-    float fb = __uint_as_float(kMagic + kPack + (uint32_t)i + ((uint32_t)j << 11));
+    float dd = 0.0f, fb = __uint_as_float(first);
     asm("" : "+v"(qo), "+v"(to));
     int ib = 0;
     for (; ib + 12 < full; ib += 16) {
@@ -331,6 +318,30 @@ __device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int 
     for (; ib < cells; ib += 8) {
       CTH_DDMS_8CELL(0, ib + 4 < cells)
       CTH_DDMS_ADVANCE(8)
+    }
+  };
+  // upper diagonals, j = len2>>2 .. 0 step 2: query index i with template index
+  // j + i; lower ones, i = len1>>2 .. 1: query index i + j with template index
+  // j.  (len - (len >> 2) grows with len, so the shortest lists give the
+  // shortest diagonals.)
+  {
+    int j = len2 >> 2, to = tr + 4 * (1 + j), left = len2 - j;
+    uint32_t first = kMagic + kPack + ((uint32_t)j << 11);
+    int most = n.tmin - (n.tmin >> 2);
+    for (int k = n.tmax >> 3; k >= 0; k--) {
+      if (j >= 0) diagonal(qr + 4, to, first, min(len1, left), min(n.qmin, most));
+      j -= 2; to -= 8; left += 2; most += 2;
+      first -= 2u << 11;
+    }
+  }
+  {
+    int i = len1 >> 2, qo = qr + 4 * (1 + i), left = len1 - i;
+    uint32_t first = kMagic + kPack + (uint32_t)i;
+    int most = n.qmin - (n.qmin >> 2);
+    for (int k = ((n.qmax >> 2) + 1) >> 1; k > 0; k--) {
+      if (i >= 1) diagonal(qo, tr + 4, first, min(left, len2), min(most, n.tmin));
+      i -= 2; qo -= 8; left += 2; most += 2;
+      first -= 2u;
     }
   }
   float s = 0.0f;
@@ -360,15 +371,17 @@ __device__ __forceinline__ float ddms_cell(const char* lds, int qr, int tr, int 
 // 64 x 1 would be 43, 31 and 19%, but its query lists take the LDS of eight
 // workgroups.
 //
-// Bound by VALU issue: by the counters 15,600 instructions a wavefront in 9,500
+// Bound by VALU issue: by the counters 15,500 instructions a wavefront in 9,400
 // issue slots of its 9,800 cycles (1 x 64 cells with every step's arithmetic
 // taken: 25,300 in 14,700).  The score stage of 250 positions against 4000
-// templates (median 220) takes 62.0 ms; with 16 x 4 cells, lists read an entry
-// at a time and no test for a step without sums 73.4, with 16 rows and words
-// of two 16-bit entries added by SDWA (which issue alone) 68.4.  Workgroups of
-// 512 lanes: 67.0 against 65.9 (a wavefront's place waits for the seven others).
-// Tiles of the fewest rows that hold a query's last ones: 40 positions against
-// 6000 templates 5.05 ms, with 32 x 8 tiles alone 6.4.
+// templates (median 220) takes 61.1 ms.  With one loop over both kinds of
+// diagonals, whose starts are then built anew each time, 61.9; with 16 x 4
+// cells, lists read an entry at a time and no test for a step without sums
+// 73.4; with 16 rows and words of two 16-bit entries added by SDWA (which issue
+// alone) 68.4.  Workgroups of 512 lanes: 67.0 against 65.9 (a wavefront's place
+// waits for the seven others).  Tiles of the fewest rows that hold a query's
+// last ones: 40 positions against 6000 templates 5.05 ms, with 32 x 8 tiles
+// alone 6.4.
 // kBatch: the row tiles of several queries in one launch, ytab[blockIdx.y /
 // ysplit] giving query and first row of ysplit tiles of kDRows rows.
 template <bool kBatch>
