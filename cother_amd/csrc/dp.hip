@@ -347,25 +347,33 @@ __device__ __forceinline__ void dp_pair(const cth_dpset& q, int qp, const cth_dp
       const bool fix = __builtin_amdgcn_ballot_w64(cf < lo || cf + 31 > hc) != 0;
       const int crel = cf - lo;
       const uint32_t span = (uint32_t)(hc - lo);
-      for (int j0 = 0; j0 < 32 && 32 * k - 64 + j0 < lt; j0 += 8) {
-        const score8 cur = nxt;
-        nxt = score_load8(srow + max(-8, min(cf + j0 + 8, lt)));
-        uint32_t bk[2];
-        if (fix)
-          dp_steps8<kTrace, kSel, true>(d, qt, j0, rg + j0, inA + j0, inB + j0, outA + 16 * j0, outB + 4 * j0, mask, crel + j0,
-                                        span, cf + j0, (uint32_t)lt, cur, mv, ms, bk);
-        else
-          dp_steps8<kTrace, kSel, false>(d, qt, j0, rg + j0, inA + j0, inB + j0, outA + 16 * j0, outB + 4 * j0, mask, 0, 0u,
-                                         cf + j0, (uint32_t)lt, cur, mv, ms, bk);
+      // (with traceback 16 steps a turn: a lane's bytes go to its own row, so a
+      // store touches 64 cache lines however few bytes it has: 372 positions
+      // against 1500 templates 0.80 -> 0.70 ms)
+      constexpr int kTurn = kTrace ? 16 : 8;
+      for (int j0 = 0; j0 < 32 && 32 * k - 64 + j0 < lt; j0 += kTurn) {
+        uint32_t bk[kTurn / 4];
+#pragma unroll
+        for (int h = 0; h < kTurn; h += 8) {
+          const int jh = j0 + h;
+          const score8 cur = nxt;
+          nxt = score_load8(srow + max(-8, min(cf + jh + 8, lt)));
+          if (fix)
+            dp_steps8<kTrace, kSel, true>(d, qt, jh, rg + jh, inA + jh, inB + jh, outA + 16 * jh, outB + 4 * jh, mask,
+                                          crel + jh, span, cf + jh, (uint32_t)lt, cur, mv, ms, bk + h / 4);
+          else
+            dp_steps8<kTrace, kSel, false>(d, qt, jh, rg + jh, inA + jh, inB + jh, outA + 16 * jh, outB + 4 * jh, mask,
+                                           0, 0u, cf + jh, (uint32_t)lt, cur, mv, ms, bk + h / 4);
+        }
         if constexpr (kTrace) {
           if (y < lq) {
             const int c = cf + j0;
             uint8_t* const at = btck + (int64_t)y * ldsc + colp + c;
-            if (0 <= c && c + 7 < lt) {
-              memcpy(at, bk, 8);
+            if (0 <= c && c + kTurn - 1 < lt) {
+              memcpy(at, bk, kTurn);
             } else {
 #pragma unroll
-              for (int j = 0; j < 8; j++)
+              for (int j = 0; j < kTurn; j++)
                 if (0 <= c + j && c + j < lt) at[j] = (uint8_t)(bk[j >> 2] >> (8 * (j & 3)));
             }
           }
@@ -584,7 +592,7 @@ namespace {
 // share over those that fit it, plus half as many again as the longest pair's,
 // which few others accompany and which start first (databases are sorted).  372
 // positions against 1500 templates (235 on average, up to 700), with
-// traceback: 0.72 ms with three or four, 1.19 with six; 600 against 6000
+// traceback (8 bytes a store): 0.8 ms with three or four, 1.19 with six; 600 against 6000
 // without: 2.0 with three, 2.8 with eight.  Five to seven where there are more
 // stripes load the four SIMDs unevenly (800 against 3000: 2.17 ms, with eight
 // 1.77, with three 1.36).
