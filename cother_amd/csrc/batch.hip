@@ -191,6 +191,24 @@ struct batch_layout {
   int* cand; int* passed; int* hitl; int* hist; int* ctr; double* zrow; cth_hit* hits; char* alnout; float* grow; float* back;
 };
 
+// The cell buffers in one piece: byte offsets of a batch of `cells` cells.  The
+// sweeps read up to 8 floats to either side of their matrices: the traceback
+// bytes come first, and a pad follows the last matrix.
+struct cell_layout {
+  size_t btck, scores, mods, post, bytes;
+};
+cell_layout lay_cells(size_t cells, bool map) {
+  cell_layout C{};
+  size_t o = 0;
+  auto take = [&](size_t n) { const size_t at = o; o += up256(n); return at; };
+  C.btck = take(cells);
+  C.scores = take(4 * cells);
+  C.mods = take(4 * cells);
+  C.post = map ? take(4 * cells) : 0;
+  C.bytes = o + CTH_SCORE_PAD * sizeof(float);
+  return C;
+}
+
 // One batch's description on the host.
 struct batch_plan {
   int q0, q1;                       // entries [q0,q1) of the query list
@@ -580,7 +598,7 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
     const size_t alnbytes = opt->alnbuf && opt->do_map ? (size_t)npairs * 5 * (size_t)rowcap : 0;
     // device buffers
     const size_t cells = (size_t)P.cells;
-    const size_t cbytes = up256(4 * cells) * (opt->do_map ? 3 : 2) + up256(cells);
+    const cell_layout cell = lay_cells(cells, opt->do_map != 0);
     const int small_max = std::max(1, std::min(npairs, ncu * 32));
     const size_t backbytes =
         opt->do_map ? cth_map_split_bytes(P.lqmax, ltmax, cth_map_split(P.lqmax, ltmax, npairs)) : 0;
@@ -592,17 +610,15 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
                           3 * up256(sizeof(int) * npairs) + up256(sizeof(int) * kNCtr) +
                           up256(sizeof(int) * hist_ints(npairs)) + up256(sizeof(double) * (size_t)small_max * P.lqmax) + up256(sizeof(cth_hit) * npairs) +
                           up256(alnbytes) + up256(growbytes) + up256(backbytes);
-    if (cth_ctx_reserve(c, &c->bcells, &c->cap_bcells, cbytes)) return -1;
+    if (cth_ctx_reserve(c, &c->bcells, &c->cap_bcells, cell.bytes)) return -1;
     if (cth_ctx_reserve(c, &c->bsmall, &c->cap_bsmall, sbytes)) return -1;
     batch_layout L{};
     {
-      uint8_t* o = (uint8_t*)c->bcells;
-      auto take = [&](size_t n) { uint8_t* p = o; o += up256(n); return p; };
-      // (traceback bytes first: the DP sweeps read up to 8 floats to either side of the scores)
-      L.btck = take(cells);
-      L.scores = (float*)take(4 * cells);
-      L.mods = (float*)take(4 * cells);
-      L.post = opt->do_map ? (float*)take(4 * cells) : nullptr;
+      uint8_t* const o = (uint8_t*)c->bcells;
+      L.btck = o + cell.btck;
+      L.scores = (float*)(o + cell.scores);
+      L.mods = (float*)(o + cell.mods);
+      L.post = opt->do_map ? (float*)(o + cell.post) : nullptr;
       uint8_t* s = (uint8_t*)c->bsmall;
       auto takes = [&](size_t n) { uint8_t* p = s; s += up256(n); return p; };
       L.bq = (cth_bquery*)takes(sizeof(cth_bquery) * P.bq.size());
@@ -746,6 +762,13 @@ extern "C" int cth_search_batch_list(cth_ctx* c, const int32_t* qidx, int nq, co
     ql[k] = q;
   }
   return search_batch_list(c, ql.data(), nq, opt, hits, maxhits, nhits, stats);
+}
+
+// Host check of the cell buffers' layout: byte offsets of the traceback bytes,
+// scores, modular scores and posteriors, and the size of the whole.
+extern "C" void cth_selftest_batch_cells(uint64_t cells, int do_map, uint64_t out[5]) {
+  const cell_layout C = lay_cells((size_t)cells, do_map != 0);
+  out[0] = C.btck; out[1] = C.scores; out[2] = C.mods; out[3] = C.post; out[4] = C.bytes;
 }
 
 // Counts of graph captures and replays of the batched search on a context
