@@ -40,13 +40,21 @@ struct cth_dpset {
 #define CTH_DD_MISSING 21
 
 // What an upload finds in a set's values.  CTH_SET_FINITE: frequencies in
-// [0, 1.5], backgrounds in [0, 4], SS probabilities in [0, 1], transitions
-// within +-1e6; CTH_SET_BKG: every background at least 2^-14.  Scores of two
-// finite sets, one with backgrounds, are finite or -inf (log-odds quotients
+// [0, 1.5], backgrounds in [0, 4], SS probabilities in [0, 1], transitions in
+// [-1e6, CTH_TRN_TOP]; CTH_SET_BKG: every background at least 2^-14.  Scores of
+// two finite sets, one with backgrounds, are finite or -inf (log-odds quotients
 // of at most 1.5^2 2^15, which FP16 holds too, and no 0/0), so no step of the
 // DPs over them gives a NaN.
+//
+// The phase-1 DP over such sets also takes no maximum from the 32 columns
+// before the profile without testing for them: a path there leaves the zero
+// states by at most 32 query transitions and returns to a match state by one
+// more and a template transition, which is CTH_LOG0 = -32768 there, so with
+// transitions of at most 256 (log-probabilities are at most 0; 992 would do)
+// no match state of those columns is positive.
 #define CTH_SET_FINITE 1
 #define CTH_SET_BKG 2
+#define CTH_TRN_TOP 256.0f
 static inline bool cth_finite_scores(const cth_dpset* q, const cth_dpset* db) {
   return (q->finite & db->finite & CTH_SET_FINITE) && ((q->finite | db->finite) & CTH_SET_BKG);
 }

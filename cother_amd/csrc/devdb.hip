@@ -49,7 +49,7 @@ __global__ __launch_bounds__(256) void k_check_values(cth_dpset d, int* bad) {
     for (int a = 0; a < CTH_NSS; a++) out |= !within(d.ss[a * d.ld + i], 0.0f, 1.0f);
   }
   for (int64_t i = i0; i < d.npos + d.nprof; i += step)
-    for (int a = 0; a < CTH_NTRN; a++) out |= !within(d.trn[a * d.ldtr + i], -1e6f, 1e6f);
+    for (int a = 0; a < CTH_NTRN; a++) out |= !within(d.trn[a * d.ldtr + i], -1e6f, CTH_TRN_TOP);
   for (int64_t i = i0; i < (int64_t)d.nprof * CTH_NAA; i += step) {
     out |= !within(d.bkg[i], 0.0f, 4.0f);
     small |= !(d.bkg[i] >= 0x1p-14f);

@@ -55,7 +55,7 @@ __host__ __device__ constexpr size_t dp_row_lds(int lt, bool grow) {
 // the max the recursion takes.  kSel: the reference's select a < b ? b : a,
 // whose result differs from the hardware's max only for NaN operands (and in
 // the sign of a zero, which no result depends on); the hardware's max runs
-// when neither set can give a NaN (cth_dpset.tame)
+// when neither set can give a NaN (cth_dpset.finite)
 template <bool kSel>
 __device__ __forceinline__ float mx(float a, float b) {
   if constexpr (kSel) return a < b ? b : a;
@@ -153,7 +153,8 @@ __device__ __forceinline__ void store_bottom(uint32_t outA, uint32_t outB, uint6
 // relative to it.  kFix: scores outside the valid columns are -9 (cells of
 // the ignored corners and outside the matrix, CuBatchDP_init_btck.cu:245).
 // mv, ms: the lane's running maximum and the step that set it (kSel: at
-// columns c + j below clt only, an infinite state passes any transition).
+// columns c + j in 0 .. clt-1 only; else no match state outside them is
+// positive, CTH_SET_FINITE and kPast).
 template <bool kTrace, bool kSel, bool kFix>
 __device__ __forceinline__ void dp_steps8(dp_state& d, const float* qt, int j0, const float4* __restrict__ ring,
                                           const float4* __restrict__ inA, const float* __restrict__ inB,
