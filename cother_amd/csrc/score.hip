@@ -843,6 +843,36 @@ extern "C" int cth_score_tile_rows(int ddms, int64_t rows, int64_t ncols) {
 static_assert(CTH_DDMS_TILE % kDRows == 0 && kDRows >= CTH_SCORE_TILE_MIN && kPlainRowsMin >= CTH_SCORE_TILE_MIN,
               "row tiles");
 
+// Columns of the distance-match launch that starts at column c: it takes 32
+// work-items a column, and a grid dimension of 2^32 work-items or more is
+// refused.  (A search's chunks have at most 6M columns, so they take one
+// launch; a launch of 8M leaves its tail behind by far.)
+static int ddms_slice(int ncols, int c) { return std::min(ncols - c, 1 << 23); }
+
+template <bool kBatch>
+static int launch_ddms(const cth_dpset* q, int qp, const cth_dpset* db, int64_t col0, int ncols, int64_t ldsc,
+                       const cth_tables* dtabs, float* scores, float* mods, const int32_t* qoff, int ytiles,
+                       const cth_bytile* ytab, int ysplit, const cth_bquery* bq, hipStream_t st) {
+  for (int c = 0, n; c < ncols; c += n) {
+    n = ddms_slice(ncols, c);
+    hipLaunchKernelGGL(k_score_ddms<kBatch>, dim3((n + kDColsMin - 1) / kDColsMin, ytiles), dim3(kDThreads), 0, st, *q,
+                       qp, *db, col0 + c, n, ldsc, dtabs, scores + c, mods + c, qoff, ytab, ysplit, bq);
+    CTH_HIP_CHECK(hipGetLastError());
+  }
+  return 0;
+}
+
+// Host check of the launches over ncols columns: the largest grid's work-items,
+// and the columns that all of them cover.
+extern "C" void cth_selftest_ddms_launches(int ncols, uint64_t out[2]) {
+  out[0] = out[1] = 0;
+  for (int c = 0, n; c < ncols; c += n) {
+    n = ddms_slice(ncols, c);
+    out[0] = std::max<uint64_t>(out[0], (uint64_t)((n + kDColsMin - 1) / kDColsMin) * kDThreads);
+    out[1] += (uint64_t)n;
+  }
+}
+
 // Launch the score stage for query profile qp against template positions
 // [col0, col0+ncols) of db; outputs are [Lq][ldsc].
 // contraction 0: the FP32 log-odds term of the reference; 1 / 2: the term
@@ -874,11 +904,8 @@ extern "C" int cth_launch_score(const cth_dpset* q, const int32_t* qoff, const f
   }
   CTH_HIP_CHECK(hipGetLastError());
   if (!ddms) return 0;
-  hipLaunchKernelGGL(k_score_ddms<false>, dim3((ncols + kDColsMin - 1) / kDColsMin, (lq + kDRows - 1) / kDRows),
-                     dim3(kDThreads), 0, st, *q, qp, *db, col0, ncols, ldsc, dtabs, scores, mods, qoff, nullptr, 1,
-                     nullptr);
-  CTH_HIP_CHECK(hipGetLastError());
-  return 0;
+  return launch_ddms<false>(q, qp, db, col0, ncols, ldsc, dtabs, scores, mods, qoff, (lq + kDRows - 1) / kDRows,
+                            nullptr, 1, nullptr, st);
 }
 
 // The score stage of a batch of queries: nytiles row tiles (ytab: query of
@@ -901,10 +928,7 @@ extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, c
                      mods, tile, ytab, bq);
   CTH_HIP_CHECK(hipGetLastError());
   if (!ddms) return 0;
-  hipLaunchKernelGGL(k_score_ddms<true>, dim3((ncols + kDColsMin - 1) / kDColsMin, nytiles * ysplit), dim3(kDThreads), 0, st,
-                     *q, 0, *db, (int64_t)0, ncols, ldsc, dtabs, scores, mods, qoff, ytab, ysplit, bq);
-  CTH_HIP_CHECK(hipGetLastError());
-  return 0;
+  return launch_ddms<true>(q, 0, db, 0, ncols, ldsc, dtabs, scores, mods, qoff, nytiles * ysplit, ytab, ysplit, bq, st);
 }
 
 // The records of an uploaded query set that the plain kernel reads (256 bytes
