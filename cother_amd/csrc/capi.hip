@@ -6,6 +6,7 @@
 // message available from cth_last_error(); nothing throws across the ABI.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -259,16 +260,23 @@ extern "C" size_t cth_map_row_bytes(int njobs, int ltmax);
 // has room for up to three bytes more)
 static __global__ void k_pack_rows(const uint8_t* __restrict__ src, int64_t ld, int64_t cols, int64_t n,
                                    uint8_t* __restrict__ dst) {
-  const int64_t i = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
-  if (i >= n) return;
-  int64_t r = i / cols, x = i - r * cols;
-  uint32_t v = 0;
-  for (int k = 0; k < 4 && i + k < n; k++) {
-    v |= (uint32_t)src[r * ld + x] << (8 * k);
-    if (++x == cols) { x = 0; r++; }
+  // (a bounded grid: rows x cols may have more bytes than a grid has work-items)
+  for (int64_t i = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x); i < n;
+       i += 4 * (int64_t)gridDim.x * blockDim.x) {
+    int64_t r = i / cols, x = i - r * cols;
+    uint32_t v = 0;
+    for (int k = 0; k < 4 && i + k < n; k++) {
+      v |= (uint32_t)src[r * ld + x] << (8 * k);
+      if (++x == cols) { x = 0; r++; }
+    }
+    *reinterpret_cast<uint32_t*>(dst + i) = v;
   }
-  *reinterpret_cast<uint32_t*>(dst + i) = v;
 }
+constexpr int kPackGrid = 4096;
+static int pack_blocks(int64_t n) { return (int)std::min<int64_t>(kPackGrid, (n / 4 + 256) / 256); }
+
+// Host check of k_pack_rows' grid for n bytes: its work-items
+extern "C" uint64_t cth_selftest_pack_grid(uint64_t n) { return (uint64_t)(uint32_t)pack_blocks((int64_t)n) * 256; }
 
 // Phase 1 (score matrix, DP, finalisation) of query qidx against template
 // profiles [p0,p1); per-profile results to res (p1-p0 records of 6 words:
@@ -306,7 +314,7 @@ extern "C" int cth_phase1_block(cth_ctx* c, int qidx, int p0, int p1, float scor
     // the bytes without the rows' padding (which the traceback needs), in the
     // modular scores' place: they go back as one piece, as cth_score_block's
     const int64_t n = (int64_t)lq * ncols;
-    hipLaunchKernelGGL(k_pack_rows, dim3((unsigned)((n / 4 + 256) / 256)), dim3(256), 0, c->st, c->btck, ldsc, ncols, n,
+    hipLaunchKernelGGL(k_pack_rows, dim3((unsigned)pack_blocks(n)), dim3(256), 0, c->st, c->btck, ldsc, ncols, n,
                        (uint8_t*)c->mods);
     CTH_HIP_CHECK(hipGetLastError());
     CTH_HIP_CHECK(hipStreamSynchronize(c->st));
