@@ -590,15 +590,14 @@ namespace {
 // 0.82 with three.  But from a third of a stripe's phases on a wavefront waits
 // for the stripe above, and it takes registers and LDS from other pairs.
 // Taken is the number of phases that is least for all pairs: a compute unit's
-// share over those that fit it, plus half as many again as the longest pair's,
+// share (of the device's ncu) over those that fit it, plus half as many again as the longest pair's,
 // which few others accompany and which start first (databases are sorted).  372
 // positions against 1500 templates (235 on average, up to 700), with
 // traceback (8 bytes a store): 0.8 ms with three or four, 1.19 with six; 600 against 6000
 // without: 2.0 with three, 2.8 with eight.  Five to seven where there are more
 // stripes load the four SIMDs unevenly (800 against 3000: 2.17 ms, with eight
 // 1.77, with three 1.36).
-int dp_waves(int lq, int ltmean, int ltmax, int np, bool global, bool trace) {
-  constexpr int kCUs = 256;
+int dp_waves(int lq, int ltmean, int ltmax, int np, bool global, bool trace, int ncu) {
   constexpr size_t kUnitLds = (size_t)160 << 10;
   const int unit = trace ? 12 : 16;  // wavefronts a compute unit holds, by their registers
   const int ns = std::max(1, (lq + 63) / 64), most = std::min(kMaxWaves, ns);
@@ -608,7 +607,7 @@ int dp_waves(int lq, int ltmean, int ltmax, int np, bool global, bool trace) {
   for (int W = most; W >= 1; W = std::min(W - 1, 4)) {
     const size_t lds = W * dp_wave_lds(global) + dp_row_lds(ltmax, global);
     const int fit = std::max(1, std::min((int)(kUnitLds / lds), unit / W));
-    const double t = (double)np / (kCUs * fit) * schedule(W, ltmean) + 1.5 * schedule(W, ltmax);
+    const double t = (double)np / (ncu * fit) * schedule(W, ltmean) + 1.5 * schedule(W, ltmax);
     if (W == most || t < least) {
       least = t;
       best = W;
@@ -664,7 +663,10 @@ extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_
   if (ltmax > CTH_MAXCOLUMNS) { cth_set_error("dp: profile length %d over %d", ltmax, CTH_MAXCOLUMNS); return -1; }
   const bool global = ltmax > CTH_DP_GLOBAL_FROM;
   if (global && !grow) { cth_set_error("dp: profile length %d needs global boundary rows", ltmax); return -1; }
-  const int W = dp_waves(lq, ltmean, ltmax, np, global, btck != nullptr);
+  int dev = 0, ncu = 0;
+  CTH_HIP_CHECK(hipGetDevice(&dev));
+  CTH_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  const int W = dp_waves(lq, ltmean, ltmax, np, global, btck != nullptr, ncu);
   const size_t lds = W * dp_wave_lds(global) + dp_row_lds(ltmax, global);
   const int64_t gs = (int64_t)7 * ltmax;
   if (global) {
@@ -684,6 +686,11 @@ extern "C" int cth_launch_dp_list(const cth_dpset* q, int qp, int lq, const cth_
     CTH_HIP_CHECK(hipGetLastError());
   }
   return 0;
+}
+
+// Host check of the rule for the wavefronts per pair, on a device of ncu compute units.
+extern "C" int cth_selftest_dp_waves(int lq, int ltmean, int ltmax, int np, int trace, int ncu) {
+  return dp_waves(lq, ltmean, ltmax, np, ltmax > CTH_DP_GLOBAL_FROM, trace != 0, ncu);
 }
 
 extern "C" int cth_launch_dp(const cth_dpset* q, int qp, int lq, const cth_dpset* db, int p0, int np, int ltmean,
