@@ -558,7 +558,8 @@ __global__ __launch_bounds__(256) void k_query_records(cth_dpset q, const cth_ta
   rec[i] = r;
 }
 
-// kBatch: as k_score_ddms's (ytab[blockIdx.y] a tile of `tile` rows).
+// kBatch: as k_score_ddms's (ytab[blockIdx.y] a tile of `tile` rows, at most
+// kPlainRowsMax).
 // kPrec 1, 2: the log-odds sum from the BF16 / FP16 product on the matrix
 // cores, 0: in FP32.
 //
@@ -640,13 +641,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   // rows have an operand outside those ranges divides (quot).
   float tf[CTH_NAA], den[CTH_NAA], y[CTH_NAA];
   bool quot = true;
-  // Every row of the tile within the ranges: looked at by all 64 lanes, before
-  // those past the last column leave.  (The product does not ask, but the look
-  // brings the rows' records near: without it 0.51 ms instead of 0.48 for 142
+  // Whether every row of the tile is within the ranges: its rows' flags, one a
+  // lane, under way with the column's loads and looked at by all 64 lanes before
+  // those past the last column leave.  (Loaded when they are looked at, 1.9%
+  // more of a launch of 32-row tiles.  The product does not ask, but the loads
+  // bring the rows' records near: without them 0.51 ms instead of 0.48 for 142
   // Mcells.)
+  int rowquot[kPlainRowsMax / 64];
+#pragma unroll
+  for (int k = 0; k < kPlainRowsMax / 64; k++)
+    rowquot[k] = row0 + 64 * k < row1 ? rec[q0 + min(row0 + 64 * k + lane, row1 - 1)].quot : 1;
   auto rows_in_range = [&] {
-    for (int r = row0; r < row1; r += 64)
-      quot = quot && __builtin_amdgcn_ballot_w64(r + lane < row1 && rec[q0 + min(r + lane, row1 - 1)].quot == 0) == 0;
+#pragma unroll
+    for (int k = 0; k < kPlainRowsMax / 64; k++) quot = quot && __builtin_amdgcn_ballot_w64(rowquot[k] == 0) == 0;
   };
   v8s pb[2][2];  // the product's column operands of this lane
   if constexpr (!kPrec) {
@@ -840,6 +847,7 @@ extern "C" int cth_score_tile_rows(int ddms, int64_t rows, int64_t ncols) {
   const int64_t fit = rows * cols / kPlainFill;  // rows per tile that leave kPlainFill workgroups
   return (int)std::max<int64_t>(kPlainRowsMin, std::min<int64_t>({(rows + 3) / 4 * 4, fit / 4 * 4, kPlainRowsMax}));
 }
+static_assert(CTH_DDMS_TILE <= kPlainRowsMax && kPlainRowsMax % 64 == 0, "rows whose flags a lane holds");
 static_assert(CTH_DDMS_TILE % kDRows == 0 && kDRows >= CTH_SCORE_TILE_MIN && kPlainRowsMin >= CTH_SCORE_TILE_MIN,
               "row tiles");
 
