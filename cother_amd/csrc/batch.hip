@@ -119,11 +119,14 @@ __global__ void k_select_hits(const cth_bquery* __restrict__ bq, const cth_bpair
 }
 
 // the hit records of the listed pairs, with the fields cth_search fills;
-// alnoff holds the pair's slot in the list (its rows' place in alnout)
+// alnoff holds the pair's slot in the list (its rows' place in alnout).  head:
+// null, or where the counters go in front of the records
 __global__ void k_gather_hits(const cth_bquery* __restrict__ bq, const cth_bpair* __restrict__ pairs,
                               const cth_dpres* __restrict__ res, const double* __restrict__ stats,
                               const cth_mapres* __restrict__ mres, int do_map, const int* __restrict__ list,
-                              const int* __restrict__ count, cth_hit* __restrict__ hits) {
+                              const int* __restrict__ count, cth_hit* __restrict__ hits,
+                              const int* __restrict__ ctr, int* __restrict__ head) {
+  if (head && blockIdx.x == 0 && threadIdx.x < kNCtr) head[threadIdx.x] = ctr[threadIdx.x];
   const int n = *count;
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
     const int i = list[k];
@@ -292,7 +295,7 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
                              cth_map_split(P.lqmax, ltmax, npairs), L.back, st))
       return -1;
     hipLaunchKernelGGL(k_gather_hits, dim3(sel_grid), dim3(256), 0, st, L.bq, L.pairs, L.res, L.stats, L.mres,
-                       opt->do_map, L.hitl, L.ctr + kCtrHits, L.hits);
+                       opt->do_map, L.hitl, L.ctr + kCtrHits, L.hits, nullptr, nullptr);
     CTH_HIP_CHECK(hipGetLastError());
     if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[4], st));
     return 0;
@@ -324,58 +327,86 @@ __global__ void k_chunk_tables(cth_bquery Q, int p0, int np, cth_bquery* __restr
   if (i == 0) *bq = Q;
 }
 
-// hit records that come back with the counters
-constexpr int kFirstHits = 128;
+// hit records that come back with the counters, and list entries
+constexpr int kFirstHits = 128, kFirstList = 1024;
+// what lies in front of either in device and in pinned memory
+constexpr size_t kHead = 256;
 // the MAP stage's workgroups per compute unit, as choose_shape's
 constexpr int kChunkMapGrid = 16;
 
+// A chunk's lists and records, by profile.
 struct chunk_layout {
-  cth_bquery* bq; cth_bpair* pairs; double* stats; cth_mapres* mres; int* cand; int* passed; int* hitl; int* hist;
-  double* zrow; int* ctr; cth_hit* hits; char* alnout; float* back;
-  int nsplit;
+  cth_bquery* bq; cth_bpair* pairs; double* stats; cth_mapres* mres; int* cand; int* passed; int* hist;
+  int* ctr; int* hitl;  // (the list follows the counters at kHead bytes)
   size_t bytes;
 };
-chunk_layout chunk_lay(const cth_chunk& k, int ncu, void* base) {
+chunk_layout chunk_lay(int np, void* base) {
   chunk_layout L;
   size_t o = 0;
   auto take = [&](size_t n) { void* p = (uint8_t*)base + o; o += up256(n); return p; };
-  const size_t np = (size_t)k.np;
   L.bq = (cth_bquery*)take(sizeof(cth_bquery));
   L.pairs = (cth_bpair*)take(sizeof(cth_bpair) * np);
   L.stats = (double*)take(sizeof(double) * CTH_STATS_NOUT * np);
   L.mres = (cth_mapres*)take(sizeof(cth_mapres) * np);
   L.cand = (int*)take(sizeof(int) * np);
   L.passed = (int*)take(sizeof(int) * np);
+  L.hist = (int*)take(sizeof(int) * hist_ints(np));
+  L.ctr = (int*)take(kHead);
   L.hitl = (int*)take(sizeof(int) * np);
-  L.hist = (int*)take(sizeof(int) * hist_ints(k.np));
-  L.zrow = (double*)take(sizeof(double) * std::min<size_t>(np, kChunkMapGrid * ncu) * k.lq);
-  L.ctr = (int*)take(sizeof(int) * 64);  // (the hit records follow at 256 bytes)
-  L.hits = (cth_hit*)take(sizeof(cth_hit) * np);
-  L.alnout = k.rows ? (char*)take(np * 5 * (size_t)(k.lq + k.ltmax)) : nullptr;
-  L.nsplit = k.post ? cth_map_split(k.lq, k.ltmax, k.np) : 0;
-  L.back = (float*)take(cth_map_split_bytes(k.lq, k.ltmax, L.nsplit));
   L.bytes = o;
   return L;
 }
 
+// What the MAP stage and the hit records of n hits take, templates of up to
+// ltmax positions: nsplit and grid as cth_launch_map_batch takes them.
+struct hits_layout {
+  int* head; cth_hit* hits;  // (the records follow the counters' copy at kHead bytes)
+  double* zrow; float* back; char* alnout;
+  size_t bytes;
+};
+hits_layout hits_lay(int lq, int ltmax, int n, bool rows, int nsplit, int grid, void* base) {
+  hits_layout M;
+  size_t o = 0;
+  auto take = [&](size_t b) { void* p = (uint8_t*)base + o; o += up256(b); return p; };
+  M.head = (int*)take(kHead);
+  M.hits = (cth_hit*)take(sizeof(cth_hit) * n);
+  M.zrow = (double*)take(sizeof(double) * std::max(grid, nsplit) * (size_t)lq);
+  M.back = (float*)take(cth_map_split_bytes(lq, ltmax, nsplit));
+  M.alnout = rows ? (char*)take((size_t)n * 5 * (size_t)(lq + ltmax)) : nullptr;
+  M.bytes = o;
+  return M;
+}
+
 }  // namespace
 
-size_t cth_chunk_work_bytes(const cth_chunk& k, int ncu) { return chunk_lay(k, ncu, nullptr).bytes; }
-
 // The stages after a chunk's first DP pass, chosen and run on the device as
-// the batched search does: one synchronisation, where the host's choice of the
-// next stage's profiles took four with copies of all records between them
-// (0.2-0.45 ms of a search).
-int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt, int ncu, void* work, hipEvent_t* ev,
+// the batched search does, where the host's choice of the next stage's profiles
+// took four synchronisations with copies of all records between them (0.2-0.45
+// ms of a search).
+//
+// The MAP stage's memory is sized for the hits, whose number and lengths come
+// back first (kEarlyBytes: unless room for all profiles as hits is a few
+// megabytes; then MAP follows at once, which saves the ~15 us between).  Known
+// hits also need no grid for any number of them: of 4096 workgroups nearly all
+// left at once, after 20 us.
+int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt, int ncu, bool timing,
                      cth_chunk_hits& out) {
+  constexpr size_t kEarlyBytes = (size_t)8 << 20;
   hipStream_t st = c->st;
   const cth_dpset *q = &c->q.d, *db = &c->db.d;
-  const chunk_layout L = chunk_lay(k, ncu, work);
+  out.hits.clear();
+  out.rows.clear();
+  out.rowcap = 0;
+  out.npassed = 0;
+  out.ms_stats = out.ms_map = 0.0f;
+  if (cth_ctx_reserve(c, &c->work, &c->cap_work, chunk_lay(k.np, nullptr).bytes)) return -1;
+  const chunk_layout L = chunk_lay(k.np, c->work);
+  constexpr size_t kPinned = kHead + std::max(sizeof(cth_hit) * kFirstHits, sizeof(int) * kFirstList);
   if (!c->h_pin) {
-    const size_t n = 256 + sizeof(cth_hit) * kFirstHits;
-    CTH_HIP_CHECK(hipHostMalloc(&c->h_pin, n));
-    c->cap_pin = n;
+    CTH_HIP_CHECK(hipHostMalloc(&c->h_pin, kPinned));
+    c->cap_pin = kPinned;
   }
+  const int* const ctr = (const int*)c->h_pin;
   cth_bquery Q{};
   Q.qp = k.qi;
   Q.lq = k.lq;
@@ -400,39 +431,80 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
   hipLaunchKernelGGL(k_select_passed, dim3(sel), dim3(256), 0, st, k.res, k.traced ? nullptr : L.cand,
                      L.ctr + kCtrCand, k.np, L.passed, L.ctr + kCtrPassed);
   CTH_HIP_CHECK(hipGetLastError());
-  if (ev) CTH_HIP_CHECK(hipEventRecord(ev[0], st));
+  if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[2], st));
   if (cth_launch_stats_batch(q, db, L.bq, L.pairs, L.passed, L.ctr + kCtrPassed, k.ldsc, k.scores, k.res,
                              opt->ssemodel, k.lq, L.hist, std::min(k.np, kHistCap), L.stats, grid, st))
     return -1;
   hipLaunchKernelGGL(k_select_hits, dim3(sel), dim3(256), 0, st, L.bq, L.pairs, L.stats, L.passed,
                      L.ctr + kCtrPassed, L.hitl, L.ctr + kCtrHits);
   CTH_HIP_CHECK(hipGetLastError());
-  if (ev) CTH_HIP_CHECK(hipEventRecord(ev[1], st));
-  out.rowcap = k.lq + k.ltmax;
-  if (opt->do_map &&
-      cth_launch_map_batch(q, db, L.bq, L.pairs, L.hitl, L.ctr + kCtrHits, k.ltmax, k.lq, k.ldsc, k.scores, k.mods,
-                           k.post, k.btck, L.stats, L.zrow, opt->minpp > 0.0f ? opt->minpp : CTH_MINPP, L.alnout,
-                           out.rowcap, L.mres, std::min(kChunkMapGrid * ncu, k.np), W, L.nsplit, L.back, st))
+  if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[3], st));
+  // the posteriors, which mem_budget counts, while the device is at work (0.3 ms
+  // for 0.9 GB, on a context's first search)
+  if (opt->do_map && cth_ctx_reserve(c, (void**)&c->mapbuf, &c->cap_mapbuf,
+                                     sizeof(float) * ((size_t)k.lq * (size_t)k.ldsc + 2 * CTH_SCORE_PAD)))
     return -1;
-  hipLaunchKernelGGL(k_gather_hits, dim3(sel), dim3(256), 0, st, L.bq, L.pairs, k.res, L.stats, L.mres, opt->do_map,
-                     L.hitl, L.ctr + kCtrHits, L.hits);
+  // the MAP stage's shape for any number of hits
+  int nhit = k.np, ltmax = k.ltmax;
+  int nsplit = opt->do_map ? cth_map_split(k.lq, ltmax, nhit) : 0;
+  int mapgrid = opt->do_map ? std::min(kChunkMapGrid * ncu, nhit) : 0;
+  const bool early = hits_lay(k.lq, ltmax, nhit, k.rows, nsplit, mapgrid, nullptr).bytes <= kEarlyBytes;
+  if (!early) {
+    // or, where that takes much memory, for those there are
+    const int first = std::min(k.np, kFirstList);
+    CTH_HIP_CHECK(hipMemcpyAsync(c->h_pin, L.ctr, kHead + sizeof(int) * first, hipMemcpyDeviceToHost, st));
+    CTH_HIP_CHECK(hipStreamSynchronize(st));
+    if (timing) CTH_HIP_CHECK(hipEventElapsedTime(&out.ms_stats, c->ev[2], c->ev[3]));
+    nhit = ctr[kCtrHits];
+    out.npassed = ctr[kCtrPassed];
+    if (!nhit) return 0;
+    if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[3], st));
+    std::vector<int> list((size_t)nhit);
+    memcpy(list.data(), (const uint8_t*)c->h_pin + kHead, sizeof(int) * std::min(nhit, first));
+    if (nhit > first) {
+      CTH_HIP_CHECK(hipMemcpyAsync(list.data() + first, L.hitl + first, sizeof(int) * (nhit - first),
+                                   hipMemcpyDeviceToHost, st));
+      CTH_HIP_CHECK(hipStreamSynchronize(st));
+    }
+    ltmax = 0;
+    for (int i : list) ltmax = std::max(ltmax, c->db.h_len[k.p0 + i]);
+    if (opt->do_map) {
+      nsplit = cth_map_split(k.lq, ltmax, nhit) >= nhit ? nhit : 0;
+      mapgrid = nsplit ? 0 : std::min(kChunkMapGrid * ncu, nhit);
+    }
+  }
+  out.rowcap = k.lq + ltmax;
+  if (cth_ctx_reserve(c, &c->mapwork, &c->cap_mapwork,
+                      hits_lay(k.lq, ltmax, nhit, k.rows, nsplit, mapgrid, nullptr).bytes))
+    return -1;
+  const hits_layout M = hits_lay(k.lq, ltmax, nhit, k.rows, nsplit, mapgrid, c->mapwork);
+  if (opt->do_map &&
+      cth_launch_map_batch(q, db, L.bq, L.pairs, L.hitl, L.ctr + kCtrHits, ltmax, k.lq, k.ldsc, k.scores, k.mods,
+                           c->mapbuf + CTH_SCORE_PAD, k.btck, L.stats, M.zrow,
+                           opt->minpp > 0.0f ? opt->minpp : CTH_MINPP, M.alnout, out.rowcap, L.mres, mapgrid, W,
+                           nsplit, M.back, st))
+    return -1;
+  hipLaunchKernelGGL(k_gather_hits, dim3(std::max(1, std::min(1024, (nhit + 255) / 256))), dim3(256), 0, st, L.bq,
+                     L.pairs, k.res, L.stats, L.mres, opt->do_map, L.hitl, L.ctr + kCtrHits, M.hits, L.ctr, M.head);
   CTH_HIP_CHECK(hipGetLastError());
-  if (ev) CTH_HIP_CHECK(hipEventRecord(ev[2], st));
-  const int first = std::min(k.np, kFirstHits);
-  CTH_HIP_CHECK(hipMemcpyAsync(c->h_pin, L.ctr, 256 + sizeof(cth_hit) * first, hipMemcpyDeviceToHost, st));
+  if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[4], st));
+  const int first = std::min(nhit, kFirstHits);
+  CTH_HIP_CHECK(hipMemcpyAsync(c->h_pin, M.head, kHead + sizeof(cth_hit) * first, hipMemcpyDeviceToHost, st));
   CTH_HIP_CHECK(hipStreamSynchronize(st));
-  const int* const ctr = (const int*)c->h_pin;
+  if (timing) {
+    if (early) CTH_HIP_CHECK(hipEventElapsedTime(&out.ms_stats, c->ev[2], c->ev[3]));
+    CTH_HIP_CHECK(hipEventElapsedTime(&out.ms_map, c->ev[3], c->ev[4]));
+  }
   const int nb = ctr[kCtrHits];
   out.npassed = ctr[kCtrPassed];
   out.hits.resize(nb);
-  out.rows.clear();
-  if (nb) memcpy(out.hits.data(), (const uint8_t*)c->h_pin + 256, sizeof(cth_hit) * std::min(nb, first));
+  if (nb) memcpy(out.hits.data(), (const uint8_t*)c->h_pin + kHead, sizeof(cth_hit) * std::min(nb, first));
   if (nb > first)
-    CTH_HIP_CHECK(hipMemcpyAsync(out.hits.data() + first, L.hits + first, sizeof(cth_hit) * (nb - first),
+    CTH_HIP_CHECK(hipMemcpyAsync(out.hits.data() + first, M.hits + first, sizeof(cth_hit) * (nb - first),
                                  hipMemcpyDeviceToHost, st));
-  if (nb && L.alnout && opt->do_map) {
+  if (nb && M.alnout) {
     out.rows.resize((size_t)nb * 5 * out.rowcap);
-    CTH_HIP_CHECK(hipMemcpyAsync(out.rows.data(), L.alnout, out.rows.size(), hipMemcpyDeviceToHost, st));
+    CTH_HIP_CHECK(hipMemcpyAsync(out.rows.data(), M.alnout, out.rows.size(), hipMemcpyDeviceToHost, st));
   }
   if (nb > first || !out.rows.empty()) CTH_HIP_CHECK(hipStreamSynchronize(st));
   std::sort(out.hits.begin(), out.hits.end(), [](const cth_hit& a, const cth_hit& b) { return a.profile < b.profile; });

@@ -108,7 +108,8 @@ extern "C" int cth_ctx_create_shared(cth_ctx* parent, cth_ctx** out) {
 extern "C" void cth_ctx_trim(cth_ctx* c, size_t keep) {
   struct { void** p; size_t* cap; } bufs[] = {
       {(void**)&c->scores, &c->cap_scores}, {(void**)&c->mods, &c->cap_mods}, {(void**)&c->btck, &c->cap_btck},
-      {(void**)&c->mapbuf, &c->cap_mapbuf}, {&c->work, &c->cap_work}, {(void**)&c->grow, &c->cap_grow}};
+      {(void**)&c->mapbuf, &c->cap_mapbuf}, {&c->work, &c->cap_work}, {(void**)&c->grow, &c->cap_grow},
+      {&c->mapwork, &c->cap_mapwork}};
   for (auto& b : bufs)
     if (*b.p && *b.cap > keep) {
       (void)hipFree(*b.p);
@@ -127,7 +128,7 @@ extern "C" void cth_ctx_destroy(cth_ctx* c) {
     cth_devset_free(&c->db);
     if (c->dtab) (void)hipFree(c->dtab);
   }
-  void* bufs[] = {c->scores, c->mods, c->btck, c->dpout, c->work, c->mapbuf, c->grow};
+  void* bufs[] = {c->scores, c->mods, c->btck, c->dpout, c->work, c->mapbuf, c->grow, c->mapwork};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   if (c->h_pin) (void)hipHostFree(c->h_pin);

@@ -16,7 +16,7 @@ extern "C" void cth_query_thresholds(float eval, uint64_t lq, uint64_t dbsize, u
 
 // One query against the resident profiles [p0, p0+np), whose scores, modular
 // scores and first-pass records (res) are on their way on the context's stream.
-// Buffers as cth_launch_dp_list and cth_launch_map take them, column 0 at col0.
+// Buffers as cth_launch_dp_list takes them, column 0 at col0.
 struct cth_chunk {
   int qi, lq, p0, np, ltmax;
   int64_t col0, ldsc;
@@ -24,7 +24,6 @@ struct cth_chunk {
   double sspace;
   const float* scores;
   const float* mods;
-  float* post;
   uint8_t* btck;
   cth_dpres* res;
   int rows;    // alignment rows wanted
@@ -38,9 +37,10 @@ struct cth_chunk_hits {
   std::vector<char> rows;
   int rowcap;
   int npassed;
+  float ms_stats, ms_map;  // with stage timing
 };
-// bytes of the work area cth_chunk_finish takes, and the call itself; ev: with
-// stage timing, events recorded after phase 1, the statistics and MAP
-size_t cth_chunk_work_bytes(const cth_chunk& k, int ncu);
-int cth_chunk_finish(struct cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt, int ncu, void* work,
-                     hipEvent_t* ev, cth_chunk_hits& out);
+// The call itself.  The context's work area holds its lists and records (about
+// 250 bytes a profile), its mapbuf and mapwork the MAP stage's; timing: the
+// context's events 2 to 4 are recorded after phase 1, the statistics and MAP.
+int cth_chunk_finish(struct cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt, int ncu, bool timing,
+                     cth_chunk_hits& out);

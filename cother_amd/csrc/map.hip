@@ -1028,9 +1028,10 @@ extern "C" int cth_launch_map(const cth_dpset* q, int qp, int lq, const cth_dpse
 
 // The batched MAP stage (k_map_batch) on a persistent grid of `grid`
 // workgroups of W wavefronts over the *count pairs of list; ltmax: the
-// database's longest profile (boundary rows in LDS); zrow: max(grid, nsplit) x
-// lqmax doubles; nsplit: cth_map_split(lqmax, ltmax, pairs), back:
-// cth_map_split_bytes of them; buffers as in cth_launch_map.
+// longest profile (boundary rows in LDS); zrow: max(grid, nsplit) x lqmax
+// doubles; nsplit: how many pairs the kSplit form takes, at most
+// cth_map_split(lqmax, ltmax, pairs), back: cth_map_split_bytes of them; grid 0
+// where *count is known to be within nsplit; buffers as in cth_launch_map.
 extern "C" int cth_launch_map_batch(const cth_dpset* q, const cth_dpset* db, const cth_bquery* bq,
                                     const cth_bpair* pairs, const int* list, const int* count, int ltmax, int lqmax,
                                     int64_t ldsc, const float* scores, const float* mods, float* post, uint8_t* btck,
@@ -1039,7 +1040,6 @@ extern "C" int cth_launch_map_batch(const cth_dpset* q, const cth_dpset* db, con
   if (ltmax > CTH_LDS_ROW_MAX) { cth_set_error("map batch: profile length %d over the LDS row limit", ltmax); return -1; }
   if (ldsc % 4) { cth_set_error("map batch: rows of %lld traceback bytes", (long long)ldsc); return -1; }
   if (W < 1 || W > kMaxWaves) { cth_set_error("map batch: %d wavefronts per pair", W); return -1; }
-  if (grid < 1) return 0;
   const bool finite = cth_finite_scores(q, db);
   auto launch = [&](auto kernel, int n, int waves, size_t lds) {
     hipLaunchKernelGGL(kernel, dim3(n), dim3(64 * waves), lds, st, *q, *db, bq, pairs, list, count, ldsc, scores, mods,
@@ -1051,6 +1051,7 @@ extern "C" int cth_launch_map_batch(const cth_dpset* q, const cth_dpset* db, con
     else launch(k_map_batch<true, true>, nsplit, 2 * split_waves(lqmax), split_lds(lqmax, ltmax));
     CTH_HIP_CHECK(hipGetLastError());
   }
+  if (grid < 1) return 0;
   const size_t lds = W * map_wave_lds(false) + map_row_lds(ltmax, false);
   if (finite) launch(k_map_batch<false, false>, grid, W, lds);
   else launch(k_map_batch<true, false>, grid, W, lds);

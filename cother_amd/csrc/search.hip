@@ -378,7 +378,7 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
       // kRowsCap
       constexpr size_t kRowsCap = (size_t)256 << 20;
       const int np = p1 - p0;
-      cth_chunk k{qi, lq, p0, np, ltchunk, col0, ldsc, scorethld, logethld, sspace, scores, mods, nullptr, btck,
+      cth_chunk k{qi, lq, p0, np, ltchunk, col0, ldsc, scorethld, logethld, sspace, scores, mods, btck,
                   dpout, opt->alnbuf && opt->do_map ? 1 : 0, 0};
       const bool ondevice = !bufs.fixed && ltchunk <= CTH_DP_GLOBAL_FROM &&
                             (!k.rows || (size_t)np * 5 * (size_t)(lq + ltchunk) <= kRowsCap);
@@ -427,18 +427,16 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
         }
       }
       if (ondevice) {
-        if (opt->do_map && !(k.post = bufs.map_buffer(lq, ldsc))) return -1;
-        void* const work = bufs.work(cth_chunk_work_bytes(k, ncu));
-        if (!work) return -1;
         cth_chunk_hits got;
-        if (cth_chunk_finish(c, k, opt, ncu, work, timing ? c->ev + 2 : nullptr, got)) return -1;
+        if (cth_chunk_finish(c, k, opt, ncu, timing, got)) return -1;
         if (timing) {
-          float ms[4];
-          for (int e = 0; e < 4; e++) CTH_HIP_CHECK(hipEventElapsedTime(&ms[e], c->ev[e], c->ev[e + 1]));
-          st.ms_k_score += ms[0];
-          st.ms_k_dp += ms[1];
-          st.ms_k_stats += ms[2];
-          st.ms_k_map += ms[3];
+          float a = 0.0f, b = 0.0f;
+          CTH_HIP_CHECK(hipEventElapsedTime(&a, c->ev[0], c->ev[1]));
+          CTH_HIP_CHECK(hipEventElapsedTime(&b, c->ev[1], c->ev[2]));
+          st.ms_k_score += a;
+          st.ms_k_dp += b;
+          st.ms_k_stats += got.ms_stats;
+          st.ms_k_map += got.ms_map;
         }
         st.ms_phase1 += now_ms() - t0;
         st.cells += (double)lq * (double)ncols;
