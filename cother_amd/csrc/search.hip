@@ -373,15 +373,12 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
         return -1;
       if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[1], c->st));
       // the stages after the first DP pass on the device, unless the buffers are
-      // fixed, profiles need boundary rows in global memory (sized for the
-      // candidates), or the alignment rows of all profiles would be more than
-      // kRowsCap
-      constexpr size_t kRowsCap = (size_t)256 << 20;
+      // fixed or profiles need boundary rows in global memory (sized for the
+      // candidates)
       const int np = p1 - p0;
       cth_chunk k{qi, lq, p0, np, ltchunk, col0, ldsc, scorethld, logethld, sspace, scores, mods, btck,
                   dpout, opt->alnbuf && opt->do_map ? 1 : 0, 0};
-      const bool ondevice = !bufs.fixed && ltchunk <= CTH_DP_GLOBAL_FROM &&
-                            (!k.rows || (size_t)np * 5 * (size_t)(lq + ltchunk) <= kRowsCap);
+      const bool ondevice = !bufs.fixed && ltchunk <= CTH_DP_GLOBAL_FROM;
       // phase 1 in two passes: the DP of every profile without traceback,
       // then, for the profiles whose maximum exceeds the score threshold (the
       // only ones FinalizeDPPro traces back, cudp/CuBatchDP_final.cu:144),
