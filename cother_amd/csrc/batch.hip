@@ -69,6 +69,10 @@ extern "C" size_t cth_map_split_bytes(int lq, int ltmax, int n);
 namespace {
 
 enum { kCtrNext1 = 0, kCtrNext2, kCtrCand, kCtrPassed, kCtrHits, kNCtr = 8 };
+// the device's clock where statistics begin and where the host takes over, as
+// two 64-bit words behind a chunk's counters
+enum { kMarkStats = 0, kMarkBack, kNMark };
+static_assert(kNCtr % 2 == 0, "marks are aligned");
 
 __global__ void k_batch_reset(int* ctr) {
   if (threadIdx.x < kNCtr) ctr[threadIdx.x] = 0;
@@ -94,10 +98,11 @@ __global__ void k_select_cand(const cth_bquery* __restrict__ bq, const cth_bpair
 }
 
 // passed pairs of the traceback pass -> list; that pass took the *ncand pairs of
-// cand, or (null) all npairs
+// cand, or (null) all npairs.  mark: null, or where the clock goes
 __global__ void k_select_passed(const cth_dpres* __restrict__ res, const int* __restrict__ cand,
                                 const int* __restrict__ ncand, int npairs, int* __restrict__ list,
-                                int* __restrict__ count) {
+                                int* __restrict__ count, int64_t* __restrict__ mark) {
+  if (mark && blockIdx.x == 0 && threadIdx.x == 0) mark[kMarkStats] = wall_clock64();
   const int n = cand ? *ncand : npairs;
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
     const int i = cand ? cand[k] : k;
@@ -106,10 +111,12 @@ __global__ void k_select_passed(const cth_dpres* __restrict__ res, const int* __
 }
 
 // passed pairs within their query's E-value threshold -> list (the profiles
-// the MAP stage realigns, cumapdp/CuBatchMAPDP_fwd.cu:127-130)
+// the MAP stage realigns, cumapdp/CuBatchMAPDP_fwd.cu:127-130); mark as above
 __global__ void k_select_hits(const cth_bquery* __restrict__ bq, const cth_bpair* __restrict__ pairs,
                               const double* __restrict__ stats, const int* __restrict__ passed,
-                              const int* __restrict__ npassed, int* __restrict__ list, int* __restrict__ count) {
+                              const int* __restrict__ npassed, int* __restrict__ list, int* __restrict__ count,
+                              int64_t* __restrict__ mark) {
+  if (mark && blockIdx.x == 0 && threadIdx.x == 0) mark[kMarkBack] = wall_clock64();
   const int n = *npassed;
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
     const int i = passed[k];
@@ -120,13 +127,18 @@ __global__ void k_select_hits(const cth_bquery* __restrict__ bq, const cth_bpair
 
 // the hit records of the listed pairs, with the fields cth_search fills;
 // alnoff holds the pair's slot in the list (its rows' place in alnout).  head:
-// null, or where the counters go in front of the records
+// null, or where the counters and marks go in front of the records
 __global__ void k_gather_hits(const cth_bquery* __restrict__ bq, const cth_bpair* __restrict__ pairs,
                               const cth_dpres* __restrict__ res, const double* __restrict__ stats,
                               const cth_mapres* __restrict__ mres, int do_map, const int* __restrict__ list,
                               const int* __restrict__ count, cth_hit* __restrict__ hits,
                               const int* __restrict__ ctr, int* __restrict__ head) {
-  if (head && blockIdx.x == 0 && threadIdx.x < kNCtr) head[threadIdx.x] = ctr[threadIdx.x];
+  if (head && blockIdx.x == 0) {
+    int64_t* const mark = reinterpret_cast<int64_t*>(head + kNCtr);
+    if (threadIdx.x < kNCtr) head[threadIdx.x] = ctr[threadIdx.x];
+    if (threadIdx.x == kMarkStats) mark[kMarkStats] = reinterpret_cast<const int64_t*>(ctr + kNCtr)[kMarkStats];
+    if (threadIdx.x == kMarkBack) mark[kMarkBack] = wall_clock64();
+  }
   const int n = *count;
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
     const int i = list[k];
@@ -277,7 +289,7 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
                             S.trace_waves, st))
       return -1;
     hipLaunchKernelGGL(k_select_passed, dim3(sel_grid), dim3(256), 0, st, L.res, L.cand, L.ctr + kCtrCand, npairs,
-                       L.passed, L.ctr + kCtrPassed);
+                       L.passed, L.ctr + kCtrPassed, nullptr);
     CTH_HIP_CHECK(hipGetLastError());
     if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[2], st));
     if (cth_launch_stats_batch(&c->q.d, &db.d, L.bq, L.pairs, L.passed, L.ctr + kCtrPassed, ldsc, L.scores, L.res,
@@ -285,7 +297,7 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
                                std::min(S.small_grid, npairs), st))
       return -1;
     hipLaunchKernelGGL(k_select_hits, dim3(sel_grid), dim3(256), 0, st, L.bq, L.pairs, L.stats, L.passed,
-                       L.ctr + kCtrPassed, L.hitl, L.ctr + kCtrHits);
+                       L.ctr + kCtrPassed, L.hitl, L.ctr + kCtrHits, nullptr);
     CTH_HIP_CHECK(hipGetLastError());
     if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[3], st));
     if (opt->do_map &&
@@ -399,6 +411,9 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
   out.rowcap = 0;
   out.npassed = 0;
   out.ms_stats = out.ms_map = 0.0f;
+  out.ms_phase2 = 0.0;
+  int clock_khz = 0;
+  CTH_HIP_CHECK(hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, c->device));
   if (cth_ctx_reserve(c, &c->work, &c->cap_work, chunk_lay(k.np, nullptr).bytes)) return -1;
   const chunk_layout L = chunk_lay(k.np, c->work);
   constexpr size_t kPinned = kHead + std::max(sizeof(cth_hit) * kFirstHits, sizeof(int) * kFirstList);
@@ -407,6 +422,14 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
     c->cap_pin = kPinned;
   }
   const int* const ctr = (const int*)c->h_pin;
+  // The statistics begin where the host does not look: their time until it is
+  // back is the device clock's.
+  double back = 0.0;
+  auto host_back = [&] {
+    const int64_t* const mark = (const int64_t*)(ctr + kNCtr);
+    back = now_ms();
+    if (clock_khz > 0) back -= (double)(mark[kMarkBack] - mark[kMarkStats]) / clock_khz;
+  };
   cth_bquery Q{};
   Q.qp = k.qi;
   Q.lq = k.lq;
@@ -429,14 +452,14 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
       return -1;
   }
   hipLaunchKernelGGL(k_select_passed, dim3(sel), dim3(256), 0, st, k.res, k.traced ? nullptr : L.cand,
-                     L.ctr + kCtrCand, k.np, L.passed, L.ctr + kCtrPassed);
+                     L.ctr + kCtrCand, k.np, L.passed, L.ctr + kCtrPassed, (int64_t*)(L.ctr + kNCtr));
   CTH_HIP_CHECK(hipGetLastError());
   if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[2], st));
   if (cth_launch_stats_batch(q, db, L.bq, L.pairs, L.passed, L.ctr + kCtrPassed, k.ldsc, k.scores, k.res,
                              opt->ssemodel, k.lq, L.hist, std::min(k.np, kHistCap), L.stats, grid, st))
     return -1;
   hipLaunchKernelGGL(k_select_hits, dim3(sel), dim3(256), 0, st, L.bq, L.pairs, L.stats, L.passed,
-                     L.ctr + kCtrPassed, L.hitl, L.ctr + kCtrHits);
+                     L.ctr + kCtrPassed, L.hitl, L.ctr + kCtrHits, (int64_t*)(L.ctr + kNCtr));
   CTH_HIP_CHECK(hipGetLastError());
   if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[3], st));
   // the posteriors, which mem_budget counts, while the device is at work (0.3 ms
@@ -455,9 +478,13 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
     CTH_HIP_CHECK(hipMemcpyAsync(c->h_pin, L.ctr, kHead + sizeof(int) * first, hipMemcpyDeviceToHost, st));
     CTH_HIP_CHECK(hipStreamSynchronize(st));
     if (timing) CTH_HIP_CHECK(hipEventElapsedTime(&out.ms_stats, c->ev[2], c->ev[3]));
+    host_back();
     nhit = ctr[kCtrHits];
     out.npassed = ctr[kCtrPassed];
-    if (!nhit) return 0;
+    if (!nhit) {
+      out.ms_phase2 = now_ms() - back;
+      return 0;
+    }
     if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[3], st));
     std::vector<int> list((size_t)nhit);
     memcpy(list.data(), (const uint8_t*)c->h_pin + kHead, sizeof(int) * std::min(nhit, first));
@@ -495,6 +522,7 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
     if (early) CTH_HIP_CHECK(hipEventElapsedTime(&out.ms_stats, c->ev[2], c->ev[3]));
     CTH_HIP_CHECK(hipEventElapsedTime(&out.ms_map, c->ev[3], c->ev[4]));
   }
+  if (early) host_back();
   const int nb = ctr[kCtrHits];
   out.npassed = ctr[kCtrPassed];
   out.hits.resize(nb);
@@ -508,6 +536,7 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
   }
   if (nb > first || !out.rows.empty()) CTH_HIP_CHECK(hipStreamSynchronize(st));
   std::sort(out.hits.begin(), out.hits.end(), [](const cth_hit& a, const cth_hit& b) { return a.profile < b.profile; });
+  out.ms_phase2 = now_ms() - back;
   return 0;
 }
 

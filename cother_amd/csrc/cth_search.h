@@ -37,6 +37,7 @@ struct cth_chunk_hits {
   std::vector<char> rows;
   int rowcap;
   int npassed;
+  double ms_phase2;        // wall time from the end of phase 1 on
   float ms_stats, ms_map;  // with stage timing
 };
 // The call itself.  The context's work area holds its lists and records (about

@@ -435,7 +435,8 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
           st.ms_k_stats += got.ms_stats;
           st.ms_k_map += got.ms_map;
         }
-        st.ms_phase1 += now_ms() - t0;
+        st.ms_phase1 += now_ms() - t0 - got.ms_phase2;
+        st.ms_phase2 += got.ms_phase2;
         st.cells += (double)lq * (double)ncols;
         st.npassed += got.npassed;
         st.nchunks += 1;

@@ -228,8 +228,8 @@ typedef struct cth_hit {
 
 typedef struct cth_search_stats {
   double cells;       /* sum over queries of Lq x database positions */
-  double ms_phase1;   /* wall time of score + DP + finalisation */
-  double ms_phase2;   /* wall time of statistics (+ MAP) */
+  double ms_phase1;   /* wall time of score + DP + finalisation (of a batch: of all its stages) */
+  double ms_phase2;   /* wall time of statistics (+ MAP) (of a batch: 0) */
   double npassed;     /* profiles passed to phase 2 */
   double nchunks;     /* database chunks processed (score-kernel launches) */
   double ms_k_score;  /* with timing: HIP-event time of the score-matrix kernels */
