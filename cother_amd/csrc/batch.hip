@@ -236,10 +236,10 @@ struct batch_plan {
   int tile = 0;                     // rows of the score kernel's tiles
 };
 
-// Grids of the persistent launches (workgroups) and wavefronts per pair of
-// the two DP passes.
+// Grids of the persistent launches (workgroups), wavefronts per pair of the two
+// DP passes, and pairs that the MAP stage may take in its split form.
 struct launch_shape {
-  int dp_grid, dp_waves, small_grid, map_grid, trace_waves;
+  int dp_grid, dp_waves, trace_grid, small_grid, map_grid, trace_waves, map_split;
 };
 
 // One wavefront per pair where the pairs fill the chip (128,000 pairs of 99 x
@@ -249,14 +249,29 @@ struct launch_shape {
 // take the pairs that are left (8 per unit: 7.2 ms, 10: 6.9, 12: 6.9, 16:
 // 6.8).  Boundary rows in global memory are reserved per workgroup, so half
 // as many then.  The traceback pass has few pairs: one wavefront per stripe.
-launch_shape choose_shape(int ncu, int npairs, int lqmax, int ltmax) {
+//
+// The boundary rows and the split form's backward values are not among the
+// bytes that the budget counts: each takes an eighth of the batch's cell
+// buffers at most (or the rows of one workgroup per compute unit, and 8 MB).
+launch_shape choose_shape(int ncu, int npairs, int lqmax, int ltmax, size_t cellbytes, bool map) {
   launch_shape S;
   const int stripes = std::min(8, std::max(1, (lqmax + 63) / 64));
   S.dp_waves = npairs >= ncu * 8 ? 1 : stripes;
   S.trace_waves = stripes;
   S.dp_grid = ncu * (ltmax > CTH_DP_GLOBAL_FROM ? 8 : 16);
   S.small_grid = ncu * 4;
+  S.trace_grid = S.small_grid;
+  if (const size_t row = cth_dp_batch_row_bytes(1, ltmax)) {
+    const int fit = (int)std::max<size_t>(ncu, std::min<size_t>(S.dp_grid, cellbytes / 8 / row));
+    S.dp_grid = std::min(S.dp_grid, fit);
+    S.trace_grid = std::min(S.trace_grid, fit);
+  }
   S.map_grid = ncu * 16;  // (2000 pairs of 130 positions: 2.85 ms with four per unit, 2.1 with one per pair)
+  S.map_split = map ? cth_map_split(lqmax, ltmax, npairs) : 0;
+  if (S.map_split) {
+    const size_t each = cth_map_split_bytes(lqmax, ltmax, 1);
+    S.map_split = (int)std::min<size_t>(S.map_split, std::max((size_t)8 << 20, cellbytes / 8) / each);
+  }
   return S;
 }
 
@@ -285,7 +300,7 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
                        L.ctr + kCtrCand, L.hist, hist_ints(npairs));
     CTH_HIP_CHECK(hipGetLastError());
     if (cth_launch_dp_batch(&c->q.d, &db.d, L.bq, L.pairs, L.cand, L.ctr + kCtrCand, 0, L.ctr + kCtrNext2, ltmax,
-                            ldsc, L.scores, L.btck, L.res, L.grow, std::min(S.small_grid, npairs),
+                            ldsc, L.scores, L.btck, L.res, L.grow, std::min(S.trace_grid, npairs),
                             S.trace_waves, st))
       return -1;
     hipLaunchKernelGGL(k_select_passed, dim3(sel_grid), dim3(256), 0, st, L.res, L.cand, L.ctr + kCtrCand, npairs,
@@ -303,8 +318,8 @@ int capture_or_launch(cth_ctx* c, const batch_plan& P, const batch_layout& L, co
     if (opt->do_map &&
         cth_launch_map_batch(&c->q.d, &db.d, L.bq, L.pairs, L.hitl, L.ctr + kCtrHits, ltmax, P.lqmax, ldsc, L.scores,
                              L.mods, L.post, L.btck, L.stats, L.zrow, opt->minpp > 0.0f ? opt->minpp : CTH_MINPP,
-                             L.alnout, rowcap, L.mres, std::min(S.map_grid, npairs), S.trace_waves,
-                             cth_map_split(P.lqmax, ltmax, npairs), L.back, st))
+                             L.alnout, rowcap, L.mres, std::min(S.map_grid, npairs), S.trace_waves, S.map_split,
+                             L.back, st))
       return -1;
     hipLaunchKernelGGL(k_gather_hits, dim3(sel_grid), dim3(256), 0, st, L.bq, L.pairs, L.res, L.stats, L.mres,
                        opt->do_map, L.hitl, L.ctr + kCtrHits, L.hits, nullptr, nullptr);
@@ -701,10 +716,9 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
     const size_t cells = (size_t)P.cells;
     const cell_layout cell = lay_cells(cells, opt->do_map != 0);
     const int small_max = std::max(1, std::min(npairs, ncu * 32));
-    const size_t backbytes =
-        opt->do_map ? cth_map_split_bytes(P.lqmax, ltmax, cth_map_split(P.lqmax, ltmax, npairs)) : 0;
-    const launch_shape S = choose_shape(ncu, npairs, P.lqmax, ltmax);
-    const size_t growbytes = cth_dp_batch_row_bytes(std::min(npairs, std::max(S.dp_grid, S.small_grid)), ltmax);
+    const launch_shape S = choose_shape(ncu, npairs, P.lqmax, ltmax, cell.bytes, opt->do_map != 0);
+    const size_t backbytes = cth_map_split_bytes(P.lqmax, ltmax, S.map_split);
+    const size_t growbytes = cth_dp_batch_row_bytes(std::min(npairs, std::max(S.dp_grid, S.trace_grid)), ltmax);
     const size_t sbytes = up256(sizeof(cth_bquery) * P.bq.size()) + up256(sizeof(cth_bytile) * P.ytab.size()) +
                           up256(sizeof(cth_bpair) * npairs) + up256(sizeof(cth_dpres) * npairs) +
                           up256(sizeof(double) * CTH_STATS_NOUT * npairs) + up256(sizeof(cth_mapres) * npairs) +
@@ -749,10 +763,11 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
     // (buffers and their layout, sizes, options, the uploaded sets)
     uint32_t mp;
     memcpy(&mp, &opt->minpp, sizeof mp);
-    uint64_t key[14] = {(uint64_t)(uintptr_t)c->bcells, (uint64_t)(uintptr_t)c->bsmall, (uint64_t)npairs,
+    uint64_t key[15] = {(uint64_t)(uintptr_t)c->bcells, (uint64_t)(uintptr_t)c->bsmall, (uint64_t)npairs,
                         (uint64_t)P.ytab.size() | ((uint64_t)P.bq.size() << 32), (uint64_t)P.tile,
                         (uint64_t)P.cells, (uint64_t)P.lqmax | ((uint64_t)rowcap << 32),
                         (uint64_t)S.dp_grid | ((uint64_t)S.small_grid << 32),
+                        (uint64_t)S.trace_grid | ((uint64_t)S.map_split << 32),
                         (uint64_t)opt->do_map | ((uint64_t)opt->ssemodel << 8) | ((uint64_t)(alnbytes != 0) << 17) |
                             ((uint64_t)P.ddms << 18) | ((uint64_t)S.dp_waves << 20) |
                             ((uint64_t)S.trace_waves << 24) | ((uint64_t)mp << 32),

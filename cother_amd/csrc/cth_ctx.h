@@ -37,7 +37,7 @@ struct cth_ctx {
   // captured graph of the last batch shape
   void* bcells; size_t cap_bcells;
   void* bsmall; size_t cap_bsmall;
-  hipGraphExec_t bgraph; int has_bgraph; uint64_t bkey[14];
+  hipGraphExec_t bgraph; int has_bgraph; uint64_t bkey[15];
   int64_t nbgraph_captures, nbgraph_replays;
   // a context made by cth_ctx_create_shared reads its parent's tables,
   // queries and database and frees only its own stream and scratch

@@ -28,7 +28,8 @@
 //    synchronizes the device, which would stall the other slots), except
 //    that scratch beyond both its share of the budget (mem_budget / nslots)
 //    and its next request's footprint is returned first, so the slots hold
-//    at most about max(mem_budget, one footprint per slot).
+//    at most about max(mem_budget, one footprint per slot), and beside it the
+//    records and working memory that cth_search_opts.mem_budget names.
 //
 // Results are those of cth_search for the same query: requests do not
 // share buffers, and every kernel's output depends only on its own inputs.
