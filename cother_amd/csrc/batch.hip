@@ -8,7 +8,7 @@
 // does for a chunk of the database, cth_chunk_finish below):
 //   1. scores of every query of the batch (one launch, row tiles of all
 //      queries);
-//   2. phase-1 DP of every pair without traceback (persistent wavefronts
+//   2. phase-1 DP of every pair without traceback (persistent workgroups
 //      taking pairs, longest first, from a device counter);
 //   3. pairs over their query's score threshold -> list (device compaction);
 //   4. DP with traceback and finalisation of the listed pairs (persistent);
@@ -26,9 +26,9 @@
 // lists' order varies, the hit order is restored by the (log E-value,
 // profile) sort.
 //
-// Covered: the FP32 contraction and databases whose profiles fit the LDS
-// boundary rows (CTH_DP_LDS_ROW_MAX positions); other searches, and queries
-// whose buffers alone exceed the budget, run through cth_search.
+// Covered: the FP32 contraction and databases of profiles of up to
+// CTH_BATCH_LEN_MAX positions; other searches, and queries whose buffers alone
+// exceed the budget, run through cth_search.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -567,9 +567,9 @@ int search_batch_list(cth_ctx* c, const int* ql, int nq, const cth_search_opts* 
   const int64_t npos = db.d.npos;
   const int ltmax = nprof ? *std::max_element(db.h_len, db.h_len + nprof) : 0;
   cth_search_stats st{};
-  // the batched form covers the FP32 contraction and profiles within the LDS
-  // row limit; otherwise the queries run through cth_search
-  if (opt->contraction != 0 || ltmax > CTH_DP_LDS_ROW_MAX || nprof == 0) {
+  // the batched form covers the FP32 contraction and profiles within its
+  // limit; otherwise the queries run through cth_search
+  if (opt->contraction != 0 || ltmax > CTH_BATCH_LEN_MAX || nprof == 0) {
     int nh = 0;
     uint64_t used = 0;
     for (int k = 0; k < nq; k++) {

@@ -303,7 +303,7 @@ extern "C" int cth_phase1_block(cth_ctx* c, int qidx, int p0, int p1, float scor
   if (cth_launch_score(&c->q.d, c->q.ddoff, c->q.qrec, qidx, &c->db.d, col0, (int)ncols, ldsc, c->dtab, lq, c->scores + CTH_SCORE_PAD, c->mods, 0,
                        ddms_of(c, qidx, p0, p1), c->st))
     return -1;
-  // boundary rows in global memory for profiles over the LDS row limit
+  // boundary rows in global memory for profiles over CTH_DP_GLOBAL_FROM
   const size_t rows = cth_dp_row_bytes(p1 - p0, ltmax);
   if (rows && cth_ctx_reserve(c, (void**)&c->grow, &c->cap_grow, rows)) return -1;
   if (cth_launch_dp(&c->q.d, qidx, lq, &c->db.d, p0, p1 - p0, (int)(ncols / (p1 - p0)), ltmax, col0, ldsc, c->scores + CTH_SCORE_PAD, c->btck, scorethld,

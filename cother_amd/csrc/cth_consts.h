@@ -19,8 +19,9 @@
 // workgroup's 160 KiB of LDS beside the transition rings of eight wavefronts;
 // longer ones keep them in global memory
 #define CTH_LDS_ROW_MAX 6000
-// longest profile of a database that the batched search covers
-#define CTH_DP_LDS_ROW_MAX 5824
+// longest profile of a database that the batched search covers (its MAP
+// kernel keeps its boundary rows in LDS; longer ones run query by query)
+#define CTH_BATCH_LEN_MAX 5824
 // the phase-1 DP keeps its boundary rows and the reference's buffer of maxima
 // (28 bytes per column) in global memory from this profile length on: the
 // LDS holds them beside the transition rings of eight wavefronts up to here

@@ -28,7 +28,7 @@ struct cth_ctx {
   void* work; size_t cap_work;
   float* mapbuf; size_t cap_mapbuf;  // MAP posteriors [Lq][ldsc]
   void* mapwork; size_t cap_mapwork; // hit records, rows and scratch of a search's MAP stage (cth_chunk_finish)
-  float* grow; size_t cap_grow;      // DP/MAP stripe boundary rows of profiles over the LDS row limit
+  float* grow; size_t cap_grow;      // DP/MAP stripe boundary rows of profiles too long for LDS
   void* h_pin; size_t cap_pin;
   // stage events of cth_search's timing mode (created on first use; the
   // batched search uses a fifth)

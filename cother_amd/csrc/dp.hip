@@ -537,8 +537,8 @@ __global__ __launch_bounds__(64) void k_dpfin(cth_dpset db, int pbase, const int
   if (threadIdx.x == 0) res[blockIdx.x] = r;
 }
 
-// Batched finalisation over the *count pairs listed in list (persistent,
-// lane 0 of each wavefront), each against its query's threshold.
+// Batched finalisation over the *count pairs listed in list (persistent, a
+// wavefront per pair at a time), each against its query's threshold.
 __global__ __launch_bounds__(64) void k_dpfin_batch(cth_dpset db, const cth_bquery* __restrict__ bq,
                                                     const cth_bpair* __restrict__ pairs, const int* __restrict__ list,
                                                     const int* __restrict__ count, int64_t ldsc,

@@ -465,7 +465,7 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
         st.ms_k_score += a;
         st.ms_k_dp += b;
       }
-      // candidates for the traceback pass: profiles within the LDS row limit
+      // candidates for the traceback pass: profiles within CTH_DP_GLOBAL_FROM
       // first, then the longer ones (global boundary rows, in batches)
       std::vector<int> cand, cand_abs, cand_long;
       int ltc = 0, ltl = 0;
@@ -555,7 +555,7 @@ int search_run(cth_ctx* c, int q0, int q1, const cth_search_opts* opt, cth_hit* 
       // MAP stage for the passed profiles within the E-value threshold (the
       // reference's MAP kernels return early for the others,
       // cumapdp/CuBatchMAPDP_fwd.cu:127-130)
-      // (jobs within the LDS row limit first, then the longer ones)
+      // (jobs within CTH_LDS_ROW_MAX first, then the longer ones)
       std::vector<int> sel, sel_long;
       for (int j = 0; j < np2; j++)
         if (!(logethld < (float)sv[(size_t)j * CTH_STATS_NOUT + CTH_ST_LOGE]))

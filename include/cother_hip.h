@@ -196,8 +196,9 @@ typedef struct cth_search_opts {
   int do_map;         /* realign passed hits by MAP (MAPALN, default 1) */
   int timing;         /* record HIP events around each stage on the context's stream */
   uint64_t mem_budget;/* bytes for the per-chunk score/traceback/posterior buffers (0: 64 GiB).  Beside them
-                         come records of about 250 bytes a (query, profile) pair, what the hits there are
-                         need (rows, MAP scratch) and, in a batch, up to a quarter of them */
+                         come records of about 250 bytes a (query, profile) pair and what the hits there are
+                         need (rows, MAP scratch); in a batch the rows of every pair (with alnbuf) and up
+                         to a quarter of the buffers again */
   float minpp;        /* MAP posterior threshold (MINPP; 0: the default 0.28) */
   int contraction;    /* log-odds term: 0 FP32 as the reference (default); 1 BF16, 2 FP16 operands on
                          the matrix cores with FP32 accumulation (no reference counterpart) */
