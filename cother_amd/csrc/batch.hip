@@ -500,7 +500,6 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
       out.ms_phase2 = now_ms() - back;
       return 0;
     }
-    if (timing) CTH_HIP_CHECK(hipEventRecord(c->ev[3], st));
     std::vector<int> list((size_t)nhit);
     memcpy(list.data(), (const uint8_t*)c->h_pin + kHead, sizeof(int) * std::min(nhit, first));
     if (nhit > first) {
@@ -520,6 +519,7 @@ int cth_chunk_finish(cth_ctx* c, const cth_chunk& k, const cth_search_opts* opt,
                       hits_lay(k.lq, ltmax, nhit, k.rows, nsplit, mapgrid, nullptr).bytes))
     return -1;
   const hits_layout M = hits_lay(k.lq, ltmax, nhit, k.rows, nsplit, mapgrid, c->mapwork);
+  if (timing && !early) CTH_HIP_CHECK(hipEventRecord(c->ev[3], st));
   if (opt->do_map &&
       cth_launch_map_batch(q, db, L.bq, L.pairs, L.hitl, L.ctr + kCtrHits, ltmax, k.lq, k.ldsc, k.scores, k.mods,
                            c->mapbuf + CTH_SCORE_PAD, k.btck, L.stats, M.zrow,
