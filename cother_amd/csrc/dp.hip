@@ -9,8 +9,11 @@
 // on wavefronts of one workgroup.  Cell values and the maximum with its cell
 // equal the reference's (dp_pair below).
 //
-// Bound by VALU issue (dp_pair: ~40 instructions per step in ~26 issue
-// slots).  Measured against one wavefront per pair with the boundary tests
+// Bound by VALU issue together with the LDS of its rows: 43 VALU instructions per
+// step (56 with traceback) in 37 (52) issue slots, which fill 73% of the cycles of a
+// first pass of 128,000 pairs at 2.3 wavefronts a SIMD, 56% of one of 6000 pairs and
+// 40% of a traceback pass of 1500, whose ends have few pairs in flight (counters in
+// profiles/k_dp_pmc.txt).  Measured against one wavefront per pair with the boundary tests
 // and the transitions' lane-to-lane moves in every step (~190 VALU): first
 // pass of 128,000 pairs of 99 x 231 positions 16.6 -> 5.7 ms; a query of 2000
 // positions against 130 templates of 1000-3000, whose rows were in global

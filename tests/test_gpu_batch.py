@@ -1,11 +1,10 @@
 """cth_search_batch (many queries per launch, device-side selection of each
-stage's pairs, graph capture and replay, autotuned persistent grids)
+stage's pairs, graph capture and replay, persistent grids)
 against cth_search: every hit field, the hit order and the alignment rows
 identical; also against the oracle directly, across several batches of one
 call, without MAP, for each significance model, for templates without
 distance lists, over graph replays with other searches in between, and for
-databases the batched form hands to cth_search (a profile over the LDS row
-limit)."""
+databases the batched form hands to cth_search (a profile over its limit)."""
 import numpy as np
 import pytest
 

@@ -1,7 +1,9 @@
-"""The plain score kernel (no cell with a distance term): the logarithm it
-uses, ragged tiles, rows and columns outside the quotient correction's ranges
-(it divides there), and the reduced-precision contraction's route through it
-against the route through the general kernel."""
+"""The plain score kernel (every term but the distance one): the logarithm it
+uses, ragged tiles, rows and columns outside the quotient correction's ranges,
+and the reduced-precision contraction over databases with and without distance
+lists, which take the same kernel (test_gpu_product_host.py holds the product
+against one formed on the host, test_gpu_score_quotient.py rows that have to be
+divided in ragged blocks)."""
 import ctypes
 
 import numpy as np
