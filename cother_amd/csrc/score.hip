@@ -930,7 +930,10 @@ extern "C" int cth_launch_score_batch(const cth_dpset* q, const int32_t* qoff, c
   if (!qoff || !qrec) { cth_set_error("score batch: query distance offsets or records not built"); return -1; }
   if (ldsc < ncols) { cth_set_error("score batch: ldsc %lld < ncols %d", (long long)ldsc, ncols); return -1; }
   const int ysplit = ddms ? tile / kDRows : 1;
-  if (ddms && tile % kDRows) { cth_set_error("score batch: row tiles of %d", tile); return -1; }
+  if (tile < 1 || tile > kPlainRowsMax || (ddms && tile % kDRows)) {
+    cth_set_error("score batch: row tiles of %d", tile);
+    return -1;
+  }
   if ((int64_t)nytiles * ysplit > 65535) { cth_set_error("score batch: %d row tiles", nytiles); return -1; }
   hipLaunchKernelGGL((k_score_plain<0, true>), dim3((ncols + kCols - 1) / kCols, nytiles), dim3(256), 0, st, *q,
                      reinterpret_cast<const query_record*>(qrec), 0, *db, (int64_t)0, ncols, ldsc, dtabs, scores,
